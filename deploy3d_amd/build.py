@@ -20,7 +20,7 @@ OBJ = os.path.join(LIBS, "obj")
 ENGINE_LIB = os.path.join(LIBS, "libdeploy3d_amd.so")
 SYNTH_LIB = os.path.join(LIBS, "libd3d_synth.so")
 
-ENGINE_SOURCES = ["rulebook.hip", "conv.hip", "conv_half.hip", "conv_bf16.hip", "conv_int8.hip", "conv_pipe_half.hip",
+ENGINE_SOURCES = ["rulebook.hip", "conv.hip", "conv_half.hip", "conv_bf16.hip", "conv_int8.hip", "conv_f32.hip", "conv_pipe_half.hip",
                   "conv_pipe_bf16.hip", "conv_pipe_int8.hip", "densify.hip", "voxelize.hip", "scratch.hip", "plugin.cpp", "schedule.cpp"]
 ENGINE_HEADERS = ["common.h", "conv_kernels.h", "conv_pipe.h", os.path.join(ROOT, "include", "d3d_spconv.h")]
 # per-source extra flags
@@ -28,6 +28,7 @@ EXTRA_FLAGS = {
     # keeps the MFMA accumulators of the pipelined kernel in VGPRs (see the header of the two files)
     "conv_pipe_half.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "conv_pipe_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "conv_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "conv_pipe_int8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 PEAKS_BIN = os.path.join(LIBS, "d3d_peaks")

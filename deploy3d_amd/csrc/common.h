@@ -187,6 +187,8 @@ int32_t launchMfmaInt8(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeHalf(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeBf16(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeInt8(const ConvArgs& a, hipStream_t stream);
+// Both kernels for fp32 storage (conv_f32.hip).
+int32_t launchMfmaFloat(const ConvArgs& a, hipStream_t stream);
 
 // True if the MFMA kernel family covers (dtype, cin, cout); otherwise the
 // narrow-channel kernel runs.

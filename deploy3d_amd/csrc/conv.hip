@@ -294,12 +294,12 @@ padRows(const uint8_t* __restrict__ in, int64_t rows, int inBytes, int outBytes,
 
 bool convUsesMfma(int32_t dtype, int cin, int cout) {
   if (dtype == D3D_INT8) return (cin == 32 || cin == 64 || cin == 128) && isMfmaChannels(cout);
-  return (dtype == D3D_HALF || dtype == D3D_BF16) && isMfmaChannels(cin) && isMfmaChannels(cout);
+  return (dtype == D3D_HALF || dtype == D3D_BF16 || dtype == D3D_FLOAT) && isMfmaChannels(cin) && isMfmaChannels(cout);
 }
 
 int paddedMfmaChannels(int32_t dtype, int cin, int cout) {
   if (!isMfmaChannels(cout) || cin < 1 || cin > 128) return cin;
-  if (dtype == D3D_HALF || dtype == D3D_BF16) {
+  if (dtype == D3D_HALF || dtype == D3D_BF16 || dtype == D3D_FLOAT) {
     int c = 16;
     while (c < cin) c *= 2;
     return c;
@@ -357,15 +357,17 @@ int32_t launchConv(const ConvArgs& a, hipStream_t stream) {
   } else if (convUsesMfma(a.dtype, a.cin, a.cout) && aligned && a.weightsMfma && a.zeros) {
     rc = D3D_ERR_UNSUPPORTED;
     if (a.pipe >= 0 && a.staged == 0 && a.tileRows == 0)
-      rc = a.dtype == D3D_HALF ? launchPipeHalf(a, stream) : launchPipeBf16(a, stream);
-    if (rc == D3D_ERR_UNSUPPORTED) rc = a.dtype == D3D_HALF ? launchMfmaHalf(a, stream) : launchMfmaBf16(a, stream);
+      rc = a.dtype == D3D_FLOAT ? launchMfmaFloat(a, stream)
+                                : (a.dtype == D3D_HALF ? launchPipeHalf(a, stream) : launchPipeBf16(a, stream));
+    if (rc == D3D_ERR_UNSUPPORTED && a.dtype != D3D_FLOAT) rc = a.dtype == D3D_HALF ? launchMfmaHalf(a, stream) : launchMfmaBf16(a, stream);
     if (rc == D3D_ERR_UNSUPPORTED && a.weightsF32 && a.inNarrow) {
       // no MFMA instantiation fits (a kernel volume whose index rows exceed LDS, 7x7x7 at 128 channels say): the
       // narrow kernel takes any kernel volume (the reference accepts any, trt/spconv/mm.h:35-71)
       ConvArgs b = a;
       b.in = a.inNarrow;
       b.cin = a.cinNarrow;
-      rc = a.dtype == D3D_HALF ? launchNarrow<_Float16>(b, stream) : launchNarrow<__bf16>(b, stream);
+      rc = a.dtype == D3D_FLOAT ? launchNarrow<float>(b, stream)
+                                : (a.dtype == D3D_HALF ? launchNarrow<_Float16>(b, stream) : launchNarrow<__bf16>(b, stream));
     }
   } else {
     const char* rowsEnv = debugEnv("D3D_CONV_NARROW_ROWS");  // =0: keep the tile kernel (tests)

@@ -13,6 +13,7 @@ bool convReadsNarrowRows(int32_t dtype, int kVol, int cin, int cout) {
   // two-byte types: rows below 16 channels read element by element (16.3 us against 17.6 with the widening pass
   // on that layer, and no widened copy to keep)
   if (dtype == D3D_HALF || dtype == D3D_BF16) return cin < 16 && convk::residentFits(kVol, 16, cout, 2);
+  if (dtype == D3D_FLOAT) return cin < 16 && convk::residentFits(kVol, 16, cout, 4);
   return false;
 }
 

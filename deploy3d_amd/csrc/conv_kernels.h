@@ -67,6 +67,20 @@ template <> struct Mfma<__bf16> {
   }
 };
 
+// fp32: a lane's 16 bytes are four channels; v_mfma_f32_16x16x4 contracts one channel of each of the four lane groups,
+// so four of them contract the 16 channels (64 bytes of a row) that the two-byte types contract in one.  Channel
+// 4 * (lane / 16) + j meets its weight in step j: the fragment order of the packed weights is the same formula.
+template <> struct Mfma<float> {
+  using Acc = float4v;
+  __device__ static float4v k32(const u32x4& a, const u32x4& b, const float4v& c) {
+    const float4v x = __builtin_bit_cast(float4v, a), y = __builtin_bit_cast(float4v, b);
+    float4v r = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], y[0], c, 0, 0, 0);
+    r = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], y[1], r, 0, 0, 0);
+    r = __builtin_amdgcn_mfma_f32_16x16x4f32(x[2], y[2], r, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x[3], y[3], r, 0, 0, 0);
+  }
+};
+
 // int8 operands, int32 accumulators: 16x16x64 takes 16 bytes per lane, 16x16x32 takes 8.
 template <> struct Mfma<int8_t> {
   using Acc = int4v;
@@ -328,7 +342,7 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
   constexpr int THREADS = 64 * WAVES;
   constexpr int MT = 1;
   constexpr int NT = COUT / 16;
-  constexpr int ES = static_cast<int>(sizeof(T));              // 2: fp16 / bf16, 1: int8
+  constexpr int ES = static_cast<int>(sizeof(T));              // 4: fp32, 2: fp16 / bf16, 1: int8
   constexpr bool WIDE = CIN * ES >= 64;                        // 16-byte operand fragments (else 8-byte)
   constexpr int KSTEP = (WIDE ? 64 : 32) / ES;                 // channels one MFMA contracts
   constexpr int KK = CIN / KSTEP;
@@ -337,7 +351,7 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
   constexpr int WCHUNKS = CIN * COUT * ES / 16;
   using F = typename std::conditional<WIDE, u32x4, u32x2>::type;
   using Acc = typename Mfma<T>::Acc;
-  static_assert(CIN % KSTEP == 0 && (CROW == CIN || (KK == 1 && !WIDE && (CROW < 0 || CROW % KG == 0))), "whole MFMA steps");
+  static_assert(CIN % KSTEP == 0 && (CROW == CIN || (KK == 1 && (!WIDE || ES == 4) && (CROW < 0 || CROW % KG == 0))), "whole MFMA steps");
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   F* wLds = reinterpret_cast<F*>(smem);                                              // [kVol][WFRAGS]
@@ -476,8 +490,12 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
             v[j] = acc[n][j] + (bias ? bias[col + j] : 0.f);
             if (relu) v[j] = v[j] > 0.f ? v[j] : 0.f;
           }
-          T packed[4] = {static_cast<T>(v[0]), static_cast<T>(v[1]), static_cast<T>(v[2]), static_cast<T>(v[3])};
-          *reinterpret_cast<u32x2*>(out + static_cast<size_t>(row) * COUT + col) = __builtin_bit_cast(u32x2, packed);
+          if constexpr (ES == 4) {
+            *reinterpret_cast<float4v*>(out + static_cast<size_t>(row) * COUT + col) = float4v{v[0], v[1], v[2], v[3]};
+          } else {
+            T packed[4] = {static_cast<T>(v[0]), static_cast<T>(v[1]), static_cast<T>(v[2]), static_cast<T>(v[3])};
+            *reinterpret_cast<u32x2*>(out + static_cast<size_t>(row) * COUT + col) = __builtin_bit_cast(u32x2, packed);
+          }
         }
       }
     }
@@ -1106,6 +1124,21 @@ int32_t launchMfma(const ConvArgs& a, hipStream_t stream) {
     case 64: return launchMfmaCout<T, 64>(a, stream);
     case 128: return launchMfmaCout<T, 128>(a, stream);
   }
+  return D3D_ERR_UNSUPPORTED;
+}
+
+// fp32 layers of at most 16 -> 32 or 32 -> 16 channels: weights resident, rows below 16 channels read as stored.
+template <class T = float>
+int32_t launchFloatResident(const ConvArgs& a, hipStream_t stream) {
+  if (!residentFits(a.kVol, a.cin, a.cout, sizeof(T))) return D3D_ERR_UNSUPPORTED;
+  if (a.rowChannels > 0) {
+    if (a.cin == 16 && a.cout == 16) return launchMfmaResident<T, 16, 16, -1>(a, stream);
+    if (a.cin == 16 && a.cout == 32) return launchMfmaResident<T, 16, 32, -1>(a, stream);
+    return D3D_ERR_UNSUPPORTED;
+  }
+  if (a.cin == 16 && a.cout == 16) return launchMfmaResident<T, 16, 16>(a, stream);
+  if (a.cin == 16 && a.cout == 32) return launchMfmaResident<T, 16, 32>(a, stream);
+  if (a.cin == 32 && a.cout == 16) return launchMfmaResident<T, 32, 16>(a, stream);
   return D3D_ERR_UNSUPPORTED;
 }
 

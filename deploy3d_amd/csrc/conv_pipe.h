@@ -1,5 +1,5 @@
 // Software-pipelined MFMA convolution for gfx950 (fp16 / bf16 storage with fp32 accumulation; int8 storage with
-// int32 accumulation and a requantizing store, for rows of 64 or 128 bytes).
+// int32 accumulation and a requantizing store, for rows of 64 or 128 bytes; fp32).
 //
 // Same mathematics and data layouts as convStaged (conv_kernels.h): output-stationary tiles, rows of a tap
 // gathered through the neighbour table into an XOR-swizzled LDS stage, weights in fragment-major order streamed
@@ -63,8 +63,8 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   constexpr int IL = (WM + 63) / 64;                           // index loads per step
   constexpr int SLOTS = WM * CH;                               // 16-byte slots of one stage
   constexpr int PER = TM / 64;                                 // tile masks per workgroup tile
-  constexpr int ROWSHIFT = CIN * ES == 64 ? 6 : (CIN * ES == 128 ? 7 : 8);
-  static_assert((ES == 2 || ES == 1) && (CS * ES == 64 || CS * ES == 128) && CIN % CS == 0 && WM % RPI == 0 && TM % 64 == 0, "shape");
+  constexpr int ROWSHIFT = CIN * ES == 64 ? 6 : (CIN * ES == 128 ? 7 : (CIN * ES == 256 ? 8 : 9));
+  static_assert((ES == 4 || ES == 2 || ES == 1) && (CS * ES == 64 || CS * ES == 128) && CIN % CS == 0 && WM % RPI == 0 && TM % 64 == 0, "shape");
   static_assert((1 << ROWSHIFT) == CIN * ES && WCH % 64 == 0 && MT >= 2 && MT * NT * 4 <= 128, "shape");
   static_assert(WM < 64 || WM % 64 == 0, "an index load covers 64 rows: a wavefront tile is below 64 rows or whole multiples");
   using F = u32x4;
@@ -212,9 +212,29 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   // MFMAs a lane holds, per channel tile n, 4 consecutive channels (8 bytes) of one row; two 16-lane row swaps
   // per pair of channel tiles hand every lane 8 consecutive channels instead, so a store instruction writes
   // 16 bytes per lane and 64 contiguous bytes per row.
-  static_assert(NT % 2 == 0, "channel tiles are stored in pairs");
+  // (fp32: 4 consecutive channels are those 16 bytes already.)
+  static_assert(NT % 2 == 0 || ES == 4, "channel tiles are stored in pairs");
   auto storeTile = [&](int pos) __attribute__((always_inline)) {
     const int64_t row0 = static_cast<int64_t>(tileAt(pos)) * TM + wave * WM;
+    if constexpr (ES == 4) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const int col = n * 16 + kgrp * 4;
+        const float4v b = bias ? *reinterpret_cast<const float4v*>(bias + col) : float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float4v v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            v[j] = acc[m][n][j] + b[j];
+            if (relu) v[j] = v[j] > 0.f ? v[j] : 0.f;
+          }
+          acc[m][n] = Acc{0, 0, 0, 0};
+          const int64_t row = row0 + m * 16 + r16;
+          if (row < outRows) *reinterpret_cast<float4v*>(out + static_cast<size_t>(row) * COUT + col) = v;
+        }
+      }
+    } else {
 #pragma unroll
     for (int n = 0; n < NT; n += 2) {
       const int col0 = n * 16 + kgrp * 4, col1 = col0 + 16;
@@ -284,6 +304,7 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
         if (row < outRows) *reinterpret_cast<u32x4*>(out + static_cast<size_t>(row) * COUT + outCol) = line;
       }
       }
+    }
     }
   };
 
@@ -457,7 +478,16 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   // shapes go by the bytes of an input row (the stage) and by the output channels (the accumulators): an int8 layer
   // takes the shape of the two-byte layer with half its input channels
   constexpr int RB = CIN * static_cast<int>(sizeof(T));
-  if constexpr (RB == 128 && COUT == 64) {
+  if constexpr (sizeof(T) == 4) {
+    // fp32: a step's MFMAs take eight times the cycles of a two-byte step with the same bytes, so the matrix pipe is
+    // the bound and the tile only has to spread over the CUs: 128 rows (two workgroups per CU) up to 64 output
+    // channels, eight wavefronts at 128, where one workgroup's weights leave no room for a second.  64 -> 64 with
+    // 150 000 rows runs in 285 us = 118 TFLOP/s of issued MFMAs against the 157 of the pipe (630 us on the vector
+    // kernel); skipping a 16-row group's MFMAs when none of its rows has the tap gained 15-20 us on strided and
+    // inverse layers and cost as much on the dense ones: the barrier waits for the fullest group either way
+    if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+    else return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
+  } else if constexpr (RB == 128 && COUT == 64) {
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else if constexpr (COUT >= 128) {
     // 8, 6 or 4 wavefronts of 32 rows: the workgroup size whose tiles load the busiest CU least (rounds of tiles
@@ -512,7 +542,11 @@ template <class T>
 int32_t launchPipe(const ConvArgs& a, hipStream_t stream) {
 #define D3D_PIPE_CASE(CI, CO) \
   if (a.cin == CI && a.cout == CO) return launchPipeShape<T, CI, CO>(a, stream);
-  if constexpr (sizeof(T) == 2) {  // rows of 64 bytes at least
+  if constexpr (sizeof(T) == 4) {
+    D3D_PIPE_CASE(16, 64)
+    D3D_PIPE_CASE(16, 128)
+  }
+  if constexpr (sizeof(T) >= 2) {  // rows of 64 bytes at least
     D3D_PIPE_CASE(32, 32)
     D3D_PIPE_CASE(32, 64)
     D3D_PIPE_CASE(32, 128)

@@ -828,43 +828,44 @@ struct MMPlugin final : d3d_plugin {
     std::vector<float> w(nW), b(withBias ? cout : 0);
     std::memcpy(w.data(), blob.data() + weightOffset, nW * 4);
     if (withBias) std::memcpy(b.data(), blob.data() + weightOffset + nW * 4, static_cast<size_t>(cout) * 4);
-    std::vector<uint16_t> packed;
-    int cinMfma = 0;
-    if (dtype == D3D_HALF || dtype == D3D_BF16) {
-      const bool half = dtype == D3D_HALF;
-      auto rnd = [&](float v, uint16_t* bits) {
-        *bits = half ? floatToHalfBits(v) : floatToBf16Bits(v);
-        return half ? halfBitsToFloat(*bits) : bf16BitsToFloat(*bits);
-      };
-      const int cinP = paddedMfmaChannels(dtype, cin, cout);
-      const bool mfma = convUsesMfma(dtype, cinP, cout);
-      if (mfma) packed.assign(static_cast<size_t>(kernelVol) * cinP * cout, 0);
-      cinMfma = mfma ? cinP : 0;
-      // fragment-major copy for the MFMA kernel: Wf[tap][kk][n][lane][j] = W[tap][kk*KS + (lane/16)*KG + j][n*16 + lane%16]
-      // with KS = 32 (16 when cin == 16) and KG = KS/4, so one wavefront load fetches one whole operand fragment;
-      // rows past cin (a narrow layer widened to 16 channels) stay zero
-      const int ks = cinP >= 32 ? 32 : 16, kg = ks / 4, nt = cout / 16, kkN = cinP / ks;
-      for (int k = 0; k < kernelVol; ++k)
-        for (int ci = 0; ci < cin; ++ci)
-          for (int co = 0; co < cout; ++co) {
-            const size_t src = (static_cast<size_t>(k) * cin + ci) * cout + co;
-            uint16_t bits;
-            w[src] = rnd(w[src], &bits);
-            if (mfma) {
-              const int kk = ci / ks, within = ci % ks, lane = (within / kg) * 16 + co % 16, j = within % kg;
-              const size_t dst = (((static_cast<size_t>(k) * kkN + kk) * nt + co / 16) * 64 + lane) * kg + j;
-              packed[dst] = bits;
-            }
-          }
-      for (auto& v : b) {
-        uint16_t bits;
-        v = rnd(v, &bits);
+    const int es = dtypeBytes(dtype);
+    // the value rounded to the storage type, and its bits
+    auto rnd = [&](float v, uint32_t* bits) {
+      if (dtype == D3D_FLOAT) {
+        std::memcpy(bits, &v, 4);
+        return v;
       }
+      const uint16_t h = dtype == D3D_HALF ? floatToHalfBits(v) : floatToBf16Bits(v);
+      *bits = h;
+      return dtype == D3D_HALF ? halfBitsToFloat(h) : bf16BitsToFloat(h);
+    };
+    const int cinP = paddedMfmaChannels(dtype, cin, cout);
+    const bool mfma = convUsesMfma(dtype, cinP, cout);
+    std::vector<uint8_t> packed(mfma ? static_cast<size_t>(kernelVol) * cinP * cout * es : 0, 0);
+    // fragment-major copy for the MFMA kernels: Wf[tap][kk][n][lane][j] = W[tap][kk*KS + (lane/16)*KG + j][n*16 + lane%16]
+    // with KS = 64 bytes of channels (32 bytes for 16 two-byte channels) and KG = KS/4, so one wavefront load fetches one
+    // whole operand fragment; rows past cin (a narrow layer widened to 16 channels) stay zero
+    const int ks = cinP * es >= 64 ? 64 / es : 16, kg = ks / 4, nt = cout / 16, kkN = cinP / ks;
+    for (int k = 0; k < kernelVol; ++k)
+      for (int ci = 0; ci < cin; ++ci)
+        for (int co = 0; co < cout; ++co) {
+          const size_t src = (static_cast<size_t>(k) * cin + ci) * cout + co;
+          uint32_t bits;
+          w[src] = rnd(w[src], &bits);
+          if (mfma) {
+            const int kk = ci / ks, within = ci % ks, lane = (within / kg) * 16 + co % 16, j = within % kg;
+            const size_t dst = (((static_cast<size_t>(k) * kkN + kk) * nt + co / 16) * 64 + lane) * kg + j;
+            std::memcpy(packed.data() + dst * es, &bits, es);
+          }
+        }
+    for (auto& v : b) {
+      uint32_t bits;
+      v = rnd(v, &bits);
     }
     int32_t rc = dev->f32.upload(w.data(), nW * 4);
     if (rc != D3D_OK) return rc;
     if (!packed.empty()) {
-      rc = dev->mfma.upload(packed.data(), packed.size() * 2);
+      rc = dev->mfma.upload(packed.data(), packed.size());
       if (rc != D3D_OK) return rc;
     }
     if (withBias) {
@@ -875,7 +876,7 @@ struct MMPlugin final : d3d_plugin {
       setError("SPConvMM: could not allocate the zero row");
       return D3D_ERR_DEVICE;
     }
-    dev->cinMfma = cinMfma;
+    dev->cinMfma = mfma ? cinP : 0;
     dev->dtype = dtype;
     return D3D_OK;
   }

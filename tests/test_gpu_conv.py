@@ -106,6 +106,18 @@ def test_narrow_tile_kernel_still_matches(engine, monkeypatch, cin, cout, dtype)
     run_case(2500, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, seed=41)
 
 
+@pytest.mark.parametrize("cin,cout", [(3, 16), (5, 32), (16, 32), (32, 16), (16, 64), (12, 64), (32, 32), (64, 32), (32, 64),
+                                      (64, 64), (16, 128), (64, 128), (128, 64), (128, 128)])
+def test_mfma_fp32(engine, cin, cout):
+    """fp32 layers on the matrix pipe: resident weights (at most 16 -> 32 or 32 -> 16 channels, rows below 16 channels
+    as stored) and the pipelined kernel, around its 128-row tiles, with and without tile masks, strided and inverse."""
+    for n in (1, 127, 128, 129, 2500):
+        run_case(n, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, "float32", True, relu=(n == 129),
+                 cap_extra=n % 3, link=n != 128)
+    run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, "float32", False)
+    run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, "float32", False, inverse=True, with_bias=False)
+
+
 def test_narrow_strided_fp32(engine):
     run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), 16, 16, "float32", False)
 
