@@ -6,23 +6,15 @@ right shape, this one returns the map.
 import numpy as np
 import torch
 
-from .plugin import Plugin, TensorDesc
+from .plugin import Launch, LaunchCache, Plugin, TensorDesc, current_stream, scratch
 
 _plugins = {}
-_workspaces = {}
+_launches = LaunchCache()
 
 
 def densify_blob(out_channels):
     """BEVDensifyPluginParam (trt/spconv/bev_densify_trt.cu:43-47; writer: bev_densify.py:38)."""
     return np.array([out_channels], dtype=np.int32).tobytes()
-
-
-def _workspace(nbytes, device):
-    key = (str(device), torch.cuda.current_stream().cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = _workspaces[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    return ws
 
 
 def bev_densify(in_feats, in_coors, num_act_in, in_spatial_shape, out_channels, out=None):
@@ -38,16 +30,21 @@ def bev_densify(in_feats, in_coors, num_act_in, in_spatial_shape, out_channels, 
         raise TypeError("coordinates and counts must be int32")
     in_feats = in_feats.contiguous()
     in_coors = in_coors.contiguous()
-    plugin = _plugins.get(int(out_channels))
-    if plugin is None:
-        plugin = _plugins[int(out_channels)] = Plugin("BEVDensify", densify_blob(out_channels))
-    in_descs = [TensorDesc.of_tensor(in_feats), TensorDesc.of_tensor(in_coors), TensorDesc.of_tensor(num_act_in),
-                TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]
-    out_descs = plugin.output_descs(in_descs)
+    # the tensors' devices and types decide nothing else: shape inference and descriptors are made once per signature
+    key = (int(out_channels), in_feats.shape, in_feats.dtype, in_coors.shape, num_act_in.shape, in_spatial_shape.shape)
+    launch = _launches.get(key)
+    if launch is None:
+        plugin = _plugins.get(key[0])
+        if plugin is None:
+            plugin = _plugins[key[0]] = Plugin("BEVDensify", densify_blob(out_channels))
+        launch = _launches.put(key, Launch(plugin, [
+            TensorDesc.of_tensor(in_feats), TensorDesc.of_tensor(in_coors), TensorDesc.of_tensor(num_act_in),
+            TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]))
+    dev = in_feats.device
+    stream = current_stream(dev)
     if out is None:
-        out = torch.empty(out_descs[0].shape(), dtype=in_feats.dtype, device=in_feats.device)
-    ws = _workspace(plugin.workspace_size(in_descs, out_descs), in_feats.device)
-    plugin.enqueue(in_descs, out_descs, [in_feats, in_coors, num_act_in, None], [out], ws)
+        out = torch.empty(launch.shapes[0], dtype=in_feats.dtype, device=dev)
+    launch((in_feats, in_coors, num_act_in, None), (out,), scratch(launch.nbytes, dev, stream), stream)
     return out
 
 

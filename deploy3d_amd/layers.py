@@ -9,7 +9,7 @@ it can be captured into a HIP graph.
 import numpy as np
 import torch
 
-from .plugin import OPT_INDEX_UNUSED, OPT_PERSISTENT_INDEX, Plugin, Schedule, TensorDesc
+from .plugin import OPT_INDEX_UNUSED, OPT_PERSISTENT_INDEX, Launch, Plugin, Schedule, TensorDesc, current_stream
 from .spconv_index import index_blob
 from .spconv_mm import mm_blob
 
@@ -82,19 +82,19 @@ class SparseConvLayer:
         if self._idx_state is None or self._idx_state["cap"] != x.capacity:
             in_descs = [TensorDesc.of_tensor(x.coors), TensorDesc.of_tensor(x.num_act),
                         TensorDesc.of((x.batch, 0) + tuple(x.grid), torch.int32)]
-            out_descs = self.idx_plugin.output_descs(in_descs)
+            launch = Launch(self.idx_plugin, in_descs)
+            out_descs = launch.out_descs
             outs = [torch.empty(d.shape(), dtype=torch.int32, device=self.device) if 0 not in d.shape() else None
                     for d in out_descs]
-            ws = torch.empty(max(1, self.idx_plugin.workspace_size(in_descs, out_descs)), dtype=torch.uint8,
-                             device=self.device)
-            self._idx_state = dict(cap=x.capacity, in_descs=in_descs, out_descs=out_descs, outs=outs, ws=ws)
+            ws = torch.empty(max(1, launch.nbytes), dtype=torch.uint8, device=self.device)
+            self._idx_state = dict(cap=x.capacity, in_descs=in_descs, out_descs=out_descs, outs=outs, ws=ws, launch=launch)
             # a SubM rulebook on the outputs of a strided one reuses that operator's occupancy map; a strided one
             # derives the occupancy of its own map from it
             if self.extensions and not self.spec.get("inverse", False):
                 self.idx_plugin.link_coords(x.producer)
             self.idx_plugin.configure(in_descs, out_descs)  # reserves the maps an operator keeps between passes
         st = self._idx_state
-        self.idx_plugin.enqueue(st["in_descs"], st["out_descs"], [x.coors, x.num_act, None], st["outs"], st["ws"])
+        st["launch"]((x.coors, x.num_act, None), st["outs"], st["ws"], current_stream())
         outs = st["outs"]
         if self.spec["subm"]:  # SubM: outputs sit on the input voxels (test_middle_encoder.py:68-69)
             return Rulebook(outs[0], outs[1], x.coors, x.num_act, x.grid, x, self.idx_plugin)
@@ -114,15 +114,16 @@ class SparseConvLayer:
         num_in, num_out = (rb.num_act_out, rb.num_act_in) if inverse else (rb.num_act_in, rb.num_act_out)
         if self._mm_state is None or self._mm_state["in_rows"] != feats.shape[0] or self._mm_state["rb"] is not rb.plugin:
             in_descs = [TensorDesc.of_tensor(t) for t in (feats, num_in, num_out, rb.index, rb.num_index)]
-            out_descs = self.mm_plugin.output_descs(in_descs)
+            launch = Launch(self.mm_plugin, in_descs)
+            out_descs = launch.out_descs
             if self.extensions:
                 self.mm_plugin.link_rulebook(rb.plugin)
             self.mm_plugin.configure(in_descs, out_descs)
             out = torch.empty(out_descs[0].shape(), dtype=self.dtype, device=self.device)
-            self._mm_state = dict(in_rows=feats.shape[0], in_descs=in_descs, out_descs=out_descs, out=out, rb=rb.plugin)
+            self._mm_state = dict(in_rows=feats.shape[0], in_descs=in_descs, out_descs=out_descs, out=out, rb=rb.plugin,
+                                  launch=launch)
         st = self._mm_state
-        self.mm_plugin.enqueue(st["in_descs"], st["out_descs"], [feats, num_in, num_out, rb.index, rb.num_index],
-                               [st["out"]])
+        st["launch"]((feats, num_in, num_out, rb.index, rb.num_index), (st["out"],), None, current_stream())
         if inverse:
             return SparseTensor(st["out"], rb.in_coors, rb.num_act_in, rb.in_grid, x.batch, rb.in_producer)
         return SparseTensor(st["out"], rb.out_coors, rb.num_act_out, rb.out_grid, x.batch,

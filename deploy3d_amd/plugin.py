@@ -137,6 +137,37 @@ def _check(status):
         raise EngineError(status, load_library().d3d_last_error().decode())
 
 
+# hipStream_t of the current stream of a device: the accessor torch's own generated code uses where it is there (0.1 us;
+# building a Stream object first takes 3)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def current_stream(device=None):
+    """hipStream_t of the current stream of ``device`` (a tensor's torch.device; None = the current device)."""
+    if _raw_stream is None or (device is not None and device.index is None):
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if device is None else device.index)
+
+
+def _pointers(tensors):
+    """Array of device pointers; null for tensors of which only the shape matters."""
+    return (ctypes.c_void_p * max(1, len(tensors)))(*[
+        t.data_ptr() if t is not None and t.numel() else None for t in tensors])
+
+
+_scratch = {}
+
+
+def scratch(nbytes, device, stream):
+    """Workspace of the functional operators: one buffer per stream, grown to the largest request (kernels of one stream
+    run in order, so consecutive calls may share it)."""
+    key = (device, stream)
+    ws = _scratch.get(key)
+    if ws is None or ws.numel() < nbytes:
+        ws = _scratch[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    return ws
+
+
 def _desc_array(descs):
     arr = (TensorDesc * max(1, len(descs)))()
     for i, d in enumerate(descs):
@@ -231,22 +262,53 @@ class Plugin:
 
     def enqueue(self, in_descs, out_descs, inputs, outputs, workspace=None, stream=None):
         """inputs / outputs: torch tensors (or None for shape-only tensors); returns the raw status check."""
-        def ptrs(ts):
-            arr = (ctypes.c_void_p * max(1, len(ts)))()
-            for i, t in enumerate(ts):
-                arr[i] = None if t is None or t.numel() == 0 else t.data_ptr()
-            return arr
         static = isinstance(workspace, str)
         ws_ptr = None if workspace is None or static else workspace.data_ptr()
         ws_bytes = 0 if workspace is None or static else workspace.numel() * workspace.element_size()
         if stream is None:
-            stream = torch.cuda.current_stream().cuda_stream
+            stream = current_stream()
         if static:  # workspace="static" -> d3d_enqueue_static: the library's own fixed scratch array, no allocation
-            _check(self._lib.d3d_enqueue_static(self._h, _desc_array(in_descs), _desc_array(out_descs), ptrs(inputs),
-                                                ptrs(outputs), ctypes.c_void_p(stream)))
+            _check(self._lib.d3d_enqueue_static(self._h, _desc_array(in_descs), _desc_array(out_descs), _pointers(inputs),
+                                                _pointers(outputs), ctypes.c_void_p(stream)))
             return
-        _check(self._lib.d3d_enqueue(self._h, _desc_array(in_descs), _desc_array(out_descs), ptrs(inputs),
-                                     ptrs(outputs), ws_ptr, ws_bytes, ctypes.c_void_p(stream)))
+        _check(self._lib.d3d_enqueue(self._h, _desc_array(in_descs), _desc_array(out_descs), _pointers(inputs),
+                                     _pointers(outputs), ws_ptr, ws_bytes, ctypes.c_void_p(stream)))
+
+
+class Launch:
+    """Enqueues of one operator at one set of descriptors: shape inference, workspace size and descriptor arrays are made
+    once, a call passes pointers only.  ``shapes``: the operator's outputs."""
+
+    def __init__(self, plugin, in_descs):
+        out_descs = plugin.output_descs(in_descs)
+        self.plugin, self.in_descs, self.out_descs = plugin, in_descs, out_descs
+        self.nbytes = plugin.workspace_size(in_descs, out_descs)
+        self.shapes = [d.shape() for d in out_descs]
+        self._in, self._out = _desc_array(in_descs), _desc_array(out_descs)
+        self._enqueue = plugin._lib.d3d_enqueue
+
+    def __call__(self, inputs, outputs, workspace, stream):
+        ws, nbytes = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.nbytes)
+        rc = self._enqueue(self.plugin._h, self._in, self._out, _pointers(inputs), _pointers(outputs), ws, nbytes, stream)
+        if rc:
+            _check(rc)
+
+
+class LaunchCache:
+    """The Launches of a functional operator by call signature.  Bounded: a caller whose shapes never repeat starts over
+    every ``limit`` signatures."""
+
+    def __init__(self, limit=256):
+        self._items, self._limit = {}, limit
+
+    def get(self, key):
+        return self._items.get(key)
+
+    def put(self, key, launch):
+        if len(self._items) >= self._limit:
+            self._items = {}
+        self._items[key] = launch
+        return launch
 
 
 class Schedule:
@@ -264,16 +326,12 @@ class Schedule:
 
     def add(self, plugin, in_descs, out_descs, inputs, outputs, workspace=None, lane=0, after=()):
         """Appends ``plugin.enqueue(in_descs, out_descs, inputs, outputs, workspace)``; returns the step's index."""
-        def ptrs(ts):
-            arr = (ctypes.c_void_p * max(1, len(ts)))()
-            for i, t in enumerate(ts):
-                arr[i] = None if t is None or t.numel() == 0 else t.data_ptr()
-            return arr
         ws_ptr = None if workspace is None else workspace.data_ptr()
         ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
         dep = (ctypes.c_int32 * max(1, len(after)))(*[int(a) for a in after])
         rc = self._lib.d3d_schedule_add(self._h, plugin._h, _desc_array(in_descs), len(in_descs),
-                                        _desc_array(out_descs), len(out_descs), ptrs(inputs), ptrs(outputs), ws_ptr,
+                                        _desc_array(out_descs), len(out_descs), _pointers(inputs),
+                                        _pointers(outputs), ws_ptr,
                                         ws_bytes, int(lane), dep, len(after))
         if rc < 0:
             _check(rc)
@@ -285,7 +343,7 @@ class Schedule:
 
     def run(self, stream=None):
         if stream is None:
-            stream = torch.cuda.current_stream().cuda_stream
+            stream = current_stream()
         _check(self._lib.d3d_schedule_run(self._h, ctypes.c_void_p(stream)))
 
     def __del__(self):

@@ -6,23 +6,15 @@ shape, this one returns the voxels.
 import numpy as np
 import torch
 
-from .plugin import Plugin, TensorDesc
+from .plugin import Launch, LaunchCache, Plugin, TensorDesc, current_stream, scratch
 
 _plugins = {}
-_workspaces = {}
+_launches = LaunchCache()
 
 
 def simple_mean_blob(max_num_act_out):
     """SimpleMeanEncoderPluginParam (trt/voxel_encoder/simple_mean_trt.cu:176-180; writer: simple_mean.py:44)."""
     return np.array([max_num_act_out], dtype=np.int32).tobytes()
-
-
-def _workspace(nbytes, device):
-    key = (str(device), torch.cuda.current_stream().cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = _workspaces[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    return ws
 
 
 def simple_mean_encoder(batch_point_feats, batch_indices, voxel_config, in_spatial_shape, max_num_act_out):
@@ -42,20 +34,25 @@ def simple_mean_encoder(batch_point_feats, batch_indices, voxel_config, in_spati
     batch_point_feats = batch_point_feats.contiguous()
     batch_indices = batch_indices.contiguous()
     dev = batch_point_feats.device
-    voxel_config = voxel_config.to(dev).contiguous()
-    plugin = _plugins.get(int(max_num_act_out))
-    if plugin is None:
-        plugin = _plugins[int(max_num_act_out)] = Plugin("SimpleMeanEncoder", simple_mean_blob(max_num_act_out))
-    in_descs = [TensorDesc.of_tensor(batch_point_feats), TensorDesc.of_tensor(batch_indices),
-                TensorDesc.of_tensor(voxel_config), TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]
-    out_descs = plugin.output_descs(in_descs)
-    out_feats = torch.empty(out_descs[0].shape(), dtype=torch.float32, device=dev)
-    out_coors = torch.empty(out_descs[1].shape(), dtype=torch.int32, device=dev)
-    num_act_out = torch.empty(out_descs[2].shape(), dtype=torch.int32, device=dev)
-    ws = _workspace(plugin.workspace_size(in_descs, out_descs), dev)
-    plugin.enqueue(in_descs, out_descs, [batch_point_feats, batch_indices, voxel_config, None],
-                   [out_feats, out_coors, num_act_out], ws)
-    return out_feats, out_coors, num_act_out
+    if voxel_config.device != dev:
+        voxel_config = voxel_config.to(dev)
+    voxel_config = voxel_config.contiguous()
+    key = (int(max_num_act_out), batch_point_feats.shape, batch_indices.shape, voxel_config.shape, in_spatial_shape.shape)
+    launch = _launches.get(key)
+    if launch is None:
+        plugin = _plugins.get(key[0])
+        if plugin is None:
+            plugin = _plugins[key[0]] = Plugin("SimpleMeanEncoder", simple_mean_blob(max_num_act_out))
+        launch = _launches.put(key, Launch(plugin, [
+            TensorDesc.of_tensor(batch_point_feats), TensorDesc.of_tensor(batch_indices),
+            TensorDesc.of_tensor(voxel_config), TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]))
+    feats_shape, coors_shape, num_shape = launch.shapes
+    outs = (torch.empty(feats_shape, dtype=torch.float32, device=dev),
+            torch.empty(coors_shape, dtype=torch.int32, device=dev),
+            torch.empty(num_shape, dtype=torch.int32, device=dev))
+    stream = current_stream(dev)
+    launch((batch_point_feats, batch_indices, voxel_config, None), outs, scratch(launch.nbytes, dev, stream), stream)
+    return outs
 
 
 class SimpleMeanEncoder:

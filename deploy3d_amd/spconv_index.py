@@ -7,10 +7,10 @@ import hashlib
 import numpy as np
 import torch
 
-from .plugin import Plugin, TensorDesc
+from .plugin import Launch, LaunchCache, Plugin, TensorDesc, current_stream, scratch
 
 _plugins = {}
-_workspaces = {}
+_launches = LaunchCache()
 
 
 def index_blob(kernel_size, stride, padding, dilation, out_padding, max_num_act_out, subm, transpose):
@@ -31,14 +31,6 @@ def _plugin(name, blob):
     return p
 
 
-def _workspace(nbytes, device):
-    key = (str(device), torch.cuda.current_stream().cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = _workspaces[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    return ws
-
-
 def index_plugin(kernel_size, stride, padding, dilation, out_padding, max_num_act_out, subm, transpose):
     """The operator instance ``spconv_index_nd`` runs for these attributes (one per distinct attribute blob); what
     ``spconv_mm(..., rulebook=...)`` links a convolution to."""
@@ -56,21 +48,22 @@ def spconv_index_nd(in_coors, num_act_in, in_spatial_shape, kernel_size, stride,
     Returns (index [3, kVol*(cap+128)], num_index [1]) for SubM, else also
     (out_coors [max_num_act_out, N+1], num_act_out [1], out_spatial_shape).
     """
-    nd = len(kernel_size)
     if in_coors.dtype != torch.int32 or num_act_in.dtype != torch.int32:
         raise TypeError("coordinates and counts must be int32")
     in_coors = in_coors.contiguous()
-    plugin = index_plugin(kernel_size, stride, padding, dilation, out_padding, max_num_act_out, subm, transpose)
-    in_descs = [TensorDesc.of_tensor(in_coors), TensorDesc.of_tensor(num_act_in),
-                TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]
-    out_descs = plugin.output_descs(in_descs)
+    key = (tuple(kernel_size), tuple(stride), tuple(padding), tuple(dilation), tuple(out_padding), int(max_num_act_out),
+           bool(subm), bool(transpose), in_coors.shape, num_act_in.shape, in_spatial_shape.shape)
+    launch = _launches.get(key)
+    if launch is None:
+        plugin = index_plugin(kernel_size, stride, padding, dilation, out_padding, max_num_act_out, subm, transpose)
+        launch = _launches.put(key, Launch(plugin, [
+            TensorDesc.of_tensor(in_coors), TensorDesc.of_tensor(num_act_in),
+            TensorDesc.of(tuple(in_spatial_shape.shape), torch.int32)]))
     dev = in_coors.device
-    outs = []
-    for i, d in enumerate(out_descs):
-        outs.append(torch.empty(d.shape(), dtype=torch.int32, device=dev))
-    ws = _workspace(plugin.workspace_size(in_descs, out_descs), dev)
-    plugin.enqueue(in_descs, out_descs, [in_coors, num_act_in, None], outs, ws)
-    return tuple(outs)
+    outs = tuple([torch.empty(shape, dtype=torch.int32, device=dev) for shape in launch.shapes])
+    queue = current_stream(dev)
+    launch((in_coors, num_act_in, None), outs, scratch(launch.nbytes, dev, queue), queue)
+    return outs
 
 
 def spconv_index(in_coors, num_act_in, in_spatial_shape, kernel_size, stride, padding, dilation, out_padding,

@@ -3,15 +3,20 @@
 HIP engine.  ``relu`` (fused ReLU) and the activation scales are this build's
 extensions, carried in an extension record after the reference's blob.
 """
+import ctypes
 import hashlib
 import struct
 
 import numpy as np
 import torch
 
-from .plugin import Plugin, TensorDesc
+from .plugin import Launch, LaunchCache, Plugin, TensorDesc, current_stream
 
 _plugins = {}
+_by_attributes = {}  # attributes of a convolution -> [(plugin, weight, bias)], copies of the values it was made from
+_launches = LaunchCache()
+_memcmp = ctypes.CDLL(None).memcmp
+_memcmp.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
 EXT_MAGIC = 0x58443344  # "D3DX"
 
 
@@ -41,12 +46,36 @@ def get_plugin(blob):
     return p
 
 
+def _same(a, b):
+    return a is b or (a is not None and b is not None and a.size == b.size and
+                      _memcmp(a.ctypes.data, b.ctypes.data, a.nbytes) == 0)
+
+
+def _plugin_of(attributes, weight, bias):
+    """The operator instance of these attributes and values.  The caller's arrays are compared value by value with those
+    of the instances that exist (a memcmp, which ends at the first difference), most recent first: packing and hashing
+    the whole blob on every call took several times as long as the convolution's kernels."""
+    weight = np.ascontiguousarray(weight, dtype=np.float32)
+    bias = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
+    known = _by_attributes.setdefault(attributes, [])
+    for plugin, w, b in list(known):
+        if _same(w, weight) and _same(b, bias):
+            return plugin
+    plugin = get_plugin(mm_blob(*attributes[:6], weight, bias, *attributes[6:]))
+    known.insert(0, (plugin, weight.copy(), None if bias is None else bias.copy()))
+    return plugin
+
+
 def run_mm(plugin, in_feats, num_act_in, num_act_out, index, num_index, out=None):
-    in_descs = [TensorDesc.of_tensor(t) for t in (in_feats, num_act_in, num_act_out, index, num_index)]
-    out_descs = plugin.output_descs(in_descs)
+    key = (id(plugin), in_feats.shape, in_feats.dtype, num_act_in.shape, num_act_in.dtype, num_act_out.shape,
+           num_act_out.dtype, index.shape, index.dtype, num_index.shape, num_index.dtype)
+    launch = _launches.get(key)
+    if launch is None or launch.plugin is not plugin:
+        launch = _launches.put(key, Launch(plugin, [
+            TensorDesc.of_tensor(t) for t in (in_feats, num_act_in, num_act_out, index, num_index)]))
     if out is None:
-        out = torch.empty(out_descs[0].shape(), dtype=in_feats.dtype, device=in_feats.device)
-    plugin.enqueue(in_descs, out_descs, [in_feats, num_act_in, num_act_out, index, num_index], [out])
+        out = torch.empty(launch.shapes[0], dtype=in_feats.dtype, device=in_feats.device)
+    launch((in_feats, num_act_in, num_act_out, index, num_index), (out,), None, current_stream(in_feats.device))
     return out
 
 
@@ -62,9 +91,9 @@ def spconv_mm(in_feats, num_act_in, num_act_out, index, num_index, kernel_size, 
     convolution is linked to it and reads the neighbour table that operator wrote instead of deriving one from the
     index tensor (which is what happens without it, and for any tensor that operator did not write last).
     """
-    blob = mm_blob(kernel_size, in_channels, out_channels, max_num_act_out, subm, inverse, weight, bias, relu,
-                   act_scale_in, act_scale_out)
-    plugin = get_plugin(blob)
+    size = int(kernel_size) if np.isscalar(kernel_size) else tuple(kernel_size)
+    plugin = _plugin_of((size, int(in_channels), int(out_channels), int(max_num_act_out), bool(subm), bool(inverse),
+                         bool(relu), float(act_scale_in), float(act_scale_out)), weight, bias)
     plugin.link_rulebook(rulebook)
     return run_mm(plugin, in_feats.contiguous(), num_act_in, num_act_out, index, num_index)
 
