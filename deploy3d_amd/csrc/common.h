@@ -33,6 +33,10 @@ inline const char* debugEnv(const char* name) {
 void setError(const char* fmt, ...);
 const char* lastError();
 
+// Changes to an operator (options, links, reserved buffers, the way its builds keep their state between passes) that make
+// an earlier capture of its enqueue differ from what an enqueue would do now.  Only ever grows.
+uint64_t pluginChanges(const d3d_plugin* p);
+
 #define D3D_HIP_CHECK(expr)                                                              \
   do {                                                                                   \
     hipError_t e_ = (expr);                                                              \
@@ -200,6 +204,11 @@ int paddedMfmaChannels(int32_t dtype, int cin, int cout);
 // paddedMfmaChannels() of them (ConvArgs::rowChannels): no widened copy of the input is needed.
 bool convReadsNarrowRows(int32_t dtype, int kVol, int cin, int cout);
 int32_t launchPadRows(const void* in, int64_t rows, int inBytes, int outBytes, void* out, hipStream_t stream);
+
+// Elementwise steps of a schedule (elementwise.hip): out = a + b for n elements of `dtype` (float, half, bf16; the sum of the
+// fp32 values, rounded once), and out = a converted from float to `dtype` (half, bf16).
+int32_t launchSum(int32_t dtype, const void* a, const void* b, void* out, int64_t n, hipStream_t stream);
+int32_t launchCastFromFloat(int32_t dtype, const float* a, void* out, int64_t n, hipStream_t stream);
 
 // Sparse rows -> dense [B, C, Z, Y, X] map (densify.hip).  The workspace holds one int32 per cell.
 struct DensifyArgs {

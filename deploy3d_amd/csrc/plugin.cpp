@@ -6,6 +6,7 @@
 // and SPConvMMPlugin (trt/spconv/mm_trt.cu:39-206).
 #include <dlfcn.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -171,6 +172,8 @@ int dtypeBytes(int32_t dtype) {
 // ---------------------------------------------------------------------------
 struct RulebookLink {
   std::mutex mutex;
+  std::atomic<uint64_t> changes{0};  // see pluginChanges
+  uint64_t buildKind = 0;            // how the last build kept its state between passes (a digest; a change counts)
   bool wanted = false;            // some convolution is linked: the operator writes the table
   bool wantMasks = false;         // ... and one of them runs a kernel that reads tile masks
   DeviceBuffer table, masks, fillState;
@@ -283,6 +286,7 @@ struct d3d_plugin {
   virtual size_t workspaceSize(const d3d_tensor_desc* in, int32_t nbIn) const = 0;
   virtual int32_t enqueue(const d3d_tensor_desc* inDesc, const d3d_tensor_desc* outDesc, const void* const* inputs,
                           void* const* outputs, void* workspace, size_t workspaceBytes, hipStream_t stream) = 0;
+  virtual uint64_t changeCount() const { return 0; }
   virtual int32_t setOption(int32_t option, int64_t) {
     d3d::setError("%s: option %d not known to this operator", type.c_str(), option);
     return D3D_ERR_UNSUPPORTED;
@@ -358,6 +362,8 @@ struct IdxPlugin final : d3d_plugin {
   // Called when a convolution is linked: from now on enqueue also writes the neighbour table and the tile masks.
   int32_t wantByProducts(bool masks) {
     std::lock_guard<std::mutex> lock(link->mutex);
+    const bool hadMasks = link->wantMasks;
+    const void* const oldTable = link->table.ptr;
     link->wantMasks = link->wantMasks || (masks && kVol() <= 64);
     if (maxNumActOut > 0) {
       int32_t rc = link->table.reserve(static_cast<size_t>(kVol()) * static_cast<size_t>(maxNumActOut) * sizeof(int32_t));
@@ -365,13 +371,19 @@ struct IdxPlugin final : d3d_plugin {
       rc = link->masks.reserve(maskEntries(maxNumActOut) * sizeof(unsigned long long));
       if (rc != D3D_OK) return rc;
     }
+    if (!link->wanted || link->table.ptr != oldTable || link->wantMasks != hadMasks) ++link->changes;
     link->wanted = true;
     return D3D_OK;
   }
 
+  // options, by-products wanted, maps and tables reallocated, another kind of build - here or at the operator whose
+  // map this one reads
+  uint64_t changeCount() const override { return link->changes + (coordSource ? coordSource->changes.load() : 0); }
+
   int32_t setOption(int32_t option, int64_t value) override {
     if (option == D3D_OPT_INDEX_UNUSED) {
       std::lock_guard<std::mutex> lock(link->mutex);
+      ++link->changes;
       indexUnused = value != 0;
       link->primedIndex = nullptr;
       return D3D_OK;
@@ -382,6 +394,7 @@ struct IdxPlugin final : d3d_plugin {
       int32_t rc = link->fillState.reallocZeroed(256);
       if (rc != D3D_OK) return rc;
     }
+    ++link->changes;
     persistentIndex = value != 0;
     link->primedIndex = nullptr;
     return D3D_OK;
@@ -454,6 +467,7 @@ struct IdxPlugin final : d3d_plugin {
              link->mapState.bytes >= stateBytes && link->mapStride * 16 == static_cast<int64_t>(recBytes);
     };
     if (!have() && mayAllocate) {
+      ++link->changes;
       link->mapStride = 0;
       if (link->mapRecords.reallocZeroed(2 * recBytes) == D3D_OK && link->mapChunkBase.reserve(chunkBytes) == D3D_OK &&
           link->mapState.reallocZeroed(stateBytes) == D3D_OK) {
@@ -619,6 +633,23 @@ struct IdxPlugin final : d3d_plugin {
                                 subM ? nullptr : static_cast<int32_t*>(outputs[3]), workspace, workspaceBytes, side,
                                 stream);
     if (rc == D3D_OK) {
+      // what a captured copy of this enqueue has baked in besides its tensors
+      uint64_t kind = 1469598103934665603ull;
+      auto mix = [&](uint64_t v) { kind = (kind ^ v) * 1099511628211ull; };
+      mix(reinterpret_cast<uintptr_t>(outputs[0]));
+      mix(static_cast<uint64_t>(cap));
+      mix(reinterpret_cast<uintptr_t>(side.nbr));
+      mix(reinterpret_cast<uintptr_t>(side.masks));
+      mix(reinterpret_cast<uintptr_t>(side.fillState));
+      mix(reinterpret_cast<uintptr_t>(side.mapRecords));
+      mix(reinterpret_cast<uintptr_t>(side.srcRecords));
+      mix((side.incrementalFill ? 1u : 0u) | (side.useSharedMap ? 2u : 0u) | (side.mapDouble ? 4u : 0u) |
+          (side.srcDouble ? 8u : 0u) | (side.indexWritten ? 16u : 0u) | (side.masksWritten ? 32u : 0u) |
+          (side.sourceMapUsed ? 64u : 0u));
+      if (kind != link->buildKind) {
+        link->buildKind = kind;
+        ++link->changes;
+      }
       link->index = outputs[0];
       link->numIndex = outputs[1];
       link->kVol = kVol();
@@ -693,6 +724,7 @@ constexpr size_t kMMHeader = 19;
 
 struct MMDeviceWeights {
   int32_t dtype = -1;
+  std::atomic<uint64_t> changes{0};  // uploads so far
   int cinMfma = 0;  // input channels of the packed MFMA weights (cin widened with zero rows), 0 = no MFMA copy
   DeviceBuffer f32, mfma, bias, requantM;  // int8: bias holds bias / s_out, requantM holds s_in * s_w[c] / s_out
 };
@@ -708,6 +740,10 @@ struct MMPlugin final : d3d_plugin {
   std::shared_ptr<DeviceBuffer> derived;       // neighbour table derived from the index tensor (no link, foreign
                                                // tensor, inverse)
   std::shared_ptr<DeviceBuffer> widened;       // input rows widened to the MFMA channel count (narrow layers)
+  uint64_t changes = 0;                        // buffers reserved, tables switched; links count in the upper half
+  const int32_t* lastTable = nullptr;          // neighbour table of the last enqueue
+
+  uint64_t changeCount() const override { return changes + dev->changes + (linked ? linked->changes.load() : 0); }
 
   static int32_t parse(const void* data, size_t len, MMPlugin** out) {
     if (!data || len < kMMHeader) {
@@ -802,6 +838,7 @@ struct MMPlugin final : d3d_plugin {
     {
       std::lock_guard<std::mutex> lock(*devMutex);
       if (dev->dtype != dtype) {
+        ++dev->changes;
         const int32_t rc = dtype == D3D_INT8 ? configureInt8() : configureFloat(dtype);
         if (rc != D3D_OK) return rc;
       }
@@ -812,12 +849,16 @@ struct MMPlugin final : d3d_plugin {
     if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && dev->cinMfma > cin &&
         !convReadsNarrowRows(dtype, kernelVol, cin, cout)) {
       if (!widened) widened = std::make_shared<DeviceBuffer>();
+      const void* const before = widened->ptr;
       const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * dev->cinMfma * dtypeBytes(dtype));
+      if (widened->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
     if ((!linked || inverse) && maxNumActOut > 0) {
       if (!derived) derived = std::make_shared<DeviceBuffer>();
+      const void* const before = derived->ptr;
       const int32_t rc = derived->reserve(static_cast<size_t>(kernelVol) * static_cast<size_t>(maxNumActOut) * sizeof(int32_t));
+      if (derived->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
     return D3D_OK;
@@ -1000,12 +1041,17 @@ struct MMPlugin final : d3d_plugin {
                  "capture (configure the node at these shapes, or enqueue it once, first)", bytes);
         return D3D_ERR_UNSUPPORTED;
       }
+      if (derived->bytes < bytes) ++changes;
       rc = derived->reserve(bytes);
       if (rc != D3D_OK) return rc;
       rc = launchBuildNeighbours(static_cast<const int32_t*>(inputs[3]), rowLen, static_cast<const int32_t*>(inputs[4]),
                                  inverse, kernelVol, outRows, inDesc[0].dims[0], static_cast<int32_t*>(derived->ptr), stream);
       if (rc != D3D_OK) return rc;
       nbr = static_cast<const int32_t*>(derived->ptr);
+    }
+    if (nbr != lastTable) {
+      lastTable = nbr;
+      ++changes;
     }
     const void* zeros = zeroRow();
     ConvArgs a{};
@@ -1033,6 +1079,7 @@ struct MMPlugin final : d3d_plugin {
         setError("SPConvMM: %zu bytes for the widened input rows were not reserved before the capture", wideBytes);
         return D3D_ERR_UNSUPPORTED;
       }
+      if (widened->bytes < wideBytes) ++changes;
       rc = widened->reserve(wideBytes);
       if (rc != D3D_OK) return rc;
       rc = launchPadRows(inputs[0], a.inRows, cin * es, dev->cinMfma * es, widened->ptr, stream);
@@ -1302,6 +1349,10 @@ using namespace d3d;
     return ret;                                    \
   }
 
+namespace d3d {
+uint64_t pluginChanges(const d3d_plugin* p) { return p->changeCount(); }
+}  // namespace d3d
+
 extern "C" {
 
 int32_t d3d_create(const char* name, const char* version, const void* blob, size_t len, d3d_plugin** out) {
@@ -1443,6 +1494,7 @@ int32_t d3d_link_rulebook(d3d_plugin* mm, d3d_plugin* idx) {
     return D3D_ERR_BAD_ARG;
   }
   if (!idx) {
+    if (m->linked) m->changes += 1ull << 32;
     m->linked.reset();
     return D3D_OK;
   }
@@ -1466,6 +1518,7 @@ int32_t d3d_link_rulebook(d3d_plugin* mm, d3d_plugin* idx) {
   // tile masks are read by the kernels of layers with at least 32 (widened) input channels
   int32_t rc = r->wantByProducts(m->cin > 16);
   if (rc != D3D_OK) return rc;
+  if (m->linked != r->link) m->changes += 1ull << 32;
   m->linked = r->link;
   return D3D_OK;
   D3D_GUARD_END(D3D_ERR_BAD_ARG)
@@ -1478,6 +1531,7 @@ int32_t d3d_link_coords(d3d_plugin* subm, d3d_plugin* producer) {
     setError("d3d_link_coords: the first handle must be an SPConvIdx{N}d");
     return D3D_ERR_BAD_ARG;
   }
+  s->link->changes += 1ull << 32;
   if (!producer) {
     s->coordSource.reset();
     return D3D_OK;
@@ -1489,6 +1543,7 @@ int32_t d3d_link_coords(d3d_plugin* subm, d3d_plugin* producer) {
   }
   {
     std::lock_guard<std::mutex> lock(r->link->mutex);
+    if (!r->link->shareMap) ++r->link->changes;
     r->link->shareMap = true;
   }
   s->coordSource = r->link;

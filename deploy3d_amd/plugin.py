@@ -28,7 +28,7 @@ EXPORTS = [
     "d3d_serialize", "d3d_num_outputs", "d3d_output_dims", "d3d_output_dtype", "d3d_supports_format",
     "d3d_configure", "d3d_workspace_size", "d3d_enqueue", "d3d_last_error", "d3d_num_ops", "d3d_op_name",
     "d3d_enqueue_static", "d3d_link_rulebook", "d3d_link_coords", "d3d_set_option",
-    "d3d_schedule_create", "d3d_schedule_add", "d3d_schedule_size", "d3d_schedule_run", "d3d_schedule_destroy",
+    "d3d_schedule_create", "d3d_schedule_add", "d3d_schedule_add_sum", "d3d_schedule_add_cast", "d3d_schedule_size", "d3d_schedule_run", "d3d_schedule_destroy",
 ]
 OPT_PERSISTENT_INDEX = 1
 OPT_INDEX_UNUSED = 2
@@ -122,6 +122,10 @@ def load_library(path=None):
     lib.d3d_schedule_add.restype = i32
     lib.d3d_schedule_add.argtypes = [vp, vp, descp, i32, descp, i32, ctypes.POINTER(vp), ctypes.POINTER(vp), vp, sz,
                                      i32, ctypes.POINTER(i32), i32]
+    lib.d3d_schedule_add_sum.restype = i32
+    lib.d3d_schedule_add_sum.argtypes = [vp, i32, vp, vp, vp, ctypes.c_int64, i32, ctypes.POINTER(i32), i32]
+    lib.d3d_schedule_add_cast.restype = i32
+    lib.d3d_schedule_add_cast.argtypes = [vp, i32, vp, vp, ctypes.c_int64, i32, ctypes.POINTER(i32), i32]
     lib.d3d_schedule_size.restype = i32
     lib.d3d_schedule_size.argtypes = [vp]
     lib.d3d_schedule_run.restype = i32
@@ -314,7 +318,8 @@ class LaunchCache:
 class Schedule:
     """A pass recorded once and enqueued by one native call (d3d_schedule_*): steps are operator enqueues with their
     descriptors, tensors and workspace, each on a lane (lane 0 = the stream of ``run``; the others are streams the
-    schedule owns) and behind the earlier steps it names.  Keeps the tensors and operators it was given alive."""
+    schedule owns) and behind the earlier steps it names.  From the third run on a pass is one HIP-graph launch (see
+    d3d_schedule_run).  Keeps the tensors and operators it was given alive."""
 
     def __init__(self, lanes=1):
         self._lib = load_library()
@@ -328,14 +333,31 @@ class Schedule:
         """Appends ``plugin.enqueue(in_descs, out_descs, inputs, outputs, workspace)``; returns the step's index."""
         ws_ptr = None if workspace is None else workspace.data_ptr()
         ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-        dep = (ctypes.c_int32 * max(1, len(after)))(*[int(a) for a in after])
         rc = self._lib.d3d_schedule_add(self._h, plugin._h, _desc_array(in_descs), len(in_descs),
                                         _desc_array(out_descs), len(out_descs), _pointers(inputs),
-                                        _pointers(outputs), ws_ptr,
-                                        ws_bytes, int(lane), dep, len(after))
+                                        _pointers(outputs), ws_ptr, ws_bytes, int(lane), *self._after(after))
+        return self._appended(rc, (plugin, list(inputs), list(outputs), workspace))
+
+    def add_sum(self, a, b, out, lane=0, after=()):
+        """Appends ``out = a + b`` (float32 / float16 / bfloat16 tensors of one shape)."""
+        rc = self._lib.d3d_schedule_add_sum(self._h, _TORCH_TO_D3D[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(),
+                                            a.numel(), int(lane), *self._after(after))
+        return self._appended(rc, (a, b, out))
+
+    def add_cast(self, a, out, lane=0, after=()):
+        """Appends ``out = a.to(out.dtype)`` (a float32, out float16 / bfloat16)."""
+        rc = self._lib.d3d_schedule_add_cast(self._h, _TORCH_TO_D3D[out.dtype], a.data_ptr(), out.data_ptr(), a.numel(),
+                                             int(lane), *self._after(after))
+        return self._appended(rc, (a, out))
+
+    @staticmethod
+    def _after(after):
+        return (ctypes.c_int32 * max(1, len(after)))(*[int(a) for a in after]), len(after)
+
+    def _appended(self, rc, kept):
         if rc < 0:
             _check(rc)
-        self._keep.append((plugin, list(inputs), list(outputs), workspace))
+        self._keep.append(kept)
         return rc
 
     def __len__(self):

@@ -220,9 +220,15 @@ int32_t d3d_set_option(d3d_plugin* p, int32_t option, int64_t value);
  *   added.  Descriptors and pointer arrays are copied; the operator, the tensors and the workspace must outlive the
  *   schedule's runs, and the operator must be configured as for d3d_enqueue.  Returns the step's index (>= 0) or a
  *   negative status.
+ * d3d_schedule_add_sum / d3d_schedule_add_cast: appends an elementwise step over `count` elements: out = a + b (tensors of
+ *   D3D_FLOAT, D3D_HALF or D3D_BF16; the residual sums of a network), or out = the float tensor a converted to D3D_HALF
+ *   or D3D_BF16.  Lane, waits and result as for d3d_schedule_add.
  * d3d_schedule_run: enqueues all steps; the owned lanes start behind what `stream` holds at the call and `stream`
  *   continues behind all of them, so for the caller the run is stream-ordered work on `stream`.  No host
- *   synchronisation.  Returns the first failing status; steps behind a failed one are not enqueued.  Refused with
+ *   synchronisation.  The first two runs enqueue step by step; when nothing about the operators has changed since
+ *   (options, links, capacities, reserved buffers), the steps are captured into one HIP graph, which the schedule keeps and
+ *   later runs launch - until something changes.  Returns the first failing status; steps behind a failed one are not
+ *   enqueued.  Refused with
  *   D3D_ERR_UNSUPPORTED while `stream` is capturing (capture the operators' own enqueues instead).  One thread at
  *   a time per schedule.
  * d3d_schedule_destroy: waits for the owned lanes, then frees them; the operators stay the caller's. */
@@ -232,6 +238,10 @@ int32_t d3d_schedule_add(d3d_schedule* s, d3d_plugin* plugin, const d3d_tensor_d
                          const d3d_tensor_desc* out_desc, int32_t nb_out, const void* const* inputs,
                          void* const* outputs, void* workspace, size_t workspace_bytes, int32_t lane,
                          const int32_t* after, int32_t nb_after);
+int32_t d3d_schedule_add_sum(d3d_schedule* s, int32_t dtype, const void* a, const void* b, void* out, int64_t count,
+                             int32_t lane, const int32_t* after, int32_t nb_after);
+int32_t d3d_schedule_add_cast(d3d_schedule* s, int32_t dtype, const void* a, void* out, int64_t count, int32_t lane,
+                              const int32_t* after, int32_t nb_after);
 int32_t d3d_schedule_size(const d3d_schedule* s);
 int32_t d3d_schedule_run(d3d_schedule* s, void* stream);
 void d3d_schedule_destroy(d3d_schedule* s);

@@ -165,6 +165,68 @@ def test_schedule_on_one_lane_and_back_to_back_runs(engine):
         assert torch.equal(c, want)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+def test_repeated_passes_become_a_graph_and_follow_changes(engine, dtype):
+    """Passes that repeat on the same buffers turn into a native schedule and then into one HIP graph (residual sums
+    included): every pass equals the step-by-step one bit for bit, with other live counts in the buffers, after an
+    option of an operator changed under the graph, and after the operators served other buffers in between."""
+    from deploy3d_amd import layers, synth
+    from deploy3d_amd.plugin import OPT_INDEX_UNUSED
+    cfg = synth.config5(6000)
+    specs, weights = cfg["layers"], cfg["weights"]
+    n = len(cfg["coords"])
+    caps = layers.plan_capacities(specs, n, layers.measure_output_counts(specs, cfg["coords"], cfg["grid"]))
+    make = lambda: layers.SparseBackbone(specs, weights, caps, dtype=getattr(torch, dtype))  # noqa: E731
+    plain, net = make(), make()
+    x = layers.make_input(cfg["coords"], cfg["feats"], cfg["grid"], dtype=getattr(torch, dtype))
+    other = layers.make_input(cfg["coords"][::-1].copy(), cfg["feats"], cfg["grid"], dtype=getattr(torch, dtype))
+
+    def check(inp, live):
+        inp.num_act.fill_(live)
+        want, got = plain._forward_steps(inp), net.forward(inp)
+        k = int(want.num_act.item())
+        assert k == int(got.num_act.item())
+        assert torch.equal(want.feats, got.feats) and torch.equal(want.coors[:k], got.coors[:k])
+        for key, rb in plain.rulebooks.items():
+            if key != skipped:
+                assert torch.equal(rb.index, net.rulebooks[key].index), key
+
+    skipped = None
+    for live in (n, n // 2, n, n // 3, n, n, 1, n):
+        check(x, live)
+    assert net._plans and next(iter(net._plans.values()))
+    for inp in (other, x, x, other, other, other, other, other, x):
+        check(inp, n)
+    skipped = specs[0]["key"]
+    net.layers[0].idx_plugin.set_option(OPT_INDEX_UNUSED, 1)
+    for live in (n, n // 2, n, n):
+        check(x, live)
+
+
+def test_cast_and_sum_steps(engine):
+    """The elementwise steps of a schedule against torch, at counts around a vector's length and unaligned addresses."""
+    from deploy3d_amd.plugin import Schedule
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        for n, skip in ((1, 0), (7, 0), (8, 1), (4097, 0), (300001, 1)):
+            a = (torch.randn(n + skip, generator=g, device="cuda") * 300).to(dtype)[skip:]
+            b = (torch.randn(n + skip, generator=g, device="cuda") * 300).to(dtype)[skip:]
+            out = torch.empty(n, dtype=dtype, device="cuda")
+            sched = Schedule(lanes=1)
+            first = sched.add_sum(a, b, out)
+            wide = torch.randn(n + skip, generator=g, device="cuda")[skip:]
+            cast = torch.empty(n, dtype=dtype, device="cuda")
+            if dtype != torch.float32:
+                sched.add_cast(wide, cast, after=[first])
+            for _ in range(4):
+                out.zero_()
+                cast.zero_()
+                sched.run()
+                assert torch.equal(out, a + b)
+                if dtype != torch.float32:
+                    assert torch.equal(cast, wide.to(dtype))
+
+
 def test_down_up_chain_with_inverse_convolution(engine):
     """An encoder-decoder wiring through the layer runner: strided down (key d), SubM at the lower resolution, then
     the inverse convolution of key d back onto the input sites, then a SubM that shares the first layer's key.  The
