@@ -100,6 +100,20 @@ def test_repeated_cell_keeps_the_last_row(engine):
     assert np.array_equal(got.cpu().numpy().reshape(1, 4, 1, 4, 4)[b, :, z, y, x], feats[8].numpy())
 
 
+def test_uncleared_table_of_earlier_calls(engine):
+    """The cell -> row table is not cleared between calls: what earlier calls on the same workspace left in it (rows of
+    other cells, rows past the live count, the same cells under other rows) never shows, nor do 40 rows of one cell in
+    whatever order they arrive."""
+    shape = (1, 2, 24, 23)
+    for seed, num_act in ((1, 900), (2, 300), (3, 900), (3, 12), (4, 0), (5, 640)):
+        feats, coords = make_case(seed, num_act, "float16", cap=1000, channels=32, shape=shape)
+        if num_act == 640:
+            coords[100:140] = coords[7]
+        got = _run(feats, coords, num_act, shape)
+        want = oracle.bev_densify(feats.view(torch.int16).numpy(), coords, num_act, shape)
+        assert np.array_equal(got.cpu().view(torch.int16).numpy(), want), (seed, num_act)
+
+
 def test_backbone_tail_shape(engine):
     """The map a CenterPoint-sized backbone hands to its 2-D head: [1, 128*2, 180, 180] fp16 from about 38 000 rows."""
     shape = (1, 2, 180, 180)
