@@ -237,7 +237,7 @@ struct VoxelizeArgs {
   void* workspace;
   size_t workspaceBytes;
 };
-size_t voxelizeWorkspaceBytes(int64_t numPts, int64_t maxNumActOut);
+size_t voxelizeWorkspaceBytes(int64_t numPts, int64_t maxNumActOut, int64_t C);
 int32_t launchVoxelize(const VoxelizeArgs& a, hipStream_t stream);
 
 size_t densifyWorkspaceBytes(int64_t B, int64_t Z, int64_t Y, int64_t X);

@@ -1268,7 +1268,7 @@ struct VoxelizePlugin final : d3d_plugin {
   int32_t configure(const d3d_tensor_desc*, int32_t, const d3d_tensor_desc*, int32_t) override { return D3D_OK; }
   size_t workspaceSize(const d3d_tensor_desc* in, int32_t nbIn) const override {  // simple_mean_trt.cu:273-278
     if (!in || nbIn < 1 || in[0].nb_dims != 2) return 0;
-    return voxelizeWorkspaceBytes(in[0].dims[0], maxNumActOut);
+    return voxelizeWorkspaceBytes(in[0].dims[0], maxNumActOut, in[0].dims[1]);
   }
   int32_t enqueue(const d3d_tensor_desc* inDesc, const d3d_tensor_desc* outDesc, const void* const* inputs,
                   void* const* outputs, void* workspace, size_t workspaceBytes, hipStream_t stream) override {

@@ -16,6 +16,12 @@
 // appearance, the same on every run, and truncation keeps the voxels that
 // appear first.  Sums use fp32 atomic adds like the reference's, so the means
 // can differ in the last bits from run to run; coordinates and counts cannot.
+//
+// Three forms, chosen by size (launchVoxelize): a few thousand points fit one workgroup's LDS (one launch); otherwise
+// the table's entries carry the sums (three launches: clear, insert, emit); very many points or channels keep a table
+// of bare keys and sum in the output rows (five launches).
+#include <atomic>
+
 #include "common.h"
 
 namespace d3d {
@@ -41,6 +47,385 @@ struct VxGeom {
   int B, Z, Y, X;
 };
 
+// Features of a point: CT channels in registers (0 = any number, left in memory).  All loads are requested before the
+// first value is looked at - a chain of loads that each wait for the check of the one before cost a small call 10 us.
+template <int CT> struct VxPoint {
+  float v[CT ? CT : 3];
+  const float* p;
+  bool finite;
+  __device__ __forceinline__ VxPoint(const float* f, int C) : p(f) {
+    uint32_t worst = 0;   // largest exponent field
+#pragma unroll
+    for (int c = 0; c < (CT ? CT : 3); ++c) v[c] = f[c];
+    if constexpr (CT == 0)
+      for (int c = 3; c < C; ++c) worst = max(worst, __float_as_uint(f[c]) & 0x7F800000u);
+#pragma unroll
+    for (int c = 0; c < (CT ? CT : 3); ++c) worst = max(worst, __float_as_uint(v[c]) & 0x7F800000u);
+    finite = worst != 0x7F800000u;
+  }
+  __device__ __forceinline__ float operator[](int c) const { return CT ? v[c] : p[c]; }
+};
+
+// int((v - lo) / size) of IEEE division, usually without the division: the product with the reciprocal is off by a few
+// units in the last place, which cannot change the integer part unless the product is that close to an integer.
+__device__ __forceinline__ int vxAxis(float v, float lo, float size, float rcp) {
+  const float d = v - lo, q = d * rcp;
+  const float away = fabsf(q - rintf(q));
+  // 2^-21 |q| is four times the error bound (2 ulp); small quotients, overflows and odd sizes take the division
+  return (away > fabsf(q) * 4.76837158e-7f && fabsf(q) > 1e-3f && fabsf(q) < 1e6f && rcp < 1e30f && rcp > 1e-30f)
+             ? static_cast<int>(q)
+             : static_cast<int>(d / size);
+}
+
+struct VxConfig {
+  float lo[3], size[3], rcp[3];
+  __device__ __forceinline__ explicit VxConfig(const float* config) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      lo[q] = config[q];
+      size[q] = config[3 + q];
+      rcp[q] = 1.f / size[q];
+    }
+  }
+};
+
+// The cell of a point (simple_mean_trt.cu:36-52); false when a feature is not finite, the point is skipped or it lies
+// outside the grid.
+template <int CT>
+__device__ __forceinline__ bool vxCell(const VxPoint<CT>& f, int b, const VxConfig& v, const VxGeom& g, uint32_t* key) {
+  if (!f.finite || b < 0 || b >= g.B) return false;
+  const int x = vxAxis(f.v[0], v.lo[0], v.size[0], v.rcp[0]);
+  const int y = vxAxis(f.v[1], v.lo[1], v.size[1], v.rcp[1]);
+  const int z = vxAxis(f.v[2], v.lo[2], v.size[2], v.rcp[2]);
+  if (!(x >= 0 && x < g.X && y >= 0 && y < g.Y && z >= 0 && z < g.Z)) return false;
+  *key = ((static_cast<uint32_t>(b) * g.Z + z) * g.Y + y) * g.X + x;
+  return true;
+}
+
+// (b, z, y, x) of a cell (refnd.h:56-64)
+__device__ __forceinline__ int4 vxCoord(uint32_t key, const VxGeom& g) {
+  const uint32_t x = key % g.X;
+  key /= g.X;
+  const uint32_t y = key % g.Y;
+  key /= g.Y;
+  const uint32_t z = key % g.Z;
+  return make_int4(static_cast<int>(key / g.Z), static_cast<int>(z), static_cast<int>(y), static_cast<int>(x));
+}
+
+// ---------------------------------------------------------------------------
+// A few thousand points: table, sums and counts in the LDS of one workgroup.  Such a call is launch latency, on the
+// host (3 us per launch) and on the device: at 3 001 points one launch of 10.8 us instead of five of 17.  Bound by one
+// CU's instruction rate (16 wavefronts, about 22 000 cycles).  Workgroups past the first zero the output rows that no
+// point can reach.  Up to 4096 points: 13 us a call there, 18 with the three launches below; four points per thread
+// are also what the registers of 16 wavefronts hold.
+// ---------------------------------------------------------------------------
+constexpr int kVxSmallThreads = 1024;
+constexpr int kVxSmallItems = 4;
+
+template <int CT>
+__global__ void __launch_bounds__(kVxSmallThreads)
+vxSmall(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, const float* __restrict__ config, int32_t n,
+        int channels, VxGeom g, uint32_t mask, int32_t maxNumActOut, float* __restrict__ outFeats, int32_t* __restrict__ outCoors,
+        int32_t* __restrict__ numActOut) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char vxSmem[];
+  const int C = CT ? CT : channels;
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    const int64_t total = static_cast<int64_t>(maxNumActOut) * C;
+    for (int64_t e = static_cast<int64_t>(n) * C + static_cast<int64_t>(blockIdx.x - 1) * kVxSmallThreads + tid; e < total;
+         e += static_cast<int64_t>(gridDim.x - 1) * kVxSmallThreads)
+      outFeats[e] = 0.f;
+    return;
+  }
+  unsigned long long* table = reinterpret_cast<unsigned long long*>(vxSmem);  // [mask + 1] key << 32 | lowest point, then id
+  // [C, n]: a channel's sums of neighbouring voxels in neighbouring banks.  A voxel's representative stores its own
+  // features and the other points add to them: LDS float atomics run at about 3 lanes per clock, and with every point
+  // adding they were half of the kernel's time.
+  float* sums = reinterpret_cast<float*>(table + mask + 1);
+  uint32_t* counts = reinterpret_cast<uint32_t*>(sums + n * C);               // [n]
+  __shared__ uint32_t waveReps[kVxSmallItems][kVxSmallThreads / 64];
+  uint32_t key[kVxSmallItems], slot[kVxSmallItems];
+  // point loads are on their way while the LDS is cleared
+  float pts[kVxSmallItems][CT ? CT : 1];
+  int batch[kVxSmallItems];
+  if constexpr (CT != 0) {
+#pragma unroll
+    for (int k = 0; k < kVxSmallItems; ++k) {
+      const int i = min(k * kVxSmallThreads + tid, n - 1);   // (no branch around a load: all of them in flight together)
+      batch[k] = batchIdx[i];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) pts[k][c] = feats[static_cast<size_t>(i) * CT + c];
+    }
+  }
+  for (uint32_t e = tid; e < (mask + 1) / 2; e += kVxSmallThreads) reinterpret_cast<uint4*>(table)[e] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  const VxConfig cfg(config);
+#pragma unroll
+  for (int k = 0; k < kVxSmallItems; ++k) {
+    const int i = k * kVxSmallThreads + tid;
+    slot[k] = kVxNone;
+    if constexpr (CT != 0) {
+      const VxPoint<CT> point(pts[k], CT);
+      if (vxCell(point, i < n ? batch[k] : -1, cfg, g, &key[k])) slot[k] = 0u;
+    } else if (i < n) {
+      const VxPoint<0> point(feats + static_cast<size_t>(i) * C, C);
+      if (vxCell(point, batchIdx[i], cfg, g, &key[k])) slot[k] = 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kVxSmallItems; ++k) {
+    if (slot[k] == kVxNone) continue;
+    const unsigned long long mine = (static_cast<unsigned long long>(key[k]) << 32) | static_cast<uint32_t>(k * kVxSmallThreads + tid);
+    uint32_t s = vxMix(key[k]) & mask;
+    for (uint32_t tries = 0; tries <= mask; ++tries) {
+      const unsigned long long old = atomicCAS(&table[s], kVxEmpty, mine);
+      if (old == kVxEmpty) break;
+      if (static_cast<uint32_t>(old >> 32) == key[k]) {
+        if (old > mine) atomicMin(&table[s], mine);
+        break;
+      }
+      s = (s + 1) & mask;
+    }
+    slot[k] = s;
+  }
+  __syncthreads();
+  // voxel ids: representatives counted in point order
+  const int lane = tid & 63, wave = tid >> 6;
+  uint32_t below[kVxSmallItems];
+  bool rep[kVxSmallItems];
+#pragma unroll
+  for (int k = 0; k < kVxSmallItems; ++k) {
+    rep[k] = slot[k] != kVxNone && static_cast<uint32_t>(table[slot[k]]) == static_cast<uint32_t>(k * kVxSmallThreads + tid);
+    const unsigned long long m = __ballot(rep[k]);
+    below[k] = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+    if (lane == 0) waveReps[k][wave] = static_cast<uint32_t>(__popcll(m));
+  }
+  __syncthreads();
+  uint32_t total = 0;
+#pragma unroll
+  for (int k = 0; k < kVxSmallItems; ++k) {
+    uint32_t id = total + below[k];
+#pragma unroll
+    for (int w = 0; w < kVxSmallThreads / 64; ++w) {
+      if (w < wave) id += waveReps[k][w];
+      total += waveReps[k][w];
+    }
+    if (rep[k]) {
+      reinterpret_cast<uint32_t*>(&table[slot[k]])[0] = id;
+      if (id < static_cast<uint32_t>(maxNumActOut)) {
+        reinterpret_cast<int4*>(outCoors)[id] = vxCoord(key[k], g);
+        counts[id] = 1u;
+        const float* f = feats + static_cast<size_t>(k * kVxSmallThreads + tid) * C;
+        for (int c = 0; c < C; ++c) sums[c * n + id] = CT ? pts[k][c] : f[c];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kVxSmallItems; ++k) {
+    if (slot[k] == kVxNone || rep[k]) continue;
+    const uint32_t id = static_cast<uint32_t>(table[slot[k]]);
+    if (id >= static_cast<uint32_t>(maxNumActOut)) continue;
+    if constexpr (CT != 0) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) unsafeAtomicAdd(sums + c * n + id, pts[k][c]);
+    } else {
+      const float* f = feats + static_cast<size_t>(k * kVxSmallThreads + tid) * C;
+      for (int c = 0; c < C; ++c) unsafeAtomicAdd(sums + c * n + id, f[c]);
+    }
+    atomicAdd(counts + id, 1u);
+  }
+  __syncthreads();
+  const int rows = static_cast<int>(total < static_cast<uint32_t>(maxNumActOut) ? total : static_cast<uint32_t>(maxNumActOut));
+  const int lastRow = n < maxNumActOut ? n : maxNumActOut;
+  for (int r = tid; r < lastRow; r += kVxSmallThreads) {
+    const bool live = r < rows;
+    const float points = live ? static_cast<float>(counts[r]) : 1.f;
+    if constexpr (CT == 4) {
+      float mean[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) mean[c] = live ? sums[c * n + r] / points : 0.f;
+      __builtin_memcpy(outFeats + r * 4, mean, 16);
+    } else {
+      for (int c = 0; c < C; ++c) outFeats[r * C + c] = live ? sums[c * n + r] / points : 0.f;
+    }
+  }
+  if (tid == 0) *numActOut = rows;
+}
+
+// ---------------------------------------------------------------------------
+// The usual form: a table entry holds key and lowest point, the point that claimed it, and count and feature sums of
+// the others - one cache line per voxel for everything:
+//   { u64 key << 32 | lowest point; u32 claiming point; u32 further points; float sums[C]; pad to 16 bytes }
+// The claiming point's own features are not added here (most voxels of a scan hold one or two points, so most points
+// then cost one compare-and-swap and no other atomic): the emitting pass reads them where they are.
+// 200 000 points: 42.6 us of kernels in five launches before, 34 in three (clear 8, insert 15, emit 10), bound by the
+// random compare-and-swaps; up to 50 000 points the call is bound by its three launches on the host (18 us).
+// ---------------------------------------------------------------------------
+constexpr int kVxMaxWide = 12;  // channels an entry carries
+
+__host__ __device__ constexpr int vxEntryBytes(int C) { return (16 + 4 * C + 15) / 16 * 16; }
+
+// Entries empty, output rows zero (simple_mean_trt.cu:139-143), chunk states zero.
+template <int PER>
+__global__ void __launch_bounds__(kVxThreads)
+vxClearWide(uint4* table, uint32_t pieces, float* outFeats, int64_t nFeats, unsigned long long* states,
+            uint32_t nStates) {
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (uint32_t i = static_cast<uint32_t>(tid); i < pieces; i += static_cast<uint32_t>(stride))
+    table[i] = i % PER == 0 ? make_uint4(~0u, ~0u, 0u, 0u) : make_uint4(0u, 0u, 0u, 0u);
+  for (int64_t i = tid; i < nFeats; i += stride) outFeats[i] = 0.f;
+  for (int64_t i = tid; i < nStates; i += stride) states[i] = 0ull;
+}
+
+// pointSlot[i] = entry of point i when it may be its voxel's lowest point, else none.
+template <int CT>
+__global__ void __launch_bounds__(kVxThreads)
+vxInsertWide(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, const float* __restrict__ config, int32_t n,
+             int channels, VxGeom g, unsigned char* table, uint32_t slots, uint32_t* __restrict__ pointSlot) {
+  const int C = CT ? CT : channels;
+  const int32_t i = blockIdx.x * kVxThreads + threadIdx.x;
+  if (i >= n) return;
+  const VxPoint<CT> f(feats + static_cast<size_t>(i) * C, C);
+  const VxConfig cfg(config);
+  uint32_t key, slot = kVxNone;
+  if (vxCell(f, batchIdx[i], cfg, g, &key)) {
+    const unsigned long long mine = (static_cast<unsigned long long>(key) << 32) | static_cast<uint32_t>(i);
+    // the hash spread over the table by its high bits: any number of slots will do
+    uint32_t s = static_cast<uint32_t>((static_cast<unsigned long long>(vxMix(key)) * slots) >> 32);
+    for (uint32_t tries = 0; tries < slots; ++tries) {
+      unsigned char* entry = table + static_cast<size_t>(s) * vxEntryBytes(C);
+      auto* head = reinterpret_cast<unsigned long long*>(entry);
+      const unsigned long long old = atomicCAS(head, kVxEmpty, mine);
+      if (old == kVxEmpty) {
+        reinterpret_cast<uint32_t*>(entry)[2] = static_cast<uint32_t>(i);
+        slot = s;
+        break;
+      }
+      if (static_cast<uint32_t>(old >> 32) == key) {
+        if (old > mine) {
+          atomicMin(head, mine);
+          slot = s;
+        }
+        float* sums = reinterpret_cast<float*>(entry + 16);
+        for (int c = 0; c < C; ++c) unsafeAtomicAdd(sums + c, f[c]);
+        atomicAdd(reinterpret_cast<uint32_t*>(entry) + 3, 1u);
+        break;
+      }
+      s = s + 1 == slots ? 0u : s + 1;
+    }
+  }
+  pointSlot[i] = slot;
+}
+
+constexpr unsigned long long kVxAggregate = 1ull << 32, kVxPrefix = 2ull << 32;
+constexpr int kVxSpins = 1 << 16;
+
+// One chunk of 1024 points per workgroup: representatives are ranked in point order, the workgroup publishes its count,
+// reads how many the chunks before it have (64 of their states at a time, waiting for those that are not there yet),
+// and writes mean and coordinate of its own voxels.  A state is one 64-bit word, flag and value together, so relaxed
+// device-scope accesses are enough.  The wait cannot deadlock - a chunk waits for lower ones only, and those were
+// dispatched before it - and it is bounded all the same: after kVxSpins looks the wavefront counts the earlier chunks'
+// representatives itself.
+template <int CT>
+__global__ void __launch_bounds__(kVxThreads)
+vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, const unsigned char* __restrict__ table,
+           const uint32_t* __restrict__ pointSlot, unsigned long long* states, int32_t maxNumActOut, float* __restrict__ outFeats,
+           int32_t* __restrict__ outCoors, int32_t* __restrict__ numActOut) {
+  const int C = CT ? CT : channels;
+  const size_t entryBytes = vxEntryBytes(C);
+  __shared__ uint32_t waveReps[kVxItems][kVxThreads / 64];
+  __shared__ uint32_t baseShared;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t chunk = blockIdx.x;
+  uint4 head[kVxItems];
+  bool rep[kVxItems];
+  uint32_t slot[kVxItems], below[kVxItems];
+#pragma unroll
+  for (int k = 0; k < kVxItems; ++k) {
+    const int64_t i = static_cast<int64_t>(chunk) * kVxChunk + k * kVxThreads + tid;
+    slot[k] = i < n ? pointSlot[i] : kVxNone;
+  }
+#pragma unroll
+  for (int k = 0; k < kVxItems; ++k)
+    head[k] = slot[k] != kVxNone ? *reinterpret_cast<const uint4*>(table + slot[k] * entryBytes) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int k = 0; k < kVxItems; ++k) {
+    rep[k] = slot[k] != kVxNone && head[k].x == chunk * kVxChunk + k * kVxThreads + tid;
+    const unsigned long long m = __ballot(rep[k]);
+    below[k] = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+    if (lane == 0) waveReps[k][wave] = static_cast<uint32_t>(__popcll(m));
+  }
+  __syncthreads();
+  uint32_t total = 0, rank[kVxItems];
+#pragma unroll
+  for (int k = 0; k < kVxItems; ++k) {
+    rank[k] = total + below[k];
+#pragma unroll
+    for (int w = 0; w < kVxThreads / 64; ++w) {
+      if (w < wave) rank[k] += waveReps[k][w];
+      total += waveReps[k][w];
+    }
+  }
+  if (wave == 0) {
+    if (lane == 0)
+      __hip_atomic_store(&states[chunk], (chunk ? kVxAggregate : kVxPrefix) | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t base = 0;
+    int spins = 0;
+    for (int64_t top = static_cast<int64_t>(chunk) - 1; top >= 0;) {
+      const int64_t p = top - lane;
+      const unsigned long long st =
+          p >= 0 ? __hip_atomic_load(&states[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kVxPrefix;
+      const unsigned long long prefixes = __ballot((st >> 32) == 2u), missing = __ballot((st >> 32) == 0u);
+      const int last = prefixes ? __builtin_ctzll(prefixes) : 63;   // lanes up to here are needed
+      if (missing & (last == 63 ? ~0ull : (2ull << last) - 1ull)) {
+        if (++spins < kVxSpins) {
+          __builtin_amdgcn_s_sleep(1);
+          continue;
+        }
+        base = 0;
+        for (int64_t q = lane; q < static_cast<int64_t>(chunk) * kVxChunk; q += 64) {
+          const uint32_t qs = pointSlot[q];
+          if (qs != kVxNone && *reinterpret_cast<const uint32_t*>(table + qs * entryBytes) == static_cast<uint32_t>(q)) ++base;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) base += __shfl_xor(base, off, 64);
+        break;
+      }
+      uint32_t v = lane <= last ? static_cast<uint32_t>(st) : 0u;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      base += v;
+      if (prefixes) break;
+      top -= 64;
+    }
+    if (lane == 0) {
+      if (chunk)
+        __hip_atomic_store(&states[chunk], kVxPrefix | (base + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      baseShared = base;
+      if (chunk == gridDim.x - 1)
+        *numActOut = static_cast<int32_t>(base + total < static_cast<uint32_t>(maxNumActOut) ? base + total : maxNumActOut);
+    }
+  }
+  __syncthreads();
+  const uint32_t base = baseShared;
+#pragma unroll
+  for (int k = 0; k < kVxItems; ++k) {
+    const uint32_t id = base + rank[k];
+    if (!rep[k] || id >= static_cast<uint32_t>(maxNumActOut)) continue;
+    const float* sums = reinterpret_cast<const float*>(table + slot[k] * entryBytes + 16);
+    const float* f = feats + static_cast<size_t>(head[k].z) * C;
+    float* row = outFeats + static_cast<size_t>(id) * C;
+    const float points = static_cast<float>(head[k].w + 1u);
+    for (int c = 0; c < C; ++c) row[c] = (f[c] + sums[c]) / points;
+    reinterpret_cast<int4*>(outCoors)[id] = vxCoord(head[k].y, g);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Very many points or channels: a table of keys, sums in the output rows.
+// ---------------------------------------------------------------------------
 // table = empty, outFeats = 0 (simple_mean_trt.cu:139-143), counts = 0, ticket = 0
 __global__ void __launch_bounds__(kVxThreads)
 vxReset(unsigned long long* table, int64_t slots, float* outFeats, int64_t nFeats, uint32_t* counts, int64_t nCounts,
@@ -59,32 +444,23 @@ vxInsert(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, 
          int C, VxGeom g, unsigned long long* table, uint32_t mask, uint32_t* __restrict__ pointSlot) {
   const int32_t i = blockIdx.x * kVxThreads + threadIdx.x;
   if (i >= n) return;
-  const float* f = feats + static_cast<size_t>(i) * C;
-  bool ok = true;
-  for (int c = 0; c < C; ++c) ok = ok && isfinite(f[c]);
-  const int b = batchIdx[i];
-  uint32_t slot = kVxNone;
-  if (ok && b >= 0 && b < g.B) {
-    const int x = static_cast<int>((f[0] - config[0]) / config[3]);
-    const int y = static_cast<int>((f[1] - config[1]) / config[4]);
-    const int z = static_cast<int>((f[2] - config[2]) / config[5]);
-    if (x >= 0 && x < g.X && y >= 0 && y < g.Y && z >= 0 && z < g.Z) {
-      const uint32_t key = ((static_cast<uint32_t>(b) * g.Z + z) * g.Y + y) * g.X + x;
-      const unsigned long long mine = (static_cast<unsigned long long>(key) << 32) | static_cast<uint32_t>(i);
-      uint32_t s = vxMix(key) & mask;
-      for (uint32_t tries = 0; tries <= mask; ++tries) {  // at most half the slots are ever taken
-        const unsigned long long old = atomicCAS(&table[s], kVxEmpty, mine);
-        if (old == kVxEmpty) {
-          slot = s;
-          break;
-        }
-        if (static_cast<uint32_t>(old >> 32) == key) {
-          if (old > mine) atomicMin(&table[s], mine);
-          slot = s;
-          break;
-        }
-        s = (s + 1) & mask;
+  const VxConfig cfg(config);
+  uint32_t key, slot = kVxNone;
+  if (vxCell(VxPoint<0>(feats + static_cast<size_t>(i) * C, C), batchIdx[i], cfg, g, &key)) {
+    const unsigned long long mine = (static_cast<unsigned long long>(key) << 32) | static_cast<uint32_t>(i);
+    uint32_t s = vxMix(key) & mask;
+    for (uint32_t tries = 0; tries <= mask; ++tries) {  // at most half the slots are ever taken
+      const unsigned long long old = atomicCAS(&table[s], kVxEmpty, mine);
+      if (old == kVxEmpty) {
+        slot = s;
+        break;
       }
+      if (static_cast<uint32_t>(old >> 32) == key) {
+        if (old > mine) atomicMin(&table[s], mine);
+        slot = s;
+        break;
+      }
+      s = (s + 1) & mask;
     }
   }
   pointSlot[i] = slot;
@@ -188,17 +564,8 @@ vxAccumulate(const float* __restrict__ feats, int32_t n, int C, VxGeom g, const 
   float* row = outFeats + static_cast<size_t>(id) * C;
   for (int c = 0; c < C; ++c) unsafeAtomicAdd(row + c, f[c]);
   atomicAdd(counts + id, 1u);
-  if (rep == static_cast<uint32_t>(i)) {
-    uint32_t off = static_cast<uint32_t>(entry >> 32);
-    const uint32_t x = off % g.X;
-    off /= g.X;
-    const uint32_t y = off % g.Y;
-    off /= g.Y;
-    const uint32_t z = off % g.Z;
-    off /= g.Z;
-    reinterpret_cast<int4*>(outCoors)[id] = make_int4(static_cast<int>(off), static_cast<int>(z), static_cast<int>(y),
-                                                      static_cast<int>(x));
-  }
+  if (rep == static_cast<uint32_t>(i))
+    reinterpret_cast<int4*>(outCoors)[id] = vxCoord(static_cast<uint32_t>(entry >> 32), g);
 }
 
 // kernel::meanFeats (simple_mean_trt.cu:93-101)
@@ -219,15 +586,31 @@ uint32_t pow2AtLeast(uint64_t v) {
 size_t alignUp256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 struct VxPlan {
+  bool wide;              // entries carry the sums
   uint32_t slots, nChunks;
   size_t table, pointSlot, local, chunkBase, counts, ticket, total;
 };
 
-VxPlan planVoxelize(int64_t numPts, int64_t maxNumActOut) {
+// Entries with sums are cleared and read whole (2 slots per point: 64 bytes per point at 4 channels), so the form is kept
+// to what the fixed scratch array of d3d_enqueue_static holds: about a million points at 4 channels.
+VxPlan planVoxelize(int64_t numPts, int64_t maxNumActOut, int64_t C) {
   VxPlan p{};
   const int64_t n = numPts < 1 ? 1 : numPts;
-  p.slots = pow2AtLeast(static_cast<uint64_t>(n) * 2);  // the reference's hashSpace = 2 (simple_mean_trt.cu:110)
   p.nChunks = static_cast<uint32_t>((n + kVxChunk - 1) / kVxChunk);
+  if (C <= kVxMaxWide && n < (1 << 30)) {
+    p.wide = true;
+    p.slots = static_cast<uint32_t>(2 * n < 1024 ? 1024 : 2 * n);  // the reference's hashSpace = 2 (simple_mean_trt.cu:110)
+    size_t off = alignUp256(static_cast<size_t>(p.slots) * vxEntryBytes(static_cast<int>(C)));
+    p.pointSlot = off;
+    off = alignUp256(off + static_cast<size_t>(n) * 4);
+    p.chunkBase = off;  // chunk states, u64
+    off = alignUp256(off + static_cast<size_t>(p.nChunks) * 8);
+    p.total = off;
+    if (p.total <= kStaticScratchBytes) return p;
+    p = VxPlan{};
+    p.nChunks = static_cast<uint32_t>((n + kVxChunk - 1) / kVxChunk);
+  }
+  p.slots = pow2AtLeast(static_cast<uint64_t>(n) * 2);
   size_t off = 0;
   p.table = off;
   off = alignUp256(off + static_cast<size_t>(p.slots) * 8);
@@ -245,12 +628,62 @@ VxPlan planVoxelize(int64_t numPts, int64_t maxNumActOut) {
   return p;
 }
 
+// One workgroup's form: at most kVxSmallItems points per thread, table and sums within a CU's LDS.
+bool smallFits(int64_t numPts, int64_t C, uint32_t* slots, size_t* lds) {
+  if (numPts < 1 || numPts > kVxSmallThreads * kVxSmallItems) return false;
+  *slots = pow2AtLeast(static_cast<uint64_t>(numPts) * 2);
+  *lds = static_cast<size_t>(*slots) * 8 + static_cast<size_t>(numPts) * (C + 1) * 4;
+  return *lds <= 150 * 1024;
+}
+
+template <int CT>
+int32_t launchSmall(const VoxelizeArgs& a, const VxGeom& g, uint32_t slots, size_t lds, hipStream_t stream) {
+  static std::atomic<bool> granted{false};
+  if (lds > 64 * 1024 && !granted.load(std::memory_order_acquire)) {
+    D3D_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&vxSmall<CT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      150 * 1024));
+    granted.store(true, std::memory_order_release);
+  }
+  const int64_t beyond = (static_cast<int64_t>(a.maxNumActOut) - a.numPts) * a.C;
+  int64_t zeroing = beyond > 0 ? (beyond + kVxSmallThreads * 4 - 1) / (kVxSmallThreads * 4) : 0;
+  if (zeroing > 512) zeroing = 512;
+  hipLaunchKernelGGL(vxSmall<CT>, dim3(static_cast<unsigned>(1 + zeroing)), dim3(kVxSmallThreads), lds, stream, a.feats, a.batchIdx,
+                     a.config, static_cast<int32_t>(a.numPts), a.C, g, slots - 1, a.maxNumActOut, a.outFeats, a.outCoors,
+                     a.numActOut);
+  D3D_HIP_CHECK(hipGetLastError());
+  return D3D_OK;
+}
+
+template <int CT>
+void launchWide(const VoxelizeArgs& a, const VxPlan& p, const VxGeom& g, char* ws, hipStream_t stream) {
+  auto* table = reinterpret_cast<unsigned char*>(ws);
+  auto* pointSlot = reinterpret_cast<uint32_t*>(ws + p.pointSlot);
+  auto* states = reinterpret_cast<unsigned long long*>(ws + p.chunkBase);
+  const int perEntry = vxEntryBytes(a.C) / 16;
+  const int64_t pieces = static_cast<int64_t>(p.slots) * perEntry, nFeats = static_cast<int64_t>(a.maxNumActOut) * a.C;
+  int64_t blocks = (pieces + kVxThreads * 4 - 1) / (kVxThreads * 4);
+  if (blocks > 4096) blocks = 4096;
+#define D3D_VX_CLEAR(PER)                                                                                                       \
+  hipLaunchKernelGGL(vxClearWide<PER>, dim3(static_cast<unsigned>(blocks)), dim3(kVxThreads), 0, stream,                        \
+                     reinterpret_cast<uint4*>(table), static_cast<uint32_t>(pieces), a.outFeats, nFeats, states, p.nChunks)
+  if (perEntry == 2) D3D_VX_CLEAR(2);
+  else if (perEntry == 3) D3D_VX_CLEAR(3);
+  else D3D_VX_CLEAR(4);
+#undef D3D_VX_CLEAR
+  hipLaunchKernelGGL(vxInsertWide<CT>, dim3(static_cast<unsigned>((a.numPts + kVxThreads - 1) / kVxThreads)), dim3(kVxThreads), 0,
+                     stream, a.feats, a.batchIdx, a.config, static_cast<int32_t>(a.numPts), a.C, g, table, p.slots, pointSlot);
+  hipLaunchKernelGGL(vxEmitWide<CT>, dim3(p.nChunks), dim3(kVxThreads), 0, stream, a.feats, static_cast<int32_t>(a.numPts), a.C, g,
+                     table, pointSlot, states, a.maxNumActOut, a.outFeats, a.outCoors, a.numActOut);
+}
+
 }  // namespace
 
-size_t voxelizeWorkspaceBytes(int64_t numPts, int64_t maxNumActOut) { return planVoxelize(numPts, maxNumActOut).total; }
+size_t voxelizeWorkspaceBytes(int64_t numPts, int64_t maxNumActOut, int64_t C) {
+  return planVoxelize(numPts, maxNumActOut, C).total;
+}
 
 int32_t launchVoxelize(const VoxelizeArgs& a, hipStream_t stream) {
-  const VxPlan p = planVoxelize(a.numPts, a.maxNumActOut);
+  const VxPlan p = planVoxelize(a.numPts, a.maxNumActOut, a.C);
   if (!a.workspace || a.workspaceBytes < p.total) {
     setError("SimpleMeanEncoder: workspace of %zu bytes, %zu needed", a.workspaceBytes, p.total);
     return D3D_ERR_WORKSPACE;
@@ -265,14 +698,42 @@ int32_t launchVoxelize(const VoxelizeArgs& a, hipStream_t stream) {
     return D3D_ERR_UNSUPPORTED;
   }
   char* ws = static_cast<char*>(a.workspace);
+  const VxGeom g{a.B, a.Z, a.Y, a.X};
+  if (a.numPts > 0 && a.maxNumActOut > 0 && cells > 0) {
+    uint32_t slots = 0;
+    size_t lds = 0;
+    if (smallFits(a.numPts, a.C, &slots, &lds)) {
+      switch (a.C) {
+        case 3: return launchSmall<3>(a, g, slots, lds, stream);
+        case 4: return launchSmall<4>(a, g, slots, lds, stream);
+        case 5: return launchSmall<5>(a, g, slots, lds, stream);
+        default: return launchSmall<0>(a, g, slots, lds, stream);
+      }
+    }
+    if (p.wide) {
+      switch (a.C) {
+        case 3: launchWide<3>(a, p, g, ws, stream); break;
+        case 4: launchWide<4>(a, p, g, ws, stream); break;
+        case 5: launchWide<5>(a, p, g, ws, stream); break;
+        default: launchWide<0>(a, p, g, ws, stream);
+      }
+      D3D_HIP_CHECK(hipGetLastError());
+      return D3D_OK;
+    }
+  }
   auto* table = reinterpret_cast<unsigned long long*>(ws + p.table);
   auto* pointSlot = reinterpret_cast<uint32_t*>(ws + p.pointSlot);
   auto* local = reinterpret_cast<uint32_t*>(ws + p.local);
   auto* chunkBase = reinterpret_cast<uint32_t*>(ws + p.chunkBase);
   auto* counts = reinterpret_cast<uint32_t*>(ws + p.counts);
   auto* ticket = reinterpret_cast<uint32_t*>(ws + p.ticket);
-  const VxGeom g{a.B, a.Z, a.Y, a.X};
   const int64_t nFeats = static_cast<int64_t>(a.maxNumActOut) * a.C;
+  if (p.wide) {  // nothing to insert: only the outputs' zeros (the plan has no table of bare keys)
+    hipLaunchKernelGGL(vxReset, dim3(static_cast<unsigned>(nFeats < 1 ? 1 : (nFeats / kVxThreads > 4095 ? 4096 : nFeats / kVxThreads + 1))),
+                       dim3(kVxThreads), 0, stream, nullptr, int64_t(0), a.outFeats, nFeats, nullptr, int64_t(0), a.numActOut);
+    D3D_HIP_CHECK(hipGetLastError());
+    return D3D_OK;
+  }
   const int64_t resetItems = static_cast<int64_t>(p.slots) + nFeats;
   int64_t resetBlocks = (resetItems + kVxThreads - 1) / kVxThreads;
   if (resetBlocks > 4096) resetBlocks = 4096;

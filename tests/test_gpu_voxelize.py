@@ -119,6 +119,31 @@ def test_crowded_voxels_and_channel_counts(engine, channels):
     np.testing.assert_allclose(got_f[:128][go], ref_f[:128][ro], rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("n,channels,max_out", [(1, 3, 4), (63, 4, 5000), (1024, 5, 300), (1025, 4, 1025), (4096, 4, 4096),
+                                                (4096, 9, 9000), (4097, 4, 100000), (5000, 6, 700), (70001, 12, 70001),
+                                                (66000, 13, 30000)])
+def test_sizes_around_the_forms(engine, n, channels, max_out):
+    """One workgroup (up to 4096 points), entries with sums (up to 12 channels) and bare keys, around their limits and
+    with capacities below and above the voxel count: rows in order of first appearance, means, zero tail - three times
+    over, the last two on a workspace that holds the calls before."""
+    rng = np.random.default_rng(n + channels)
+    pts = rng.uniform(-0.5, 8.5, (n, channels)).astype(np.float32)
+    pts[:, 2] *= max(1.0, n / 2000)
+    batch = rng.integers(-1, 3, n).astype(np.int32)
+    cfg = np.array([0, 0, 0, 0.5, 0.5, 0.5], np.float32)
+    shape = (2, int(18 * max(1.0, n / 2000)), 17, 16)
+    want = _first_appearance(pts, batch, cfg, shape)
+    ref_f, ref_c, ref_n = oracle.simple_mean(pts, batch, cfg, shape, n)
+    lut = {tuple(r): i for i, r in enumerate(ref_c[:ref_n].tolist())}
+    for _ in range(3):
+        got_f, got_c, got_n = _run(pts, batch, cfg, shape, max_out)
+        assert got_n == min(max_out, len(want))
+        assert np.array_equal(got_c[:got_n], want[:got_n])
+        rows = np.array([lut[tuple(r)] for r in got_c[:got_n].tolist()], dtype=np.int64)
+        np.testing.assert_allclose(got_f[:got_n], ref_f[rows], rtol=2e-5, atol=2e-5)
+        assert not got_f[got_n:].any()
+
+
 def test_wrong_dtype_is_unsupported(engine):
     from deploy3d_amd import EngineError, Plugin, TensorDesc
     from deploy3d_amd.simple_mean import simple_mean_blob
