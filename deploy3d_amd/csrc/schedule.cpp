@@ -92,16 +92,33 @@ bool captureGraph(d3d_schedule* s) {
   hipStream_t q = nullptr;
   if (hipGraphCreate(&graph, 0) != hipSuccess) return false;
   bool ok = hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
-  std::vector<std::vector<hipGraphNode_t>> tail(s->steps.size());
-  for (size_t i = 0; ok && i < s->steps.size(); ++i) {
+  const size_t count = s->steps.size();
+  std::vector<std::vector<hipGraphNode_t>> tail(count);
+  // What each step comes after, directly or not.  A dependency that another one implies gets no edge: every edge
+  // between branches is a wait packet in front of the kernel, 6 us even when the other branch is long done (a
+  // VoxelNet backbone of 9 000 voxels: 374 us with the implied edges, 324 without; 120 000 voxels: 708 and 700).
+  std::vector<std::vector<bool>> behindOf(count, std::vector<bool>(count));
+  for (size_t i = 0; ok && i < count; ++i) {
     const d3d_schedule::Step& st = s->steps[i];
+    std::vector<int> direct(st.after);
+    if (st.before >= 0) direct.insert(direct.begin(), st.before);
+    for (int d : direct) {
+      behindOf[i][static_cast<size_t>(d)] = true;
+      for (size_t k = 0; k < count; ++k)
+        if (behindOf[static_cast<size_t>(d)][k]) behindOf[i][k] = true;
+    }
+    auto implied = [&](int d) {
+      for (int other : direct)
+        if (behindOf[static_cast<size_t>(other)][static_cast<size_t>(d)]) return true;
+      return false;
+    };
     std::vector<hipGraphNode_t> deps;
     auto behind = [&](int step) {
       for (hipGraphNode_t n : tail[static_cast<size_t>(step)])
         if (std::find(deps.begin(), deps.end(), n) == deps.end()) deps.push_back(n);
     };
-    if (st.before >= 0) behind(st.before);
-    for (int dep : st.after) behind(dep);
+    for (int d : direct)
+      if (!implied(d)) behind(d);
     if (hipStreamBeginCaptureToGraph(q, graph, deps.empty() ? nullptr : deps.data(), nullptr, deps.size(),
                                      hipStreamCaptureModeThreadLocal) != hipSuccess) {
       ok = false;
