@@ -332,8 +332,9 @@ convMfma(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
 // the lanes that would read the others multiply zeros (their weights are zero rows as well); CROW < 0: the rows
 // store `rowCh` channels, any number below CIN, and are read element by element (a 5-channel input: no widened
 // copy, and the few bytes of such rows do not need vector loads).
+// (launch bounds: layers whose weights leave room for two workgroups per CU keep to 64 registers)
 template <class T, int CIN, int COUT, int WAVES, int CROW = CIN>
-__global__ void __launch_bounds__(64 * WAVES)
+__global__ void __launch_bounds__(64 * WAVES, CIN * COUT * static_cast<int>(sizeof(T)) <= 1024 ? 8 : 4)
 convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
                  const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr,
                  int64_t nbrPitch, int tapMirror, const T* __restrict__ zeros, int kVol, int64_t inRows,
@@ -391,23 +392,44 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
   const int wavesPerXcd = (gridDim.x >> xcdShift) * WAVES;
   const TileOrder order(groups, static_cast<int>((liveOutRows(numActOut, outRows) + 15) / 16), xcdShift,
                         blockIdx.x & ((1 << xcdShift) - 1));
-  for (int local = (blockIdx.x >> xcdShift) * WAVES + wave; local < order.count(); local += wavesPerXcd) {
+  // The neighbour slice of a group is requested while the group before it multiplies (kernel volumes up to 28: seven
+  // registers): table, gathers and multiplications of a group otherwise run one after the other.
+  constexpr int AHEAD = 7;
+  const bool ahead = kVol <= 4 * AHEAD;
+  int32_t next[AHEAD];
+  auto tableEntry = [&](int64_t row0, int t0) __attribute__((always_inline)) -> int32_t {
+    const int tap = t0 + kgrp;
+    const int64_t row = row0 + r16;
+    const bool ok = tap < kVol && row < outRows;
+    const int32_t v = nbr[ok ? static_cast<int64_t>(tapMirror ? kVol - 1 - tap : tap) * nbrPitch + row : 0];
+    return !ok || v >= inRows ? -1 : v;
+  };
+  auto requestTable = [&](int local) __attribute__((always_inline)) {
+    if (!ahead || local >= order.count()) return;
+    const int64_t row0 = static_cast<int64_t>(order.tile(local)) * 16;
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) next[q] = tableEntry(row0, 4 * q);
+  };
+  const int firstLocal = (blockIdx.x >> xcdShift) * WAVES + wave;
+  requestTable(firstLocal);
+  for (int local = firstLocal; local < order.count(); local += wavesPerXcd) {
     const int group = order.tile(local);
     const int64_t row0 = static_cast<int64_t>(group) * 16;
 
     // private neighbour slice and the taps that occur in it (wavefront-uniform masks)
     unsigned long long active[2] = {0ull, 0ull};
-    for (int t0 = 0; t0 < kVol; t0 += 4) {
-      const int tap = t0 + kgrp;
-      const int64_t row = row0 + r16;
-      const bool ok = tap < kVol && row < outRows;
-      int32_t v = nbr[ok ? static_cast<int64_t>(tapMirror ? kVol - 1 - tap : tap) * nbrPitch + row : 0];
-      if (!ok || v >= inRows) v = -1;
-      if (tap < kVol) nb[tap * 16 + r16] = v;
+    auto noteTaps = [&](int t0, int32_t v) __attribute__((always_inline)) {
+      if (t0 + kgrp < kVol) nb[(t0 + kgrp) * 16 + r16] = v;
       const unsigned long long hit = __ballot(v >= 0);
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if ((hit >> (16 * q)) & 0xFFFFull) active[(t0 + q) >> 6] |= 1ull << ((t0 + q) & 63);
+    };
+    if (ahead) {
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) noteTaps(4 * q, next[q]);
+    } else {
+      for (int t0 = 0; t0 < kVol; t0 += 4) noteTaps(t0, tableEntry(row0, t0));
     }
     auto nextTap = [&]() __attribute__((always_inline)) -> int {  // -1 once the list is exhausted
       if (active[0]) {
@@ -448,6 +470,7 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
     int tA = nextTap(), tB = nextTap(), tC;
     gatherRows(tA, bufA);
     gatherRows(tB, bufB);
+    requestTable(local + wavesPerXcd);
     while (tA >= 0) {  // three steps per iteration, no branch between them (see convMfma)
       tC = nextTap();
       gatherRows(tC, bufC);
