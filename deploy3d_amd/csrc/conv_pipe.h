@@ -122,35 +122,36 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
     return m ? m : 1ull;
   };
 
-  // A walk over the workgroup's steps (tile, tap, part), one per consumer; each consumer asks for its steps in
-  // order.  Past the last step a walk stays on it: the loads issued for steps that do not exist repeat valid
-  // addresses and nothing in the loop has to branch on "is there such a step".
-  struct Walk {
-    int pos;                       // ordinal of the tile among this workgroup's
-    unsigned long long rem, next;  // taps of this tile still to walk; taps of the following tile
-    int tap, part;
-  };
-  auto walkInit = [&]() __attribute__((always_inline)) { return Walk{0, maskAt(0), maskAt(1), 0, 0}; };
-  // moves to the walk's next step; returns its step id (tap * KS + part).  *newTile = the step opens a tile.
-  auto walkNext = [&](Walk& w, bool* newTile) __attribute__((always_inline)) -> int {
+  // The workgroup's steps (tile, tap, part) in order.  One walk serves all consumers: the index loads run four steps
+  // ahead of the multiplication, the weight loads three, the gathers two, so a step's id is made once, by the index
+  // load, and handed down a chain of scalars (a walk per consumer took a third of a 32-channel step's instructions).
+  // Past the last step the walk stays on it: the loads issued for steps that do not exist repeat valid addresses and
+  // nothing in the loop has to branch on "is there such a step".
+  constexpr uint32_t kLastOfTile = 1u << 31;
+  int walkPos = 0;                                   // ordinal of the walk's tile among this workgroup's
+  unsigned long long walkRem = maskAt(0), walkTaps = maskAt(1);  // taps of it still to walk; taps of the next tile
+  int walkTap = 0, walkPart = 0;
+  // moves to the next step; returns its id (tap * KS + part), flagged when it ends its tile.  *newTile = it opens one.
+  auto walkNext = [&](bool* newTile) __attribute__((always_inline)) -> uint32_t {
     *newTile = false;
-    if (w.part == 0) {
-      if (w.rem == 0 && w.pos + 1 < nMine) {
-        ++w.pos;
-        w.rem = w.next;
-        w.next = maskAt(w.pos + 1);
+    if (walkPart == 0) {
+      if (walkRem == 0 && walkPos + 1 < nMine) {
+        ++walkPos;
+        walkRem = walkTaps;
+        walkTaps = maskAt(walkPos + 1);
         *newTile = true;
       }
-      if (w.rem) {
-        w.tap = __builtin_ctzll(w.rem);
-        w.rem &= w.rem - 1;
+      if (walkRem) {
+        walkTap = __builtin_ctzll(walkRem);
+        walkRem &= walkRem - 1;
       }
     }
-    const int s = w.tap * KS + w.part;
-    w.part = w.part + 1 == KS ? 0 : w.part + 1;
-    return s;
+    const uint32_t s = static_cast<uint32_t>(walkTap * KS + walkPart);
+    walkPart = walkPart + 1 == KS ? 0 : walkPart + 1;
+    return s | (walkRem == 0 && walkPart == 0 ? kLastOfTile : 0u);
   };
-  Walk walkIndex = walkInit(), walkWeights = walkInit(), walkRows = walkInit(), walkMul = walkInit();
+  uint32_t ids[5];                                   // steps a .. a+4
+  int mulPos = 0;                                    // ordinal of the tile that multiplies
 
   F rowBuf[2][KK];                                   // row fragments of the group that multiplies / of the next
   int32_t ixBuf[2][GPM];                             // neighbour indices for the gathers of this group / the next
@@ -164,11 +165,12 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   // indices of the index walk's next step -> ring slot `seq % NI` (asynchronous, straight into LDS); rows past
   // the table read as 0 and are never stored
   uint32_t idxOff[IL];
-  auto loadIndex = [&](int seq) __attribute__((always_inline)) {
+  auto loadIndex = [&](int seq) __attribute__((always_inline)) -> uint32_t {
     bool newTile;
-    const int tap = walkNext(walkIndex, &newTile) / KS;
+    const uint32_t id = walkNext(&newTile);
+    const int tap = walkTap;
     if (newTile || seq == 0) {
-      const uint32_t rowBase = static_cast<uint32_t>(tileAt(walkIndex.pos)) * TM;
+      const uint32_t rowBase = static_cast<uint32_t>(tileAt(walkPos)) * TM;
 #pragma unroll
       for (int i = 0; i < IL; ++i) idxOff[i] = (rowBase + idxRow[i]) * 4u;
     }
@@ -179,6 +181,7 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
         __builtin_amdgcn_raw_ptr_buffer_load_lds(nbrBuf, (LdsVoidPtr)(idxLds + (seq & (NI - 1)) * WM + i * 64), 4,
                                                  base + idxOff[i], 0, 0, 0);
     }
+    return id;
   };
   // the GPM indices of row group m of ring slot `seq % NI`, for this lane's gathers
   auto readIndex = [&](int seq, int m, int32_t (&dst)[GPM]) __attribute__((always_inline)) {
@@ -309,20 +312,17 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   };
 
   // ---- prologue: indices of steps 0..3, weights of steps 0..2, rows of steps 0 and 1 in flight ----
-  bool opened;
-  loadIndex(0);
-  loadIndex(1);
-  loadIndex(2);
-  loadIndex(3);
-  for (int wseq = 0; wseq < 3; ++wseq) {
-    const int s = walkNext(walkWeights, &opened);
 #pragma unroll
-    for (int q = 0; q < WL; ++q) weightLoad(q, s, wseq);
+  for (int t = 0; t < 4; ++t) ids[t] = loadIndex(t);
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+#pragma unroll
+    for (int q = 0; q < WL; ++q) weightLoad(q, static_cast<int>(ids[t] & ~kLastOfTile), t);
   }
   waitVmcnt<0>();
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    const int s0 = walkNext(walkRows, &opened);
+    const int s0 = static_cast<int>(ids[t] & ~kLastOfTile);
     const uint32_t p0 = chunkOff + static_cast<uint32_t>((s0 % KS) * CS * ES);
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -362,12 +362,9 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
     constexpr int freeBeforeWait = (MT - 1) * FREE; // free slots ahead of the wait (which opens the last group)
     constexpr int extraBeforeWait = (freeBeforeWait >= 1 ? IL : 0) +
                                     (freeBeforeWait - 1 > WL ? WL : (freeBeforeWait - 1 > 0 ? freeBeforeWait - 1 : 0));
-    bool open;
-    walkNext(walkMul, &open);
-    const bool lastOfTile = walkMul.rem == 0 && walkMul.part == 0;
-    const int sRows = walkNext(walkRows, &open);
-    const uint32_t partOff = chunkOff + static_cast<uint32_t>((sRows % KS) * CS * ES);
-    const int sW = walkNext(walkWeights, &open);
+    const bool lastOfTile = (ids[0] & kLastOfTile) != 0;
+    const uint32_t partOff = chunkOff + ((ids[2] & ~kLastOfTile) % KS) * static_cast<uint32_t>(CS * ES);
+    const int sW = static_cast<int>(ids[3] & ~kLastOfTile);
     const int nextBuf = wbuf + 1 == NWB ? 0 : wbuf + 1;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -396,13 +393,15 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
         if (q < GPM) gatherOne(m * GPM + q, ix[q], partOff, SLOT);
         if (q >= GPM) {
           const int u = m * FREE + q - GPM;         // ordinal of this free slot within the step
-          if (u == 0) loadIndex(a + 4);
+          if (u == 0) ids[4] = loadIndex(a + 4);
           if (u >= 1 && u <= WL) weightLoad(u - 1, sW, wbuf);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     wbuf = nextBuf;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) ids[t] = ids[t + 1];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     return lastOfTile;
@@ -410,12 +409,12 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
 
   for (int a = 0;; a += 2) {
     if (step(a, std::integral_constant<int, 0>{}, wtsA, wtsB)) {
-      storeTile(walkMul.pos);
-      if (walkMul.pos + 1 >= nMine) break;
+      storeTile(mulPos);
+      if (++mulPos >= nMine) break;
     }
     if (step(a + 1, std::integral_constant<int, 1>{}, wtsB, wtsA)) {
-      storeTile(walkMul.pos);
-      if (walkMul.pos + 1 >= nMine) break;
+      storeTile(mulPos);
+      if (++mulPos >= nMine) break;
     }
   }
   waitVmcnt<0>();                                   // loads issued for steps that do not exist, and the stores
