@@ -456,17 +456,12 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
 // 16 * MT, wavefronts per workgroup.  64 x 64 and narrower tiles afford 8 wavefronts (4 wavefronts of 128 rows,
 // which read half the weight fragments per MFMA, measured slower on a 64 -> 64 layer: 68 us against 58 - one
 // wavefront per SIMD has nobody to hide its waits); 128 output channels double the accumulators, so the wavefront
-// tile halves.  32 -> 32 takes 8 wavefronts as well (two workgroups of 78 KB per CU, 16 wavefronts): 38 us against
-// 41 with 4, 40 with three 4-wavefront workgroups per CU, 41 with 128-row and 42 with 48-row wavefront tiles; with gathers and MFMAs
-// both taken out of it the kernel still runs 27 us on that layer (25 with the table reads served from cache), so
-// what is left is the per-step bookkeeping of a 32-channel step, not a memory or matrix limit.  Two taps per step
+// tile halves.  32 -> 32 (more taps than conv_solo.h keeps resident) takes 8
+// wavefronts as well (two workgroups of 78 KB per CU): with 27 taps 38 us against 41 with 4, 40 with three
+// 4-wavefront workgroups per CU, 41 with 128-row and 42 with 48-row wavefront tiles.  Two taps per step
 // (a stage row holding the neighbours under two taps side by side, the step of a 64-channel layer) measured slower
-// on both 32-channel layers in every tile shape tried (32 -> 32: 44-58 us against 37.5; 32 -> 64: 45-57 against
-// 36): the stage doubles, one workgroup fits a CU instead of two, and the layer needs the wavefronts more than
-// the longer steps.  Smaller tiles for the sake of balance do not pay either: 351 000 rows are 686 tiles of 512 rows
-// on 512 workgroup slots (the busiest workgroup takes two), yet 384-row tiles (busiest: 768 rows) run the layer in
-// 43 us and 256-row tiles in 49 - a step costs about the same whatever its rows, because a CU's 16 wavefronts
-// move about 168 KB through LDS per step (gathered rows in and out, weight fragments) at 128 bytes per clock.
+// on 32 -> 64 in every tile shape tried (45-57 us against 36): the stage doubles, one workgroup fits a CU instead of
+// two, and the layer needs the wavefronts more than the longer steps.
 // Layers with few
 // rows (the 128-channel stages: 47 000 rows are 186 tiles of 256 rows for 256 CUs) pick the workgroup shape by
 // tile count: the time of a layer that fits one round is that of ONE tile, so 248 tiles of 192 rows beat 186 of

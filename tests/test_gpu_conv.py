@@ -118,6 +118,19 @@ def test_mfma_fp32(engine, cin, cout):
     run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, "float32", False, inverse=True, with_bias=False)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (3, 1, 3), (1, 1, 1), (3, 3, 5)])
+def test_resident_32_to_32(engine, ksize, dtype):
+    """32 -> 32 channels with the weights of up to 27 taps resident (45 taps: the pipelined kernel), around its 64-row
+    tiles, with rows past the live count, with and without tile masks, strided and inverse."""
+    pad = tuple(k // 2 for k in ksize)
+    for n in (1, 63, 64, 65, 2500):
+        run_case(n, (10, 36, 30), ksize, (1, 1, 1), pad, 32, 32, dtype, True, relu=(n == 65), cap_extra=n % 3 * 40, link=n != 64)
+    if ksize == (3, 3, 3):
+        run_case(2500, (10, 36, 30), ksize, (2, 2, 2), pad, 32, 32, dtype, False, with_bias=False)
+        run_case(2500, (10, 36, 30), ksize, (2, 2, 2), pad, 32, 32, dtype, False, inverse=True)
+
+
 def test_narrow_strided_fp32(engine):
     run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), 16, 16, "float32", False)
 
