@@ -482,6 +482,14 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
     else return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
   } else if constexpr (RB == 128 && COUT == 64) {
+    // 512-row tiles; few rows take the smallest of 128, 256 and 512 whose tiles still fit one round of the CUs (64 -> 64:
+    // 15 600 rows 16 us against 25 with 512-row tiles, 43 000 rows 19 against 26; with 118 000 rows, more than one round
+    // of 256-row tiles, those take 35 against 30)
+    if constexpr (sizeof(T) == 2) {
+      const int64_t cus = chipLayout().cus;
+      if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
+      if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+    }
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else if constexpr (COUT >= 128) {
     // 8, 6 or 4 wavefronts of 32 rows: the workgroup size whose tiles load the busiest CU least (rounds of tiles
@@ -489,6 +497,11 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     // wavefronts of 48 rows - one per SIMD - instead of six of 32, which load two SIMDs twice as much as the
     // others (conv4_x: 45 us against 48); over several rounds the eight-wavefront shapes hide their waits better
     // (a 64 -> 128 layer of 10 rounds: 105 us with 8 x 32 rows, 138 us with 4 x 48).
+    // Fewer rows than one round of 64-row tiles take those, two wavefronts each (128 -> 128 with 10 200 rows: 29 us
+    // against 33 with 128-row tiles; with 23 000 rows, more than a round, 41 against 34).
+    if constexpr (sizeof(T) == 2 && CIN >= 64)
+      if (a.outRows <= 64 * static_cast<int64_t>(chipLayout().cus) && !debugEnv("D3D_CONV_PIPE_SHAPE"))
+        return launchPipeCfg<T, CIN, COUT, 2, 2>(a, stream);
     static const int kCand[4][2] = {{32, 8}, {32, 6}, {32, 4}, {48, 4}};
     // int8 128 -> 128: the wider workgroups (two wavefronts per SIMD, 256 registers each) spill - 84-97 us against
     // 33-44 on a 47 000-row layer - so only the four-wavefront shapes are candidates, the larger tile winning ties
@@ -528,6 +541,10 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   } else if constexpr (RB == 64 && COUT == 32) {
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else {
+    // 256-row tiles; 128-row ones while those fit the two workgroups that a CU holds (32 -> 64: 15 600 rows 12.7 us
+    // against 15.7, 43 000 rows 14.4 against 16.4, but 118 000 rows, nearly four per CU, 26 against 21)
+    if constexpr (sizeof(T) == 2 && CIN == 32 && COUT == 64)
+      if (a.outRows <= 256 * static_cast<int64_t>(chipLayout().cus)) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
     return launchPipeCfg<T, CIN, COUT, 4, 4>(a, stream);
   }
 }

@@ -334,6 +334,14 @@ def test_pipelined_tile_shapes_of_wide_layers(engine, monkeypatch, shape, cin, c
         run_case(70000, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=True)
 
 
+@pytest.mark.parametrize("cin,cout", [(32, 64), (64, 64), (64, 128), (128, 128)])
+def test_pipelined_tile_shapes_by_row_count(engine, cin, cout):
+    """Row counts on both sides of the lines (64, 128 and 256 rows per CU) at which the pipelined kernel takes another
+    tile; smaller layers of the other tests run the smallest tiles."""
+    for k, n in enumerate((64 * 256, 64 * 256 + 1, 128 * 256 + 1, 256 * 256 + 1)):
+        run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, ("float16", "bfloat16")[k % 2], True, relu=True)
+
+
 @pytest.mark.parametrize("cfg", ["off", "4,8,2", "2,8,3", "2,8,2", "4,4,2", "4,4,3", "4,8,3,1", "2,8,3,1"])
 @pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128), (128, 16)])
 def test_staged_configurations(engine, monkeypatch, cfg, cin, cout):
