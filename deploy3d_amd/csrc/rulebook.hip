@@ -53,16 +53,15 @@ __device__ __forceinline__ uint32_t fmix32(uint32_t k) {
 // Inserts (key, value); on a key that is already present keeps the smaller
 // value.  Returns the slot, or kNone if the table is full (cannot happen at
 // load factor <= 1/2).  At most `mask + 1` probes, so every lane terminates.
+// A probe is one compare-and-swap, which returns what the slot holds: most slots are free when a key arrives, and a
+// plain read in front of it would double the chain of memory round trips that this pass consists of.
 __device__ __forceinline__ uint32_t hashInsertMin(unsigned long long* table, uint32_t mask, uint32_t key,
                                                   uint32_t value) {
   const unsigned long long packed = (static_cast<unsigned long long>(key) << 32) | value;
   uint32_t slot = fmix32(key) & mask;
   for (uint32_t probe = 0; probe <= mask; ++probe) {
-    unsigned long long cur = __builtin_nontemporal_load(table + slot);
-    if (cur == kEmptySlot) {
-      cur = atomicCAS(table + slot, kEmptySlot, packed);
-      if (cur == kEmptySlot) return slot;
-    }
+    const unsigned long long cur = atomicCAS(table + slot, kEmptySlot, packed);
+    if (cur == kEmptySlot) return slot;
     if (static_cast<uint32_t>(cur >> 32) == key) {
       // values only ever decrease, so a (possibly stale) smaller value settles it
       if (packed < cur) atomicMin(table + slot, packed);
@@ -73,15 +72,49 @@ __device__ __forceinline__ uint32_t hashInsertMin(unsigned long long* table, uin
   return kNone;
 }
 
-__device__ __forceinline__ uint32_t hashLookup(const unsigned long long* table, uint32_t mask, uint32_t key) {
-  uint32_t slot = fmix32(key) & mask;
-  for (uint32_t probe = 0; probe <= mask; ++probe) {
-    const unsigned long long cur = table[slot];
-    if (static_cast<uint32_t>(cur >> 32) == key) return static_cast<uint32_t>(cur);
-    if (cur == kEmptySlot) return kNone;
-    slot = (slot + 1) & mask;
+constexpr uint32_t kHashGroup = 4;  // slots that one step of a lookup reads (32 bytes; tables hold 1024 slots at least)
+
+// Looks up N keys; a key of want[j] == false is not looked up.  The probes of all keys travel together and cover a
+// group of slots each: a wavefront waits for the longest of its 64 * N chains, which at load factor 1/3 is five to
+// ten slots long, as many round trips when they are read one by one.
+template <int N>
+__device__ __forceinline__ void hashLookup(const unsigned long long* table, uint32_t mask, const uint32_t (&key)[N],
+                                           const bool (&want)[N], uint32_t (&value)[N]) {
+  uint32_t group[N], first[N];
+  bool open[N];
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const uint32_t slot = fmix32(key[j]) & mask;
+    group[j] = slot / kHashGroup;
+    first[j] = slot % kHashGroup;
+    open[j] = want[j];
+    any = any || want[j];
+    value[j] = kNone;
   }
-  return kNone;
+  for (uint32_t probe = 0; any && probe <= mask / kHashGroup + 1; ++probe) {
+    uint4 cur[N][2];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        cur[j][h] = reinterpret_cast<const uint4*>(table)[(open[j] ? group[j] : 0u) * 2 + h];
+    any = false;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+      for (uint32_t e = 0; e < kHashGroup; ++e) {
+        const uint4& v = cur[j][e / 2];
+        const uint32_t lo = e % 2 ? v.z : v.x, hi = e % 2 ? v.w : v.y;
+        const bool here = open[j] && e >= first[j];
+        if (here && hi == key[j]) value[j] = lo;
+        open[j] = open[j] && !(here && (hi == key[j] || (hi & lo) == ~0u));
+      }
+      any = any || open[j];
+      first[j] = 0;
+      group[j] = (group[j] + 1) & (mask / kHashGroup);
+    }
+  }
 }
 
 // Loads coordinate row `i` widened to (batch, 4 spatial).
@@ -98,15 +131,19 @@ __device__ __forceinline__ void loadCoord(const int32_t* coors, int nd, int64_t 
   for (int dim = 0; dim < kMaxSpatial; ++dim) c[dim + 1] = dim >= pad ? row[1 + dim - pad] : 0;
 }
 
+__device__ __forceinline__ bool inputInGrid(const RbGeom& g, const int c[5]) {
+  bool ok = true;
+#pragma unroll
+  for (int dim = 0; dim <= kMaxSpatial; ++dim) ok = ok && c[dim] >= 0 && c[dim] < g.inShape[dim];
+  return ok;
+}
+
 // Loads input row `i`; false if its coordinate lies outside the input grid.  Such a row takes part in no pair, on
 // every structure (the reference hashes its linear offset unchecked, so it aliases into another cell there:
 // trt/spconv/index.cu:174-182).
 __device__ __forceinline__ bool loadInput(const RbGeom& g, const int32_t* coors, int64_t i, int c[5]) {
   loadCoord(coors, g.nd, i, c);
-  bool ok = true;
-#pragma unroll
-  for (int dim = 0; dim <= kMaxSpatial; ++dim) ok = ok && c[dim] >= 0 && c[dim] < g.inShape[dim];
-  return ok;
+  return inputInGrid(g, c);
 }
 
 __device__ __forceinline__ bool coordInGrid(const RbGeom& g, const int c[5]) {
@@ -343,18 +380,37 @@ rbSubmProbe(RbGeom g, const int32_t* __restrict__ coors, const int32_t* __restri
   if (static_cast<int64_t>(blockIdx.x) * kRbChunk < n) {  // workgroup-uniform
     int idx[kMaxSpatial];
     tapPositions(g, tap, idx);
-    uint32_t row[kRbItems];
+    uint32_t row[kRbItems], off[kRbItems];
+    bool want[kRbItems];
+    int c[kRbItems][5];
 #pragma unroll
-    for (int j = 0; j < kRbItems; ++j) {
-      row[j] = kNone;
-      const int64_t i = first + j;
-      if (i < n) {
-        int c[5];
-        uint32_t off;
-        if (loadInput(g, coors, i, c) && tapTarget(g, c, idx, &off)) row[j] = hashLookup(table, mask, off);
+    for (int j = 0; j < kRbItems; ++j) loadCoord(coors, g.nd, first + j < n ? first + j : 0, c[j]);  // n > 0 here
+    if (!g.transpose && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1 && g.s[3] == 1) {
+      // stride 1 (every SubM layer in use): the tap moves all inputs by the same cells, no general walk per dim and input
+      int move[kMaxSpatial];
+#pragma unroll
+      for (int dim = 0; dim < kMaxSpatial; ++dim) move[dim] = g.p[dim] - idx[dim] * g.d[dim];
+#pragma unroll
+      for (int j = 0; j < kRbItems; ++j) {
+        want[j] = first + j < n && inputInGrid(g, c[j]) && c[j][0] < g.shape[0];
+        off[j] = static_cast<uint32_t>(c[j][0]);
+#pragma unroll
+        for (int dim = 0; dim < kMaxSpatial; ++dim) {
+          const uint32_t to = static_cast<uint32_t>(c[j][dim + 1] + move[dim]);
+          want[j] = want[j] && to < static_cast<uint32_t>(g.shape[dim + 1]);
+          off[j] = off[j] * static_cast<uint32_t>(g.shape[dim + 1]) + to;
+        }
       }
-      found += row[j] != kNone;
+    } else {
+#pragma unroll
+      for (int j = 0; j < kRbItems; ++j) {
+        off[j] = 0;
+        want[j] = first + j < n && inputInGrid(g, c[j]) && tapTarget(g, c[j], idx, &off[j]);
+      }
     }
+    hashLookup(table, mask, off, want, row);
+#pragma unroll
+    for (int j = 0; j < kRbItems; ++j) found += row[j] != kNone;
     if (first < n) *reinterpret_cast<uint4*>(staging + static_cast<int64_t>(tap) * pitch + first) =
         make_uint4(row[0], row[1], row[2], row[3]);
   }
