@@ -945,7 +945,18 @@ struct BlockMap {
   int shift[kMaxSpatial];  // log2 brick extent per spatial dim (extents multiply to 64)
   int nb[kMaxSpatial];     // bricks per dim
   uint32_t records;        // batch * product of nb
+  int chunkShift;          // log2 of the records per chunk of the rank prefix (chunkShiftOf)
 };
+
+// Records per chunk: 1024, scanned by one workgroup; small maps (two million cells and less: the deep levels of a
+// backbone) go in chunks of one wavefront, because their scan is bound by the loads of too few CUs - 2 700 records in
+// chunks of 1024 keep three CUs busy.  Deriving 22 300 / 2 700 occupancies from the level above (27 loads each): 13.4 /
+// 14.8 us with chunks of 1024, 12.1 / 9.1 with chunks of 64.  Beyond, the totals that the last workgroup scans get many.
+constexpr int kChunkShift = 10, kSmallChunkShift = 6;
+constexpr uint64_t kSmallMapRecords = 1u << 15;
+__host__ __device__ constexpr int chunkShiftOf(uint64_t records) {
+  return records <= kSmallMapRecords ? kSmallChunkShift : kChunkShift;
+}
 
 __device__ __forceinline__ void bmLocate(const BlockMap& m, const int c[5], uint32_t* rec, uint32_t* bit) {
   uint32_t r = static_cast<uint32_t>(c[0]);
@@ -973,10 +984,10 @@ __device__ __forceinline__ bool tapTargetCoord(const RbGeom& g, const int c[5], 
   return ok;
 }
 
-// rank = occupied cells in earlier chunks of 1024 records + in earlier records of the chunk + below the bit
-__device__ __forceinline__ uint32_t bmRank(const BmRecord& r, uint32_t bit, const uint32_t* __restrict__ chunkBase,
-                                           uint32_t rec) {
-  return chunkBase[rec / kRbChunk] + r.prefix + static_cast<uint32_t>(__popcll(r.bits & ((1ull << bit) - 1ull)));
+// rank = occupied cells in earlier chunks of records + in earlier records of the chunk + below the bit
+__device__ __forceinline__ uint32_t bmRank(const BlockMap& m, const BmRecord& r, uint32_t bit,
+                                           const uint32_t* __restrict__ chunkBase, uint32_t rec) {
+  return chunkBase[rec >> m.chunkShift] + r.prefix + static_cast<uint32_t>(__popcll(r.bits & ((1ull << bit) - 1ull)));
 }
 
 // reset for the block-map path: records = 0, index tensor = -1, counters = 0
@@ -1206,7 +1217,7 @@ __device__ __forceinline__ unsigned long long gatherOccupancy(const GatherArgs& 
       if (!inside) continue;
       const uint4 r = *reinterpret_cast<const uint4*>(src + at);
       unsigned long long bits = (static_cast<unsigned long long>(r.y) << 32) | r.x;
-      if (bits) bits = cutToLive(bits, ga.srcChunkBase[at / kRbChunk] + r.z, nLive);
+      if (bits) bits = cutToLive(bits, ga.srcChunkBase[at >> ga.mi.chunkShift] + r.z, nLive);
       // (a loop that is not unrolled: the brick is chosen by arithmetic, not by a constant index)
       const int a = (e / NA) % NA, c = e % NA;
 #pragma unroll
@@ -1222,6 +1233,105 @@ __device__ __forceinline__ unsigned long long gatherOccupancy(const GatherArgs& 
     // 17 x 17 input cells under the 8 x 8 outputs: rows folded first (per brick column), then cells
     return foldCells(foldRows(under[0][0], under[1][0], under[2][0]), foldRows(under[0][1], under[1][1], under[2][1]),
                      foldRows(under[0][2], under[1][2], under[2][2]));
+  }
+}
+
+// Occupancy of output record `rec`, cut to the rows of the input and the cells of the output grid.
+template <int GATHER>
+__device__ __forceinline__ unsigned long long gatheredBits(const GatherArgs& ga, uint32_t rec, uint32_t nRecords) {
+  const BmRecord* __restrict__ src = ga.src.get();
+  const int32_t live = *ga.numActIn;
+  const uint32_t nLive = live < 0 ? 0u : (static_cast<uint32_t>(live) < ga.inCap ? static_cast<uint32_t>(live) : ga.inCap);
+  const bool checkRanks = nLive >= ga.inCap;  // fewer rows than the capacity: nothing was cut off
+  unsigned long long bits = rec < nRecords ? gatherOccupancy<GATHER>(ga, src, rec, nLive, checkRanks) : 0ull;
+  if (bits) {  // cells of the brick past the edge of the output grid are no outputs
+    const uint32_t q1 = divSmall(rec, static_cast<uint32_t>(ga.mo.nb[3]), ga.rcpX);
+    const int bx = static_cast<int>(rec - q1 * static_cast<uint32_t>(ga.mo.nb[3]));
+    const int by = static_cast<int>(q1 - divSmall(q1, static_cast<uint32_t>(ga.mo.nb[2]), ga.rcpY) * static_cast<uint32_t>(ga.mo.nb[2]));
+    const int rows = ga.shapeY - 8 * by, cols = ga.shapeX - 8 * bx;
+    if (rows < 8) bits &= (1ull << (8 * rows)) - 1ull;
+    if (cols < 8) bits &= 0x0101010101010101ull * ((1ull << cols) - 1ull);
+  }
+  return bits;
+}
+
+// Exclusive scan over the workgroup (of one wavefront or kRbThreads threads).
+template <int THREADS>
+__device__ __forceinline__ uint32_t chunkScan(uint32_t v, uint32_t* scratch, uint32_t* total) {
+  if constexpr (THREADS == 64) {
+    const uint32_t incl = waveInclusiveScan(v);
+    *total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+    return incl - v;
+  } else {
+    static_assert(THREADS == kRbThreads, "one wavefront or a whole workgroup");
+    return blockExclusiveScan(v, scratch, total);
+  }
+}
+
+// End of a scan: the workgroup's total is published, and the workgroup that comes last turns all totals into prefixes.
+template <bool ORDERED, int THREADS>
+__device__ __forceinline__ void finishScan(uint32_t total, const RecRef& recRef, uint32_t epoch, uint32_t* chunkBase,
+                                           uint32_t nChunks, uint32_t* ticket, uint32_t* groupTickets, int32_t* numActOut,
+                                           int32_t maxNumActOut, uint32_t* scratch, uint32_t* isLast) {
+  if (threadIdx.x == 0) {
+    // The chunk totals are the only data that passes between workgroups inside this kernel, and every access to
+    // them is a device-scope atomic.  ORDERED makes the hand-off formal: acquire-release tickets, i.e. a
+    // device-scope release per workgroup, which on this part writes the L2 back - measured 6.3 -> 10.9 us per
+    // launch on average and 17 -> 50 us on a 1.3 M-record grid, 37 us per pass of eight rulebooks.  The default
+    // does without: the total is published with a RETURNING device-scope atomic, which has been performed where
+    // every XCD sees it once its result is back (the s_waitcnt below), and only then is the ticket taken, so the
+    // workgroup that draws the last ticket cannot read an older total.
+    uint32_t old = __hip_atomic_exchange(&chunkBase[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(old)::"memory");
+    // Atomics on one address are performed one after the other (about 18 ns each across the XCDs), so the
+    // tickets are taken in two levels: one counter per kScanGroup workgroups, and only the last of each group
+    // goes on to the counter of the whole grid.
+    const uint32_t group = blockIdx.x / kScanGroup;
+    const uint32_t groupSize = min(kScanGroup, nChunks - group * kScanGroup);
+    const uint32_t nGroups = (nChunks + kScanGroup - 1) / kScanGroup;
+    uint32_t last = 0;
+    constexpr int kOrder = ORDERED ? __ATOMIC_ACQ_REL : __ATOMIC_RELAXED;
+    if (__hip_atomic_fetch_add(&groupTickets[group], 1u, kOrder, __HIP_MEMORY_SCOPE_AGENT) == groupSize - 1)
+      last = __hip_atomic_fetch_add(ticket, 1u, kOrder, __HIP_MEMORY_SCOPE_AGENT) == nGroups - 1 ? 1u : 0u;
+    *isLast = last;
+  }
+  __syncthreads();
+  if (!*isLast) return;
+  // one exclusive scan over all chunk totals: thread t takes a contiguous run of them (all loads in flight at
+  // once), scans it in registers, and a single workgroup scan of the run sums supplies the offsets
+  constexpr uint32_t kRun = 8;
+  uint32_t running = 0;
+  for (uint32_t base = 0; base < nChunks; base += kRun * THREADS) {
+    const uint32_t q0 = base + threadIdx.x * kRun;
+    uint32_t v[kRun];
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j)
+      v[j] = q0 + j < nChunks ? __hip_atomic_load(&chunkBase[q0 + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    uint32_t mineSum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j) mineSum += v[j];
+    uint32_t sum;
+    uint32_t at = running + chunkScan<THREADS>(mineSum, scratch, &sum);
+#pragma unroll
+    for (uint32_t j = 0; j < kRun; ++j) {
+      if (q0 + j < nChunks) chunkBase[q0 + j] = at;
+      at += v[j];
+    }
+    running += sum;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && numActOut)
+    *numActOut = static_cast<int32_t>(running < static_cast<uint32_t>(maxNumActOut) ? running : maxNumActOut);
+  // Every other workgroup has drawn its tickets (and read the scan count before that): the counters go back to
+  // zero for the next pass, and with two maps the count moves on - the passes behind this one see this map as
+  // the finished one, the next build marks the other.
+  if (recRef.epoch) {
+    const uint32_t nGroups = (nChunks + kScanGroup - 1) / kScanGroup;
+    for (uint32_t q = threadIdx.x; q < nGroups; q += THREADS) groupTickets[q] = 0u;
+    if (threadIdx.x == 0) {
+      *ticket = 0u;
+      *recRef.epoch = epoch + 1u;
+    }
   }
 }
 
@@ -1250,21 +1360,8 @@ bmScan(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, 
   if constexpr (GATHER != 0) {
     __shared__ unsigned long long chunkBits[kRbChunk];
     {
-      const BmRecord* __restrict__ src = ga.src.get();
-      const int32_t live = *ga.numActIn;
-      const uint32_t nLive = live < 0 ? 0u : (static_cast<uint32_t>(live) < ga.inCap ? static_cast<uint32_t>(live) : ga.inCap);
-      const bool checkRanks = nLive >= ga.inCap;  // fewer rows than the capacity: nothing was cut off
       const uint32_t rec = blockIdx.x * kRbChunk + threadIdx.x;
-      unsigned long long bits = rec < nRecords ? gatherOccupancy<GATHER>(ga, src, rec, nLive, checkRanks) : 0ull;
-      if (bits) {  // cells of the brick past the edge of the output grid are no outputs
-        const uint32_t q1 = divSmall(rec, static_cast<uint32_t>(ga.mo.nb[3]), ga.rcpX);
-        const int bx = static_cast<int>(rec - q1 * static_cast<uint32_t>(ga.mo.nb[3]));
-        const int by = static_cast<int>(q1 - divSmall(q1, static_cast<uint32_t>(ga.mo.nb[2]), ga.rcpY) * static_cast<uint32_t>(ga.mo.nb[2]));
-        const int rows = ga.shapeY - 8 * by, cols = ga.shapeX - 8 * bx;
-        if (rows < 8) bits &= (1ull << (8 * rows)) - 1ull;
-        if (cols < 8) bits &= 0x0101010101010101ull * ((1ull << cols) - 1ull);
-      }
-      chunkBits[threadIdx.x] = bits;
+      chunkBits[threadIdx.x] = gatheredBits<GATHER>(ga, rec, nRecords);
     }
     __syncthreads();
     if (threadIdx.x >= kRbThreads) return;  // (a wavefront that has ended no longer counts at a barrier)
@@ -1314,68 +1411,36 @@ bmScan(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, 
     }
     rank += rowSum[j];
   }
-  if (threadIdx.x == 0) {
-    // The chunk totals are the only data that passes between workgroups inside this kernel, and every access to
-    // them is a device-scope atomic.  ORDERED makes the hand-off formal: acquire-release tickets, i.e. a
-    // device-scope release per workgroup, which on this part writes the L2 back - measured 6.3 -> 10.9 us per
-    // launch on average and 17 -> 50 us on a 1.3 M-record grid, 37 us per pass of eight rulebooks.  The default
-    // does without: the total is published with a RETURNING device-scope atomic, which has been performed where
-    // every XCD sees it once its result is back (the s_waitcnt below), and only then is the ticket taken, so the
-    // workgroup that draws the last ticket cannot read an older total.
-    uint32_t old = __hip_atomic_exchange(&chunkBase[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(old)::"memory");
-    // Atomics on one address are performed one after the other (about 18 ns each across the XCDs), so the
-    // tickets are taken in two levels: one counter per kScanGroup workgroups, and only the last of each group
-    // goes on to the counter of the whole grid.
-    const uint32_t group = blockIdx.x / kScanGroup;
-    const uint32_t groupSize = min(kScanGroup, nChunks - group * kScanGroup);
-    const uint32_t nGroups = (nChunks + kScanGroup - 1) / kScanGroup;
-    uint32_t last = 0;
-    constexpr int kOrder = ORDERED ? __ATOMIC_ACQ_REL : __ATOMIC_RELAXED;
-    if (__hip_atomic_fetch_add(&groupTickets[group], 1u, kOrder, __HIP_MEMORY_SCOPE_AGENT) == groupSize - 1)
-      last = __hip_atomic_fetch_add(ticket, 1u, kOrder, __HIP_MEMORY_SCOPE_AGENT) == nGroups - 1 ? 1u : 0u;
-    isLast = last;
-  }
-  __syncthreads();
-  if (!isLast) return;
-  // one exclusive scan over all chunk totals: thread t takes a contiguous run of them (all loads in flight at
-  // once), scans it in registers, and a single workgroup scan of the run sums supplies the offsets
-  constexpr uint32_t kRun = 8;
-  uint32_t running = 0;
-  for (uint32_t base = 0; base < nChunks; base += kRun * kRbThreads) {
-    const uint32_t q0 = base + threadIdx.x * kRun;
-    uint32_t v[kRun];
-#pragma unroll
-    for (uint32_t j = 0; j < kRun; ++j)
-      v[j] = q0 + j < nChunks ? __hip_atomic_load(&chunkBase[q0 + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-    uint32_t mineSum = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kRun; ++j) mineSum += v[j];
-    uint32_t sum;
-    uint32_t at = running + blockExclusiveScan(mineSum, scratch, &sum);
-#pragma unroll
-    for (uint32_t j = 0; j < kRun; ++j) {
-      if (q0 + j < nChunks) chunkBase[q0 + j] = at;
-      at += v[j];
-    }
-    running += sum;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && numActOut)
-    *numActOut = static_cast<int32_t>(running < static_cast<uint32_t>(maxNumActOut) ? running : maxNumActOut);
-  // Every other workgroup has drawn its tickets (and read the scan count before that): the counters go back to
-  // zero for the next pass, and with two maps the count moves on - the passes behind this one see this map as
-  // the finished one, the next build marks the other.
-  if (recRef.epoch) {
-    const uint32_t nGroups = (nChunks + kScanGroup - 1) / kScanGroup;
-    for (uint32_t q = threadIdx.x; q < nGroups; q += kRbThreads) groupTickets[q] = 0u;
-    if (threadIdx.x == 0) {
-      *ticket = 0u;
-      *recRef.epoch = epoch + 1u;
-    }
-  }
+  finishScan<ORDERED, kRbThreads>(total, recRef, epoch, chunkBase, nChunks, ticket, groupTickets, numActOut, maxNumActOut,
+                                  scratch, &isLast);
 }
 
+// The same scan in chunks of 64 records, one per lane of a workgroup of one wavefront (small maps, see chunkShiftOf).
+template <bool ORDERED, int GATHER>
+__global__ void __launch_bounds__(64)
+bmScanSmall(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, uint32_t* ticket,
+            uint32_t* groupTickets, int32_t* numActOut, int32_t maxNumActOut, GatherArgs ga) {
+  __shared__ uint32_t isLast;
+  const uint32_t epoch = recRef.epoch ? *recRef.epoch : 0u;
+  BmRecord* __restrict__ records = recRef.base + static_cast<size_t>(epoch & 1u) * (recRef.epoch ? recRef.stride : 0u);
+  BmRecord* __restrict__ other = recRef.epoch ? recRef.base + static_cast<size_t>((epoch + 1u) & 1u) * recRef.stride : nullptr;
+  const uint32_t rec = blockIdx.x * 64 + threadIdx.x;
+  unsigned long long bits = 0ull;
+  if constexpr (GATHER != 0) bits = gatheredBits<GATHER>(ga, rec, nRecords);
+  else if (rec < nRecords) bits = records[rec].bits;
+  if (other && rec < nRecords) other[rec].bits = 0ull;
+  const uint32_t count = static_cast<uint32_t>(__popcll(bits));
+  const uint32_t incl = waveInclusiveScan(count);
+  if (count) {  // an empty record is never ranked
+    if constexpr (GATHER != 0)
+      *reinterpret_cast<uint4*>(records + rec) =
+          make_uint4(static_cast<uint32_t>(bits), static_cast<uint32_t>(bits >> 32), incl - count, 0u);
+    else
+      records[rec].prefix = incl - count;
+  }
+  finishScan<ORDERED, 64>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63)), recRef, epoch, chunkBase,
+                          nChunks, ticket, groupTickets, numActOut, maxNumActOut, nullptr, &isLast);
+}
 
 constexpr uint32_t kEmitGroup = 8;  // records per wavefront of the coordinate pass
 
@@ -1421,7 +1486,7 @@ __device__ __forceinline__ void emitRecordCoords(const RbGeom& g, const BlockMap
   }
   unsigned long long occupied = __ballot((lo | hi) != 0u);
   if (occupied == 0ull) return;
-  prefix += chunkBase[((lane < kEmitGroup && rec0 + lane < nRecords) ? rec0 + lane : rec0) / kRbChunk];
+  prefix += chunkBase[((lane < kEmitGroup && rec0 + lane < nRecords) ? rec0 + lane : rec0) >> m.chunkShift];
   while (occupied) {
     const int r = __builtin_ctzll(occupied);
     occupied &= occupied - 1ull;
@@ -1453,7 +1518,7 @@ __device__ __forceinline__ void permuteRow(const RbGeom& g, const BlockMap& m, c
   if (!loadInput(g, coors, i, c) || !coordInGrid(g, c)) return;
   uint32_t rec, bit;
   bmLocate(m, c, &rec, &bit);
-  const uint32_t rank = bmRank(records[rec], bit, chunkBase, rec);
+  const uint32_t rank = bmRank(m, records[rec], bit, chunkBase, rec);
   perm[rank] = static_cast<uint32_t>(i);
   if (rank != static_cast<uint32_t>(i)) *permShuffled = 1u;
 }
@@ -1497,7 +1562,7 @@ bmProbe(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int32_t* 
           bmLocate(m, o, &rec, &bit);
           const BmRecord r = records[rec];
           if ((r.bits >> bit) & 1ull) {
-            const uint32_t rank = bmRank(r, bit, chunkBase, rec);
+            const uint32_t rank = bmRank(m, r, bit, chunkBase, rec);
             if (SUBM ? rank < static_cast<uint32_t>(n) : rank < static_cast<uint32_t>(maxNumActOut))
               row[j] = rank;  // SubM: the compaction turns ranks into rows through perm[] when rows are shuffled
           }
@@ -1760,7 +1825,7 @@ bmProbeNear(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int32
 #pragma unroll
   for (int e = 0; e < kNearGroup; ++e) {
     loaded[e] = *reinterpret_cast<const uint4*>(records + (live ? rec[e] : 0u));
-    base[e] = chunkBase[(live ? rec[e] : 0u) / kRbChunk];
+    base[e] = chunkBase[(live ? rec[e] : 0u) >> m.chunkShift];
   }
 #pragma unroll
   for (int e = 0; e < kNearGroup; ++e) {
@@ -1909,7 +1974,7 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
       const bool present = ok1[q1] && base2 + (e >> 1) < m.nb[2] && base3 + (e & 1) < m.nb[3];
       const uint32_t rec = present ? rec0 + static_cast<uint32_t>((e >> 1) * m.nb[3] + (e & 1)) : 0u;
       const uint4 r = *reinterpret_cast<const uint4*>(records + rec);
-      const uint32_t base = chunkBase[rec / kRbChunk];
+      const uint32_t base = chunkBase[rec >> m.chunkShift];
       lo[q1][e] = present ? r.x : 0u;
       hi[q1][e] = present ? r.y : 0u;
       pre[q1][e] = r.z + base;  // in-chunk prefix -> global prefix
@@ -1999,6 +2064,7 @@ BlockMap makeBlockMap(const RbGeom& g, uint64_t* records) {
   }
   *records = n;
   m.records = static_cast<uint32_t>(n < 0xFFFFFFFFull ? n : 0xFFFFFFFFull);
+  m.chunkShift = chunkShiftOf(n);
   return m;
 }
 
@@ -2030,7 +2096,8 @@ RbWorkspace planWith(const RbGeom& g, int64_t cap, bool subM, bool blockMap) {
     uint64_t records;
     makeBlockMap(g, &records);
     w.nRecords = static_cast<uint32_t>(records);
-    w.nChunks = static_cast<uint32_t>((records + kRbChunk - 1) / kRbChunk);
+    const int chunkShift = chunkShiftOf(records);
+    w.nChunks = static_cast<uint32_t>((records + (1u << chunkShift) - 1) >> chunkShift);
     w.table = off;  // BmRecord [nRecords]
     off = alignUp(off + static_cast<size_t>(records) * sizeof(BmRecord));
     w.ids = off;    // SubM: perm u32 [cap]
@@ -2348,8 +2415,15 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     }
     // D3D_RULEBOOK_ORDERED_SCAN=1: acquire-release tickets (see bmScan)
 #define D3D_LAUNCH_SCAN(ORDERED, GATHER)                                                                          \
-  hipLaunchKernelGGL((bmScan<ORDERED, GATHER>), perChunk, dim3(GATHER ? kRbChunk : kRbThreads), 0, stream, recBefore, w.nRecords, chunkBase, \
-                     w.nChunks, scanTicket, scanTicket + 1, subM ? nullptr : numActOut, maxNumActOut, ga)
+  do {                                                                                                                \
+    if (m.chunkShift == kSmallChunkShift)                                                                             \
+      hipLaunchKernelGGL((bmScanSmall<ORDERED, GATHER>), perChunk, dim3(64), 0, stream, recBefore, w.nRecords, chunkBase, \
+                         w.nChunks, scanTicket, scanTicket + 1, subM ? nullptr : numActOut, maxNumActOut, ga);        \
+    else                                                                                                              \
+      hipLaunchKernelGGL((bmScan<ORDERED, GATHER>), perChunk, dim3(GATHER ? kRbChunk : kRbThreads), 0, stream, recBefore, \
+                         w.nRecords, chunkBase, w.nChunks, scanTicket, scanTicket + 1, subM ? nullptr : numActOut,    \
+                         maxNumActOut, ga);                                                                           \
+  } while (0)
     const bool ordered = debugEnv("D3D_RULEBOOK_ORDERED_SCAN") != nullptr;
     if (sharedMap) {
     } else if (gather == 1) {

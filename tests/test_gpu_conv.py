@@ -342,6 +342,14 @@ def test_pipelined_tile_shapes_by_row_count(engine, cin, cout):
         run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, ("float16", "bfloat16")[k % 2], True, relu=True)
 
 
+@pytest.mark.parametrize("levels", [1, 13, 14])
+def test_map_sizes_around_the_scan_forms(engine, levels):
+    """Occupancy maps of 50 x 50 bricks per level, on both sides of the 32 768 records at which their scan takes another
+    form, as the map of a SubM layer and of a strided one."""
+    run_case(3000, (levels, 400, 400), (3, 3, 3), (1, 1, 1), (1, 1, 1), 16, 16, "float16", True)
+    run_case(3000, (2 * levels - 1, 800, 800), (3, 3, 3), (2, 2, 2), (1, 1, 1), 16, 16, "float16", False)
+
+
 @pytest.mark.parametrize("cfg", ["off", "4,8,2", "2,8,3", "2,8,2", "4,4,2", "4,4,3", "4,8,3,1", "2,8,3,1"])
 @pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128), (128, 16)])
 def test_staged_configurations(engine, monkeypatch, cfg, cin, cout):
