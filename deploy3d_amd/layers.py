@@ -172,8 +172,9 @@ class SparseBackbone:
         self.index_tensors = index_tensors
         self.overlap = overlap
         self._side = None
-        self._plans = {}        # buffers of the input -> the pass on them as a native schedule (None: not possible)
-        self._last, self._repeats = None, 0
+        self._plans = {}        # buffers of the input -> the pass on them as a native schedule (False: not possible)
+        self._last = None       # (buffers of the input, what was made on them) of the pass before, if ``forward`` made it
+        self._repeats = 0       # passes on those buffers in a row before it
 
     def forward(self, x):
         """One pass on ``x``; returns the last layer's SparseTensor (every layer's is in ``outputs``).
@@ -184,24 +185,34 @@ class SparseBackbone:
         first).  Other buffers, and a stream that is being captured, take the operators one by one."""
         if torch.cuda.is_current_stream_capturing():
             return self._forward_steps(x)
-        key = (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr(), x.feats.shape, x.feats.dtype, x.coors.shape,
-               x.batch, tuple(x.grid), id(x.producer))
+        key = self._buffers_of(x)
         plan = self._plans.get(key)
-        self._repeats = self._repeats + 1 if key == self._last else 0
+        again = self._last is not None and self._last[0] == key
+        self._repeats = self._repeats + 1 if again else 0
         if plan is None and self._repeats >= 2:
             if len(self._plans) >= self._PLANS:
                 self._plans.pop(next(iter(self._plans)))
-            plan = self._plans[key] = self._record(x)
-        self._last = key
+            plan = self._plans[key] = self._record(self._last[1])
         if not plan:
-            return self._forward_steps(x)
-        sched, self.rulebooks, self.inputs, self.outputs = plan
+            y = self._forward_steps(x)
+            self._last = (key, (self.rulebooks, self.inputs, self.outputs))
+            return y
+        sched, made = plan
+        self.rulebooks, self.inputs, self.outputs = made
+        self._last = (key, made)
         sched.run()
         return self.outputs[self.specs[-1]["name"]]
 
     _PLANS = 4  # sets of input buffers whose passes are kept as schedules
 
+    @staticmethod
+    def _buffers_of(x):
+        """What a recorded pass on ``x`` depends on besides the contents of its tensors."""
+        return (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr(), x.feats.shape, x.feats.dtype,
+                x.coors.shape, x.batch, tuple(x.grid), id(x.producer))
+
     def _forward_steps(self, x):
+        self._last = None  # a capture or a schedule of the caller's is not a pass that ``forward`` repeats
         main = side = None
         if self.overlap:
             if self._side is None:  # strided rulebooks feed each other; SubM rulebooks hang off them
@@ -264,22 +275,23 @@ class SparseBackbone:
 
 
     # -- the pass as one native call -------------------------------------------------------------------------
-    def _record(self, x):
-        """The pass just made on ``x`` as a native schedule: convolutions and sums on lane 0 (the caller's stream),
-        strided rulebooks on lane 1, SubM rulebooks on lane 2; a convolution waits for its rulebook, a SubM rulebook
-        for the strided rulebook that wrote its coordinates (directly - no detour through the main stream, which only
-        stream capture needs).  Returns (schedule, rulebooks, inputs, outputs), or False when the pass holds something
-        a schedule does not (a sum of int8 maps, buffers replaced since)."""
+    def _record(self, made):
+        """A pass - ``made`` is the (rulebooks, inputs, outputs) it left behind - as a native schedule: convolutions and
+        sums on lane 0 (the caller's stream), strided rulebooks on lane 1, SubM rulebooks on lane 2; a convolution waits
+        for its rulebook, a SubM rulebook for the strided rulebook that wrote its coordinates (directly - no detour
+        through the main stream, which only stream capture needs).  Returns (schedule, made), or False when the pass
+        holds something a schedule does not (a sum of int8 maps, buffers replaced since)."""
+        rulebooks, inputs, outputs = made
         lanes = (0, 1, 2) if self.overlap else (0, 0, 0)
         sched = Schedule(lanes=3 if self.overlap else 1)
         rb_step, by_plugin = {}, {}
         for spec, lyr in zip(self.specs, self.layers):
-            inp, out = self.inputs[spec["name"]], self.outputs[spec["name"]]
+            inp, out = inputs[spec["name"]], outputs[spec["name"]]
             key = spec["key"]
-            rb = self.rulebooks[key]
+            rb = rulebooks[key]
             src = spec.get("src") or ""
             if "+" in src:
-                a, b = (self.outputs[s].feats for s in src.split("+"))
+                a, b = (outputs[s].feats for s in src.split("+"))
                 if a.dtype not in (torch.float32, torch.float16, torch.bfloat16) or a.shape != b.shape:
                     return False
                 sched.add_sum(a, b, inp.feats, lane=lanes[0])
@@ -298,7 +310,7 @@ class SparseBackbone:
                 return False
             sched.add(lyr.mm_plugin, st["in_descs"], st["out_descs"], [inp.feats, num_in, num_out, rb.index, rb.num_index],
                       [st["out"]], None, lane=lanes[0], after=[rb_step[key]])
-        return sched, self.rulebooks, self.inputs, self.outputs
+        return sched, made
 
     def build_schedule(self, x):
         """Records the pass on ``x`` as a native schedule (see _record).  Runs one ordinary pass first so that every
@@ -307,18 +319,20 @@ class SparseBackbone:
             raise NotImplementedError("a schedule holds operator steps only; this chain adds feature maps in between")
         self._forward_steps(x)
         overlap, self.overlap = self.overlap, True
-        sched = self._record(x)[0]
+        sched, made = self._record((self.rulebooks, self.inputs, self.outputs))
         self.overlap = overlap
-        self._schedule = (sched, (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr()))
+        self._schedule = (sched, self._buffers_of(x), made)
         return sched
 
     def forward_scheduled(self, x):
         """The pass through the native schedule (recorded at the first call, and again when ``x`` is another set of
         buffers); same output tensors as ``forward``."""
-        sig = (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr())
-        if getattr(self, "_schedule", None) is None or self._schedule[1] != sig:
+        if getattr(self, "_schedule", None) is None or self._schedule[1] != self._buffers_of(x):
             self.build_schedule(x)
-        self._schedule[0].run()
+        sched, _, made = self._schedule
+        self.rulebooks, self.inputs, self.outputs = made
+        self._last = None
+        sched.run()
         return self.outputs[self.specs[-1]["name"]]
 
 

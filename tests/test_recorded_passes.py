@@ -1,0 +1,124 @@
+"""Which pass a recorded schedule holds, on the CPU: the operators and the schedule are replaced by stand-ins that run on host
+tensors (a convolution fills its output with one more than the mean of its input, so every result names the input it came
+from), everything else - buffers, keys, what is recorded when and what is handed out - is the product's own code."""
+import numpy as np
+import pytest
+import torch
+
+from deploy3d_amd import layers, onnx_graph, plugin, synth
+
+GRID = (4, 8, 8)
+
+
+def _apply(op, inputs, outputs):
+    if op.name == "SPConvMM":
+        outputs[0].fill_(float(inputs[0].float().mean()) + 1)
+
+
+class _HostSchedule(plugin.Schedule):
+    def __init__(self, lanes=1, **options):
+        super().__init__(lanes=1, **options)  # one lane needs no device
+
+    def add(self, op, in_descs, out_descs, inputs, outputs, workspace=None, lane=0, after=()):
+        self._steps = getattr(self, "_steps", []) + [lambda: _apply(op, inputs, outputs)]
+        return super().add(op, in_descs, out_descs, inputs, outputs, workspace, 0, after)
+
+    def add_sum(self, a, b, out, lane=0, after=()):
+        n = a.numel()
+        flat = lambda t: torch.as_strided(t, (n,), (1,))  # noqa: E731  (the step knows an address and a count)
+        self._steps = getattr(self, "_steps", []) + [lambda: torch.add(flat(a), flat(b), out=flat(out))]
+        return super().add_sum(a, b, out, 0, after)
+
+    def add_cast(self, a, out, lane=0, after=()):
+        n = a.numel()
+        self._steps = getattr(self, "_steps", []) + [
+            lambda: torch.as_strided(out, (n,), (1,)).copy_(torch.as_strided(a, (n,), (1,)))]
+        return super().add_cast(a, out, 0, after)
+
+    def run(self, stream=None):
+        for step in self._steps:
+            step()
+
+
+@pytest.fixture
+def host(monkeypatch):
+    """The stand-ins; ``host.capturing`` is what the stream is asked."""
+    class State:
+        capturing = False
+    monkeypatch.setattr(plugin.Launch, "__call__", lambda self, ins, outs, ws, stream: _apply(self.plugin, ins, outs))
+    monkeypatch.setattr(plugin.Plugin, "configure", lambda self, *a: None)
+    monkeypatch.setattr(plugin.Plugin, "set_option", lambda self, *a: None)
+    monkeypatch.setattr(plugin.Plugin, "link_rulebook", lambda self, *a: None)
+    monkeypatch.setattr(plugin.Plugin, "enqueue", lambda self, ind, outd, ins, outs, ws=None, stream=None:
+                        _apply(self, ins, outs))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: State.capturing)
+    for module in (layers, onnx_graph):
+        monkeypatch.setattr(module, "Schedule", _HostSchedule)
+    monkeypatch.setattr(layers, "current_stream", lambda *a: 0)
+    return State
+
+
+def _specs(last_sum=False):
+    p = dict(padding=(1, 1, 1))
+    specs = [synth.layer("a", "s", True, (3, 3, 3), 4, 4, **p), synth.layer("b", "s", True, (3, 3, 3), 4, 4, **p)]
+    if last_sum:
+        specs.append(synth.layer("c", "s", True, (3, 3, 3), 4, 4, src="b+input", **p))
+    return specs
+
+
+def _net(specs, rows=16):
+    weights = [synth.layer_weights(0, i, s) for i, s in enumerate(specs)]
+    net = layers.SparseBackbone(specs, weights, [rows] * len(specs), dtype=torch.float32, device="cpu", overlap=False,
+                                extensions=False)
+    for lyr in net.layers:  # one lane of host tensors
+        lyr.device = "cpu"
+    return net
+
+
+def _input(value, rows=16):
+    coords = np.zeros((rows, 4), np.int32)
+    return layers.make_input(coords, np.full((rows, 4), value, np.float32), GRID, dtype=torch.float32, device="cpu")
+
+
+def _expect(y, value, convolutions=2):
+    assert float(y.feats.min()) == float(y.feats.max()) == value + convolutions
+
+
+@pytest.mark.parametrize("between", ["capture", "scheduled", "build", "steps"])
+def test_a_recorded_pass_reads_its_own_input(host, between):
+    """Warm up on ``a``, make one pass on other buffers in another way, go on with ``a``: every result is of its input."""
+    net, a, static = _net(_specs()), _input(10.0), _input(500.0)
+    _expect(net.forward(a), 10.0)
+    _expect(net.forward(a), 10.0)
+    if between == "capture":
+        host.capturing = True
+        _expect(net.forward(static), 500.0)
+        host.capturing = False
+    elif between == "scheduled":
+        _expect(net.forward_scheduled(static), 500.0)
+    elif between == "build":
+        net.build_schedule(static)
+    else:
+        net._forward_steps(static)
+    for _ in range(6):
+        y = net.forward(a)
+        _expect(y, 10.0)
+        assert y.coors is a.coors and net.outputs["input"].feats is a.feats
+    assert any(net._plans.values())  # the pass did become a schedule
+
+
+def test_a_scheduled_pass_hands_out_its_own_tensors(host):
+    net, a, b = _net(_specs()), _input(10.0), _input(500.0)
+    net.forward_scheduled(a)
+    _expect(net.forward(b), 500.0)
+    y = net.forward_scheduled(a)
+    _expect(y, 10.0)
+    assert y.coors is a.coors and net.inputs["a"].feats is a.feats
+
+
+def test_a_schedule_is_not_reused_for_other_shapes_at_the_same_address(host):
+    net, whole = _net(_specs()), _input(10.0, rows=32)
+    part = layers.SparseTensor(whole.feats[:16], whole.coors[:16], whole.num_act, GRID)
+    for x in (whole, part, whole):
+        net.forward_scheduled(x)
+        assert net.inputs["a"].feats.shape == x.feats.shape
