@@ -208,8 +208,8 @@ class SparseBackbone:
     @staticmethod
     def _buffers_of(x):
         """What a recorded pass on ``x`` depends on besides the contents of its tensors."""
-        return (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr(), x.feats.shape, x.feats.dtype,
-                x.coors.shape, x.batch, tuple(x.grid), id(x.producer))
+        return (x.feats.data_ptr(), x.coors.data_ptr(), x.num_act.data_ptr(), x.feats.shape, x.feats.stride(),
+                x.feats.dtype, x.coors.shape, x.coors.stride(), x.batch, tuple(x.grid), id(x.producer))
 
     def _forward_steps(self, x):
         self._last = None  # a capture or a schedule of the caller's is not a pass that ``forward`` repeats
@@ -280,7 +280,8 @@ class SparseBackbone:
         sums on lane 0 (the caller's stream), strided rulebooks on lane 1, SubM rulebooks on lane 2; a convolution waits
         for its rulebook, a SubM rulebook for the strided rulebook that wrote its coordinates (directly - no detour
         through the main stream, which only stream capture needs).  Returns (schedule, made), or False when the pass
-        holds something a schedule does not (a sum of int8 maps, buffers replaced since)."""
+        holds something a schedule does not (a sum of int8 maps, of two types or of strided views; buffers
+        replaced since)."""
         rulebooks, inputs, outputs = made
         lanes = (0, 1, 2) if self.overlap else (0, 0, 0)
         sched = Schedule(lanes=3 if self.overlap else 1)
@@ -292,7 +293,7 @@ class SparseBackbone:
             src = spec.get("src") or ""
             if "+" in src:
                 a, b = (outputs[s].feats for s in src.split("+"))
-                if a.dtype not in (torch.float32, torch.float16, torch.bfloat16) or a.shape != b.shape:
+                if not Schedule.holds_sum(a, b, inp.feats):
                     return False
                 sched.add_sum(a, b, inp.feats, lane=lanes[0])
             if key not in rb_step:

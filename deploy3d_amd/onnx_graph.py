@@ -446,8 +446,11 @@ class GraphExecutor:
             for name, t in zip(n.outputs, outs):
                 values[name] = t
             plan.append(("plugin", p, in_descs, out_descs, ins, outs, ws))
-        self._bound = dict(shapes={k: (tuple(v.shape), v.dtype, v.data_ptr()) for k, v in inputs.items()},
-                           values=values, plan=plan)
+        self._bound = dict(signature=self._signature(inputs), values=values, plan=plan)
+
+    @staticmethod
+    def _signature(inputs):
+        return {k: (tuple(v.shape), v.stride(), v.dtype, v.data_ptr()) for k, v in inputs.items()}
 
     def run(self, **inputs):
         """inputs: name -> device tensor for every graph input (a zero-element tensor for a spatial shape).
@@ -455,8 +458,7 @@ class GraphExecutor:
         missing = [v.name for v in self.model.inputs if v.name not in inputs]
         if missing:
             raise ValueError("missing graph inputs: %s" % missing)
-        sig = {k: (tuple(v.shape), v.dtype, v.data_ptr()) for k, v in inputs.items()}
-        if self._bound is None or self._bound["shapes"] != sig:
+        if self._bound is None or self._bound["signature"] != self._signature(inputs):
             self._bind(inputs)
         elif not torch.cuda.is_current_stream_capturing():
             # the third pass on the same buffers and later ones: a native schedule, one graph launch from its third run
@@ -482,18 +484,18 @@ class GraphExecutor:
     def _record(self):
         """The bound graph as a native schedule: every node a step that waits for the steps its inputs come from,
         rulebook nodes on lanes of their own (strided 1, SubM 2), everything else on lane 0.  None when a node is
-        something a schedule does not hold (a sum of int8 maps, a cast that is not from float to a 2-byte type)."""
+        something a schedule does not hold (a sum of int8 maps, a cast that is not from float to a 2-byte type, either of
+        a strided view)."""
         sched = Schedule(lanes=3)
         made = {}  # tensor name -> step that writes it
         for n, step in zip(self.nodes, self._bound["plan"]):
             after = sorted({made[name] for name in n.inputs if name in made})
             if step[0] == "add":
-                a, b = step[1]
-                if a.dtype not in (torch.float32, torch.float16, torch.bfloat16) or a.shape != b.shape or a.dtype != b.dtype:
+                if not Schedule.holds_sum(*step[1], step[2]):
                     return None
-                at = sched.add_sum(a, b, step[2], after=after)
+                at = sched.add_sum(*step[1], step[2], after=after)
             elif step[0] == "cast":
-                if step[1][0].dtype != torch.float32 or step[2].dtype not in (torch.float16, torch.bfloat16):
+                if not Schedule.holds_cast(step[1][0], step[2]):
                     return None
                 at = sched.add_cast(step[1][0], step[2], after=after)
             else:
@@ -510,8 +512,7 @@ class GraphExecutor:
         """``run`` through a native schedule (d3d_schedule_*): every node becomes a step that waits for the steps
         its inputs come from; rulebook nodes get lanes of their own (strided 1, SubM 2), everything else runs on
         the current stream.  Graphs of plugin nodes only (an ``Add`` needs the step-by-step ``run``)."""
-        sig = {k: (tuple(v.shape), v.dtype, v.data_ptr()) for k, v in inputs.items()}
-        if self._bound is None or self._bound["shapes"] != sig:
+        if self._bound is None or self._bound["signature"] != self._signature(inputs):
             self.run(**inputs)  # binds, and brings every operator's buffers into being
         if "schedule" not in self._bound:
             if any(step[0] != "plugin" for step in self._bound["plan"]):

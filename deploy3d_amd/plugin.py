@@ -338,14 +338,27 @@ class Schedule:
                                         _pointers(outputs), ws_ptr, ws_bytes, int(lane), *self._after(after))
         return self._appended(rc, (plugin, list(inputs), list(outputs), workspace))
 
+    @staticmethod
+    def holds_sum(a, b, out):
+        """Whether ``add_sum`` does what ``torch.add(a, b, out=out)`` does: a step knows addresses and a count, so it takes
+        tensors of one shape and type that lie in memory in the order of their elements."""
+        return (a.dtype in (torch.float32, torch.float16, torch.bfloat16) and a.dtype == b.dtype == out.dtype and
+                a.shape == b.shape == out.shape and a.is_contiguous() and b.is_contiguous() and out.is_contiguous())
+
+    @staticmethod
+    def holds_cast(a, out):
+        """Whether ``add_cast`` does what ``out.copy_(a)`` does (see holds_sum)."""
+        return (a.dtype == torch.float32 and out.dtype in (torch.float16, torch.bfloat16) and a.shape == out.shape and
+                a.is_contiguous() and out.is_contiguous())
+
     def add_sum(self, a, b, out, lane=0, after=()):
-        """Appends ``out = a + b`` (float32 / float16 / bfloat16 tensors of one shape)."""
+        """Appends ``out = a + b`` (tensors that ``holds_sum``)."""
         rc = self._lib.d3d_schedule_add_sum(self._h, _TORCH_TO_D3D[a.dtype], a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                             a.numel(), int(lane), *self._after(after))
         return self._appended(rc, (a, b, out))
 
     def add_cast(self, a, out, lane=0, after=()):
-        """Appends ``out = a.to(out.dtype)`` (a float32, out float16 / bfloat16)."""
+        """Appends ``out = a.to(out.dtype)`` (tensors that ``holds_cast``)."""
         rc = self._lib.d3d_schedule_add_cast(self._h, _TORCH_TO_D3D[out.dtype], a.data_ptr(), out.data_ptr(), a.numel(),
                                              int(lane), *self._after(after))
         return self._appended(rc, (a, out))

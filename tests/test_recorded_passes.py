@@ -122,3 +122,48 @@ def test_a_schedule_is_not_reused_for_other_shapes_at_the_same_address(host):
     for x in (whole, part, whole):
         net.forward_scheduled(x)
         assert net.inputs["a"].feats.shape == x.feats.shape
+
+
+def test_a_sum_of_strided_features_is_not_recorded(host):
+    """torch adds views of any stride; a schedule's sum step reads memory in order, so such a pass stays step by step."""
+    net, x = _net(_specs(last_sum=True)), _input(0.0)
+    wide = torch.zeros(16, 8)
+    wide[:, :4] = 10.0
+    wide[:, 4:] = 1000.0
+    x.feats = wide[:, :4]
+    for _ in range(5):
+        y = net.forward(x)
+        assert float(y.feats.max()) == 10.0 + 2 + 10.0 + 1
+    assert not any(net._plans.values())
+
+
+@pytest.mark.parametrize("node", ["Cast", "Add"])
+@pytest.mark.parametrize("view", ["columns", "transposed", "plain"])
+def test_elementwise_nodes_of_graph_inputs_that_are_views(host, node, view):
+    """Runs on one binding become a schedule from the third on; a Cast or an Add of a strided view stays what torch makes
+    of it, run after run, with contents that change in between.  Dense tensors do become steps."""
+    base = torch.empty(16, 16)
+    x = {"columns": base[:, 4:8], "transposed": base.t(), "plain": base}[view]
+    elem = onnx_graph.FLOAT
+    make = onnx_graph.Node("Cast", ["x"], ["y"], dict(to=onnx_graph.FLOAT16)) if node == "Cast" else \
+        onnx_graph.Node("Add", ["x", "z"], ["y"])
+    names = ["x"] if node == "Cast" else ["x", "z"]
+    model = onnx_graph.Model([make], [onnx_graph.Value(n, elem, list(x.shape)) for n in names],
+                             [onnx_graph.Value("y", elem, list(x.shape))])
+    ex = onnx_graph.GraphExecutor(model, device="cpu")
+    z = torch.arange(float(x.numel())).reshape(x.shape)
+    for i in range(8):
+        base.copy_(torch.randn(16, 16, generator=torch.Generator().manual_seed(i)))
+        y = ex.run(**dict(x=x, z=z) if node == "Add" else dict(x=x))["y"]
+        assert torch.equal(y, x.half() if node == "Cast" else x + z)
+    assert (ex._bound["native"] is not None) == (view == "plain")
+
+
+def test_a_view_of_other_strides_at_the_same_address_is_bound_anew(host):
+    base = torch.randn(16, 16, generator=torch.Generator().manual_seed(0))
+    model = onnx_graph.Model([onnx_graph.Node("Cast", ["x"], ["y"], dict(to=onnx_graph.FLOAT16))],
+                             [onnx_graph.Value("x", onnx_graph.FLOAT, [16, 16])],
+                             [onnx_graph.Value("y", onnx_graph.FLOAT16, [16, 16])])
+    ex = onnx_graph.GraphExecutor(model, device="cpu")
+    for x in (base, base.t(), base, base.t()):
+        assert torch.equal(ex.run(x=x)["y"], x.half())
