@@ -167,3 +167,29 @@ def test_a_view_of_other_strides_at_the_same_address_is_bound_anew(host):
     ex = onnx_graph.GraphExecutor(model, device="cpu")
     for x in (base, base.t(), base, base.t()):
         assert torch.equal(ex.run(x=x)["y"], x.half())
+
+
+def test_results_are_the_callers_own_objects(host):
+    """Rebinding tensors on what a pass returned, on its outputs or rulebooks, or on the input afterwards, reaches neither
+    the recorded pass nor a later result - while passes run step by step, when they are recorded, and after."""
+    net, x = _net(_specs(last_sum=True)), _input(10.0)
+    seen = []
+    for _ in range(8):
+        y = net.forward(x)
+        assert y is net.outputs["c"] and net.outputs["input"] is x and net.inputs["b"] is net.outputs["a"]
+        _expect(y, 10.0, 2 + 10 + 1)
+        assert all(y is not s for s in seen)
+        seen.append(y)
+        y.feats = y.feats.double() * 0 - 1                 # a float copy, say
+        net.outputs["a"].feats = torch.full((16, 4), 99.0)
+        net.outputs["b"].coors = None
+        net.rulebooks["s"].num_act_in = None
+        net.outputs.clear()
+    assert any(net._plans.values())
+    feats, same = x.feats, layers.SparseTensor(x.feats, x.coors, x.num_act, GRID)
+    net = _net(_specs())
+    net.forward(x)
+    net.forward(x)
+    x.feats = torch.full((16, 4), 700.0)                   # the object now names other features, `same` the old ones
+    for _ in range(4):
+        _expect(net.forward(same), float(feats[0, 0]))
