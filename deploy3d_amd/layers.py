@@ -10,6 +10,7 @@ import copy
 
 import numpy as np
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from .plugin import OPT_INDEX_UNUSED, OPT_PERSISTENT_INDEX, Launch, Plugin, Schedule, TensorDesc, current_stream
 from .spconv_index import index_blob
@@ -132,6 +133,32 @@ class SparseConvLayer:
                             x.producer if self.spec["subm"] else rb.plugin)
 
 
+class _Plan:
+    """A recorded pass of SparseBackbone.forward: its schedule and what the pass left behind.  Neither keeps the input's
+    tensors alive - in ``made`` their names stand for them - so a caller who drops an input gets its memory back, and a
+    plan whose input is gone (``expired``) is never run: another tensor may have its address by then."""
+
+    def __init__(self, schedule, made):
+        rulebooks, inputs, outputs = made
+        x = outputs["input"]
+        name_of = {id(getattr(x, name)): name for name in ("feats", "coors", "num_act")}
+        without = {}
+
+        def named(t):
+            if id(t) not in without:
+                without[id(t)] = copy.copy(t)
+                vars(without[id(t)]).update((k, name_of[id(v)]) for k, v in vars(t).items() if id(v) in name_of)
+            return without[id(t)]
+
+        self.made = tuple({k: named(t) for k, t in part.items()} for part in made)
+        self._storages = [StorageWeakRef(getattr(x, name).untyped_storage()) for name in ("feats", "coors", "num_act")]
+        self.schedule = schedule
+        schedule.release((x.feats, x.coors, x.num_act))
+
+    def expired(self):
+        return any(s.expired() for s in self._storages)
+
+
 class SparseBackbone:
     """A chain (or small DAG, via ``src``) of SparseConvLayers sharing rulebooks by indice key.
 
@@ -189,20 +216,25 @@ class SparseBackbone:
             return self._forward_steps(x)
         key = self._buffers_of(x)
         plan = self._plans.get(key)
+        if not plan or plan.expired():
+            for k in [k for k, p in self._plans.items() if p and p.expired()]:
+                del self._plans[k]
+                self._last = None
+            plan = self._plans.get(key)
         again = self._last is not None and self._last[0] == key
         self._repeats = self._repeats + 1 if again else 0
         if plan is None and self._repeats >= 2:
             if len(self._plans) >= self._PLANS:
                 self._plans.pop(next(iter(self._plans)))
-            plan = self._plans[key] = self._record(self._last[1])
+            sched = self._record(self._last[1])
+            plan = self._plans[key] = sched and _Plan(sched, self._last[1])
         if not plan:
             y = self._forward_steps(x)
             self._last = (key, self._made)
             return y
-        sched, made = plan
-        self._last = (key, made)
-        sched.run()
-        return self._hand_out(made, x)
+        self._last = (key, None)
+        plan.schedule.run()
+        return self._hand_out(plan.made, x)
 
     # What a pass left behind goes to the caller as objects of that pass's own (over the same tensors): what is rebound on
     # a result is neither in what is recorded nor in the next pass's result.  Made when asked for: 70 us of a VoxelNet pass.
@@ -210,12 +242,18 @@ class SparseBackbone:
         """``made``, a pass on the buffers of ``x``, is the pass whose results are shown; returns its last SparseTensor."""
         self._made, self._shown = made, {}
         self._own_of = {id(made[2]["input"]): x}
+        self._input = dict(feats=x.feats, coors=x.coors, num_act=x.num_act)
         return self._own(made[2][self.specs[-1]["name"]])
 
     def _own(self, t):
         own = self._own_of.get(id(t))
         if own is None:
-            own = self._own_of[id(t)] = SparseTensor(t.feats, t.coors, t.num_act, t.grid, t.batch, t.producer)
+            own = self._own_of[id(t)] = copy.copy(t)
+            for name, v in vars(own).items():
+                if type(v) is str:  # a tensor of the input (see _Plan)
+                    setattr(own, name, self._input[v])
+            if isinstance(own, SparseTensor):
+                own.grid = list(t.grid)
         return own
 
     def _show(self, which, own):
@@ -226,7 +264,7 @@ class SparseBackbone:
     @property
     def rulebooks(self):
         """Indice key -> Rulebook of the latest pass."""
-        return self._show(0, copy.copy)
+        return self._show(0, self._own)
 
     @property
     def inputs(self):
@@ -310,9 +348,8 @@ class SparseBackbone:
         """A pass - ``made`` is the (rulebooks, inputs, outputs) it left behind - as a native schedule: convolutions and
         sums on lane 0 (the caller's stream), strided rulebooks on lane 1, SubM rulebooks on lane 2; a convolution waits
         for its rulebook, a SubM rulebook for the strided rulebook that wrote its coordinates (directly - no detour
-        through the main stream, which only stream capture needs).  Returns (schedule, made), or False when the pass
-        holds something a schedule does not (a sum of int8 maps, of two types or of strided views; buffers
-        replaced since)."""
+        through the main stream, which only stream capture needs).  Returns the schedule, or False when the pass holds
+        something a schedule does not (a sum of int8 maps, of two types or of strided views; buffers replaced since)."""
         rulebooks, inputs, outputs = made
         lanes = (0, 1, 2) if self.overlap else (0, 0, 0)
         sched = Schedule(lanes=3 if self.overlap else 1)
@@ -342,7 +379,7 @@ class SparseBackbone:
                 return False
             sched.add(lyr.mm_plugin, st["in_descs"], st["out_descs"], [inp.feats, num_in, num_out, rb.index, rb.num_index],
                       [st["out"]], None, lane=lanes[0], after=[rb_step[key]])
-        return sched, made
+        return sched
 
     def build_schedule(self, x):
         """Records the pass on ``x`` as a native schedule (see _record).  Runs one ordinary pass first so that every
@@ -351,9 +388,9 @@ class SparseBackbone:
             raise NotImplementedError("a schedule holds operator steps only; this chain adds feature maps in between")
         self._forward_steps(x)
         overlap, self.overlap = self.overlap, True
-        sched, made = self._record(self._made)
+        sched = self._record(self._made)
         self.overlap = overlap
-        self._schedule = (sched, self._buffers_of(x), made)
+        self._schedule = (sched, self._buffers_of(x), self._made)
         return sched
 
     def forward_scheduled(self, x):

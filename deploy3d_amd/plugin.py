@@ -336,7 +336,7 @@ class Schedule:
         rc = self._lib.d3d_schedule_add(self._h, plugin._h, _desc_array(in_descs), len(in_descs),
                                         _desc_array(out_descs), len(out_descs), _pointers(inputs),
                                         _pointers(outputs), ws_ptr, ws_bytes, int(lane), *self._after(after))
-        return self._appended(rc, (plugin, list(inputs), list(outputs), workspace))
+        return self._appended(rc, (plugin, *inputs, *outputs, workspace))
 
     @staticmethod
     def holds_sum(a, b, out):
@@ -370,8 +370,12 @@ class Schedule:
     def _appended(self, rc, kept):
         if rc < 0:
             _check(rc)
-        self._keep.append(kept)
+        self._keep.extend(k for k in kept if k is not None)
         return rc
+
+    def release(self, tensors):
+        """Stops keeping ``tensors`` alive: whoever runs the schedule from now on answers for them."""
+        self._keep = [k for k in self._keep if all(k is not t for t in tensors)]
 
     def __len__(self):
         return int(self._lib.d3d_schedule_size(self._h))

@@ -1,6 +1,9 @@
 """Which pass a recorded schedule holds, on the CPU: the operators and the schedule are replaced by stand-ins that run on host
 tensors (a convolution fills its output with one more than the mean of its input, so every result names the input it came
 from), everything else - buffers, keys, what is recorded when and what is handed out - is the product's own code."""
+import ctypes
+import weakref
+
 import numpy as np
 import pytest
 import torch
@@ -15,24 +18,32 @@ def _apply(op, inputs, outputs):
         outputs[0].fill_(float(inputs[0].float().mean()) + 1)
 
 
+def _bytes_of(t):
+    """The elements at a tensor's address in memory order: all that a step of a schedule knows of a tensor."""
+    if t is None or t.numel() == 0:
+        return None
+    raw = (ctypes.c_byte * (t.numel() * t.element_size())).from_address(t.data_ptr())
+    return torch.frombuffer(raw, dtype=t.dtype)
+
+
 class _HostSchedule(plugin.Schedule):
     def __init__(self, lanes=1, **options):
         super().__init__(lanes=1, **options)  # one lane needs no device
+        self._steps = []
 
     def add(self, op, in_descs, out_descs, inputs, outputs, workspace=None, lane=0, after=()):
-        self._steps = getattr(self, "_steps", []) + [lambda: _apply(op, inputs, outputs)]
+        ins, outs = [_bytes_of(t) for t in inputs], [_bytes_of(t) for t in outputs]
+        self._steps.append(lambda: _apply(op, ins, outs))
         return super().add(op, in_descs, out_descs, inputs, outputs, workspace, 0, after)
 
     def add_sum(self, a, b, out, lane=0, after=()):
-        n = a.numel()
-        flat = lambda t: torch.as_strided(t, (n,), (1,))  # noqa: E731  (the step knows an address and a count)
-        self._steps = getattr(self, "_steps", []) + [lambda: torch.add(flat(a), flat(b), out=flat(out))]
+        x, y, z = _bytes_of(a), _bytes_of(b), _bytes_of(out)
+        self._steps.append(lambda: torch.add(x, y, out=z))
         return super().add_sum(a, b, out, 0, after)
 
     def add_cast(self, a, out, lane=0, after=()):
-        n = a.numel()
-        self._steps = getattr(self, "_steps", []) + [
-            lambda: torch.as_strided(out, (n,), (1,)).copy_(torch.as_strided(a, (n,), (1,)))]
+        x, y = _bytes_of(a), _bytes_of(out)
+        self._steps.append(lambda: y.copy_(x))
         return super().add_cast(a, out, 0, after)
 
     def run(self, stream=None):
@@ -193,3 +204,32 @@ def test_results_are_the_callers_own_objects(host):
     x.feats = torch.full((16, 4), 700.0)                   # the object now names other features, `same` the old ones
     for _ in range(4):
         _expect(net.forward(same), float(feats[0, 0]))
+
+
+def test_a_recorded_pass_does_not_keep_a_dropped_input(host):
+    """The three tensors of an input that became a schedule are freed with the caller's last reference and the next pass,
+    and a schedule whose input is gone is dropped, also when another input comes to lie at the same addresses."""
+    net, other = _net(_specs(last_sum=True)), _input(500.0)
+    memory = torch.empty(16 * 4 * 8)
+
+    def at_the_same_address(value):
+        feats = torch.from_numpy(memory.numpy()[:64]).view(16, 4)   # a storage of its own over the same bytes
+        feats.fill_(value)
+        x = _input(0.0)
+        return layers.SparseTensor(feats, x.coors, x.num_act, GRID)
+
+    for value in (10.0, 20.0, 30.0):
+        x = at_the_same_address(value)
+        for _ in range(5):
+            _expect(net.forward(x), value, 2 + value + 1)
+        assert any(net._plans.values())
+        gone = [weakref.ref(t) for t in (x.feats, x.coors, x.num_act)]
+        del x
+        net.forward(other)
+        assert all(r() is None for r in gone)
+        net.forward(other)
+        assert not any(net._plans.values())
+    for _ in range(5):
+        y = net.forward(other)
+    assert any(net._plans.values()) and y.coors is other.coors and y.num_act is other.num_act
+    assert net.rulebooks["s"].in_coors is other.coors and net.inputs["a"] is other
