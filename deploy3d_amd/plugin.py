@@ -8,6 +8,7 @@ streams only.
 """
 import ctypes
 import os
+import threading
 
 import torch
 
@@ -159,16 +160,23 @@ def _pointers(tensors):
         t.data_ptr() if t is not None and t.numel() else None for t in tensors])
 
 
-_scratch = {}
+_scratch = threading.local()
 
 
 def scratch(nbytes, device, stream):
-    """Workspace of the functional operators: one buffer per stream, grown to the largest request (kernels of one stream
-    run in order, so consecutive calls may share it)."""
+    """Workspace of a functional operator's call on ``stream``, the current stream of ``device``.
+
+    One buffer per thread and stream, grown to the largest request: the calls a thread makes on one stream run in order,
+    so they may share it; those of two threads interleave launch by launch.  A call under stream capture gets memory of its
+    own, from the pool of the graph that is being captured: the graph reads and writes it for as long as it is replayed,
+    whatever later calls need."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    buffers = vars(_scratch)
     key = (device, stream)
-    ws = _scratch.get(key)
+    ws = buffers.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = _scratch[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+        ws = buffers[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     return ws
 
 
