@@ -14,10 +14,16 @@
 // waits for (explicit dependencies, no cross-stream events), and a run is one graph launch.  A pass of a small scan (36
 // launches, 9 000 voxels) costs the host 415 us step by step on three lanes - more than its kernels take - and 195 as a
 // graph; the device then takes 345 us.  The graph is dropped when an operator reports a change (pluginChanges).
+//
+// A dropped graph is destroyed once its last launch has run, which an event behind every launch tells: dropping one neither
+// waits nor synchronises the device, so it is also allowed while the caller captures a stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -46,6 +52,7 @@ struct d3d_schedule {
   std::vector<Step> steps;
   // the pass as a graph
   hipGraphExec_t graph = nullptr;
+  hipEvent_t graphRan = nullptr; // behind the last launch of the graph
   uint64_t graphChanges = 0;    // the operators' change count the graph was captured at
   uint64_t lastChanges = ~0ull; // ... and at the end of the last run
   int steady = 0;               // runs in a row that changed nothing
@@ -77,11 +84,56 @@ uint64_t changesOf(const d3d_schedule* s) {
   return sum;
 }
 
+// The calls below are legal while some other stream is being captured in the global mode only from a thread in the relaxed
+// mode; from any other they fail and spoil that capture.  None of them touches a capturing stream.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Graphs that no schedule launches any more, until their last launch has run.  Lives until the process ends.
+struct Retired {
+  std::mutex mutex;
+  std::atomic<size_t> count{0};
+  std::vector<std::pair<hipGraphExec_t, hipEvent_t>> graphs;
+};
+Retired& retired() {
+  static Retired* r = new Retired();
+  return *r;
+}
+
+// Destroys the retired graphs that have run.
+void reapGraphs() {
+  Retired& r = retired();
+  if (r.count.load(std::memory_order_relaxed) == 0) return;
+  const RelaxedCapture relaxed;
+  std::lock_guard<std::mutex> lock(r.mutex);
+  for (size_t i = 0; i < r.graphs.size();) {
+    if (hipEventQuery(r.graphs[i].second) != hipSuccess) {
+      (void)hipGetLastError();  // "not ready" is no error of the caller's
+      ++i;
+      continue;
+    }
+    (void)hipGraphExecDestroy(r.graphs[i].first);
+    (void)hipEventDestroy(r.graphs[i].second);
+    r.graphs[i] = r.graphs.back();
+    r.graphs.pop_back();
+  }
+  r.count.store(r.graphs.size(), std::memory_order_relaxed);
+}
+
 void dropGraph(d3d_schedule* s) {
   if (!s->graph) return;
-  (void)hipDeviceSynchronize();  // a launch of it may still be running
-  (void)hipGraphExecDestroy(s->graph);
+  {
+    Retired& r = retired();
+    std::lock_guard<std::mutex> lock(r.mutex);
+    r.graphs.emplace_back(s->graph, s->graphRan);
+    r.count.store(r.graphs.size(), std::memory_order_relaxed);
+  }
   s->graph = nullptr;
+  s->graphRan = nullptr;
+  reapGraphs();
 }
 
 // Captures every step into one graph, each behind the last nodes of the steps it waits for.  False (and no graph) if
@@ -90,8 +142,15 @@ bool captureGraph(d3d_schedule* s) {
   dropGraph(s);
   hipGraph_t graph = nullptr;
   hipStream_t q = nullptr;
-  if (hipGraphCreate(&graph, 0) != hipSuccess) return false;
-  bool ok = hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
+  bool ok;
+  {
+    const RelaxedCapture relaxed;
+    if (hipGraphCreate(&graph, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    ok = hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
+  }
   const size_t count = s->steps.size();
   std::vector<std::vector<hipGraphNode_t>> tail(count);
   // What each step comes after, directly or not.  A dependency that another one implies gets no edge: every edge
@@ -133,9 +192,15 @@ bool captureGraph(d3d_schedule* s) {
     hipGraph_t same = nullptr;
     ok = hipStreamEndCapture(q, &same) == hipSuccess && ok;
   }
+  const RelaxedCapture relaxed;
+  hipEvent_t ran = nullptr;
+  if (ok) ok = hipEventCreateWithFlags(&ran, hipEventDisableTiming) == hipSuccess;
   if (ok) ok = hipGraphInstantiateWithFlags(&s->graph, graph, 0) == hipSuccess;
-  if (!ok) {
+  if (ok) {
+    s->graphRan = ran;
+  } else {
     s->graph = nullptr;
+    if (ran) (void)hipEventDestroy(ran);
     (void)hipGetLastError();
   }
   (void)hipGraphDestroy(graph);
@@ -182,6 +247,7 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
     return D3D_ERR_BAD_ARG;
   }
   *out = nullptr;
+  reapGraphs();
   auto* s = new d3d_schedule();
   hipError_t e = hipSuccess;
   if (n_lanes > 1) e = hipEventCreateWithFlags(&s->fork, hipEventDisableTiming);  // one lane: no HIP object at all
@@ -201,17 +267,21 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
 
 void d3d_schedule_destroy(d3d_schedule* s) {
   if (!s) return;
-  dropGraph(s);
-  for (auto& st : s->steps)
-    if (st.done) (void)hipEventDestroy(st.done);
-  for (size_t l = 1; l < s->lanes.size(); ++l) {
-    if (s->lanes[l]) {
-      (void)hipStreamSynchronize(s->lanes[l]);
-      (void)hipStreamDestroy(s->lanes[l]);
+  if (s->graph || s->lanes.size() > 1) {
+    const RelaxedCapture relaxed;
+    if (s->graph) (void)hipEventSynchronize(s->graphRan);
+    dropGraph(s);
+    for (auto& st : s->steps)
+      if (st.done) (void)hipEventDestroy(st.done);
+    for (size_t l = 1; l < s->lanes.size(); ++l) {
+      if (s->joined[l]) {  // behind the lane's work of every run
+        (void)hipEventSynchronize(s->joined[l]);
+        (void)hipEventDestroy(s->joined[l]);
+      }
+      if (s->lanes[l]) (void)hipStreamDestroy(s->lanes[l]);
     }
-    if (s->joined[l]) (void)hipEventDestroy(s->joined[l]);
+    if (s->fork) (void)hipEventDestroy(s->fork);
   }
-  if (s->fork) (void)hipEventDestroy(s->fork);
   delete s;
 }
 
@@ -300,6 +370,7 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
     d3d::setError("schedule: the stream is capturing; a schedule runs eagerly");
     return D3D_ERR_UNSUPPORTED;
   }
+  reapGraphs();
   const uint64_t changes = changesOf(s);
   s->steady = s->lastChanges == changes ? s->steady + 1 : 0;
   if (!s->graphRefused && s->steady >= 2 && !(s->graph && s->graphChanges == changes)) {
@@ -314,7 +385,14 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
   if (s->graph && s->graphChanges == changes) {
     s->lastChanges = changes;
     const hipError_t launched = hipGraphLaunch(s->graph, main);
-    return launched == hipSuccess ? D3D_OK : hipFail(launched, "hipGraphLaunch");
+    if (launched != hipSuccess) return hipFail(launched, "hipGraphLaunch");
+    const hipError_t marked = hipEventRecord(s->graphRan, main);
+    if (marked != hipSuccess) {
+      s->graph = nullptr;  // never destroyed: nothing would say when it has run
+      s->graphRan = nullptr;
+      return hipFail(marked, "hipEventRecord");
+    }
+    return D3D_OK;
   }
   hipError_t e = hipSuccess;
   auto laneStream = [&](int lane) { return lane == 0 ? main : s->lanes[static_cast<size_t>(lane)]; };

@@ -231,7 +231,8 @@ int32_t d3d_set_option(d3d_plugin* p, int32_t option, int64_t value);
  *   enqueued.  Refused with
  *   D3D_ERR_UNSUPPORTED while `stream` is capturing (capture the operators' own enqueues instead).  One thread at
  *   a time per schedule.
- * d3d_schedule_destroy: waits for the owned lanes, then frees them; the operators stay the caller's. */
+ * d3d_schedule_destroy: waits for the schedule's own runs, then frees its streams and its graph; the operators stay the
+ *   caller's.  Allowed while another stream is being captured. */
 typedef struct d3d_schedule d3d_schedule;
 int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out);
 int32_t d3d_schedule_add(d3d_schedule* s, d3d_plugin* plugin, const d3d_tensor_desc* in_desc, int32_t nb_in,

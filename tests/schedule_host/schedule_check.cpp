@@ -1,0 +1,203 @@
+// Host check of csrc/schedule.cpp against a stand-in for the HIP runtime that keeps count: work counts as pending until
+// finish() is called, and while `othersCapture` is set a call that synchronises spoils that capture - from a thread that is not
+// in the relaxed mode any such call, from a relaxed one a device-wide wait.  Operators are stand-ins too.  No GPU.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <map>
+#include <set>
+
+#include "common.h"
+#include "d3d_spconv.h"
+
+namespace {
+int pendingWork = 0, graphLaunches = 0, steps = 0, captures = 0, liveGraphs = 0, liveEvents = 0, liveStreams = 0;
+bool othersCapture = false, spoiled = false, destroyedRunning = false, refuseCapture = false, deviceWait = false;
+hipStreamCaptureMode threadMode = hipStreamCaptureModeGlobal;
+uint64_t operatorChanges = 0;
+std::map<void*, bool> eventPending;
+std::set<void*> running;  // graphs launched and not finished
+uintptr_t nextHandle = 16;
+void* fresh() { return reinterpret_cast<void*>(nextHandle += 16); }
+hipError_t unsafe() {
+  if (!othersCapture || threadMode == hipStreamCaptureModeRelaxed) return hipSuccess;
+  spoiled = true;
+  return hipErrorStreamCaptureUnsupported;
+}
+void finish() {
+  pendingWork = 0;
+  running.clear();
+  for (auto& e : eventPending) e.second = false;
+}
+}  // namespace
+
+// ---- the runtime ----
+extern "C" {
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+  const hipStreamCaptureMode was = threadMode;
+  threadMode = *m;
+  *m = was;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() {
+  deviceWait = true;
+  if (othersCapture) {
+    spoiled = true;
+    return hipErrorStreamCaptureUnsupported;
+  }
+  finish();
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = static_cast<hipStream_t>(fresh());
+  ++liveStreams;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) {
+  --liveStreams;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  const hipError_t e = unsafe();
+  if (e == hipSuccess) finish();
+  return e;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = static_cast<hipEvent_t>(fresh());
+  ++liveEvents;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  eventPending.erase(e);
+  --liveEvents;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  eventPending[e] = pendingWork > 0;
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  const hipError_t r = unsafe();
+  return r != hipSuccess ? r : (eventPending[e] ? hipErrorNotReady : hipSuccess);
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  const hipError_t r = unsafe();
+  if (r == hipSuccess && eventPending[e]) finish();
+  return r;
+}
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
+  *st = hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipGraphCreate(hipGraph_t* g, unsigned) {
+  *g = static_cast<hipGraph_t>(fresh());
+  return refuseCapture ? hipErrorStreamCaptureUnsupported : hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipStreamBeginCaptureToGraph(hipStream_t, hipGraph_t, const hipGraphNode_t*, const hipGraphEdgeData*, size_t,
+                                        hipStreamCaptureMode) {
+  return hipSuccess;
+}
+hipError_t hipStreamGetCaptureInfo_v2(hipStream_t, hipStreamCaptureStatus* st, unsigned long long*, hipGraph_t*,
+                                      const hipGraphNode_t** deps, size_t* n) {
+  *st = hipStreamCaptureStatusActive;
+  *deps = nullptr;
+  *n = 0;
+  return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipSuccess; }
+hipError_t hipGraphInstantiateWithFlags(hipGraphExec_t* g, hipGraph_t, unsigned long long) {
+  *g = static_cast<hipGraphExec_t>(fresh());
+  ++captures;
+  ++liveGraphs;
+  return hipSuccess;
+}
+hipError_t hipGraphExecDestroy(hipGraphExec_t g) {
+  if (running.count(g)) destroyedRunning = true;
+  --liveGraphs;
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t g, hipStream_t) {
+  ++graphLaunches;
+  ++pendingWork;
+  running.insert(g);
+  return hipSuccess;
+}
+// ---- the operators ----
+const char* d3d_plugin_type(const d3d_plugin*) { return "BEVDensify"; }
+int32_t d3d_num_outputs(const d3d_plugin*) { return 1; }
+int32_t d3d_enqueue(d3d_plugin*, const d3d_tensor_desc*, const d3d_tensor_desc*, const void* const*, void* const*, void*, size_t,
+                    void*) {
+  ++steps;
+  ++pendingWork;
+  return D3D_OK;
+}
+}
+namespace d3d {
+void setError(const char*, ...) {}
+uint64_t pluginChanges(const d3d_plugin*) { return operatorChanges; }
+int32_t launchSum(int32_t, const void*, const void*, void*, int64_t, hipStream_t) { return D3D_OK; }
+int32_t launchCastFromFloat(int32_t, const float*, void*, int64_t, hipStream_t) { return D3D_OK; }
+}  // namespace d3d
+
+#define CHECK(cond)                                                                \
+  do {                                                                             \
+    if (!(cond)) {                                                                 \
+      std::fprintf(stderr, "schedule_check: %s failed (line %d)\n", #cond, __LINE__); \
+      return 1;                                                                    \
+    }                                                                              \
+  } while (0)
+
+namespace {
+d3d_schedule* make() {
+  d3d_schedule* s = nullptr;
+  if (d3d_schedule_create(2, &s) != D3D_OK) return nullptr;
+  static d3d_tensor_desc in[4], out[1];
+  const void* ins[4] = {};
+  void* outs[1] = {};
+  auto* op = reinterpret_cast<d3d_plugin*>(16);
+  const int32_t first = d3d_schedule_add(s, op, in, 4, out, 1, ins, outs, nullptr, 0, 1, nullptr, 0);
+  d3d_schedule_add(s, op, in, 4, out, 1, ins, outs, nullptr, 0, 0, &first, 1);
+  return s;
+}
+
+// A schedule destroyed while the caller captures another stream, its last launch still running.
+int destroyUnderCapture() {
+  d3d_schedule* s = make();
+  for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  CHECK(graphLaunches == 3 && liveGraphs == 1);
+  othersCapture = true;
+  d3d_schedule_destroy(s);
+  othersCapture = false;
+  CHECK(!spoiled && !destroyedRunning && !deviceWait);
+  CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && threadMode == hipStreamCaptureModeGlobal);
+  return 0;
+}
+
+// A change under a graph whose launch still runs: the run neither waits nor destroys it; it goes once it has run.
+int changeWithoutWaiting() {
+  d3d_schedule* s = make();
+  for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  const int launched = graphLaunches, before = captures;
+  ++operatorChanges;
+  othersCapture = true;
+  for (int i = 0; i < 3; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  CHECK(graphLaunches == launched + 1 && captures == before + 1);
+  CHECK(!spoiled && !destroyedRunning && !deviceWait && pendingWork > 0 && liveGraphs == 2);
+  othersCapture = false;
+  finish();
+  CHECK(d3d_schedule_run(s, nullptr) == D3D_OK && liveGraphs == 1);
+  d3d_schedule_destroy(s);
+  CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && !destroyedRunning);
+  return 0;
+}
+}  // namespace
+
+int main() {
+  if (destroyUnderCapture() || changeWithoutWaiting()) return 1;
+  std::puts("schedule_check ok");
+  return 0;
+}

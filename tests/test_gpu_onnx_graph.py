@@ -187,3 +187,112 @@ def test_points_to_dense_map_as_one_graph(engine):
             torch.cuda.synchronize()
             _same(y, out, ex.model)
             assert torch.equal(out["bev"], bev)
+
+
+def _points_model(dtype=torch.float16):
+    """Points -> voxels -> Cast -> four sparse layers -> dense map on a small grid, and inputs for it."""
+    from deploy3d_amd import layers, onnx_graph, synth
+    n_pts, max_vox, grid = 20000, 12000, (16, 96, 96)
+    specs = synth.voxelnet_layers()[:4]
+    weights = [synth.layer_weights(0, i, s) for i, s in enumerate(specs)]
+    caps = layers.plan_capacities(specs, max_vox)
+    model = onnx_graph.backbone_model(specs, weights, caps, max_vox, 5, grid, dtype=dtype, densify=True, points=n_pts)
+
+    def points(seed):
+        rng = np.random.default_rng(seed)
+        pts = np.empty((n_pts, 5), np.float32)
+        pts[:, 0:2] = rng.normal(0, 4.0, (n_pts, 2))
+        pts[:, 2] = np.where(rng.random(n_pts) < 0.7, rng.uniform(-1.0, -0.4, n_pts), rng.normal(0.5, 0.8, n_pts))
+        pts[:, 3:] = rng.random((n_pts, 2))
+        return torch.from_numpy(pts).cuda()
+
+    def inputs(seed):
+        return dict(points=points(seed), batch_indices=torch.zeros(n_pts, dtype=torch.int32, device="cuda"),
+                    voxel_config=torch.tensor([-9.6, -9.6, -1.0, 0.2, 0.2, 0.25], device="cuda"),
+                    spatial_shape=torch.empty((1, 0) + grid, dtype=torch.int32, device="cuda"))
+
+    net = layers.SparseBackbone(specs, weights, caps, dtype=dtype, overlap=False)
+
+    def check(ex, out, x):
+        """The graph's outputs against the stages called one by one: voxels from the voxeliser (means are sums of atomics,
+        equal up to the order of addition), everything behind it from the graph's own voxels, bit for bit."""
+        from deploy3d_amd import simple_mean_encoder
+        vals = ex._bound["values"]
+        f, c, k = simple_mean_encoder(x["points"], x["batch_indices"], x["voxel_config"], x["spatial_shape"], max_vox)
+        n = int(k.item())
+        assert n == int(vals["num_act"].item()) and torch.equal(c[:n], vals["coors"][:n])
+        torch.testing.assert_close(f[:n], vals["voxel_means"][:n], rtol=1e-5, atol=1e-6)
+        y = net._forward_steps(layers.SparseTensor(vals["voxel_means"].to(dtype), vals["coors"], vals["num_act"], list(grid), 1))
+        torch.cuda.synchronize()
+        _same(y, out, ex.model)
+        assert torch.equal(out["bev"], layers.densify(y))
+
+    return model, inputs, points, check
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_repeated_runs_of_a_points_graph(engine, dtype):
+    """Ten runs on one binding with other points in its buffers each time: step by step, recorded, and - from the sixth -
+    one captured graph that holds the voxeliser, the cast, the layers and the dense map."""
+    from deploy3d_amd import onnx_graph
+    model, inputs, points, check = _points_model(dtype)
+    ex = onnx_graph.GraphExecutor(onnx_graph.write_model(model))
+    x = inputs(0)
+    for run in range(10):
+        x["points"].copy_(points(run))
+        x["batch_indices"].zero_()
+        x["batch_indices"][:1500 * run] = -1
+        out = ex.run(**x)
+        torch.cuda.synchronize()
+        check(ex, out, x)
+    assert ex._bound["native"] is not None
+
+
+def test_repeated_runs_of_a_graph_with_sums(engine):
+    """The two-branch block (an Add node, keys shared across branches) over nine runs with changing contents."""
+    from deploy3d_amd import layers, onnx_graph, synth
+    cfg = synth.config5(9000)
+    specs, weights, n = cfg["layers"], cfg["weights"], len(cfg["coords"])
+    caps = layers.plan_capacities(specs, n, layers.measure_output_counts(specs, cfg["coords"], cfg["grid"]))
+    model = onnx_graph.backbone_model(specs, weights, caps, n, cfg["feats"].shape[1], cfg["grid"], densify=True)
+    ex = onnx_graph.GraphExecutor(onnx_graph.write_model(model))
+    net = layers.SparseBackbone(specs, weights, caps, overlap=False)
+    x = layers.make_input(cfg["coords"], cfg["feats"], cfg["grid"])
+    inputs = _graph_inputs(x, cfg["grid"])
+    for run in range(9):
+        x.num_act.fill_(n - 700 * (run % 4))
+        x.feats.mul_(-0.9)
+        y = net._forward_steps(x)
+        bev = layers.densify(y)
+        out = ex.run(**inputs)
+        torch.cuda.synchronize()
+        _same(y, out, ex.model)
+        assert torch.equal(out["bev"], bev)
+    assert ex._bound["native"] is not None
+
+
+def test_capture_on_other_buffers_after_runs_became_a_graph(engine):
+    """The binding whose runs became a graph gives way to another one while a stream is being captured, its last launch
+    perhaps still running: the capture holds, its replays and later eager runs are right."""
+    from deploy3d_amd import onnx_graph
+    model, inputs, points, check = _points_model()
+    ex = onnx_graph.GraphExecutor(onnx_graph.write_model(model))
+    first, second = inputs(1), inputs(2)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for _ in range(8):
+            ex.run(**first)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = ex.run(**second)
+        for seed in (2, 3, 4):
+            second["points"].copy_(points(seed))
+            graph.replay()
+            stream.synchronize()
+            check(ex, out, second)
+        for seed in (5, 6, 7, 8, 9, 10, 11):
+            first["points"].copy_(points(seed))
+            out = ex.run(**first)
+            stream.synchronize()
+            check(ex, out, first)
