@@ -56,7 +56,8 @@ struct d3d_schedule {
   uint64_t graphChanges = 0;    // the operators' change count the graph was captured at
   uint64_t lastChanges = ~0ull; // ... and at the end of the last run
   int steady = 0;               // runs in a row that changed nothing
-  bool graphRefused = false;    // a capture failed: this schedule stays with streams
+  int patience = kSteadyRuns;   // ... after which a capture is tried; doubled by every refusal, as it costs a pass
+  static constexpr int kSteadyRuns = 2, kMostPatience = 4096;
 };
 
 namespace {
@@ -373,13 +374,16 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
   reapGraphs();
   const uint64_t changes = changesOf(s);
   s->steady = s->lastChanges == changes ? s->steady + 1 : 0;
-  if (!s->graphRefused && s->steady >= 2 && !(s->graph && s->graphChanges == changes)) {
+  if (s->steady >= s->patience && !(s->graph && s->graphChanges == changes)) {
     // what the operators enqueue is settled, and the pass repeats: capturing it costs about what one pass does
-    s->graphRefused = !captureGraph(s);
+    const bool captured = captureGraph(s);
     s->graphChanges = changes;
-    if (s->graph && changesOf(s) != changes) {  // an operator is not settled after all: no graph for this schedule
+    if (captured && changesOf(s) == changes) {
+      s->patience = d3d_schedule::kSteadyRuns;
+    } else {  // refused, which may pass (memory, a capture in another thread), or an operator is not settled after all
       dropGraph(s);
-      s->graphRefused = true;
+      s->steady = 0;
+      s->patience = std::min(2 * s->patience, d3d_schedule::kMostPatience);
     }
   }
   if (s->graph && s->graphChanges == changes) {

@@ -227,7 +227,7 @@ int32_t d3d_set_option(d3d_plugin* p, int32_t option, int64_t value);
  *   continues behind all of them, so for the caller the run is stream-ordered work on `stream`.  No host
  *   synchronisation.  The first two runs enqueue step by step; when nothing about the operators has changed since
  *   (options, links, capacities, reserved buffers), the steps are captured into one HIP graph, which the schedule keeps and
- *   later runs launch - until something changes.  Returns the first failing status; steps behind a failed one are not
+ *   later runs launch - until something changes.  A capture that is refused is tried again after twice as many runs.  Returns the first failing status; steps behind a failed one are not
  *   enqueued.  Refused with
  *   D3D_ERR_UNSUPPORTED while `stream` is capturing (capture the operators' own enqueues instead).  One thread at
  *   a time per schedule.

@@ -11,7 +11,7 @@
 #include "d3d_spconv.h"
 
 namespace {
-int pendingWork = 0, graphLaunches = 0, steps = 0, captures = 0, liveGraphs = 0, liveEvents = 0, liveStreams = 0;
+int pendingWork = 0, graphLaunches = 0, steps = 0, captures = 0, refusals = 0, liveGraphs = 0, liveEvents = 0, liveStreams = 0;
 bool othersCapture = false, spoiled = false, destroyedRunning = false, refuseCapture = false, deviceWait = false;
 hipStreamCaptureMode threadMode = hipStreamCaptureModeGlobal;
 uint64_t operatorChanges = 0;
@@ -94,6 +94,7 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
 }
 hipError_t hipGraphCreate(hipGraph_t* g, unsigned) {
   *g = static_cast<hipGraph_t>(fresh());
+  refusals += refuseCapture;
   return refuseCapture ? hipErrorStreamCaptureUnsupported : hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
@@ -194,10 +195,29 @@ int changeWithoutWaiting() {
   CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && !destroyedRunning);
   return 0;
 }
+
+// A capture that is refused for a while: the passes run step by step, the attempts get rarer, and the graph comes in the end.
+int refusedForAWhile() {
+  d3d_schedule* s = make();
+  refuseCapture = true;
+  const int launched = graphLaunches;
+  refusals = 0;
+  for (int i = 0; i < 40; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  CHECK(graphLaunches == launched && refusals >= 3 && refusals <= 5);
+  refuseCapture = false;
+  for (int i = 0; i < 100; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  CHECK(graphLaunches > launched);
+  ++operatorChanges;  // the next graph comes as fast as the first one
+  const int before = graphLaunches;
+  for (int i = 0; i < 3; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  CHECK(graphLaunches == before + 1);
+  d3d_schedule_destroy(s);
+  return 0;
+}
 }  // namespace
 
 int main() {
-  if (destroyUnderCapture() || changeWithoutWaiting()) return 1;
+  if (destroyUnderCapture() || changeWithoutWaiting() || refusedForAWhile()) return 1;
   std::puts("schedule_check ok");
   return 0;
 }
