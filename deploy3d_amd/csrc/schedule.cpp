@@ -15,8 +15,8 @@
 // launches, 9 000 voxels) costs the host 415 us step by step on three lanes - more than its kernels take - and 195 as a
 // graph; the device then takes 345 us.  The graph is dropped when an operator reports a change (pluginChanges).
 //
-// A dropped graph is destroyed once its last launch has run, which an event behind every launch tells: dropping one neither
-// waits nor synchronises the device, so it is also allowed while the caller captures a stream.
+// A dropped graph is destroyed once its last launch has run, which an event behind every launch tells (RetiredGraph): no
+// device-wide synchronisation, which a stream under capture would not survive.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -85,40 +85,56 @@ uint64_t changesOf(const d3d_schedule* s) {
   return sum;
 }
 
-// The calls below are legal while some other stream is being captured in the global mode only from a thread in the relaxed
-// mode; from any other they fail and spoil that capture.  None of them touches a capturing stream.
+// Asking an event or waiting for one is legal while another stream is being captured in the global mode only from a thread in
+// the relaxed mode; from any other it fails and spoils that capture.
 struct RelaxedCapture {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// Graphs that no schedule launches any more, until their last launch has run.  Lives until the process ends.
+// A graph that no schedule launches any more, until its last launch has run.  The event behind that launch (`ran`) was
+// recorded on the caller's stream: if that is being captured by now, even a relaxed query of the event spoils the capture,
+// while a wait of another stream for it is merely refused.  So a stream of its own is put behind it, when that is possible,
+// and the event behind THAT (`over`) is asked.
+struct RetiredGraph {
+  hipGraphExec_t graph = nullptr;
+  hipEvent_t ran = nullptr, over = nullptr;
+  hipStream_t behind = nullptr;
+  bool ordered = false;  // `over` stands behind `ran`
+};
 struct Retired {
   std::mutex mutex;
   std::atomic<size_t> count{0};
-  std::vector<std::pair<hipGraphExec_t, hipEvent_t>> graphs;
+  std::vector<RetiredGraph> graphs;
 };
 Retired& retired() {
-  static Retired* r = new Retired();
+  static Retired* r = new Retired();  // lives until the process ends
   return *r;
 }
 
-// Destroys the retired graphs that have run.
-void reapGraphs() {
+// Destroys the retired graphs that have run; `wait`: waits for each that can be waited for.
+void reapGraphs(bool wait) {
   Retired& r = retired();
   if (r.count.load(std::memory_order_relaxed) == 0) return;
   const RelaxedCapture relaxed;
   std::lock_guard<std::mutex> lock(r.mutex);
   for (size_t i = 0; i < r.graphs.size();) {
-    if (hipEventQuery(r.graphs[i].second) != hipSuccess) {
-      (void)hipGetLastError();  // "not ready" is no error of the caller's
+    RetiredGraph& g = r.graphs[i];
+    if (!g.behind && hipStreamCreateWithFlags(&g.behind, hipStreamNonBlocking) != hipSuccess) g.behind = nullptr;
+    if (!g.over && hipEventCreateWithFlags(&g.over, hipEventDisableTiming) != hipSuccess) g.over = nullptr;
+    if (!g.ordered && g.behind && g.over)
+      g.ordered = hipStreamWaitEvent(g.behind, g.ran, 0) == hipSuccess && hipEventRecord(g.over, g.behind) == hipSuccess;
+    if (!g.ordered || (wait ? hipEventSynchronize(g.over) : hipEventQuery(g.over)) != hipSuccess) {
+      (void)hipGetLastError();  // not ready, or not now: no error of the caller's
       ++i;
       continue;
     }
-    (void)hipGraphExecDestroy(r.graphs[i].first);
-    (void)hipEventDestroy(r.graphs[i].second);
-    r.graphs[i] = r.graphs.back();
+    (void)hipGraphExecDestroy(g.graph);
+    (void)hipEventDestroy(g.ran);
+    (void)hipEventDestroy(g.over);
+    (void)hipStreamDestroy(g.behind);
+    g = r.graphs.back();
     r.graphs.pop_back();
   }
   r.count.store(r.graphs.size(), std::memory_order_relaxed);
@@ -126,15 +142,15 @@ void reapGraphs() {
 
 void dropGraph(d3d_schedule* s) {
   if (!s->graph) return;
-  {
-    Retired& r = retired();
-    std::lock_guard<std::mutex> lock(r.mutex);
-    r.graphs.emplace_back(s->graph, s->graphRan);
-    r.count.store(r.graphs.size(), std::memory_order_relaxed);
-  }
+  Retired& r = retired();
+  RetiredGraph g;
+  g.graph = s->graph;
+  g.ran = s->graphRan;
   s->graph = nullptr;
   s->graphRan = nullptr;
-  reapGraphs();
+  std::lock_guard<std::mutex> lock(r.mutex);
+  r.graphs.push_back(g);
+  r.count.store(r.graphs.size(), std::memory_order_relaxed);
 }
 
 // Captures every step into one graph, each behind the last nodes of the steps it waits for.  False (and no graph) if
@@ -248,7 +264,7 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
     return D3D_ERR_BAD_ARG;
   }
   *out = nullptr;
-  reapGraphs();
+  reapGraphs(false);
   auto* s = new d3d_schedule();
   hipError_t e = hipSuccess;
   if (n_lanes > 1) e = hipEventCreateWithFlags(&s->fork, hipEventDisableTiming);  // one lane: no HIP object at all
@@ -270,8 +286,8 @@ void d3d_schedule_destroy(d3d_schedule* s) {
   if (!s) return;
   if (s->graph || s->lanes.size() > 1) {
     const RelaxedCapture relaxed;
-    if (s->graph) (void)hipEventSynchronize(s->graphRan);
     dropGraph(s);
+    reapGraphs(true);
     for (auto& st : s->steps)
       if (st.done) (void)hipEventDestroy(st.done);
     for (size_t l = 1; l < s->lanes.size(); ++l) {
@@ -371,7 +387,7 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
     d3d::setError("schedule: the stream is capturing; a schedule runs eagerly");
     return D3D_ERR_UNSUPPORTED;
   }
-  reapGraphs();
+  reapGraphs(false);
   const uint64_t changes = changesOf(s);
   s->steady = s->lastChanges == changes ? s->steady + 1 : 0;
   if (s->steady >= s->patience && !(s->graph && s->graphChanges == changes)) {

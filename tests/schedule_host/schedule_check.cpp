@@ -1,6 +1,7 @@
 // Host check of csrc/schedule.cpp against a stand-in for the HIP runtime that keeps count: work counts as pending until
-// finish() is called, and while `othersCapture` is set a call that synchronises spoils that capture - from a thread that is not
-// in the relaxed mode any such call, from a relaxed one a device-wide wait.  Operators are stand-ins too.  No GPU.
+// finish() is called, and while a stream is being captured a call that asks or waits spoils the capture - from a thread that
+// is not in the relaxed mode any such call, from a relaxed one a device-wide wait and anything that asks an event last
+// recorded on that stream (as the runtime does on a gfx950 system).  Operators are stand-ins too.  No GPU.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -12,15 +13,18 @@
 
 namespace {
 int pendingWork = 0, graphLaunches = 0, steps = 0, captures = 0, refusals = 0, liveGraphs = 0, liveEvents = 0, liveStreams = 0;
-bool othersCapture = false, spoiled = false, destroyedRunning = false, refuseCapture = false, deviceWait = false;
+hipStream_t const kMain = reinterpret_cast<hipStream_t>(8), kOther = reinterpret_cast<hipStream_t>(12);
+hipStream_t captured = nullptr;  // the stream that the caller captures
+bool spoiled = false, destroyedRunning = false, refuseCapture = false, deviceWait = false;
 hipStreamCaptureMode threadMode = hipStreamCaptureModeGlobal;
 uint64_t operatorChanges = 0;
 std::map<void*, bool> eventPending;
+std::map<void*, hipStream_t> recordedOn;
 std::set<void*> running;  // graphs launched and not finished
 uintptr_t nextHandle = 16;
 void* fresh() { return reinterpret_cast<void*>(nextHandle += 16); }
 hipError_t unsafe() {
-  if (!othersCapture || threadMode == hipStreamCaptureModeRelaxed) return hipSuccess;
+  if (!captured || threadMode == hipStreamCaptureModeRelaxed) return hipSuccess;
   spoiled = true;
   return hipErrorStreamCaptureUnsupported;
 }
@@ -43,7 +47,7 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
 }
 hipError_t hipDeviceSynchronize() {
   deviceWait = true;
-  if (othersCapture) {
+  if (captured) {
     spoiled = true;
     return hipErrorStreamCaptureUnsupported;
   }
@@ -74,20 +78,30 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   --liveEvents;
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   eventPending[e] = pendingWork > 0;
+  recordedOn[e] = s;
   return hipSuccess;
 }
+hipError_t unsafeFor(hipEvent_t e) {
+  if (captured && recordedOn[e] == captured) {
+    spoiled = true;
+    return hipErrorCapturedEvent;
+  }
+  return unsafe();
+}
 hipError_t hipEventQuery(hipEvent_t e) {
-  const hipError_t r = unsafe();
+  const hipError_t r = unsafeFor(e);
   return r != hipSuccess ? r : (eventPending[e] ? hipErrorNotReady : hipSuccess);
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
-  const hipError_t r = unsafe();
+  const hipError_t r = unsafeFor(e);
   if (r == hipSuccess && eventPending[e]) finish();
   return r;
 }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t e, unsigned) {
+  return captured && recordedOn[e] == captured ? hipErrorStreamCaptureIsolation : hipSuccess;
+}
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
   *st = hipStreamCaptureStatusNone;
   return hipSuccess;
@@ -165,32 +179,38 @@ d3d_schedule* make() {
   return s;
 }
 
-// A schedule destroyed while the caller captures another stream, its last launch still running.
+// A schedule destroyed while the caller captures a stream, its last launch still running.
 int destroyUnderCapture() {
-  d3d_schedule* s = make();
-  for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
-  CHECK(graphLaunches == 3 && liveGraphs == 1);
-  othersCapture = true;
-  d3d_schedule_destroy(s);
-  othersCapture = false;
-  CHECK(!spoiled && !destroyedRunning && !deviceWait);
-  CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && threadMode == hipStreamCaptureModeGlobal);
+  for (hipStream_t during : {kOther, kMain}) {
+    d3d_schedule* s = make();
+    const int launched = graphLaunches;
+    for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
+    CHECK(graphLaunches == launched + 3 && liveGraphs == 1);
+    captured = during;
+    d3d_schedule_destroy(s);
+    CHECK(!spoiled && !destroyedRunning && !deviceWait && threadMode == hipStreamCaptureModeGlobal);
+    CHECK(liveGraphs == (during == kMain ? 1 : 0));
+    captured = nullptr;
+    finish();
+    d3d_schedule_destroy(make());
+    CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && !destroyedRunning);
+  }
   return 0;
 }
 
 // A change under a graph whose launch still runs: the run neither waits nor destroys it; it goes once it has run.
 int changeWithoutWaiting() {
   d3d_schedule* s = make();
-  for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  for (int i = 0; i < 5; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
   const int launched = graphLaunches, before = captures;
   ++operatorChanges;
-  othersCapture = true;
-  for (int i = 0; i < 3; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
-  CHECK(graphLaunches == launched + 1 && captures == before + 1);
+  captured = kOther;
+  for (int i = 0; i < 4; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
+  CHECK(graphLaunches == launched + 2 && captures == before + 1);
   CHECK(!spoiled && !destroyedRunning && !deviceWait && pendingWork > 0 && liveGraphs == 2);
-  othersCapture = false;
+  captured = nullptr;
   finish();
-  CHECK(d3d_schedule_run(s, nullptr) == D3D_OK && liveGraphs == 1);
+  CHECK(d3d_schedule_run(s, kMain) == D3D_OK && liveGraphs == 1);
   d3d_schedule_destroy(s);
   CHECK(liveGraphs == 0 && liveStreams == 0 && liveEvents == 0 && !destroyedRunning);
   return 0;
@@ -202,14 +222,14 @@ int refusedForAWhile() {
   refuseCapture = true;
   const int launched = graphLaunches;
   refusals = 0;
-  for (int i = 0; i < 40; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  for (int i = 0; i < 40; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
   CHECK(graphLaunches == launched && refusals >= 3 && refusals <= 5);
   refuseCapture = false;
-  for (int i = 0; i < 100; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  for (int i = 0; i < 100; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
   CHECK(graphLaunches > launched);
   ++operatorChanges;  // the next graph comes as fast as the first one
   const int before = graphLaunches;
-  for (int i = 0; i < 3; ++i) CHECK(d3d_schedule_run(s, nullptr) == D3D_OK);
+  for (int i = 0; i < 3; ++i) CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
   CHECK(graphLaunches == before + 1);
   d3d_schedule_destroy(s);
   return 0;
