@@ -191,8 +191,9 @@ int32_t launchMfmaInt8(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeHalf(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeBf16(const ConvArgs& a, hipStream_t stream);
 int32_t launchPipeInt8(const ConvArgs& a, hipStream_t stream);
-// Both kernels for fp32 storage (conv_f32.hip).
+// Both kernels for fp32 storage (conv_f32.hip), and whether one of them takes a layer of these (widened) channels.
 int32_t launchMfmaFloat(const ConvArgs& a, hipStream_t stream);
+bool floatMfmaFits(int kVol, int cin, int cout);
 
 // True if the MFMA kernel family covers (dtype, cin, cout); otherwise the
 // narrow-channel kernel runs.

@@ -274,6 +274,21 @@ int32_t launchNarrowRows(const ConvArgs& a, hipStream_t stream) {
 
 bool isMfmaChannels(int c) { return c == 16 || c == 32 || c == 64 || c == 128; }
 
+// fp32 layers that would be MFMA layers but for their kernel volume (floatMfmaFits) have the choice between the two vector
+// kernels.  The rows kernel wins until its copies of the weights into LDS, one per workgroup, outweigh the tile kernel's
+// passes through it: the sooner the larger they are, and at 32 output channels, where a wavefront holds half the rows.
+// us on the rows / the tile kernel (LiDAR-like clouds):
+//   5 -> 16, 125 taps (39 KB):   8 000 rows  24 / 78     80 000 rows  179 / 239    250 000 rows  634 / 615
+//   16 -> 16, 60 taps (60 KB):   8 000 rows  19 / 50     40 000 rows   89 / 122    120 000 rows  222 / 209
+//   3 -> 32, 125 taps (47 KB):   8 000 rows  40 / 81     30 000 rows  135 / 143     60 000 rows  266 / 217
+//   16 -> 32, 30 taps (60 KB):   8 000 rows  28 / 44     20 000 rows   65 / 73      40 000 rows  129 / 102
+bool narrowRowsPay(const ConvArgs& a) {
+  if (a.weightsMfma || !isMfmaChannels(a.cout)) return true;
+  const bool wide = a.cout > 16;
+  const size_t lds = static_cast<size_t>(a.kVol) * a.cin * (wide ? 32 : 16) * sizeof(float);
+  return a.outRows <= (lds <= 48 * 1024 ? (wide ? 32768 : 98304) : (wide ? 20480 : 49152));
+}
+
 // rows of `inBytes` bytes widened to `outBytes` (a multiple of 16) with zeros, so that a narrow first layer
 // (5 input channels, say) can run on the MFMA path
 __global__ void __launch_bounds__(256)
@@ -374,7 +389,7 @@ int32_t launchConv(const ConvArgs& a, hipStream_t stream) {
     const bool rows = !(rowsEnv && rowsEnv[0] == '0');
     switch (a.dtype) {
       case D3D_FLOAT:
-        rc = rows ? launchNarrowRows<float>(a, stream) : D3D_ERR_UNSUPPORTED;
+        rc = rows && narrowRowsPay(a) ? launchNarrowRows<float>(a, stream) : D3D_ERR_UNSUPPORTED;
         if (rc == D3D_ERR_UNSUPPORTED) rc = launchNarrow<float>(a, stream);
         break;
       case D3D_HALF:

@@ -7,6 +7,13 @@
 
 namespace d3d {
 
+// 16 -> 16, 16 -> 32 and 32 -> 16 run with resident weights or not at all; the pipelined kernel takes the rest up to 64 taps
+// (conv_pipe.h).  Beyond that the vector kernels run on the rows as stored: the layer is neither widened nor packed for an
+// MFMA.
+bool floatMfmaFits(int kVol, int cin, int cout) {
+  return cin * cout <= 512 ? convk::residentFits(kVol, cin, cout, sizeof(float)) : kVol <= 64;
+}
+
 int32_t launchMfmaFloat(const ConvArgs& a, hipStream_t stream) {
   const int32_t rc = convk::launchFloatResident<>(a, stream);
   if (rc != D3D_ERR_UNSUPPORTED || a.rowChannels > 0) return rc;

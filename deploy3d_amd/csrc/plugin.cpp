@@ -881,7 +881,7 @@ struct MMPlugin final : d3d_plugin {
       return dtype == D3D_HALF ? halfBitsToFloat(h) : bf16BitsToFloat(h);
     };
     const int cinP = paddedMfmaChannels(dtype, cin, cout);
-    const bool mfma = convUsesMfma(dtype, cinP, cout);
+    const bool mfma = convUsesMfma(dtype, cinP, cout) && (dtype != D3D_FLOAT || floatMfmaFits(kernelVol, cinP, cout));
     std::vector<uint8_t> packed(mfma ? static_cast<size_t>(kernelVol) * cinP * cout * es : 0, 0);
     // fragment-major copy for the MFMA kernels: Wf[tap][kk][n][lane][j] = W[tap][kk*KS + (lane/16)*KG + j][n*16 + lane%16]
     // with KS = 64 bytes of channels (32 bytes for 16 two-byte channels) and KG = KS/4, so one wavefront load fetches one
@@ -1089,7 +1089,7 @@ struct MMPlugin final : d3d_plugin {
     }
     a.out = outputs[0];
     a.weightsF32 = static_cast<const float*>(dev->f32.ptr);
-    a.weightsMfma = dev->mfma.ptr;
+    a.weightsMfma = dev->cinMfma > 0 ? dev->mfma.ptr : nullptr;
     a.bias = (withBias || dtype == D3D_INT8) ? static_cast<const float*>(dev->bias.ptr) : nullptr;
     a.requantM = dtype == D3D_INT8 ? static_cast<const float*>(dev->requantM.ptr) : nullptr;
     a.nbr = nbr;

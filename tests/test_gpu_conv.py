@@ -118,6 +118,38 @@ def test_mfma_fp32(engine, cin, cout):
     run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, "float32", False, inverse=True, with_bias=False)
 
 
+@pytest.mark.parametrize("ksize,cin,cout", [((5, 5, 5), 5, 16), ((3, 4, 5), 16, 16), ((2, 4, 7), 16, 16), ((2, 4, 7), 3, 16),
+                                            ((2, 2, 7), 16, 32), ((1, 5, 6), 16, 32), ((1, 5, 6), 32, 16), ((5, 5, 5), 3, 32),
+                                            ((4, 4, 4), 32, 32), ((5, 13, 1), 32, 32), ((5, 13, 1), 64, 64)])
+def test_fp32_kernel_volumes_around_the_mfma_limits(engine, ksize, cin, cout):
+    """fp32 layers on either side of the volumes that the resident-weight kernel (56 KB of weights) and the pipelined one
+    (64 taps) take; past them the vector kernels run."""
+    pad = tuple((k - 1) // 2 for k in ksize)
+    run_case(2500, (10, 36, 30), ksize, (1, 1, 1), pad, cin, cout, "float32", False, relu=True, cap_extra=3)
+    run_case(700, (10, 36, 30), ksize, (2, 2, 2), pad, cin, cout, "float32", False, inverse=True, link=False)
+
+
+@pytest.mark.parametrize("rows", [98000, 99000])
+def test_fp32_vector_kernels_by_row_count(engine, rows):
+    """125 taps of 3 -> 16 channels on either side of the rows from which the tile kernel takes over."""
+    run_case(rows, (16, 128, 128), (5, 5, 5), (1, 1, 1), (2, 2, 2), 3, 16, "float32", True)
+
+
+def test_fp32_layers_no_mfma_takes_are_not_widened(engine):
+    """A 5x5x5 layer of 5 -> 16 channels runs on its rows as stored: configuring it for four million input rows reserves no
+    16-channel copy of them (256 MB)."""
+    from deploy3d_amd import Plugin, TensorDesc
+    from deploy3d_amd.spconv_mm import mm_blob
+    rows = 1 << 22
+    op = Plugin("SPConvMM", mm_blob((5, 5, 5), 5, 16, 64, False, False, np.zeros(125 * 5 * 16, np.float32)))
+    ins = [TensorDesc.of((rows, 5), torch.float32), TensorDesc.of((1,), torch.int32), TensorDesc.of((1,), torch.int32),
+           TensorDesc.of((3, 125 * (rows + 128)), torch.int32), TensorDesc.of((1,), torch.int32)]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    op.configure(ins, op.output_descs(ins))
+    assert before - torch.cuda.mem_get_info()[0] < 128 << 20
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("ksize", [(3, 3, 3), (3, 1, 3), (1, 1, 1), (3, 3, 5)])
 def test_resident_32_to_32(engine, ksize, dtype):
