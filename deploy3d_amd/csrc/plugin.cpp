@@ -1421,6 +1421,20 @@ int32_t d3d_serialize(const d3d_plugin* p, void* buffer, size_t len) {
   return D3D_OK;
 }
 
+int32_t d3d_holds_weights(const d3d_plugin* mm, const float* weight, size_t nb_weight, const float* bias, size_t nb_bias) {
+  D3D_GUARD_BEGIN
+  const auto* m = dynamic_cast<const MMPlugin*>(mm);
+  if (!m || (nb_weight && !weight) || (nb_bias && !bias)) {
+    setError("d3d_holds_weights: the handle must be an SPConvMM and the arrays not null");
+    return D3D_ERR_BAD_ARG;
+  }
+  const size_t weights = static_cast<size_t>(m->kernelVol) * m->cin * m->cout;
+  if (nb_weight != weights || nb_bias != (m->withBias ? static_cast<size_t>(m->cout) : 0)) return 0;
+  const uint8_t* held = m->blob.data() + m->weightOffset;
+  return std::memcmp(held, weight, weights * 4) == 0 && (!nb_bias || std::memcmp(held + weights * 4, bias, nb_bias * 4) == 0);
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
+}
+
 int32_t d3d_num_outputs(const d3d_plugin* p) { return p ? p->numOutputs() : D3D_ERR_BAD_ARG; }
 
 int32_t d3d_output_dims(const d3d_plugin* p, int32_t output_index, const d3d_tensor_desc* in, int32_t nb_in,

@@ -26,7 +26,7 @@ STATUS_NAMES = {0: "OK", -1: "UNSUPPORTED", -2: "BAD_BLOB", -3: "BAD_ARG", -4: "
 
 EXPORTS = [
     "d3d_create", "d3d_clone", "d3d_destroy", "d3d_plugin_type", "d3d_plugin_version", "d3d_serialize_size",
-    "d3d_serialize", "d3d_num_outputs", "d3d_output_dims", "d3d_output_dtype", "d3d_supports_format",
+    "d3d_serialize", "d3d_holds_weights", "d3d_num_outputs", "d3d_output_dims", "d3d_output_dtype", "d3d_supports_format",
     "d3d_configure", "d3d_workspace_size", "d3d_enqueue", "d3d_last_error", "d3d_num_ops", "d3d_op_name",
     "d3d_enqueue_static", "d3d_link_rulebook", "d3d_link_coords", "d3d_set_option",
     "d3d_schedule_create", "d3d_schedule_add", "d3d_schedule_add_sum", "d3d_schedule_add_cast", "d3d_schedule_size", "d3d_schedule_run", "d3d_schedule_destroy",
@@ -92,6 +92,8 @@ def load_library(path=None):
     lib.d3d_serialize_size.argtypes = [vp]
     lib.d3d_serialize.restype = i32
     lib.d3d_serialize.argtypes = [vp, vp, sz]
+    lib.d3d_holds_weights.restype = i32
+    lib.d3d_holds_weights.argtypes = [vp, vp, sz, vp, sz]
     lib.d3d_num_outputs.restype = i32
     lib.d3d_num_outputs.argtypes = [vp]
     lib.d3d_output_dims.restype = i32
@@ -231,6 +233,14 @@ class Plugin:
         buf = ctypes.create_string_buffer(n)
         _check(self._lib.d3d_serialize(self._h, buf, n))
         return buf.raw
+
+    def holds_weights(self, weight, bias):
+        """SPConvMM only: whether this operator was made of exactly these values (contiguous float32 arrays, bias or None)."""
+        rc = self._lib.d3d_holds_weights(self._h, weight.ctypes.data, weight.size,
+                                         None if bias is None else bias.ctypes.data, 0 if bias is None else bias.size)
+        if rc < 0:
+            _check(rc)
+        return rc == 1
 
     @property
     def num_outputs(self):

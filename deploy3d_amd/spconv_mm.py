@@ -3,7 +3,6 @@
 HIP engine.  ``relu`` (fused ReLU) and the activation scales are this build's
 extensions, carried in an extension record after the reference's blob.
 """
-import ctypes
 import hashlib
 import struct
 
@@ -13,10 +12,8 @@ import torch
 from .plugin import Launch, LaunchCache, Plugin, TensorDesc, current_stream
 
 _plugins = {}
-_by_attributes = {}  # attributes of a convolution -> [(plugin, weight, bias)], copies of the values it was made from
+_by_sample = {}  # (attributes of a convolution, a few of its weights) -> operators made of such, the last one used first
 _launches = LaunchCache()
-_memcmp = ctypes.CDLL(None).memcmp
-_memcmp.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
 EXT_MAGIC = 0x58443344  # "D3DX"
 
 
@@ -46,23 +43,22 @@ def get_plugin(blob):
     return p
 
 
-def _same(a, b):
-    return a is b or (a is not None and b is not None and a.size == b.size and
-                      _memcmp(a.ctypes.data, b.ctypes.data, a.nbytes) == 0)
-
-
 def _plugin_of(attributes, weight, bias):
-    """The operator instance of these attributes and values.  The caller's arrays are compared value by value with those
-    of the instances that exist (a memcmp, which ends at the first difference), most recent first: packing and hashing
-    the whole blob on every call took several times as long as the convolution's kernels."""
+    """The operator instance of these attributes and values.  A few of the weights say which instances come into question;
+    those compare all values with the ones they hold (a memcmp): packing and hashing the whole blob on every call took
+    several times as long as the convolution's kernels."""
     weight = np.ascontiguousarray(weight, dtype=np.float32)
     bias = None if bias is None else np.ascontiguousarray(bias, dtype=np.float32)
-    known = _by_attributes.setdefault(attributes, [])
-    for plugin, w, b in list(known):
-        if _same(w, weight) and _same(b, bias):
+    flat = weight.reshape(-1)
+    key = (attributes, flat[::flat.size // 16 + 1].tobytes())
+    known = _by_sample.get(key, ())
+    for plugin in known:
+        if plugin.holds_weights(weight, bias):
+            if plugin is not known[0]:
+                _by_sample[key] = (plugin,) + tuple(p for p in known if p is not plugin)
             return plugin
     plugin = get_plugin(mm_blob(*attributes[:6], weight, bias, *attributes[6:]))
-    known.insert(0, (plugin, weight.copy(), None if bias is None else bias.copy()))
+    _by_sample[key] = (plugin,) + known
     return plugin
 
 

@@ -88,6 +88,11 @@ const char* d3d_plugin_version(const d3d_plugin* p);
 size_t d3d_serialize_size(const d3d_plugin* p);
 int32_t d3d_serialize(const d3d_plugin* p, void* buffer, size_t len);
 
+/* No counterpart in the reference.  SPConvMM: 1 if the blob holds exactly these fp32 weights and this bias (NULL, 0 = none),
+ * compared bit by bit, else 0; a negative status for other operators.  What a caller that is handed weights with every
+ * call finds the operator it has made of them with. */
+int32_t d3d_holds_weights(const d3d_plugin* mm, const float* weight, size_t nb_weight, const float* bias, size_t nb_bias);
+
 /* getNbOutputs (index_trt.cu:98-101: 2 for SubM, 5 otherwise; mm_trt.cu:97). */
 int32_t d3d_num_outputs(const d3d_plugin* p);
 
