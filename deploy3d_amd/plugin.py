@@ -162,7 +162,14 @@ def _pointers(tensors):
         t.data_ptr() if t is not None and t.numel() else None for t in tensors])
 
 
-_scratch = threading.local()
+class _Scratch(threading.local):
+    def __init__(self):
+        self.buffers = {}
+
+
+_scratch = _Scratch()
+# torch.cuda.is_current_stream_capturing without its Python frame
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
 
 
 def scratch(nbytes, device, stream):
@@ -172,13 +179,12 @@ def scratch(nbytes, device, stream):
     so they may share it; those of two threads interleave launch by launch.  A call under stream capture gets memory of its
     own, from the pool of the graph that is being captured: the graph reads and writes it for as long as it is replayed,
     whatever later calls need."""
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing():
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    buffers = vars(_scratch)
-    key = (device, stream)
-    ws = buffers.get(key)
+    buffers = _scratch.buffers
+    ws = buffers.get((device, stream))
     if ws is None or ws.numel() < nbytes:
-        ws = buffers[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+        ws = buffers[device, stream] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     return ws
 
 

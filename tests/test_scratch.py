@@ -13,8 +13,8 @@ HOST = torch.device("cpu")
 @pytest.fixture
 def capturing(monkeypatch):
     state = dict(now=False)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["now"])
-    monkeypatch.setattr(plugin, "_scratch", threading.local())
+    monkeypatch.setattr(plugin, "_capturing", lambda: state["now"])
+    monkeypatch.setattr(plugin, "_scratch", plugin._Scratch())
     return state
 
 
