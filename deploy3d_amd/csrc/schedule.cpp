@@ -15,8 +15,8 @@
 // launches, 9 000 voxels) costs the host 415 us step by step on three lanes - more than its kernels take - and 195 as a
 // graph; the device then takes 345 us.  The graph is dropped when an operator reports a change (pluginChanges).
 //
-// A dropped graph is destroyed once its last launch has run, which an event behind every launch tells (RetiredGraph): no
-// device-wide synchronisation, which a stream under capture would not survive.
+// A dropped graph is destroyed once its last launch has run (RetiredGraph): no device-wide synchronisation, which a stream
+// under capture would not survive, and no event behind every launch, which costs 4 to 6 us a pass.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,7 +52,8 @@ struct d3d_schedule {
   std::vector<Step> steps;
   // the pass as a graph
   hipGraphExec_t graph = nullptr;
-  hipEvent_t graphRan = nullptr; // behind the last launch of the graph
+  bool launched = false;        // the graph has been launched, last on launchedOn
+  hipStream_t launchedOn = nullptr;
   uint64_t graphChanges = 0;    // the operators' change count the graph was captured at
   uint64_t lastChanges = ~0ull; // ... and at the end of the last run
   int steady = 0;               // runs in a row that changed nothing
@@ -93,16 +94,30 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// A graph that no schedule launches any more, until its last launch has run.  The event behind that launch (`ran`) was
-// recorded on the caller's stream: if that is being captured by now, even a relaxed query of the event spoils the capture,
-// while a wait of another stream for it is merely refused.  So a stream of its own is put behind it, when that is possible,
-// and the event behind THAT (`over`) is asked.
+// A graph that no schedule launches any more, until its last launch has run.  What tells is an event (`over`) on a stream of
+// its own (`behind`) that waits for an event (`ran`) on the stream of the launch.  The latter itself may not be asked: if
+// that stream is being captured by then, even a relaxed query of an event last recorded on it spoils the capture.
 struct RetiredGraph {
   hipGraphExec_t graph = nullptr;
+  hipStream_t launchedOn = nullptr;  // until `ran` has been recorded there
   hipEvent_t ran = nullptr, over = nullptr;
   hipStream_t behind = nullptr;
-  bool ordered = false;  // `over` stands behind `ran`
+  bool marked = false;
 };
+
+// Puts `over` behind the graph's last launch; false while the stream of the launch is being captured.
+bool mark(RetiredGraph& g) {
+  if (g.marked) return true;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(g.launchedOn, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+  if (!g.ran && hipEventCreateWithFlags(&g.ran, hipEventDisableTiming) != hipSuccess) return false;
+  if (!g.over && hipEventCreateWithFlags(&g.over, hipEventDisableTiming) != hipSuccess) return false;
+  if (!g.behind && hipStreamCreateWithFlags(&g.behind, hipStreamNonBlocking) != hipSuccess) return false;
+  g.marked = hipEventRecord(g.ran, g.launchedOn) == hipSuccess && hipStreamWaitEvent(g.behind, g.ran, 0) == hipSuccess &&
+             hipEventRecord(g.over, g.behind) == hipSuccess;
+  return g.marked;
+}
+
 struct Retired {
   std::mutex mutex;
   std::atomic<size_t> count{0};
@@ -121,11 +136,7 @@ void reapGraphs(bool wait) {
   std::lock_guard<std::mutex> lock(r.mutex);
   for (size_t i = 0; i < r.graphs.size();) {
     RetiredGraph& g = r.graphs[i];
-    if (!g.behind && hipStreamCreateWithFlags(&g.behind, hipStreamNonBlocking) != hipSuccess) g.behind = nullptr;
-    if (!g.over && hipEventCreateWithFlags(&g.over, hipEventDisableTiming) != hipSuccess) g.over = nullptr;
-    if (!g.ordered && g.behind && g.over)
-      g.ordered = hipStreamWaitEvent(g.behind, g.ran, 0) == hipSuccess && hipEventRecord(g.over, g.behind) == hipSuccess;
-    if (!g.ordered || (wait ? hipEventSynchronize(g.over) : hipEventQuery(g.over)) != hipSuccess) {
+    if (!mark(g) || (wait ? hipEventSynchronize(g.over) : hipEventQuery(g.over)) != hipSuccess) {
       (void)hipGetLastError();  // not ready, or not now: no error of the caller's
       ++i;
       continue;
@@ -140,14 +151,21 @@ void reapGraphs(bool wait) {
   r.count.store(r.graphs.size(), std::memory_order_relaxed);
 }
 
-void dropGraph(d3d_schedule* s) {
+// `stream`: the stream of the last launch or one that the caller has ordered behind it.
+void dropGraph(d3d_schedule* s, hipStream_t stream) {
   if (!s->graph) return;
-  Retired& r = retired();
+  const RelaxedCapture relaxed;
   RetiredGraph g;
   g.graph = s->graph;
-  g.ran = s->graphRan;
+  g.launchedOn = stream;
   s->graph = nullptr;
-  s->graphRan = nullptr;
+  if (!s->launched) {
+    (void)hipGraphExecDestroy(g.graph);
+    return;
+  }
+  s->launched = false;
+  if (!mark(g)) (void)hipGetLastError();
+  Retired& r = retired();
   std::lock_guard<std::mutex> lock(r.mutex);
   r.graphs.push_back(g);
   r.count.store(r.graphs.size(), std::memory_order_relaxed);
@@ -156,7 +174,6 @@ void dropGraph(d3d_schedule* s) {
 // Captures every step into one graph, each behind the last nodes of the steps it waits for.  False (and no graph) if
 // any part of it is refused; nothing has been enqueued then.
 bool captureGraph(d3d_schedule* s) {
-  dropGraph(s);
   hipGraph_t graph = nullptr;
   hipStream_t q = nullptr;
   bool ok;
@@ -210,14 +227,9 @@ bool captureGraph(d3d_schedule* s) {
     ok = hipStreamEndCapture(q, &same) == hipSuccess && ok;
   }
   const RelaxedCapture relaxed;
-  hipEvent_t ran = nullptr;
-  if (ok) ok = hipEventCreateWithFlags(&ran, hipEventDisableTiming) == hipSuccess;
   if (ok) ok = hipGraphInstantiateWithFlags(&s->graph, graph, 0) == hipSuccess;
-  if (ok) {
-    s->graphRan = ran;
-  } else {
+  if (!ok) {
     s->graph = nullptr;
-    if (ran) (void)hipEventDestroy(ran);
     (void)hipGetLastError();
   }
   (void)hipGraphDestroy(graph);
@@ -248,7 +260,7 @@ int32_t appendStep(d3d_schedule* s, d3d_schedule::Step&& st, const int32_t* afte
   }
   for (int i = me - 1; i >= 0 && st.before < 0; --i)
     if (s->steps[static_cast<size_t>(i)].lane == st.lane) st.before = i;
-  dropGraph(s);
+  dropGraph(s, s->launchedOn);
   s->lastChanges = ~0ull;
   s->steps.push_back(std::move(st));
   return me;
@@ -286,7 +298,7 @@ void d3d_schedule_destroy(d3d_schedule* s) {
   if (!s) return;
   if (s->graph || s->lanes.size() > 1) {
     const RelaxedCapture relaxed;
-    dropGraph(s);
+    dropGraph(s, s->launchedOn);
     reapGraphs(true);
     for (auto& st : s->steps)
       if (st.done) (void)hipEventDestroy(st.done);
@@ -392,12 +404,13 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
   s->steady = s->lastChanges == changes ? s->steady + 1 : 0;
   if (s->steady >= s->patience && !(s->graph && s->graphChanges == changes)) {
     // what the operators enqueue is settled, and the pass repeats: capturing it costs about what one pass does
+    dropGraph(s, main);
     const bool captured = captureGraph(s);
     s->graphChanges = changes;
     if (captured && changesOf(s) == changes) {
       s->patience = d3d_schedule::kSteadyRuns;
     } else {  // refused, which may pass (memory, a capture in another thread), or an operator is not settled after all
-      dropGraph(s);
+      dropGraph(s, main);
       s->steady = 0;
       s->patience = std::min(2 * s->patience, d3d_schedule::kMostPatience);
     }
@@ -406,12 +419,8 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
     s->lastChanges = changes;
     const hipError_t launched = hipGraphLaunch(s->graph, main);
     if (launched != hipSuccess) return hipFail(launched, "hipGraphLaunch");
-    const hipError_t marked = hipEventRecord(s->graphRan, main);
-    if (marked != hipSuccess) {
-      s->graph = nullptr;  // never destroyed: nothing would say when it has run
-      s->graphRan = nullptr;
-      return hipFail(marked, "hipEventRecord");
-    }
+    s->launched = true;
+    s->launchedOn = main;  // runs use the same tensors, so the caller orders them: the last launch is the last to end
     return D3D_OK;
   }
   hipError_t e = hipSuccess;

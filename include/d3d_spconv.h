@@ -233,11 +233,13 @@ int32_t d3d_set_option(d3d_plugin* p, int32_t option, int64_t value);
  *   synchronisation.  The first two runs enqueue step by step; when nothing about the operators has changed since
  *   (options, links, capacities, reserved buffers), the steps are captured into one HIP graph, which the schedule keeps and
  *   later runs launch - until something changes.  A capture that is refused is tried again after twice as many runs.
- *   Returns the first failing status; steps behind a failed one are not enqueued.  Refused with D3D_ERR_UNSUPPORTED while `stream` is capturing (capture the operators' own enqueues instead).  One thread at
- *   a time per schedule.
- * d3d_schedule_destroy: waits for the schedule's runs, then frees its streams and its graph; the operators stay the
- *   caller's.  Allowed while a stream is being captured: a graph last launched on that very stream is not waited for but
- *   freed by a later call, and what its steps use must outlive it as for any run in flight. */
+ *   Returns the first failing status; steps behind a failed one are not enqueued.  Refused with D3D_ERR_UNSUPPORTED while
+ *   `stream` is capturing (capture the operators' own enqueues instead).  One thread at a time per schedule; runs use the
+ *   same tensors, so runs on different streams are the caller's to order.
+ * d3d_schedule_destroy: waits for the last run, whose stream must still exist, then frees the schedule's streams and its
+ *   graph; the operators stay the caller's.  Allowed while a stream is being captured: if that is the stream of the last
+ *   run, a graph is not waited for but freed by a later call of these functions, and what its steps use must outlive it
+ *   as for any work in flight. */
 typedef struct d3d_schedule d3d_schedule;
 int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out);
 int32_t d3d_schedule_add(d3d_schedule* s, d3d_plugin* plugin, const d3d_tensor_desc* in_desc, int32_t nb_in,

@@ -203,6 +203,53 @@ def test_repeated_passes_become_a_graph_and_follow_changes(engine, dtype):
         check(x, live)
 
 
+@pytest.mark.parametrize("between", ["capture", "scheduled"])
+def test_recorded_passes_beside_other_ways_to_run(engine, between):
+    """forward on one set of buffers, a capture or the native schedule on another in between, before and after the former
+    became a graph: every result is of its own input."""
+    from deploy3d_amd import layers, synth
+    cfg = synth.config3(8000)
+    specs, weights = cfg["layers"], cfg["weights"]
+    n = len(cfg["coords"])
+    caps = layers.plan_capacities(specs, n, layers.measure_output_counts(specs, cfg["coords"], cfg["grid"]))
+    net, plain = layers.SparseBackbone(specs, weights, caps), layers.SparseBackbone(specs, weights, caps)
+    a = layers.make_input(cfg["coords"], cfg["feats"], cfg["grid"])
+    b = layers.make_input(cfg["coords"][: n // 2], -cfg["feats"][: n // 2], cfg["grid"], capacity=n)
+
+    def want(x):
+        y = plain._forward_steps(x)
+        return y.feats.clone(), int(y.num_act.item()), y.coors.clone()
+
+    def check(y, ref):
+        assert int(y.num_act.item()) == ref[1] and torch.equal(y.feats, ref[0])
+        assert torch.equal(y.coors[:ref[1]], ref[2][:ref[1]])
+
+    want_a, want_b = want(a), want(b)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for warm in (2, 7):
+            for _ in range(warm):
+                check(net.forward(a), want_a)
+            if between == "capture":
+                stream.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=stream):
+                    y = net.forward(b)
+                for _ in range(3):
+                    y.feats.zero_()
+                    graph.replay()
+                    check(y, want_b)
+                    check(net.forward(a), want_a)
+            else:
+                for _ in range(4):
+                    check(net.forward_scheduled(b), want_b)
+                    check(net.forward(a), want_a)
+            for _ in range(4):
+                check(net.forward(a), want_a)
+        assert any(net._plans.values())
+
+
 def test_cast_and_sum_steps(engine):
     """The elementwise steps of a schedule against torch, at counts around a vector's length and unaligned addresses."""
     from deploy3d_amd.plugin import Schedule
