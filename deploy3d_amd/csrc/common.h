@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 
 #include "d3d_spconv.h"
 
@@ -45,6 +46,19 @@ uint64_t pluginChanges(const d3d_plugin* p);
       return D3D_ERR_DEVICE;                                                             \
     }                                                                                    \
   } while (0)
+
+// Body of an entry point of the C ABI: an exception ends as a status, never in the caller's language.
+#define D3D_GUARD_BEGIN try {
+#define D3D_GUARD_END(ret)                        \
+  }                                               \
+  catch (const std::bad_alloc&) {                 \
+    ::d3d::setError("out of host memory");        \
+    return ret;                                   \
+  }                                               \
+  catch (...) {                                   \
+    ::d3d::setError("unexpected C++ exception");  \
+    return ret;                                   \
+  }
 
 // Geometry of one rulebook, always widened to four spatial dims: missing
 // leading dims get kernel 1, stride 1, padding 0, dilation 1 and extent 1, so

@@ -1337,18 +1337,6 @@ constexpr const char* kVersion = "2.0";
 // ---------------------------------------------------------------------------
 using namespace d3d;
 
-#define D3D_GUARD_BEGIN try {
-#define D3D_GUARD_END(ret)                         \
-  }                                                \
-  catch (const std::bad_alloc&) {                  \
-    setError("out of host memory");                \
-    return ret;                                    \
-  }                                                \
-  catch (...) {                                    \
-    setError("unexpected C++ exception");          \
-    return ret;                                    \
-  }
-
 namespace d3d {
 uint64_t pluginChanges(const d3d_plugin* p) { return p->changeCount(); }
 }  // namespace d3d

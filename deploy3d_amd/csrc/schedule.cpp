@@ -271,6 +271,7 @@ int32_t appendStep(d3d_schedule* s, d3d_schedule::Step&& st, const int32_t* afte
 extern "C" {
 
 int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
+  D3D_GUARD_BEGIN
   if (!out || n_lanes < 1 || n_lanes > 8) {
     d3d::setError("schedule: 1 to 8 lanes");
     return D3D_ERR_BAD_ARG;
@@ -292,9 +293,11 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
   }
   *out = s;
   return D3D_OK;
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
 
 void d3d_schedule_destroy(d3d_schedule* s) {
+  D3D_GUARD_BEGIN
   if (!s) return;
   if (s->graph || s->lanes.size() > 1) {
     const RelaxedCapture relaxed;
@@ -312,12 +315,14 @@ void d3d_schedule_destroy(d3d_schedule* s) {
     if (s->fork) (void)hipEventDestroy(s->fork);
   }
   delete s;
+  D3D_GUARD_END()
 }
 
 int32_t d3d_schedule_add(d3d_schedule* s, d3d_plugin* plugin, const d3d_tensor_desc* in_desc, int32_t nb_in,
                          const d3d_tensor_desc* out_desc, int32_t nb_out, const void* const* inputs,
                          void* const* outputs, void* workspace, size_t workspace_bytes, int32_t lane,
                          const int32_t* after, int32_t nb_after) {
+  D3D_GUARD_BEGIN
   if (!s || !plugin || nb_in < 0 || nb_out < 0 || nb_after < 0 || (nb_in && (!in_desc || !inputs)) ||
       (nb_out && (!out_desc || !outputs)) || (nb_after && !after) || lane < 0 ||
       lane >= static_cast<int32_t>(s->lanes.size())) {
@@ -347,10 +352,12 @@ int32_t d3d_schedule_add(d3d_schedule* s, d3d_plugin* plugin, const d3d_tensor_d
   st.workspaceBytes = workspace_bytes;
   st.lane = lane;
   return appendStep(s, std::move(st), after, nb_after);
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
 
 int32_t d3d_schedule_add_sum(d3d_schedule* s, int32_t dtype, const void* a, const void* b, void* out, int64_t count,
                              int32_t lane, const int32_t* after, int32_t nb_after) {
+  D3D_GUARD_BEGIN
   if (!s || count < 0 || (count && (!a || !b || !out))) {
     d3d::setError("schedule: bad sum (null tensor or negative count)");
     return D3D_ERR_BAD_ARG;
@@ -367,10 +374,12 @@ int32_t d3d_schedule_add_sum(d3d_schedule* s, int32_t dtype, const void* a, cons
   st.outputs = {out};
   st.lane = lane;
   return appendStep(s, std::move(st), after, nb_after);
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
 
 int32_t d3d_schedule_add_cast(d3d_schedule* s, int32_t dtype, const void* a, void* out, int64_t count, int32_t lane,
                               const int32_t* after, int32_t nb_after) {
+  D3D_GUARD_BEGIN
   if (!s || count < 0 || (count && (!a || !out))) {
     d3d::setError("schedule: bad cast (null tensor or negative count)");
     return D3D_ERR_BAD_ARG;
@@ -387,9 +396,11 @@ int32_t d3d_schedule_add_cast(d3d_schedule* s, int32_t dtype, const void* a, voi
   st.outputs = {out};
   st.lane = lane;
   return appendStep(s, std::move(st), after, nb_after);
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
 
 int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
+  D3D_GUARD_BEGIN
   if (!s) return D3D_ERR_BAD_ARG;
   hipStream_t main = static_cast<hipStream_t>(stream);
   // A run puts event edges between streams that are not the caller's; under stream capture that is a topology
@@ -453,6 +464,7 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
   if (rc != D3D_OK || now != changes) s->steady = 0;
   s->lastChanges = rc == D3D_OK ? now : ~0ull;
   return rc;
+  D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
 
 int32_t d3d_schedule_size(const d3d_schedule* s) { return s ? static_cast<int32_t>(s->steps.size()) : D3D_ERR_BAD_ARG; }

@@ -5,11 +5,22 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
+#include <cstdlib>
 #include <map>
+#include <new>
 #include <set>
 
 #include "common.h"
 #include "d3d_spconv.h"
+
+static bool noMemory = false;  // host allocations fail
+void* operator new(size_t n) {
+  void* p = noMemory ? nullptr : std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 int pendingWork = 0, graphLaunches = 0, steps = 0, captures = 0, refusals = 0, liveGraphs = 0, liveEvents = 0, liveStreams = 0;
@@ -234,10 +245,28 @@ int refusedForAWhile() {
   d3d_schedule_destroy(s);
   return 0;
 }
+
+// Host memory that runs out is a status, not an exception in the caller's language.
+int outOfHostMemory() {
+  d3d_schedule *s = make(), *none = nullptr;
+  const int32_t size = d3d_schedule_size(s);
+  d3d_tensor_desc in[4], out[1];
+  const void* ins[4] = {};
+  void* outs[1] = {};
+  noMemory = true;
+  const int32_t created = d3d_schedule_create(1, &none);
+  const int32_t added = d3d_schedule_add(s, reinterpret_cast<d3d_plugin*>(16), in, 4, out, 1, ins, outs, nullptr, 0, 0, nullptr, 0);
+  const int32_t summed = d3d_schedule_add_sum(s, D3D_FLOAT, in, in, in, 1, 0, nullptr, 0);
+  noMemory = false;
+  CHECK(created < 0 && !none && added < 0 && summed < 0 && d3d_schedule_size(s) == size);
+  CHECK(d3d_schedule_run(s, kMain) == D3D_OK);
+  d3d_schedule_destroy(s);
+  return 0;
+}
 }  // namespace
 
 int main() {
-  if (destroyUnderCapture() || changeWithoutWaiting() || refusedForAWhile()) return 1;
+  if (destroyUnderCapture() || changeWithoutWaiting() || refusedForAWhile() || outOfHostMemory()) return 1;
   std::puts("schedule_check ok");
   return 0;
 }
