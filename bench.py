@@ -357,8 +357,8 @@ def main():
                      "outputs_equal_full_pass": bool(n2 == int(y.num_act.item()) and torch.equal(y2.feats, y.feats)
                                                      and torch.equal(y2.coors[:n2], y.coors[:n2]))}
             del net2, graph2
-        # third figure: the same pass recorded once as a native schedule (d3d_schedule_*, three lanes with direct
-        # events, no HIP graph) - what a caller without graph capture gets; its host cost per pass is reported
+        # third figure: the same pass recorded once as a native schedule (d3d_schedule_*, three lanes), which captures its
+        # steps itself after two runs - what a caller without graph capture gets; its host cost per pass is reported
         sched = None
         if not args.no_graph and not args.no_fused and all("+" not in (s.get("src") or "") for s in specs):
             net3 = layers.SparseBackbone(specs, weights, caps, dtype=dtype, overlap=False)
@@ -373,8 +373,8 @@ def main():
             torch.cuda.synchronize()
             ms3 = (time.perf_counter() - t0) * 1e3 / args.steps
             sched = {"ms_per_step": round(ms3, 4), "host_ms_per_pass": round(host3, 4),
-                     "what": "the pass enqueued by one d3d_schedule_run per step: no HIP graph, rulebooks on two "
-                             "lanes of their own, events straight between the lanes",
+                     "what": "one d3d_schedule_run per step: a launch of the HIP graph that the schedule captured from "
+                             "its steps, rulebooks on two branches of their own, dependencies straight between steps",
                      "outputs_equal_full_pass": bool(torch.equal(y3.feats, y.feats))}
             del net3
         # further figures beside `value` (same kernels, other conditions): what a caller gets who binds the operators
