@@ -179,7 +179,7 @@ def scratch(nbytes, device, stream):
     so they may share it; those of two threads interleave launch by launch.  A call under stream capture gets memory of its
     own, from the pool of the graph that is being captured: the graph reads and writes it for as long as it is replayed,
     whatever later calls need."""
-    if _capturing():
+    if stream and _capturing():  # the null stream cannot be captured
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     buffers = _scratch.buffers
     ws = buffers.get((device, stream))
