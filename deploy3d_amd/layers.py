@@ -217,10 +217,11 @@ class SparseBackbone:
         key = self._buffers_of(x)
         plan = self._plans.get(key)
         if not plan or plan.expired():
-            for k in [k for k, p in self._plans.items() if p and p.expired()]:
-                del self._plans[k]
-                self._last = None
-            plan = self._plans.get(key)
+            gone = [k for k, p in self._plans.items() if p and p.expired()]
+            if gone:
+                for k in gone:
+                    del self._plans[k]
+                self._last, plan = None, self._plans.get(key)
         again = self._last is not None and self._last[0] == key
         self._repeats = self._repeats + 1 if again else 0
         if plan is None and self._repeats >= 2:
@@ -234,47 +235,46 @@ class SparseBackbone:
             return y
         self._last = (key, None)
         plan.schedule.run()
-        return self._hand_out(plan.made, x)
+        return self._hand_out(plan.made, x, SparseTensor(x.feats, x.coors, x.num_act, x.grid))
 
     # What a pass left behind goes to the caller as objects of that pass's own (over the same tensors): what is rebound on
-    # a result is neither in what is recorded nor in the next pass's result.  Made when asked for: 70 us of a VoxelNet pass.
-    def _hand_out(self, made, x):
-        """``made``, a pass on the buffers of ``x``, is the pass whose results are shown; returns its last SparseTensor."""
-        self._made, self._shown = made, {}
+    # a result is neither in what is recorded nor in the next pass's result.  Made when asked for: 30 us for a VoxelNet pass.
+    def _hand_out(self, made, x, named=None):
+        """``made``, a pass on the buffers of ``x``, is the pass whose results are shown; returns its last SparseTensor.
+        ``named``: holds the tensors that names in ``made`` stand for (see _Plan), apart from ``x``, which the caller may
+        rebind."""
+        self._made, self._shown, self._named = made, {}, named
         self._own_of = {id(made[2]["input"]): x}
-        self._input = dict(feats=x.feats, coors=x.coors, num_act=x.num_act)
         return self._own(made[2][self.specs[-1]["name"]])
 
     def _own(self, t):
         own = self._own_of.get(id(t))
         if own is None:
-            own = self._own_of[id(t)] = copy.copy(t)
-            for name, v in vars(own).items():
-                if type(v) is str:  # a tensor of the input (see _Plan)
-                    setattr(own, name, self._input[v])
-            if isinstance(own, SparseTensor):
-                own.grid = list(t.grid)
+            own = self._own_of[id(t)] = object.__new__(type(t))
+            for name, v in t.__dict__.items():
+                kind = type(v)
+                own.__dict__[name] = list(v) if kind is list else getattr(self._named, v) if kind is str else v
         return own
 
-    def _show(self, which, own):
+    def _show(self, which):
         if which not in self._shown:
-            self._shown[which] = {name: own(t) for name, t in self._made[which].items()}
+            self._shown[which] = {name: self._own(t) for name, t in self._made[which].items()}
         return self._shown[which]
 
     @property
     def rulebooks(self):
         """Indice key -> Rulebook of the latest pass."""
-        return self._show(0, self._own)
+        return self._show(0)
 
     @property
     def inputs(self):
         """Layer name -> the SparseTensor it read in the latest pass."""
-        return self._show(1, self._own)
+        return self._show(1)
 
     @property
     def outputs(self):
         """Layer name (and "input") -> SparseTensor of the latest pass."""
-        return self._show(2, self._own)
+        return self._show(2)
 
     _PLANS = 4  # sets of input buffers whose passes are kept as schedules
 
