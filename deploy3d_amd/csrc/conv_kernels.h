@@ -676,9 +676,10 @@ convStaged(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ 
           __syncthreads();  // every wavefront has read the masks before the first index load overwrites them
         }
       }
-      present = static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(present))) |
-                (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(present >> 32)))
-                 << 32);
+      // (the builtin returns an int: without the cast a layer that has tap 31 walks taps 32..63 as well, past table and weights)
+      present = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(present))) |
+                (static_cast<unsigned long long>(static_cast<uint32_t>(
+                     __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(present >> 32)))) << 32);
     }
     const int steps = (sparseTaps ? __popcll(present) : kVol) * KS;
     // Four walks over the present taps, one per consumer (index loads, weight loads, row gathers, resident weight

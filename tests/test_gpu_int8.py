@@ -64,6 +64,12 @@ def test_int8_staged_configurations(engine, monkeypatch, cfg):
     run_int8(3001, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), 128, 32, True, False)
 
 
+@pytest.mark.parametrize("ksize", [(2, 4, 4), (1, 3, 11), (4, 4, 4)])
+def test_int8_staged_kernel_volumes_from_32(engine, ksize):
+    """32 to 64 taps on the barrier-per-tap kernel: its mask of the taps that occur has its 32nd bit set."""
+    run_int8(333, (10, 36, 30), ksize, (1, 1, 1), tuple((k - 1) // 2 for k in ksize), 32, 64, False, False)
+
+
 @pytest.mark.parametrize("shape", ["32,8", "32,6", "32,4", "48,4"])
 @pytest.mark.parametrize("cin,cout", [(64, 128), (128, 128)])
 def test_int8_pipelined_tile_shapes(engine, monkeypatch, shape, cin, cout):
