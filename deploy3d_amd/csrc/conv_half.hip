@@ -1,5 +1,5 @@
 // Instantiates the MFMA convolution kernels (conv_kernels.h) for one storage type.
-#include "conv_kernels.h"
+#include "conv_taps.h"
 
 namespace d3d {
 

@@ -92,6 +92,10 @@ template <> struct Mfma<int8_t> {
   }
 };
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t makeRawBuffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
+}
+
 // Which tiles (or row groups) a persistent workgroup serves, in which order.  Workgroups are dealt to the XCDs
 // round-robin; XCD x serves the x-th contiguous part of the tiles that hold LIVE rows (neighbouring tiles gather
 // many of the same rows: they meet behind one L2), and every n-th of the tiles past the live rows, which only
@@ -325,6 +329,8 @@ convMfma(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   }
 }
 
+// Rows of 64 bytes (fp32 layers of 16 channels, two-byte ones of 32 -> 16), and what conv_taps.h leaves: kernel volumes above 32,
+// rows of 9 to 15 channels, inputs of 3 GB and more.
 // Small layers: the weights of ALL taps fit in LDS.  A workgroup loads them once and then lives on: each of
 // its wavefronts walks, on its own, over groups of 16 output rows (group index strided by the number of
 // wavefronts in the grid), with a private slice of the neighbour table, its own list of the taps that occur
@@ -1076,6 +1082,9 @@ int32_t launchStaged(const ConvArgs& a, hipStream_t stream) {
   return D3D_ERR_UNSUPPORTED;
 }
 
+// conv_taps.h
+template <class T, int RB, int CB, int COUT> int32_t launchTaps(const ConvArgs& a, hipStream_t stream);
+
 // Does the resident-weight kernel take the layer: every tap's weights and 16 wavefronts' table slices in LDS,
 // two workgroups per CU.
 inline bool residentFits(int kVol, int cin, int cout, size_t elemBytes) {
@@ -1089,6 +1098,10 @@ template <class T, int CIN, int COUT>
 int32_t launchMfmaOne(const ConvArgs& a, hipStream_t stream) {
   if (a.rowChannels > 0 && a.rowChannels < CIN) {  // narrow rows read as stored: the resident kernel only
     if constexpr (CIN == 16 && (COUT == 16 || COUT == 32)) {
+      if (a.rowChannels <= 8) {
+        const int32_t rc = launchTaps<T, 0, 16, COUT>(a, stream);
+        if (rc != D3D_ERR_UNSUPPORTED) return rc;
+      }
       if (residentFits(a.kVol, CIN, COUT, sizeof(T))) return launchMfmaResident<T, CIN, COUT, -1>(a, stream);
     }
     return D3D_ERR_UNSUPPORTED;
@@ -1096,6 +1109,12 @@ int32_t launchMfmaOne(const ConvArgs& a, hipStream_t stream) {
   if constexpr (CIN * COUT >= 512) {
     if (a.staged >= 0) {
       const int32_t rc = launchStaged<T, CIN, COUT>(a, stream);
+      if (rc != D3D_ERR_UNSUPPORTED) return rc;
+    }
+  }
+  if constexpr (CIN == 16 && COUT <= 64) {
+    if (a.staged == 0 && a.tileRows == 0) {
+      const int32_t rc = launchTaps<T, 32, 32, COUT>(a, stream);
       if (rc != D3D_ERR_UNSUPPORTED) return rc;
     }
   }
@@ -1180,13 +1199,27 @@ template <int CIN>
 int32_t launchInt8Cout(const ConvArgs& a, hipStream_t stream) {
   if constexpr (CIN == 32) {
     int32_t rc = D3D_ERR_UNSUPPORTED;
-    if (a.rowChannels == 16) {  // rows of 16 stored channels: only the resident kernel reads them as they are
+    if (a.rowChannels == 16) {  // rows of 16 stored channels: only the resident kernels read them as they are
+      if (a.cout == 16) rc = launchTaps<int8_t, 16, 16, 16>(a, stream);
+      if (a.cout == 32) rc = launchTaps<int8_t, 16, 16, 32>(a, stream);
+      if (rc != D3D_ERR_UNSUPPORTED) return rc;
       if (a.cout == 16) return launchInt8Resident<32, 16, 16>(a, stream);
       if (a.cout == 32) return launchInt8Resident<32, 32, 16>(a, stream);
       return D3D_ERR_UNSUPPORTED;
     }
+    if (a.rowChannels > 0 && a.rowChannels <= 8) {
+      if (a.cout == 16) rc = launchTaps<int8_t, 0, 16, 16>(a, stream);
+      if (a.cout == 32) rc = launchTaps<int8_t, 0, 16, 32>(a, stream);
+      if (rc != D3D_ERR_UNSUPPORTED) return rc;
+      if (a.cout == 16) return launchInt8Resident<32, 16, -1>(a, stream);
+      if (a.cout == 32) return launchInt8Resident<32, 32, -1>(a, stream);
+    }
     if (a.rowChannels > 0) return D3D_ERR_UNSUPPORTED;
     if (a.staged == 0) {
+      if (a.cout == 16) rc = launchTaps<int8_t, 32, 32, 16>(a, stream);
+      if (a.cout == 32) rc = launchTaps<int8_t, 32, 32, 32>(a, stream);
+      if (a.cout == 64) rc = launchTaps<int8_t, 32, 32, 64>(a, stream);
+      if (rc != D3D_ERR_UNSUPPORTED) return rc;
       if (a.cout == 16) rc = launchInt8Resident<32, 16>(a, stream);
       if (a.cout == 32 && a.tileMasks == nullptr) rc = launchInt8Resident<32, 32>(a, stream);
       if (a.cout == 64 && a.tileMasks == nullptr) rc = launchInt8Resident<32, 64>(a, stream);

@@ -32,10 +32,6 @@ namespace convk {
 
 typedef __attribute__((address_space(3))) void* LdsVoidPtr;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t makeRawBuffer(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
-}
-
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
 // ceil(outRows / 64) (a workgroup reads the masks of a whole tile at once); null = every tap of every tile.
 template <class T, int CIN, int COUT, int MT, int WAVES>

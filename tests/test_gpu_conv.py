@@ -163,6 +163,21 @@ def test_resident_32_to_32(engine, ksize, dtype):
         run_case(2500, (10, 36, 30), ksize, (2, 2, 2), pad, 32, 32, dtype, False, inverse=True)
 
 
+@pytest.mark.parametrize("cin,cout", [(1, 16), (3, 32), (4, 16), (5, 16), (7, 32), (8, 16), (9, 16), (16, 16), (16, 32), (16, 64)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_rows_of_at_most_32_bytes(engine, cin, cout, dtype):
+    """Two or four taps per MFMA (conv_taps.h): around its 16-row groups, kernel volumes on either side of a multiple of four
+    and of the 32 taps it takes, rows that begin at any even byte, inputs that end with the buffer."""
+    for n in (1, 15, 16, 17, 2500):
+        run_case(n, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=(n == 17),
+                 cap_extra=n % 3 * 40, link=n != 16)
+    for ksize in ((1, 1, 1), (1, 1, 3), (2, 2, 2), (2, 3, 4), (1, 5, 5), (2, 2, 7), (1, 2, 15), (2, 4, 4), (1, 3, 11)):
+        pad = tuple((k - 1) // 2 for k in ksize)
+        run_case(333, (10, 36, 30), ksize, (1, 1, 1), pad, cin, cout, dtype, False, with_bias=ksize != (2, 2, 2))
+    run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False)
+    run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False, inverse=True)
+
+
 def test_narrow_strided_fp32(engine):
     run_case(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), 16, 16, "float32", False)
 

@@ -51,6 +51,17 @@ def test_int8_subm_bit_exact(engine, cin, cout, relu):
     run_int8(3000, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, True, relu)
 
 
+@pytest.mark.parametrize("cin,cout", [(1, 16), (3, 32), (5, 16), (8, 32), (9, 16), (16, 16), (16, 32), (32, 16), (32, 32), (32, 64)])
+def test_int8_rows_of_at_most_32_bytes(engine, cin, cout):
+    """Two or four taps per MFMA (conv_taps.h): 16-row groups, kernel volumes around a multiple of four and 32, rows that
+    begin at any byte."""
+    for n in (15, 16, 17, 2500):
+        run_int8(n, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, True, n == 17)
+    for ksize in ((1, 1, 1), (2, 2, 2), (1, 5, 5), (2, 2, 7), (1, 2, 15), (2, 4, 4), (1, 3, 11)):
+        run_int8(333, (10, 36, 30), ksize, (1, 1, 1), tuple((k - 1) // 2 for k in ksize), cin, cout, False, False)
+    run_int8(2500, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, False, True)
+
+
 @pytest.mark.parametrize("cin,cout", [(16, 32), (32, 64), (64, 128), (128, 128)])
 def test_int8_strided_bit_exact(engine, cin, cout):
     run_int8(3000, (10, 36, 30), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, False, True)
