@@ -1341,12 +1341,19 @@ __device__ __forceinline__ void finishScan(uint32_t total, const RecRef& recRef,
 // map of the input grid (gatherOccupancy) and stored with the prefix.
 // That variant runs 1024 threads per workgroup: one thread per record of the chunk gathers (27 independent loads),
 // the bits pass through LDS, and the first 256 threads go on with the scan as always.
+// Workgroups past the chunks set fill[0..nFill) to -1: the table that the probe pass of a build whose index tensor nobody
+// reads scatters into - streaming stores beside a pass that waits for loads and atomics.
 template <bool ORDERED, int GATHER>
 __global__ void __launch_bounds__(GATHER ? kRbChunk : kRbThreads)
 bmScan(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, uint32_t* ticket,
-       uint32_t* groupTickets, int32_t* numActOut, int32_t maxNumActOut, GatherArgs ga) {
+       uint32_t* groupTickets, int32_t* numActOut, int32_t maxNumActOut, GatherArgs ga, int32_t* fill, int64_t nFill) {
   __shared__ uint32_t scratch[kRbThreads / 64];
   __shared__ uint32_t isLast;
+  if (blockIdx.x >= nChunks) {
+    fillMinusOneRange(fill, nFill, static_cast<int64_t>(blockIdx.x - nChunks) * blockDim.x + threadIdx.x,
+                      static_cast<int64_t>(gridDim.x - nChunks) * blockDim.x);
+    return;
+  }
   const uint32_t epoch = recRef.epoch ? *recRef.epoch : 0u;
   BmRecord* __restrict__ records = recRef.base + static_cast<size_t>(epoch & 1u) * (recRef.epoch ? recRef.stride : 0u);
   // two maps: the occupancy bits of the one the next build marks are cleared here, record by record
@@ -1421,8 +1428,13 @@ bmScan(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, 
 template <bool ORDERED, int GATHER>
 __global__ void __launch_bounds__(64)
 bmScanSmall(RecRef recRef, uint32_t nRecords, uint32_t* chunkBase, uint32_t nChunks, uint32_t* ticket,
-            uint32_t* groupTickets, int32_t* numActOut, int32_t maxNumActOut, GatherArgs ga) {
+            uint32_t* groupTickets, int32_t* numActOut, int32_t maxNumActOut, GatherArgs ga, int32_t* fill, int64_t nFill) {
   __shared__ uint32_t isLast;
+  if (blockIdx.x >= nChunks) {
+    fillMinusOneRange(fill, nFill, static_cast<int64_t>(blockIdx.x - nChunks) * blockDim.x + threadIdx.x,
+                      static_cast<int64_t>(gridDim.x - nChunks) * blockDim.x);
+    return;
+  }
   const uint32_t epoch = recRef.epoch ? *recRef.epoch : 0u;
   BmRecord* __restrict__ records = recRef.base + static_cast<size_t>(epoch & 1u) * (recRef.epoch ? recRef.stride : 0u);
   BmRecord* __restrict__ other = recRef.epoch ? recRef.base + static_cast<size_t>((epoch + 1u) & 1u) * recRef.stride : nullptr;
@@ -2355,7 +2367,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     const bool twoMaps = mapOutside && side.mapState && side.mapStride > 0 &&
                          (sharedMap ? side.mapDouble
                                     : (side.mapStride == static_cast<int64_t>(w.nRecords) && near && ksel != 0 &&
-                                       !side.skipIndex && !side.mapDirty));
+                                       !side.mapDirty));
     side.mapDouble = twoMaps;
     uint32_t* const epochPtr = twoMaps ? side.mapState : nullptr;
     const uint32_t recStride = twoMaps ? static_cast<uint32_t>(side.mapStride) : 0u;
@@ -2370,8 +2382,8 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     const size_t nearLds = static_cast<size_t>(kNearGroup) * kRbThreads * sizeof(uint4) + static_cast<size_t>(g.kVol) * 4;
     // A build whose index tensor nobody reads (side.skipIndex) writes table and masks in the probe pass and skips
     // the compaction: for the kernel shapes of the plane probe, a SubM build with the mirrored table staged in
-    // place, or a strided build with a table to scatter into (which the reset pass then fills with -1, since the
-    // probe pass writes entries into it).
+    // place, or a strided build with a table to scatter into (which the scan pass - or the reset pass, where there is
+    // one - fills with -1, since the probe pass writes entries into it).
     skipIndex = side.skipIndex && near && ksel != 0 && nbrOut && (subM ? (mirror && inPlace) : true);
     // (with the index tensor written it does not pay: the fill, moved into the reset pass, is no longer hidden
     // beside the probe - measured 1-2 us slower per strided build)
@@ -2379,12 +2391,15 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     const bool probeMasks = subM && mirror && masks && near && ksel != 0;
     if (probeMasks) compactMasks = nullptr;
     side.indexWritten = !skipIndex;
-    int32_t* const resetFill = directScatter ? nbrOut : ((near || skipIndex) ? nullptr : fillIndex);
+    // With two maps nothing is left to reset but that table, and the scan fills it: five launches of 5 us less in a pass of
+    // eight such builds (60 000 voxels to a dense map through an imported graph: 577 -> 571 us).
+    const bool scanFills = directScatter && twoMaps;
+    int32_t* const resetFill = directScatter ? (scanFills ? nullptr : nbrOut) : ((near || skipIndex) ? nullptr : fillIndex);
     const int64_t resetFillN = directScatter ? static_cast<int64_t>(g.kVol) * nbrRows : nIndex;
     const int64_t clearRecords = sharedMap ? 0 : static_cast<int64_t>(w.nRecords);
     // A build on a shared map with the fixed-shape probe leaves nothing to zero: the probe writes counts and tile
     // masks with plain stores, the compaction sums the counts itself, numIndex is written last.
-    needReset = !((sharedMap || twoMaps) && near && ksel != 0 && !directScatter && !resetFill && compactMasks == nullptr);
+    needReset = !((sharedMap || twoMaps) && near && ksel != 0 && !resetFill && compactMasks == nullptr);
     if (needReset)
       hipLaunchKernelGGL(bmReset, fillGrid(clearRecords + (resetFill ? resetFillN / 4 : 0) + 1), block, 0,
                          stream, reinterpret_cast<uint4*>(records), clearRecords,
@@ -2443,15 +2458,23 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       hipLaunchKernelGGL(bmMarkCandidates, perTap, block, 0, stream, g, m, coors, numActIn, cap, recBefore);
     }
     // D3D_RULEBOOK_ORDERED_SCAN=1: acquire-release tickets (see bmScan)
-#define D3D_LAUNCH_SCAN(ORDERED, GATHER)                                                                          \
+    const int64_t nScanFill = scanFills ? resetFillN : 0;
+    auto scanGrid = [&](int threads) {  // a workgroup per chunk, then the ones that fill the table
+      int64_t fillers = (nScanFill / 4 + threads - 1) / threads;
+      if (fillers > 131072 / threads) fillers = 131072 / threads;
+      return dim3(static_cast<unsigned>(perChunk.x + fillers));
+    };
+#define D3D_LAUNCH_SCAN(ORDERED, GATHER)                                                                              \
   do {                                                                                                                \
     if (m.chunkShift == kSmallChunkShift)                                                                             \
-      hipLaunchKernelGGL((bmScanSmall<ORDERED, GATHER>), perChunk, dim3(64), 0, stream, recBefore, w.nRecords, chunkBase, \
-                         w.nChunks, scanTicket, scanTicket + 1, subM ? nullptr : numActOut, maxNumActOut, ga);        \
+      hipLaunchKernelGGL((bmScanSmall<ORDERED, GATHER>), scanGrid(64), dim3(64), 0, stream, recBefore, w.nRecords,    \
+                         chunkBase, perChunk.x, scanTicket, scanTicket + 1, subM ? nullptr : numActOut, maxNumActOut, \
+                         ga, scanFills ? nbrOut : nullptr, nScanFill);                                                \
     else                                                                                                              \
-      hipLaunchKernelGGL((bmScan<ORDERED, GATHER>), perChunk, dim3(GATHER ? kRbChunk : kRbThreads), 0, stream, recBefore, \
-                         w.nRecords, chunkBase, w.nChunks, scanTicket, scanTicket + 1, subM ? nullptr : numActOut,    \
-                         maxNumActOut, ga);                                                                           \
+      hipLaunchKernelGGL((bmScan<ORDERED, GATHER>), scanGrid(GATHER ? kRbChunk : kRbThreads),                         \
+                         dim3(GATHER ? kRbChunk : kRbThreads), 0, stream, recBefore, w.nRecords, chunkBase,           \
+                         perChunk.x, scanTicket, scanTicket + 1, subM ? nullptr : numActOut, maxNumActOut, ga,        \
+                         scanFills ? nbrOut : nullptr, nScanFill);                                                    \
   } while (0)
     const bool ordered = debugEnv("D3D_RULEBOOK_ORDERED_SCAN") != nullptr;
     if (sharedMap) {
