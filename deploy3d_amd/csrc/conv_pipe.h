@@ -32,14 +32,35 @@ namespace convk {
 
 typedef __attribute__((address_space(3))) void* LdsVoidPtr;
 
+// Wavefronts of the largest shape of a layer of 128 output channels.  int8 128 -> 128: the wider workgroups (two wavefronts per
+// SIMD, 256 registers each) spill - 84-97 us against 33-44 on a 47 000-row layer - so only the four-wavefront shapes count.
+template <class T, int CIN>
+constexpr int pipeWaves() { return sizeof(T) == 1 && CIN == 128 ? 4 : 8; }
+
+// Whether the 48-row shape is among those a kernel chooses from: in two-byte types it takes 278 registers, which workgroups of
+// eight wavefronts do not have (256 and a spill: 59 us where it takes 45 by itself).
+template <class T> constexpr bool kPipeTall = sizeof(T) == 1;
+
+// Shapes of those layers, rows per wavefront x wavefronts: 0: 32 x 8, 1: 32 x 6, 2: 32 x 4, 3: 48 x 4.  The one that loads the
+// busiest of `cus` CUs least with `rows` rows (rounds of tiles x rows per tile); see launchPipeShape.
+template <bool FOUR_ONLY>
+__host__ __device__ inline int pipeShapeOf(int64_t rows, int cus) {
+  auto load = [&](int tile) { return static_cast<int>((rows + static_cast<int64_t>(tile) * cus - 1) / (static_cast<int64_t>(tile) * cus)) * tile; };
+  const int l8 = load(256), l6 = load(192), l4 = load(128);
+  if (FOUR_ONLY) return l4 < l6 ? 2 : 3;
+  int best = l6 < l8 ? 1 : 0;
+  if (l4 < (best ? l6 : l8)) best = 2;
+  return best == 1 && l6 <= 192 ? 3 : best;
+}
+
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
 // ceil(outRows / 64) (a workgroup reads the masks of a whole tile at once); null = every tap of every tile.
 template <class T, int CIN, int COUT, int MT, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES)
-convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
-         const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
-         const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
-         int tileBlocks, int xcdShift, const int32_t* __restrict__ numActOut) {
+__device__ __forceinline__ void
+pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
+          const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch,
+          int tapMirror, const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
+          int xcdShift, const int32_t* __restrict__ numActOut, int blocks) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int ES = static_cast<int>(sizeof(T));
   constexpr int CS = CIN * ES > 128 ? 128 / ES : CIN;          // input channels per step (at most 128 bytes of a row); a tap takes KS steps
@@ -66,7 +87,6 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   using F = u32x4;
   using Acc = typename Mfma<T>::Acc;
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -96,9 +116,9 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
   // ---- this workgroup's tiles: XCD x serves the x-th contiguous part of the tiles that hold live rows
   // (neighbouring tiles gather many of the same rows: they should meet behind one L2) and its share of the tiles
   // past the live rows; inside an XCD, workgroups take tiles round robin ----
-  const TileOrder order(tileBlocks, static_cast<int>((liveOutRows(numActOut, outRows) + TM - 1) / TM), xcdShift,
+  const TileOrder order(static_cast<int>((outRows + TM - 1) / TM), static_cast<int>((liveOutRows(numActOut, outRows) + TM - 1) / TM), xcdShift,
                         blockIdx.x & ((1 << xcdShift) - 1));
-  const int firstLocal = blockIdx.x >> xcdShift, strideLocal = gridDim.x >> xcdShift;
+  const int firstLocal = blockIdx.x >> xcdShift, strideLocal = blocks >> xcdShift;
   const int nMine = firstLocal < order.count() ? (order.count() - 1 - firstLocal) / strideLocal + 1 : 0;
   if (nMine <= 0) return;                                // workgroup-uniform
   auto tileAt = [&](int pos) __attribute__((always_inline)) { return order.tile(firstLocal + pos * strideLocal); };
@@ -417,18 +437,89 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
 }
 
 template <class T, int CIN, int COUT, int MT, int WAVES>
-int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
-  constexpr int CS = CIN * static_cast<int>(sizeof(T)) > 128 ? 128 / static_cast<int>(sizeof(T)) : CIN;
-  constexpr int WM = 16 * MT, TM = WM * WAVES;
-  constexpr int WCH = CS * COUT * static_cast<int>(sizeof(T)) / 16;
-  const size_t lds = static_cast<size_t>(3) * WCH * 16 + static_cast<size_t>(WAVES) * 2 * WM * (CS * sizeof(T)) +
-                     static_cast<size_t>(WAVES) * 4 * WM * 4;
+__global__ void __launch_bounds__(64 * WAVES)
+convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
+         const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
+         const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
+         int xcdShift, const int32_t* __restrict__ numActOut) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  pipeTiles<T, CIN, COUT, MT, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+                                     relu, xcdShift, numActOut, gridDim.x);
+}
+
+// The workgroup shape chosen here, by the rows that are live, for layers whose time is that of a few rounds of tiles (see
+// launchPipeShape): the host knows the capacity only.  Wavefronts past the shape's end at once.
+template <class T, int CIN, int COUT, int MOST>
+__global__ void __launch_bounds__(64 * MOST)
+convPipeByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
+               const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
+               const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
+               int xcdShift, const int32_t* __restrict__ numActOut, int cus) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int shape = pipeShapeOf<MOST == 4>(liveOutRows(numActOut, outRows), cus);
+#define D3D_PIPE_BODY(MT, WAVES)                                                                                        \
+  {                                                                                                                     \
+    if (wave >= WAVES) return;                                                                                          \
+    pipeTiles<T, CIN, COUT, MT, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol,    \
+                                       inRows, outRows, relu, xcdShift, numActOut, WAVES == 4 && MT == 3 ? cus : gridDim.x); \
+  }
+  if constexpr (kPipeTall<T>) {
+    if (shape == 3) {
+      if (blockIdx.x >= static_cast<unsigned>(cus)) return;   // one round: a tile per CU, none beside another
+      D3D_PIPE_BODY(3, 4)
+      return;
+    }
+  }
+  if (shape == 2) D3D_PIPE_BODY(2, 4)
+  else if constexpr (MOST == 8) {
+    if (shape == 0) D3D_PIPE_BODY(2, 8)
+    else D3D_PIPE_BODY(2, 6)
+  }
+#undef D3D_PIPE_BODY
+}
+
+// LDS of a shape: three weight slices, two stages and four steps of indices per wavefront.
+template <class T, int CIN, int COUT>
+constexpr size_t pipeLds(int mt, int waves) {
+  const int cs = CIN * static_cast<int>(sizeof(T)) > 128 ? 128 / static_cast<int>(sizeof(T)) : CIN;
+  return static_cast<size_t>(3) * cs * COUT * sizeof(T) + static_cast<size_t>(waves) * (2 * 16 * mt * cs * sizeof(T) + 4 * 16 * mt * 4);
+}
+
+// 32-bit buffer offsets, and the 64 bits of a tap mask
+inline bool pipeTakes(const ConvArgs& a, int64_t pitch, size_t rowBytes, int tileRows) {
+  return a.kVol <= 64 && static_cast<uint64_t>(a.inRows) * rowBytes < 0xFFFF0000ull &&
+         static_cast<uint64_t>(a.kVol) * static_cast<uint64_t>(pitch) * 4 < 0xFFFF0000ull &&
+         static_cast<uint64_t>(a.outRows) + tileRows < 0x3FFFFFFFull;
+}
+
+template <class T, int CIN, int COUT>
+int32_t launchPipeByRows(const ConvArgs& a, hipStream_t stream) {
+  constexpr int WAVES = pipeWaves<T, CIN>();
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
-  if (lds > kLdsLimit || a.kVol > 64) return D3D_ERR_UNSUPPORTED;
-  if (static_cast<uint64_t>(a.inRows) * CIN * sizeof(T) >= 0xFFFF0000ull ||
-      static_cast<uint64_t>(a.kVol) * static_cast<uint64_t>(pitch) * 4 >= 0xFFFF0000ull ||
-      static_cast<uint64_t>(a.outRows) + TM >= 0x3FFFFFFFull)
-    return D3D_ERR_UNSUPPORTED;                         // 32-bit buffer offsets
+  if (!pipeTakes(a, pitch, CIN * sizeof(T), 256)) return D3D_ERR_UNSUPPORTED;
+  constexpr size_t wide = pipeLds<T, CIN, COUT>(2, WAVES), tall = kPipeTall<T> ? pipeLds<T, CIN, COUT>(3, 4) : 0;
+  constexpr size_t lds = wide > tall ? wide : tall;
+  static_assert(lds <= kLdsLimit, "every shape fits a CU");
+  static std::atomic<size_t> granted{64 * 1024};
+  const int32_t rc = grantLds(&convPipeByRows<T, CIN, COUT, WAVES>, lds, &granted);
+  if (rc != D3D_OK) return rc;
+  const ChipLayout chip = chipLayout();
+  const int nXcd = 1 << chip.xcdShift, cus = chip.cus / nXcd * nXcd;
+  const int perCu = 2 * lds <= kLdsLimit ? 2 : 1;
+  hipLaunchKernelGGL((convPipeByRows<T, CIN, COUT, WAVES>), dim3(static_cast<unsigned>(cus * perCu)), dim3(64 * WAVES), lds, stream,
+                     static_cast<const T*>(a.in), static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias,
+                     a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift,
+                     a.numActOut, cus);
+  return D3D_OK;
+}
+
+template <class T, int CIN, int COUT, int MT, int WAVES>
+int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
+  constexpr int TM = 16 * MT * WAVES;
+  constexpr size_t lds = pipeLds<T, CIN, COUT>(MT, WAVES);
+  const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
+  if (lds > kLdsLimit || !pipeTakes(a, pitch, CIN * sizeof(T), TM)) return D3D_ERR_UNSUPPORTED;
   static std::atomic<size_t> granted{64 * 1024};
   const int32_t rc = grantLds(&convPipe<T, CIN, COUT, MT, WAVES>, lds, &granted);
   if (rc != D3D_OK) return rc;
@@ -444,7 +535,7 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((convPipe<T, CIN, COUT, MT, WAVES>), dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES),
                      lds, stream, static_cast<const T*>(a.in), static_cast<T*>(a.out),
                      static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks,
-                     a.kVol, a.inRows, a.outRows, a.relu, tiles, chip.xcdShift, a.numActOut);
+                     a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut);
   return D3D_OK;
 }
 
@@ -499,29 +590,17 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       if (a.outRows <= 64 * static_cast<int64_t>(chipLayout().cus) && !debugEnv("D3D_CONV_PIPE_SHAPE"))
         return launchPipeCfg<T, CIN, COUT, 2, 2>(a, stream);
     static const int kCand[4][2] = {{32, 8}, {32, 6}, {32, 4}, {48, 4}};
-    // int8 128 -> 128: the wider workgroups (two wavefronts per SIMD, 256 registers each) spill - 84-97 us against
-    // 33-44 on a 47 000-row layer - so only the four-wavefront shapes are candidates, the larger tile winning ties
-    constexpr bool FOUR_ONLY = sizeof(T) == 1 && CIN == 128;
-    int best = FOUR_ONLY ? 3 : 0;
-    int64_t bestCost = 0;
-    const int64_t cus = chipLayout().cus;
-    auto costOf = [&](int c) {
-      const int64_t tm = kCand[c][0] * kCand[c][1], tiles = (a.outRows + tm - 1) / tm;
-      return (tiles + cus - 1) / cus * tm;              // rows the busiest CU multiplies
-    };
-    if (FOUR_ONLY) {
-      if (costOf(2) < costOf(3)) best = 2;
-    } else {
-      for (int c = 0; c < 3; ++c) {
-        const int64_t cost = costOf(c);
-        if (c == 0 || cost < bestCost) {
-          best = c;
-          bestCost = cost;
-        }
-      }
-      if (best == 1 && (a.outRows + 191) / 192 <= cus) best = 3;
-    }
-    if (const char* force = debugEnv("D3D_CONV_PIPE_SHAPE")) {  // "rows,wavefronts" of one candidate (tests)
+    constexpr bool FOUR_ONLY = pipeWaves<T, CIN>() == 4;
+    const char* const force = debugEnv("D3D_CONV_PIPE_SHAPE");  // "rows,wavefronts" of one candidate (tests)
+    // More than a round of the largest tiles: the shape is chosen from the live rows (convPipeByRows; fp16, us: 128 -> 128 with
+    // 190 000 rows at a capacity of 237 000 183 -> 154, at 199 500 202 -> 160, 64 -> 128 104 -> 88; what the host would choose
+    // at the live count takes the same).  Below, that kernel has nothing better to choose in two-byte types: 48-row
+    // wavefronts need a launch of their own, and 32 x 6 in it is no faster than 32 x 8 (53 us).  int8 128 -> 128 has two
+    // shapes, both in it: 47 500 rows at a capacity of 59 400 43 -> 33.
+    if (!force && a.outRows > (FOUR_ONLY ? 128 : 256) * static_cast<int64_t>(chipLayout().cus))
+      return launchPipeByRows<T, CIN, COUT>(a, stream);
+    int best = pipeShapeOf<FOUR_ONLY>(a.outRows, chipLayout().cus);
+    if (force) {
       for (int c = FOUR_ONLY ? 2 : 0; c < 4; ++c)
         if (std::atoi(force) == kCand[c][0] && std::strchr(force, ',') &&
             std::atoi(std::strchr(force, ',') + 1) == kCand[c][1])

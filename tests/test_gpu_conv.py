@@ -381,6 +381,14 @@ def test_pipelined_tile_shapes_of_wide_layers(engine, monkeypatch, shape, cin, c
         run_case(70000, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=True)
 
 
+@pytest.mark.parametrize("cin,dtype", [(32, "float16"), (64, "bfloat16"), (128, "float16")])
+def test_pipelined_tile_shape_by_live_rows(engine, cin, dtype):
+    """Capacities above 256 rows per CU: the kernel chooses its workgroup shape by the live rows - here one round of 128-row
+    tiles, one of 192, one of 256, and several - and serves the rows past them whatever it chose."""
+    for n in (30000, 45000, 60000, 75000):
+        run_case(n, (16, 128, 128), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, dtype, True, relu=True, cap_extra=76011 - n)
+
+
 @pytest.mark.parametrize("cin,cout", [(32, 64), (64, 64), (64, 128), (128, 128)])
 def test_pipelined_tile_shapes_by_row_count(engine, cin, cout):
     """Row counts on both sides of the lines (64, 128 and 256 rows per CU) at which the pipelined kernel takes another

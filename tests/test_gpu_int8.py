@@ -12,16 +12,16 @@ from oracle import oracle
 pytestmark = pytest.mark.gpu
 
 
-def run_int8(n, grid, ksize, stride, padding, cin, cout, subm, relu, with_bias=True, seed=0):
+def run_int8(n, grid, ksize, stride, padding, cin, cout, subm, relu, with_bias=True, seed=0, cap_extra=0):
     from deploy3d_amd import spconv_mm
     rng = np.random.default_rng(seed + 31 * cin + cout + n)
     coords = random_cloud(rng, n, grid, 1)
     n = len(coords)
     kvol = int(np.prod(ksize))
-    max_out = n if subm else 8 * n
-    rb = gpu_rulebook(coords, n, grid, 1, ksize, stride, padding, (1,) * len(ksize), max_out, subm)
+    max_out = n + cap_extra if subm else 8 * n
+    rb = gpu_rulebook(coords, n, grid, 1, ksize, stride, padding, (1,) * len(ksize), max_out, subm, cap=n + cap_extra)
     n_out = n if subm else rb["num_act_out"]
-    x_q = rng.integers(-128, 128, (n, cin)).astype(np.int8)
+    x_q = rng.integers(-128, 128, (n + cap_extra, cin)).astype(np.int8)
     w = (rng.standard_normal((kvol, cin, cout)) / np.sqrt(kvol * cin)).astype(np.float32)
     b = rng.standard_normal(cout).astype(np.float32) if with_bias else None
     s_in, s_out = np.float32(0.043), np.float32(0.057)
@@ -92,6 +92,13 @@ def test_int8_pipelined_tile_shapes(engine, monkeypatch, shape, cin, cout):
     if cin == 64:
         run_int8(5000, (12, 48, 40), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, False, False)
         run_int8(70000, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, True, True)
+
+
+@pytest.mark.parametrize("cin", [64, 128])
+def test_int8_pipelined_tile_shape_by_live_rows(engine, cin):
+    """Capacities above one round of tiles: the kernel chooses its workgroup shape by the live rows."""
+    for n in (30000, 45000, 60000):
+        run_int8(n, (16, 128, 128), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, True, True, cap_extra=76011 - n)
 
 
 @pytest.mark.parametrize("cin,cout", [(64, 32), (64, 64), (128, 64), (128, 128)])
