@@ -87,7 +87,12 @@ struct RbWorkspace {
   int64_t pitch;          // row pitch of staging, a multiple of the chunk size
   size_t table;           // hash: u64 [slots] key<<32 | value;  block map: records [nRecords]
   size_t ids;             // hash: u32 [slots] output row of an occupied slot (strided only);  block map: perm [cap] (SubM)
-  size_t staging;         // u32 [kVol, pitch] per (tap, input): slot, then output row, or ~0
+  size_t staging;         // u32 [kVol, pitch] per (tap, input): slot, then output row, or ~0;  strided builds of the
+                          // fixed-shape probe: the output rows alone, packed per (tap, 64 inputs), with
+  size_t hits;            // u64 [kVol, hitsPitch] which of the 64 inputs they belong to (block map, strided only)
+  uint32_t hitsPitch;
+  size_t offsets;
+  uint32_t offsetPitch;
   size_t ownCnt;          // hash: u32 [kVol, nBlocks] owned outputs per (tap, chunk) (strided only);  block map: chunk totals
   size_t cnt;             // u16 [kVol, cntPitch] valid pairs per (tap, block of 256 or 1024 inputs)
   size_t totals;          // u32 [2, kVol]  valid pairs per tap; owned outputs per tap

@@ -582,11 +582,17 @@ rbConvResolve(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, 
 // Both sums come from the per-(tap, block) counts the probe pass left in `cnt` with plain stores
 // (cnt[tap * cntPitch + b] = pairs of inputs [b << cntShift, (b + 1) << cntShift) under the tap): the sixteen
 // wavefronts of a workgroup sum the rows of the taps up to their own, one row per wavefront at a time, so no pass
-// keeps per-tap totals with device-wide atomics and nothing has to be zeroed before a build.  A workgroup covers
-// `iters` runs of 4096 inputs, which keeps the number of workgroups that repeat these sums small.
+// keeps per-tap totals with device-wide atomics and nothing has to be zeroed before a build.
+// What bounds it then is not bytes but the life of a workgroup (live count, counts, barrier, entries, stores: 7 us) times
+// the rounds of workgroups: 84 us for 12.4 million pairs of 1.4 million inputs, a third of the memory's rate.  From
+// kOffsetRows inputs a pass of one workgroup per tap (rbOffsets, 5 to 8 us) therefore works out where the pairs of every
+// (tap, block) go, and the compaction becomes wavefronts that share nothing: 84 -> 51 us (5.9 TB/s of entries read and
+// pairs written), 72 -> 33 us for the 4.8 million pairs of the strided build behind it.  Below, the extra launch costs
+// what it saves: 366 000 inputs 19.0 us without, 5.1 + 14.5 with; 120 000 inputs 18.0 against 4.6 + 16.5.
 // ---------------------------------------------------------------------------
-constexpr int kCompactThreads = 1024;
-constexpr int kCompactWaves = kCompactThreads / 64;
+constexpr int64_t kOffsetRows = 1 << 19;
+// Workgroups that sum the counts in front of them are large; the others need not be.
+__host__ __device__ constexpr int compactThreads(bool offsets) { return offsets ? 256 : 1024; }
 
 // Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS traffic, no index registers):
 // four shifts inside each row of 16 lanes, then the total of row 0 (2) is added to row 1 (3), then that of rows
@@ -599,6 +605,18 @@ __device__ __forceinline__ uint32_t waveInclusiveScan(uint32_t v) {
   v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xA, 0xF, false));  // row_bcast:15
   v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xC, 0xF, false));  // row_bcast:31
   return v;
+}
+
+// Bits of `v` below the calling lane's.
+__device__ __forceinline__ uint32_t lanesBelow(unsigned long long v) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(v >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(v), 0u));
+}
+
+// The value of `v` in lane `from`, wavefront-uniform.
+__device__ __forceinline__ unsigned long long laneWord(unsigned long long v, int from) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), from));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), from));
+  return static_cast<unsigned long long>(hi) << 32 | lo;
 }
 
 // Sum over the 64 lanes, the same value in every lane.
@@ -627,28 +645,103 @@ __device__ __forceinline__ uint32_t countsBelow(const uint4& v, uint32_t b0, uin
   return sum;
 }
 
+// Where the pairs of every (tap, block of inputs) go in the index tensor: one workgroup per tap sums the rows of cnt in
+// front of its own and scans its own.  Writes numIndex too (and with fillState the end of the used part).
+struct PairOffsets {
+  uint32_t* at;        // [kVol, pitch]
+  uint32_t pitch;
+  int32_t* numIndex;
+  uint32_t* fillState;
+};
+constexpr int kOffsetThreads = 1024;
+template <int THREADS>
+__device__ __forceinline__ void pairOffsets(int tap, const int32_t* __restrict__ numActIn, int64_t cap, int kVol, int shift,
+                                            const RbCount* __restrict__ cnt, uint32_t cntPitch, const PairOffsets& out) {
+  constexpr int WAVES = THREADS / 64;
+  __shared__ uint32_t segs[WAVES], sums[WAVES];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = liveCount(numActIn, cap);
+  const uint32_t live = static_cast<uint32_t>((static_cast<int64_t>(n) + (1ll << shift) - 1) >> shift);
+  uint32_t before = 0;   // segments of this wavefront's rows
+  for (int row = wave; row < tap; row += WAVES) {
+    uint32_t sum = 0;
+    for (uint32_t b = lane * 8; b < live; b += 512)
+      sum += countsBelow(*reinterpret_cast<const uint4*>(cnt + static_cast<size_t>(row) * cntPitch + b), b, live);
+    before += alignSegment(waveSum(sum));
+  }
+  if (lane == 0) segs[wave] = before;
+  __syncthreads();
+  uint32_t at = 0;
+  for (int q = 0; q < WAVES; ++q) at += segs[q];
+  const uint32_t start = at;
+  for (uint32_t base = 0; base < out.pitch; base += THREADS * 8) {
+    const uint32_t b = base + tid * 8;
+    uint4 c = make_uint4(0, 0, 0, 0);
+    if (b < live) c = *reinterpret_cast<const uint4*>(cnt + static_cast<size_t>(tap) * cntPitch + b);
+    const uint32_t mine = countsBelow(c, b, live);
+    const uint32_t incl = waveInclusiveScan(mine);
+    __syncthreads();
+    if (lane == 63) sums[wave] = incl;
+    __syncthreads();
+    uint32_t run = at + incl - mine, all = 0;
+    for (int q = 0; q < WAVES; ++q) {
+      if (q < wave) run += sums[q];
+      all += sums[q];
+    }
+    if (b < out.pitch) {
+      const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+      uint32_t o[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        o[j] = run;
+        if (b + j < live) run += (w[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
+      }
+      uint4* const to = reinterpret_cast<uint4*>(out.at + static_cast<size_t>(tap) * out.pitch + b);
+      to[0] = make_uint4(o[0], o[1], o[2], o[3]);
+      to[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    }
+    at += all;
+  }
+  if (tap == kVol - 1 && tid == 0) {
+    const uint32_t end = start + alignSegment(at - start);
+    *out.numIndex = static_cast<int32_t>(end);
+    if (out.fillState) out.fillState[1] = end;
+  }
+}
+
+__global__ void __launch_bounds__(kOffsetThreads)
+rbOffsets(const int32_t* __restrict__ numActIn, int64_t cap, int kVol, int shift, const RbCount* __restrict__ cnt, uint32_t cntPitch,
+          PairOffsets out) {
+  pairOffsets<kOffsetThreads>(blockIdx.x, numActIn, cap, kVol, shift, cnt, cntPitch, out);
+}
+
+// PACKED: staging holds the output rows of the pairs alone, those of each 64 inputs at the head of their 64 entries, and
+// `hits` which of the 64 they belong to (the strided fixed-shape probe, an eighth to a quarter of whose entries are pairs).
+// OFFSETS: the wavefront reads where its pairs go.
 // MIRROR: the table is that of a SubM rulebook with "same" padding (see below).  SKIP: the index tensor is left
 // unwritten (nothing reads it): what remains is numIndex and, where inputs were not in rank order, the ranks in
 // the mirrored table turned into rows.  SHIFT: log2 of the inputs per entry of cnt (8 or 9); a wavefront
 // compacts exactly one such block, 1 << (SHIFT - 6) consecutive inputs per lane, so its write position is the
 // workgroup's plus the counts of the workgroup's earlier blocks - after the one barrier behind the sums the
 // wavefronts run on their own, each as soon as its own staging entries have arrived.
-template <bool MIRROR, bool SKIP, int SHIFT>
-__global__ void __launch_bounds__(kCompactThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
+template <bool MIRROR, bool SKIP, int SHIFT, bool PACKED, bool OFFSETS>
+__global__ void __launch_bounds__(compactThreads(OFFSETS)) __attribute__((amdgpu_waves_per_eu(8, 8)))
 rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int kVol, const uint32_t* staging,
-          const RbCount* __restrict__ cnt, uint32_t cntPitch, int32_t* __restrict__ gather,
-          int32_t* __restrict__ scatter, int32_t* __restrict__ tapRow, int32_t* numIndex, int32_t* nbr, int64_t nbrRows,
+          const unsigned long long* __restrict__ hits, uint32_t hitsPitch,
+          const RbCount* __restrict__ cnt, uint32_t cntPitch, const uint32_t* __restrict__ offsets, uint32_t offsetPitch,
+          int32_t* __restrict__ gather, int32_t* __restrict__ scatter, int32_t* __restrict__ tapRow, int32_t* numIndex, int32_t* nbr, int64_t nbrRows,
           const uint32_t* __restrict__ perm, const uint32_t* __restrict__ permShuffled, int inPlace,
           unsigned long long* __restrict__ masks, uint32_t* fillState, int incrementalFill) {
   constexpr int ITEMS = 1 << (SHIFT - 6);           // consecutive inputs per lane
-  constexpr int RUN = kCompactThreads * ITEMS;      // inputs per workgroup
+  constexpr int WAVES = compactThreads(OFFSETS) / 64;   // blocks of cnt per workgroup
   extern __shared__ uint32_t tapTotal[];           // [kVol] pairs per tap (the taps this workgroup needs)
   __shared__ uint32_t partBefore;                   // pairs of this tap in the blocks before this workgroup's
   const int tap = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = liveCount(numActIn, cap);
-  const int64_t run0 = static_cast<int64_t>(blockIdx.x) * RUN;
-  const int64_t first = run0 + tid * ITEMS;
+  const uint32_t waveBlock = blockIdx.x * WAVES + wave;
+  const int64_t block0 = static_cast<int64_t>(waveBlock) << SHIFT;  // the wavefront's first input
+  const int64_t first = block0 + lane * ITEMS;
   const bool lastTap = tap == kVol - 1;
   const bool lastSpan = blockIdx.x == gridDim.x - 1;
   const bool shuffled = perm && *permShuffled;
@@ -672,12 +765,12 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
 
   // ---- pairs per tap (rows of cnt), pairs of this tap before this workgroup's blocks ----
   const uint32_t liveBlocks = static_cast<uint32_t>((static_cast<int64_t>(n) + (1 << SHIFT) - 1) >> SHIFT);
-  uint32_t firstBlock = blockIdx.x * kCompactWaves;
+  uint32_t firstBlock = blockIdx.x * WAVES;
   if (firstBlock > liveBlocks) firstBlock = liveBlocks;
   // pairs of this tap in the workgroup's blocks before this wavefront's: read now, summed behind the barrier
   uint32_t earlier = 0;
-  if (!SKIP && lane < wave && blockIdx.x * kCompactWaves + lane < liveBlocks)
-    earlier = cnt[static_cast<size_t>(tap) * cntPitch + blockIdx.x * kCompactWaves + lane];
+  if (!SKIP && !OFFSETS && lane < wave && blockIdx.x * WAVES + lane < liveBlocks)
+    earlier = cnt[static_cast<size_t>(tap) * cntPitch + blockIdx.x * WAVES + lane];
   // workgroups of the last tap also need that tap's total (the end of the used part of the tensor); the one
   // workgroup of a build that leaves the tensor unwritten needs every tap's
   const bool wantAll = SKIP || lastTap;
@@ -689,7 +782,7 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
     return row > lastRow ? 0u : ((row < tap || wantAll) ? liveBlocks : firstBlock);
   };
   auto loadRows = [&](int row0, uint32_t base, uint4 (&a)[3], uint4 (&b)[3]) {
-    const int row1 = row0 + kCompactWaves;
+    const int row1 = row0 + WAVES;
     const uint32_t limit0 = rowLimit(row0), limit1 = rowLimit(row1);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -702,7 +795,7 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
   };
   auto sumRows = [&](int row0, uint32_t base, const uint4 (&a)[3], const uint4 (&b)[3], uint32_t* full0,
                      uint32_t* full1, uint32_t* part) {
-    const int row1 = row0 + kCompactWaves;
+    const int row1 = row0 + WAVES;
     const uint32_t limit0 = rowLimit(row0), limit1 = rowLimit(row1);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -714,7 +807,7 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
     }
   };
   auto publishRows = [&](int row0, uint32_t full0, uint32_t full1, uint32_t part) {
-    const int row1 = row0 + kCompactWaves;
+    const int row1 = row0 + WAVES;
     full0 = waveSum(full0);
     full1 = waveSum(full1);
     if (row0 == tap || row1 == tap) part = waveSum(part);
@@ -724,97 +817,114 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
       if (row0 == tap || row1 == tap) partBefore = part;
     }
   };
+  // PACKED: lane j < ITEMS holds which of the wavefront's j-th 64 inputs have the tap
+  unsigned long long having = 0;
+  if (PACKED && lane < ITEMS && block0 < n)
+    having = hits[static_cast<size_t>(tap) * hitsPitch + (block0 >> 6) + lane];
   uint4 headA[3], headB[3];
-  loadRows(wave, 0, headA, headB);
+  uint32_t offset = 0;
+  if constexpr (OFFSETS) offset = offsets[static_cast<size_t>(tap) * offsetPitch + waveBlock];
+  else loadRows(wave, 0, headA, headB);
   // the staging entries: their latency (HBM) covers the sums below
-  uint4 s4[ITEMS / 4];
-#pragma unroll
-  for (int q = 0; q < ITEMS / 4; ++q) {
-    s4[q] = make_uint4(kNone, kNone, kNone, kNone);
-    if (!SKIP && first + 4 * q < n)
-      s4[q] = *(reinterpret_cast<const uint4*>(staging + static_cast<int64_t>(tap) * pitch + first) + q);
-  }
-  {
-    uint32_t full0 = 0, full1 = 0, part = 0;
-    sumRows(wave, 0, headA, headB, &full0, &full1, &part);
-    for (uint32_t base = 3 * 512; base < liveBlocks; base += 3 * 512) {  // more than 1536 blocks in a row
-      uint4 a[3], b[3];
-      loadRows(wave, base, a, b);
-      sumRows(wave, base, a, b, &full0, &full1, &part);
-    }
-    publishRows(wave, full0, full1, part);
-  }
-  for (int row0 = wave + 2 * kCompactWaves; row0 <= lastRow; row0 += 2 * kCompactWaves) {  // more than 32 taps
-    uint32_t full0 = 0, full1 = 0, part = 0;
-    for (uint32_t base = 0; base < liveBlocks; base += 3 * 512) {
-      uint4 a[3], b[3];
-      loadRows(row0, base, a, b);
-      sumRows(row0, base, a, b, &full0, &full1, &part);
-    }
-    publishRows(row0, full0, full1, part);
-  }
-  __syncthreads();
-  uint32_t segs = 0;  // segments of the earlier taps
-  for (int t = lane; t < tap; t += 64) segs += alignSegment(tapTotal[t]);
-  const uint32_t segStart = waveSum(segs);
-  uint32_t end = 0;   // end of the used part of the index tensor (workgroups that summed every row)
-  if (wantAll) {
-    uint32_t all = 0;
-    for (int t = lane; t < kVol; t += 64) all += alignSegment(tapTotal[t]);
-    end = waveSum(all);
-  }
-  if (SKIP) {
-    if (tid == 0) {
-      *numIndex = static_cast<int32_t>(end);
-      if (fillState) fillState[1] = end;
-    }
-    return;
-  }
-  const uint32_t at0 = segStart + partBefore + waveSum(earlier);  // where this wavefront's first pair goes
-
-  // ---- rank of this lane's pairs among the wavefront's ----
   uint32_t v[ITEMS];
+  if constexpr (!PACKED) {
 #pragma unroll
-  for (int q = 0; q < ITEMS / 4; ++q) {
-    v[4 * q] = s4[q].x;
-    v[4 * q + 1] = s4[q].y;
-    v[4 * q + 2] = s4[q].z;
-    v[4 * q + 3] = s4[q].w;
-  }
-  uint32_t mine = 0;
+    for (int q = 0; q < ITEMS / 4; ++q) {
+      uint4 s = make_uint4(kNone, kNone, kNone, kNone);
+      if (!SKIP && first + 4 * q < n)
+        s = *(reinterpret_cast<const uint4*>(staging + static_cast<int64_t>(tap) * pitch + first) + q);
+      v[4 * q] = s.x;
+      v[4 * q + 1] = s.y;
+      v[4 * q + 2] = s.z;
+      v[4 * q + 3] = s.w;
+    }
+  } else {
+    // every lane reads (one without a pair an entry of its 64's run that it drops): no branch between the loads
+    const uint32_t* const run = staging + static_cast<int64_t>(tap) * pitch + (block0 < n ? block0 : 0);
 #pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    if (first + j >= n) v[j] = kNone;
-    mine += (v[j] != kNone);
+    for (int j = 0; j < ITEMS; ++j) v[j] = run[j * 64 + lanesBelow(laneWord(having, j))];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (!((laneWord(having, j) >> lane) & 1ull)) v[j] = kNone;
   }
-  const uint32_t incl = waveInclusiveScan(mine);
-  uint32_t at = at0 + incl - mine;
+  uint32_t end = 0;   // end of the used part of the index tensor (workgroups that summed every row)
+  uint32_t at0 = offset;  // where this wavefront's first pair goes
+  if constexpr (!OFFSETS) {
+    {
+      uint32_t full0 = 0, full1 = 0, part = 0;
+      sumRows(wave, 0, headA, headB, &full0, &full1, &part);
+      for (uint32_t base = 3 * 512; base < liveBlocks; base += 3 * 512) {  // more than 1536 blocks in a row
+        uint4 a[3], b[3];
+        loadRows(wave, base, a, b);
+        sumRows(wave, base, a, b, &full0, &full1, &part);
+      }
+      publishRows(wave, full0, full1, part);
+    }
+    for (int row0 = wave + 2 * WAVES; row0 <= lastRow; row0 += 2 * WAVES) {  // more than 32 taps
+      uint32_t full0 = 0, full1 = 0, part = 0;
+      for (uint32_t base = 0; base < liveBlocks; base += 3 * 512) {
+        uint4 a[3], b[3];
+        loadRows(row0, base, a, b);
+        sumRows(row0, base, a, b, &full0, &full1, &part);
+      }
+      publishRows(row0, full0, full1, part);
+    }
+    __syncthreads();
+    uint32_t segs = 0;  // segments of the earlier taps
+    for (int t = lane; t < tap; t += 64) segs += alignSegment(tapTotal[t]);
+    const uint32_t segStart = waveSum(segs);
+    if (wantAll) {
+      uint32_t all = 0;
+      for (int t = lane; t < kVol; t += 64) all += alignSegment(tapTotal[t]);
+      end = waveSum(all);
+    }
+    if (SKIP) {
+      if (tid == 0) {
+        *numIndex = static_cast<int32_t>(end);
+        if (fillState) fillState[1] = end;
+      }
+      return;
+    }
+    at0 = segStart + partBefore + waveSum(earlier);
+  }
 
+  int32_t* nbrRow = (MIRROR && nbr) ? nbr + static_cast<int64_t>(kVol - 1 - tap) * nbrRows : nullptr;
+  static_assert(ITEMS <= 8, "64 KB of packed pairs");
+  __shared__ uint2 packed[WAVES][64 * ITEMS];
+  // ---- rank of this lane's pairs among the wavefront's ----
+  uint32_t mine = 0, slot = 0, pairs = 0;
+  if constexpr (!PACKED) {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (first + j >= n) v[j] = kNone;
+      mine += (v[j] != kNone);
+    }
+    const uint32_t incl = waveInclusiveScan(mine);
+    slot = incl - mine;
+    pairs = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+  }
+  if (shuffled) {  // block-map SubM: the probe stored ranks; rows are perm[rank]
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (v[j] != kNone) v[j] = perm[v[j]];
+  }
   // Mirror mode (SubM with "same" padding): the pair (tap, in i -> out o) has the twin (kVol-1-tap, in o -> out i),
   // so row i of the neighbour table under the mirrored tap is simply o - this thread's own staging entry.  The
   // table is then written here in whole coalesced rows, -1 included: no fill pass, no scatter.  With inPlace the
   // probe pass already used the table rows as its staging rows (staging + tap * pitch IS the row below): only
   // what the probe did not leave right is stored - entries of rows past the live count, and rows where ranks have
   // to become row numbers.
-  int32_t* nbrRow = (MIRROR && nbr) ? nbr + static_cast<int64_t>(kVol - 1 - tap) * nbrRows : nullptr;
-  auto mirrorStore = [&](const uint32_t (&o)[ITEMS]) {
-    if (!nbrRow) return;
+  if (nbrRow && (!inPlace || shuffled || first + ITEMS > n)) {
     if (first + ITEMS <= nbrRows && ((reinterpret_cast<uintptr_t>(nbrRow + first) & 15) == 0)) {
 #pragma unroll
       for (int q = 0; q < ITEMS / 4; ++q)
-        reinterpret_cast<uint4*>(nbrRow + first)[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
+        reinterpret_cast<uint4*>(nbrRow + first)[q] = make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
     } else {
 #pragma unroll
       for (int j = 0; j < ITEMS; ++j)
-        if (first + j < nbrRows) nbrRow[first + j] = static_cast<int32_t>(o[j]);
+        if (first + j < nbrRows) nbrRow[first + j] = static_cast<int32_t>(v[j]);
     }
-  };
-  if (shuffled) {  // block-map SubM: the probe stored ranks; rows are perm[rank]
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-      if (v[j] != kNone) v[j] = perm[v[j]];
   }
-  if (!inPlace || shuffled || first + ITEMS > n) mirrorStore(v);
   if (masks && MIRROR && kVol <= 64) {
     // tile masks of the convolution (bit t of masks[r / 64]: some output row of 64-row tile r / 64 has tap t).
     // Mirrored table: this thread's consecutive INPUT rows are output rows under tap kVol-1-tap; kTileLanes
@@ -824,47 +934,35 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
     if ((lane & (kTileLanes - 1)) == 0 && ((any >> lane) & ((1ull << kTileLanes) - 1ull)) && first < nbrRows)
       atomicOr(&masks[first >> 6], 1ull << (kVol - 1 - tap));
   }
-  if constexpr (ITEMS <= 8) {
-    // The wavefront's pairs are packed in LDS first (a lane's pairs start at its exclusive rank) and stored from
-    // there: lane l writes pairs l, l + 64, ... of the wavefront, so every store instruction covers 256
-    // consecutive bytes of a row instead of 64 runs of a few entries.  The buffer is the wavefront's own: LDS
-    // accesses of one wavefront are performed in order, no workgroup barrier is involved.
-    __shared__ uint2 packed[kCompactWaves][64 * ITEMS];
-    uint32_t slot = incl - mine;
+  // The block's pairs are packed in LDS first (a lane's pairs start at its exclusive rank) and stored from
+  // there: lane l writes pairs l, l + 64, ... of the block, so every store instruction covers 256
+  // consecutive bytes of a row instead of 64 runs of a few entries.  The buffer is the wavefront's own: LDS
+  // accesses of one wavefront are performed in order, no workgroup barrier is involved.
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (v[j] != kNone) {
-        packed[wave][slot++] = make_uint2(static_cast<uint32_t>(first + j), v[j]);
-        // the same pair in output-major form, for the convolution: nbr[tap][output row] = input row
-        if (nbr && !MIRROR && v[j] < static_cast<uint64_t>(nbrRows))
-          nbr[static_cast<int64_t>(tap) * nbrRows + v[j]] = static_cast<int32_t>(first + j);
-      }
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t input = static_cast<uint32_t>(PACKED ? block0 + j * 64 + lane : first + j);
+    if constexpr (PACKED) {
+      const unsigned long long set = laneWord(having, j);
+      slot = pairs + lanesBelow(set);
+      pairs += static_cast<uint32_t>(__popcll(set));
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const uint32_t pairs = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
-    for (uint32_t k = lane; k < pairs; k += 64) {
-      const uint2 e = packed[wave][k];
-      gather[at0 + k] = static_cast<int32_t>(e.x);
-      scatter[at0 + k] = static_cast<int32_t>(e.y);
-      tapRow[at0 + k] = tap;
-    }
-    (void)at;
-  } else {
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (v[j] != kNone) {
-        gather[at] = static_cast<int32_t>(first + j);
-        scatter[at] = static_cast<int32_t>(v[j]);
-        tapRow[at] = tap;
-        ++at;
-        if (nbr && !MIRROR && v[j] < static_cast<uint64_t>(nbrRows))
-          nbr[static_cast<int64_t>(tap) * nbrRows + v[j]] = static_cast<int32_t>(first + j);
-      }
-    }
+    if (v[j] == kNone) continue;
+    packed[wave][slot] = make_uint2(input, v[j]);
+    if constexpr (!PACKED) ++slot;
+    // the same pair in output-major form, for the convolution: nbr[tap][output row] = input row
+    if (nbr && !MIRROR && v[j] < static_cast<uint64_t>(nbrRows))
+      nbr[static_cast<int64_t>(tap) * nbrRows + v[j]] = static_cast<int32_t>(input);
   }
-  if (lastTap && lastSpan && tid == 0) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  for (uint32_t k = lane; k < pairs; k += 64) {
+    const uint2 e = packed[wave][k];
+    gather[at0 + k] = static_cast<int32_t>(e.x);
+    scatter[at0 + k] = static_cast<int32_t>(e.y);
+    tapRow[at0 + k] = tap;
+  }
+  if (!OFFSETS && lastTap && lastSpan && tid == 0) {
     *numIndex = static_cast<int32_t>(end);
     if (fillState) fillState[1] = end;  // what this pass uses of the index tensor: the next pass clears from here
   }
@@ -873,8 +971,8 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
   // segment up to 128 (the wavefront that holds the tap's last pairs), and behind the new end up to the old one
   // (the workgroups of the last tap, which know the new end; short unless the scene changed a lot).
   if (!incrementalFill) return;
-  if (lastSpan && wave == kCompactWaves - 1) {
-    const uint32_t pairsEnd = at0 + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+  if (lastSpan && wave == WAVES - 1) {
+    const uint32_t pairsEnd = at0 + pairs;
     const uint32_t segEnd = alignSegment(pairsEnd);
     for (uint32_t i = pairsEnd + lane; i < segEnd; i += 64) {
       gather[i] = -1;
@@ -884,7 +982,8 @@ rbCompact(const int32_t* __restrict__ numActIn, int64_t cap, int64_t pitch, int 
   }
   if (lastTap) {
     const uint32_t oldEnd = fillState[0];
-    const uint32_t gid = blockIdx.x * kCompactThreads + tid, nThreads = gridDim.x * kCompactThreads;
+    if (OFFSETS) end = fillState[1];
+    const uint32_t gid = blockIdx.x * blockDim.x + tid, nThreads = gridDim.x * blockDim.x;
     // segment ends are multiples of 128 entries: 16-byte stores when the three rows are 16-byte aligned
     if (((reinterpret_cast<uintptr_t>(gather) | reinterpret_cast<uintptr_t>(scatter) |
           reinterpret_cast<uintptr_t>(tapRow)) & 15) == 0) {
@@ -1892,15 +1991,28 @@ constexpr int kProbeThreads = 512;   // inputs per workgroup of the fixed-shape 
 constexpr int kProbeShift = 9;
 static_assert(1 << kProbeShift == kProbeThreads, "counts per workgroup");
 
-template <bool SUBM, int K1, int K2, int K3>
+// kProbeTable: the neighbour table of a strided build from the outputs' side.  Row o looks cells o * s - p + t up in the
+// finished map of the INPUT grid (the map of the strided build whose outputs the inputs are), which gives whole table rows
+// and tile masks, where pairs scattered from the inputs' side need the table filled with -1 first, write it a second
+// time in parts of lines and leave no masks.  The stage of 1.4 million inputs and 1.07 million outputs: fill and probe
+// 69, compaction with the scatter 81, convolution 176 us; now 49, 39 (with the work of rbOffsets beside it), 33 and 160.
+// Below kTableProbeRows outputs one more launch on the rulebooks' chain costs more than masks and fill give back (a pass
+// from 9 000 voxels, 20 000 to 30 000 outputs: 298 -> 305 us; 120 000 voxels: 260 000 outputs 663 -> 660, with the next
+// level's 50 000 too 665).
+constexpr int64_t kTableProbeRows = 1 << 17;
+enum ProbeMode { kProbeStrided = 0, kProbeSubM = 1, kProbeTable = 2 };
+template <int MODE, int K1, int K2, int K3>
 __global__ void __launch_bounds__(kProbeThreads)
 bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int32_t* __restrict__ numActIn, int64_t cap,
              int64_t pitch, RecRef recRef, const uint32_t* __restrict__ chunkBase,
              uint32_t* __restrict__ perm, uint32_t* permShuffled, int32_t maxNumActOut, uint32_t* __restrict__ staging,
-             RbCount* __restrict__ cnt, uint32_t cntPitch, int32_t* fillA, int64_t nFillA, int32_t* fillB,
+             unsigned long long* __restrict__ hitsOut, uint32_t hitsPitch, RbCount* __restrict__ cnt, uint32_t cntPitch,
+             int32_t* fillA, int64_t nFillA, int32_t* fillB,
              int64_t nFillB, uint32_t fillBlocks, uint32_t probeBlocks, int32_t* __restrict__ outCoors,
              uint32_t nRecords, unsigned long long* __restrict__ maskOut, int64_t nMasks, int fixTail,
-             int32_t* __restrict__ nbrDirect, int64_t nbrRows, uint32_t* fillState, int handOver) {
+             int32_t* __restrict__ nbrDirect, int64_t nbrRows, uint32_t* fillState, int handOver,
+             const int32_t* __restrict__ numActSrc, int64_t srcCap, PairOffsets offsets) {
+  constexpr bool SUBM = MODE != kProbeStrided;   // staging rows whole, in the order of the rows probed for
   const BmRecord* __restrict__ records = recRef.get();
   // Besides the staging entries the pass writes what a linked convolution reads: maskOut (SubM, staging rows =
   // rows of the mirrored table) takes the tile masks - a wavefront's 64 inputs are one 64-row tile - and fixTail
@@ -1911,6 +2023,10 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
   static_assert(KV <= 64, "one lane per tap keeps the wavefront's pair counts");
   __shared__ uint32_t ldsCnt[KV];
   if (blockIdx.x < fillBlocks) {
+    if constexpr (MODE == kProbeTable) {
+      pairOffsets<kProbeThreads>(blockIdx.x, numActSrc, srcCap, KV, kProbeShift, cnt, cntPitch, offsets);
+      return;
+    }
     const int64_t tid = static_cast<int64_t>(blockIdx.x) * kProbeThreads + threadIdx.x;
     const int64_t stride = static_cast<int64_t>(fillBlocks) * kProbeThreads;
     fillMinusOneRange(fillA, nFillA, tid, stride);
@@ -1962,6 +2078,10 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
   auto along = [&](int dim, int pos, int* cell) {
     const int st = g.s[dim];
     const int ls = st >> 1 > 1 ? 2 : st >> 1;
+    if constexpr (MODE == kProbeTable) {
+      *cell = c[dim + 1] * st + g.p[dim] - pos;
+      return *cell >= 0 && *cell < g.shape[dim + 1];
+    }
     const int num = c[dim + 1] + g.p[dim] - pos;
     *cell = num >> ls;
     return num >= 0 && (num & (st - 1)) == 0 && *cell < g.shape[dim + 1];
@@ -2017,8 +2137,10 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
     }
   }
   uint32_t mine = 0;  // lane t of a wavefront counts the wavefront's pairs of tap t
+  unsigned long long hitsOfTap = 0;  // strided: which of the wavefront's inputs have tap t (lane t)
   unsigned long long tileBits = 0;  // wavefront-uniform: (mirrored) taps that some input of the wavefront has
-  const uint32_t rankLimit = SUBM ? static_cast<uint32_t>(n) : static_cast<uint32_t>(maxNumActOut);
+  const uint32_t rankLimit = static_cast<uint32_t>(MODE == kProbeTable ? liveCount(numActSrc, srcCap)
+                                                                       : MODE == kProbeSubM ? n : maxNumActOut);
 #pragma unroll
   for (int q2 = 0; q2 < K2; ++q2) {
     const bool up = (o2[q2] >> 3) > base2;
@@ -2046,14 +2168,29 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
         const int tap = (q1 * K2 + q2) * K3 + q3;
         if (nbrDirect && row != kNone && row < static_cast<uint64_t>(nbrRows))
           nbrDirect[static_cast<int64_t>(tap) * nbrRows + row] = static_cast<int32_t>(i);
-        if (staging && inRange) staging[static_cast<int64_t>(tap) * pitch + i] = row;
-        const uint32_t hits = static_cast<uint32_t>(__popcll(__ballot(row != kNone)));
-        mine = lane == tap ? hits : mine;
-        if (hits) tileBits |= 1ull << (KV - 1 - tap);
+        const unsigned long long having = __ballot(row != kNone);
+        if constexpr (SUBM) {
+          if (staging && inRange) staging[static_cast<int64_t>(tap) * pitch + i] = row;
+          const uint32_t hits = static_cast<uint32_t>(__popcll(having));
+          mine = lane == tap ? hits : mine;
+          if (hits) tileBits |= 1ull << (KV - 1 - tap);
+        } else {
+          if (hitsOut) {
+            if (row != kNone) staging[static_cast<int64_t>(tap) * pitch + (i - lane) + lanesBelow(having)] = row;
+          } else if (staging && inRange) {
+            staging[static_cast<int64_t>(tap) * pitch + i] = row;
+          }
+          hitsOfTap = lane == tap ? having : hitsOfTap;
+        }
       }
     }
   }
   if (maskOut && lane == 0 && (i >> 6) < nMasks) maskOut[i >> 6] = tileBits;
+  if constexpr (!SUBM) {
+    mine = static_cast<uint32_t>(__popcll(hitsOfTap));
+    if (hitsOut && lane < KV) hitsOut[static_cast<size_t>(lane) * hitsPitch + (i >> 6)] = hitsOfTap;
+  }
+  if constexpr (MODE == kProbeTable) return;  // the pairs were counted from the inputs' side
   __syncthreads();  // ldsCnt zeroed
   if (mine) atomicAdd(&ldsCnt[lane], mine);
   __syncthreads();
@@ -2169,9 +2306,15 @@ RbWorkspace planWith(const RbGeom& g, int64_t cap, bool subM, bool blockMap) {
   }
   w.staging = off;
   off = alignUp(off + static_cast<size_t>(g.kVol) * w.pitch * 4);
+  w.hits = off;    // strided builds of the fixed-shape probe: u64 [kVol, hitsPitch], the inputs of 64 that have the tap
+  w.hitsPitch = static_cast<uint32_t>((cap + kProbeThreads - 1) / kProbeThreads * (kProbeThreads / 64));
+  if (blockMap && !subM) off = alignUp(off + static_cast<size_t>(g.kVol) * w.hitsPitch * 8);
   // pairs per (tap, block of inputs): rows of cntPitch words, one per 256 inputs (the fixed-shape probe) or per
   // 1024 (the others, which use the head of each row)
   w.cntPitch = static_cast<uint32_t>(((cap + kRbThreads - 1) / kRbThreads + 7) / 8 * 8);
+  w.offsets = off; // u32 [kVol, offsetPitch] where the pairs of a (tap, block) go
+  w.offsetPitch = static_cast<uint32_t>((cap + 8191) / 8192 * 16);
+  if (blockMap) off = alignUp(off + static_cast<size_t>(g.kVol) * w.offsetPitch * 4);
   w.cnt = off;     // RbCount [kVol, cntPitch], followed (the counters are cleared as one range) by
   off = alignUp(off + static_cast<size_t>(g.kVol) * w.cntPitch * sizeof(RbCount), 16);
   w.totals = off;  // [kVol, kTotalSlots] valid pairs per tap in partial sums, [kVol] owned outputs per tap, "rows not
@@ -2337,12 +2480,16 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     pitch = -nbrRows;
   }
   if (!mirror) masks = nullptr;
-  const int64_t nMasks = masks ? side.nMasks : 0;
+  int64_t nMasks = masks ? side.nMasks : 0;
   side.masksWritten = masks != nullptr;
   bool nbrFilled = mirror;
   bool skipIndex = false;                     // set below when side.skipIndex can be honoured
   bool directScatter = false;                 // the probe pass writes the scattered table itself
   bool needReset = true;                      // a reset pass opens the build
+  bool tableProbe = false;                    // the table is written by a probe of the source map (see below)
+  bool packed = false;                        // staging holds the pairs alone, packed per 64 inputs
+  auto* const hits = reinterpret_cast<unsigned long long*>(ws + w.hits);
+  const PairOffsets offsets{reinterpret_cast<uint32_t*>(ws + w.offsets), w.offsetPitch, numIndex, fillState};
   int cntShift = 8;                           // log2 of the inputs one entry of cnt covers
   unsigned long long* compactMasks = masks;   // null when the probe pass writes the masks itself
   const uint32_t* compactPerm = nullptr;      // block-map SubM: staging holds ranks, rows = perm[rank] when shuffled
@@ -2380,32 +2527,6 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       compactPermFlag = permShuffled;
     }
     const size_t nearLds = static_cast<size_t>(kNearGroup) * kRbThreads * sizeof(uint4) + static_cast<size_t>(g.kVol) * 4;
-    // A build whose index tensor nobody reads (side.skipIndex) writes table and masks in the probe pass and skips
-    // the compaction: for the kernel shapes of the plane probe, a SubM build with the mirrored table staged in
-    // place, or a strided build with a table to scatter into (which the scan pass - or the reset pass, where there is
-    // one - fills with -1, since the probe pass writes entries into it).
-    skipIndex = side.skipIndex && near && ksel != 0 && nbrOut && (subM ? (mirror && inPlace) : true);
-    // (with the index tensor written it does not pay: the fill, moved into the reset pass, is no longer hidden
-    // beside the probe - measured 1-2 us slower per strided build)
-    directScatter = skipIndex && !subM;
-    const bool probeMasks = subM && mirror && masks && near && ksel != 0;
-    if (probeMasks) compactMasks = nullptr;
-    side.indexWritten = !skipIndex;
-    // With two maps nothing is left to reset but that table, and the scan fills it: five launches of 5 us less in a pass of
-    // eight such builds (60 000 voxels to a dense map through an imported graph: 577 -> 571 us).
-    const bool scanFills = directScatter && twoMaps;
-    int32_t* const resetFill = directScatter ? (scanFills ? nullptr : nbrOut) : ((near || skipIndex) ? nullptr : fillIndex);
-    const int64_t resetFillN = directScatter ? static_cast<int64_t>(g.kVol) * nbrRows : nIndex;
-    const int64_t clearRecords = sharedMap ? 0 : static_cast<int64_t>(w.nRecords);
-    // A build on a shared map with the fixed-shape probe leaves nothing to zero: the probe writes counts and tile
-    // masks with plain stores, the compaction sums the counts itself, numIndex is written last.
-    needReset = !((sharedMap || twoMaps) && near && ksel != 0 && !resetFill && compactMasks == nullptr);
-    if (needReset)
-      hipLaunchKernelGGL(bmReset, fillGrid(clearRecords + (resetFill ? resetFillN / 4 : 0) + 1), block, 0,
-                         stream, reinterpret_cast<uint4*>(records), clearRecords,
-                         resetFill, resetFillN, reinterpret_cast<uint32_t*>(cnt),
-                         static_cast<int64_t>((w.totals - w.cnt) / 4 + totalsWords(g.kVol, w.nChunks)),
-                         numIndex, masks, nMasks, fillState);
     // A strided build on the outputs of another strided build, handed that build's finished map: the occupancy of
     // its own map is derived from it inside the scan (bmScan<.., GATHER>), the marking pass and its atomics go.
     int gather = 0;
@@ -2438,6 +2559,39 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
         ga.rcpZ = 1.0f / static_cast<float>(m.nb[1]);
       }
     }
+    // ... and its table comes from that map too, row by row of the output (tableProbe below).
+    tableProbe = gather == 1 && !side.skipIndex && nbrOut && nbrRows == maxNumActOut && nbrRows >= kTableProbeRows;
+    if (tableProbe && side.masks && g.kVol <= 64) {
+      masks = side.masks;
+      nMasks = side.nMasks;
+      side.masksWritten = true;
+    }
+    // A build whose index tensor nobody reads (side.skipIndex) writes table and masks in the probe pass and skips
+    // the compaction: for the kernel shapes of the plane probe, a SubM build with the mirrored table staged in
+    // place, or a strided build with a table to scatter into (which the scan pass - or the reset pass, where there is
+    // one - fills with -1, since the probe pass writes entries into it).
+    skipIndex = side.skipIndex && near && ksel != 0 && nbrOut && (subM ? (mirror && inPlace) : true);
+    // (with the index tensor written it does not pay: the fill, moved into the reset pass, is no longer hidden
+    // beside the probe - measured 1-2 us slower per strided build)
+    directScatter = skipIndex && !subM;
+    const bool probeMasks = subM && mirror && masks && near && ksel != 0;
+    if (probeMasks || tableProbe) compactMasks = nullptr;
+    side.indexWritten = !skipIndex;
+    // With two maps nothing is left to reset but that table, and the scan fills it: five launches of 5 us less in a pass of
+    // eight such builds (60 000 voxels to a dense map through an imported graph: 577 -> 571 us).
+    const bool scanFills = directScatter && twoMaps;
+    int32_t* const resetFill = directScatter ? (scanFills ? nullptr : nbrOut) : ((near || skipIndex) ? nullptr : fillIndex);
+    const int64_t resetFillN = directScatter ? static_cast<int64_t>(g.kVol) * nbrRows : nIndex;
+    const int64_t clearRecords = sharedMap ? 0 : static_cast<int64_t>(w.nRecords);
+    // A build on a shared map with the fixed-shape probe leaves nothing to zero: the probe writes counts and tile
+    // masks with plain stores, the compaction sums the counts itself, numIndex is written last.
+    needReset = !((sharedMap || twoMaps) && near && ksel != 0 && !resetFill && compactMasks == nullptr);
+    if (needReset)
+      hipLaunchKernelGGL(bmReset, fillGrid(clearRecords + (resetFill ? resetFillN / 4 : 0) + 1), block, 0,
+                         stream, reinterpret_cast<uint4*>(records), clearRecords,
+                         resetFill, resetFillN, reinterpret_cast<uint32_t*>(cnt),
+                         static_cast<int64_t>((w.totals - w.cnt) / 4 + totalsWords(g.kVol, w.nChunks)),
+                         numIndex, masks, nMasks, fillState);
     side.sourceMapUsed = gather != 0;
     if (sharedMap) {
       // the strided build that wrote these coordinates marked and scanned this very grid
@@ -2499,7 +2653,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       const uint32_t quads = probeBlocks;
       const uint32_t extra = sharedMap ? 0u : (subM ? probeBlocks : emitBlocks(w.nRecords, kRbThreads));
       const dim3 fused(quads * 2 + extra);
-      int32_t* fillB = (nbrOut && nbrRows > 0 && !mirror && !directScatter) ? nbrOut : nullptr;
+      int32_t* fillB = (nbrOut && nbrRows > 0 && !mirror && !directScatter && !tableProbe) ? nbrOut : nullptr;
       int32_t* const probeFillIndex = skipIndex ? nullptr : fillIndex;
       const int64_t nFillB = fillB ? static_cast<int64_t>(g.kVol) * nbrRows : 0;
       nbrFilled = true;
@@ -2507,6 +2661,9 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
   hipLaunchKernelGGL((bmProbeNear<SUBM, KSEL>), fused, block, nearLds, stream, g, m, coors, numActIn, cap, pitch,   \
                      recBehind, chunkBase, perm, permShuffled, maxNumActOut, staging, cnt, w.cntPitch, nullptr, fillIndex, \
                      nIndex, fillB, nFillB, quads, outCoors, w.nRecords)
+      // (where the compaction scatters into the table packing costs more than the staging rows it saves: 34 -> 44 us for
+      // 480 000 unsorted inputs)
+      packed = ksel != 0 && !subM && !skipIndex && !fillB;
       // fixed kernel shapes: K1 threads per input; fill workgroups only for what there is to fill
       const int64_t fillItems = (probeFillIndex ? nIndex : 0) + nFillB;
       uint32_t planeFill = static_cast<uint32_t>((fillItems / 4 + kRbThreads - 1) / kRbThreads);
@@ -2515,33 +2672,53 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       const uint32_t fixedBlocks = static_cast<uint32_t>((cap + kProbeThreads - 1) / kProbeThreads > 0 ? (cap + kProbeThreads - 1) / kProbeThreads : 1);
       const uint32_t fixedExtra = sharedMap ? 0u : (subM ? fixedBlocks : emitBlocks(w.nRecords, kProbeThreads));
       planeFill = (planeFill * kRbThreads + kProbeThreads - 1) / kProbeThreads;
-#define D3D_LAUNCH_PROBE_PLANE(SUBM, K1, K2, K3)                                                                    \
-  hipLaunchKernelGGL((bmProbeFixed<SUBM, K1, K2, K3>), dim3(planeFill + fixedBlocks + fixedExtra), dim3(kProbeThreads), 0, stream, \
+#define D3D_LAUNCH_PROBE_PLANE(MODE, K1, K2, K3)                                                                    \
+  hipLaunchKernelGGL((bmProbeFixed<MODE, K1, K2, K3>), dim3(planeFill + fixedBlocks + fixedExtra), dim3(kProbeThreads), 0, stream, \
                      g, m, coors, numActIn, cap, pitch, recBehind, chunkBase, perm, permShuffled, maxNumActOut,   \
-                     (directScatter && skipIndex) ? nullptr : staging, cnt, w.cntPitch, probeFillIndex,             \
+                     (directScatter && skipIndex) ? nullptr : staging, packed ? hits : nullptr, w.hitsPitch, cnt, w.cntPitch, probeFillIndex, \
                      nIndex, fillB, nFillB, planeFill,                                                               \
                      fixedBlocks, outCoors, w.nRecords, probeMasks ? masks : nullptr, nMasks,                        \
                      (subM && inPlace) ? 1 : 0, directScatter ? nbrOut : nullptr, nbrRows, fillState,               \
-                     needReset ? 0 : 1)
+                     needReset ? 0 : 1, nullptr, 0, PairOffsets{})
       cntShift = ksel != 0 ? kProbeShift : 8;  // the one-thread-per-input probes count per workgroup
       if (subM) {
         switch (ksel) {
-          case 1: D3D_LAUNCH_PROBE_PLANE(true, 3, 3, 3); break;
-          case 2: D3D_LAUNCH_PROBE_PLANE(true, 3, 1, 1); break;
-          case 3: D3D_LAUNCH_PROBE_PLANE(true, 3, 1, 3); break;
-          case 4: D3D_LAUNCH_PROBE_PLANE(true, 1, 3, 3); break;
+          case 1: D3D_LAUNCH_PROBE_PLANE(kProbeSubM, 3, 3, 3); break;
+          case 2: D3D_LAUNCH_PROBE_PLANE(kProbeSubM, 3, 1, 1); break;
+          case 3: D3D_LAUNCH_PROBE_PLANE(kProbeSubM, 3, 1, 3); break;
+          case 4: D3D_LAUNCH_PROBE_PLANE(kProbeSubM, 1, 3, 3); break;
           default: D3D_LAUNCH_PROBE_NEAR(true, 0);
         }
       } else {
         switch (ksel) {
-          case 1: D3D_LAUNCH_PROBE_PLANE(false, 3, 3, 3); break;
-          case 2: D3D_LAUNCH_PROBE_PLANE(false, 3, 1, 1); break;
-          case 3: D3D_LAUNCH_PROBE_PLANE(false, 3, 1, 3); break;
-          case 4: D3D_LAUNCH_PROBE_PLANE(false, 1, 3, 3); break;
+          case 1: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 3, 3); break;
+          case 2: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 1, 1); break;
+          case 3: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 1, 3); break;
+          case 4: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 1, 3, 3); break;
           default: D3D_LAUNCH_PROBE_NEAR(false, 0);
         }
       }
 #undef D3D_LAUNCH_PROBE_PLANE
+      if (tableProbe) {
+        // the outputs look their inputs up: output cell o has input cell o * s - p + t under tap t
+        RbGeom gt = g;
+        for (int dim = 0; dim <= kMaxSpatial; ++dim) {
+          gt.shape[dim] = g.inShape[dim];
+          gt.inShape[dim] = g.shape[dim];
+        }
+        for (int dim = 0; dim < kMaxSpatial; ++dim) gt.p[dim] = g.k[dim] - 1 - g.p[dim];
+        const uint32_t offsetBlocks = static_cast<uint32_t>(g.kVol);
+        const uint32_t tableBlocks = static_cast<uint32_t>((nbrRows + kProbeThreads - 1) / kProbeThreads);
+#define D3D_LAUNCH_PROBE_TABLE(K1, K2, K3)                                                                           \
+  hipLaunchKernelGGL((bmProbeFixed<kProbeTable, K1, K2, K3>), dim3(offsetBlocks + tableBlocks), dim3(kProbeThreads), 0, stream, gt, ga.mi, \
+                     static_cast<const int32_t*>(outCoors), static_cast<const int32_t*>(numActOut), nbrRows, -nbrRows, ga.src, \
+                     ga.srcChunkBase, nullptr, nullptr, 0,                                                           \
+                     reinterpret_cast<uint32_t*>(nbrOut) + static_cast<int64_t>(g.kVol - 1) * nbrRows, nullptr, 0u,  \
+                     cnt, w.cntPitch, nullptr, 0, nullptr, 0, offsetBlocks, tableBlocks, nullptr, 0u,                \
+                     masks, nMasks, 1, nullptr, 0, nullptr, 0, numActIn, cap, offsets)
+        D3D_LAUNCH_PROBE_TABLE(3, 3, 3);
+#undef D3D_LAUNCH_PROBE_TABLE
+      }
 #undef D3D_LAUNCH_PROBE_NEAR
     } else if (subM) {
       hipLaunchKernelGGL(bmProbe<true>, perTap, block, 0, stream, g, m, coors, numActIn, cap, pitch, recBehind, chunkBase, perm,
@@ -2579,27 +2756,38 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
                        static_cast<int64_t>(g.kVol) * nbrRows);
   // with the index tensor unwritten only a build that may have to turn ranks into rows needs the whole grid; the
   // others launch the one workgroup that writes numIndex
-  const int64_t compactRun = static_cast<int64_t>(kCompactWaves) << cntShift;  // a wavefront per block of counts
+  const bool withOffsets = !skipIndex && cntShift == kProbeShift && (tableProbe || cap >= kOffsetRows);
+  const int64_t compactRun = static_cast<int64_t>(compactThreads(withOffsets) / 64) << cntShift;  // a wavefront per block of counts
   const dim3 allSpans(static_cast<unsigned>((cap + compactRun - 1) / compactRun > 0 ? (cap + compactRun - 1) / compactRun : 1),
                       g.kVol);
   const dim3 compactGrid = (skipIndex && !compactPerm) ? dim3(1, 1) : allSpans;
-#define D3D_LAUNCH_COMPACT(MIRROR, SKIP, SHIFT)                                                                       \
-  hipLaunchKernelGGL((rbCompact<MIRROR, SKIP, SHIFT>), compactGrid, dim3(kCompactThreads),                            \
-                     static_cast<size_t>(g.kVol) * 4, stream, numActIn, cap, pitch, g.kVol, staging, cnt, w.cntPitch,  \
-                     index, index + rowLen, index + 2 * rowLen, numIndex,                                             \
-                     (nbrRows > 0 && !directScatter) ? nbrOut : nullptr, nbrRows, compactPerm, compactPermFlag,        \
+  if (withOffsets && !tableProbe)  // (a table probe brings them)
+    hipLaunchKernelGGL(rbOffsets, dim3(g.kVol), dim3(kOffsetThreads), 0, stream, numActIn, cap, g.kVol, kProbeShift, cnt,
+                       w.cntPitch, offsets);
+#define D3D_LAUNCH_COMPACT(MIRROR, SKIP, SHIFT, PACKED, OFFSETS)                                                       \
+  hipLaunchKernelGGL((rbCompact<MIRROR, SKIP, SHIFT, PACKED, OFFSETS>), compactGrid, dim3(compactThreads(OFFSETS)),    \
+                     static_cast<size_t>(g.kVol) * 4, stream, numActIn, cap, pitch, g.kVol, staging, hits,  \
+                     w.hitsPitch, cnt, w.cntPitch, offsets.at, offsets.pitch, index, index + rowLen, index + 2 * rowLen, numIndex, \
+                     (nbrRows > 0 && !directScatter && !tableProbe) ? nbrOut : nullptr, nbrRows, compactPerm, compactPermFlag, \
                      inPlace ? 1 : 0, compactMasks, fillState, incremental ? 1 : 0)
-#define D3D_LAUNCH_COMPACT_SHIFT(MIRROR, SKIP)                        \
-  do {                                                                \
-    if (cntShift == 8) D3D_LAUNCH_COMPACT(MIRROR, SKIP, 8);           \
-    else D3D_LAUNCH_COMPACT(MIRROR, SKIP, 9);                         \
+#define D3D_LAUNCH_COMPACT_FORM(SHIFT, OFFSETS)                                                  \
+  do {                                                                                           \
+    if (mirror) D3D_LAUNCH_COMPACT(true, false, SHIFT, false, OFFSETS);                          \
+    else if (packed) D3D_LAUNCH_COMPACT(false, false, SHIFT, true, OFFSETS);                     \
+    else D3D_LAUNCH_COMPACT(false, false, SHIFT, false, OFFSETS);                                \
   } while (0)
-  if (skipIndex) {
-    if (mirror) D3D_LAUNCH_COMPACT_SHIFT(true, true); else D3D_LAUNCH_COMPACT_SHIFT(false, true);
+  if (skipIndex) {  // (the fixed-shape probe's counts)
+    if (mirror) D3D_LAUNCH_COMPACT(true, true, kProbeShift, false, false);
+    else D3D_LAUNCH_COMPACT(false, true, kProbeShift, false, false);
+  } else if (cntShift != kProbeShift) {
+    if (mirror) D3D_LAUNCH_COMPACT(true, false, 8, false, false);
+    else D3D_LAUNCH_COMPACT(false, false, 8, false, false);
+  } else if (withOffsets) {
+    D3D_LAUNCH_COMPACT_FORM(kProbeShift, true);
   } else {
-    if (mirror) D3D_LAUNCH_COMPACT_SHIFT(true, false); else D3D_LAUNCH_COMPACT_SHIFT(false, false);
+    D3D_LAUNCH_COMPACT_FORM(kProbeShift, false);
   }
-#undef D3D_LAUNCH_COMPACT_SHIFT
+#undef D3D_LAUNCH_COMPACT_FORM
 #undef D3D_LAUNCH_COMPACT
   D3D_HIP_CHECK(hipGetLastError());
   return D3D_OK;

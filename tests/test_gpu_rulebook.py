@@ -263,6 +263,48 @@ def test_strided_operator_on_a_strided_operators_map(engine, second):
         consumer.link_coords(None)
 
 
+@pytest.mark.parametrize("max1,max2", [(32000, 1 << 17), (900, 1 << 17), (1 << 19, 1 << 17), (1 << 19, 30000)])
+def test_large_strided_operator_on_a_strided_operators_map(engine, max1, max2):
+    """At capacities from 131072 outputs the table of a linked 3x3x3 stride-2 operator is looked up in the producer's map
+    (with its tile masks), and from 524288 inputs the places of the pairs are worked out before the compaction: the
+    convolution on that table gives the bits of one that derives its table from the index tensor of the unlinked
+    operator, and both operators write the same index tensor.  A producer that truncates (its map holds cells without a
+    row), live counts that end inside a tile and at 0, changing clouds; a submanifold operator of the same capacity."""
+    import torch
+    from deploy3d_amd import spconv_index_nd, spconv_mm
+    from deploy3d_amd.spconv_index import index_plugin
+    grid, batch = (13, 45, 38), 2
+    rng = np.random.default_rng(31)
+    geometry = ((3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1), (0, 0, 0))
+    near = ((3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1), (0, 0, 0))
+    shape = torch.empty((batch, 0) + grid, dtype=torch.int32, device="cuda")
+    producer = index_plugin(*geometry, max1, False, False)
+    consumer, subm = index_plugin(*geometry, max2, False, False), index_plugin(*near, max1, True, False)
+    weight = rng.standard_normal(27 * 32 * 64).astype(np.float32) * 0.1
+    feats = torch.from_numpy(rng.standard_normal((max1, 32)).astype(np.float32)).cuda().half()
+    for m in (4000, 4000, 777, 0, 2500):
+        coords = random_cloud(rng, 4000, grid, batch)[:m]
+        c = torch.zeros((4000, 4), dtype=torch.int32, device="cuda")
+        c[:len(coords)] = torch.from_numpy(coords).cuda()
+        num = torch.tensor([len(coords)], dtype=torch.int32, device="cuda")
+        got = []
+        for linked in (True, False):
+            consumer.link_coords(producer if linked else None)
+            subm.link_coords(producer if linked else None)
+            _, _, oc, no, osh = spconv_index_nd(c, num, shape, *geometry, max1, False, False)
+            si, sn = spconv_index_nd(oc, no, osh, *near, max1, True, False)
+            index, num_index, oc2, no2, _ = spconv_index_nd(oc, no, osh, *geometry, max2, False, False)
+            out = spconv_mm(feats, no, no2, index, num_index, (3, 3, 3), 32, 64, max2, False, False, weight,
+                            rulebook=consumer if linked else None)
+            sout = spconv_mm(feats, no, no, si, sn, (3, 3, 3), 32, 64, max1, True, False, weight, rulebook=subm if linked else None)
+            live, live1 = min(int(no2.item()), max2), min(int(no.item()), max1)
+            got.append([index, num_index, oc2[:live], no2, out[:live], si, sn, sout[:live1]])
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
+    consumer.link_coords(None)
+    subm.link_coords(None)
+
+
 def test_ordered_scan_variant(engine, monkeypatch):
     """D3D_RULEBOOK_ORDERED_SCAN=1 selects acquire-release tickets in the scan pass of the block map: same results."""
     monkeypatch.setenv("D3D_RULEBOOK_ORDERED_SCAN", "1")
