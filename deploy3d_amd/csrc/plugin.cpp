@@ -193,6 +193,7 @@ struct RulebookLink {
   // an operator that keeps its map between passes holds two of them (mapStride records apart) and the state
   // words of RbSide::mapState: its builds then need no reset pass
   DeviceBuffer mapState;
+  DeviceBuffer mapList;           // SubM: RbSide::mapList
   int64_t mapStride = 0;
   bool mapDouble = false;         // the last build alternated between the two maps
   bool mapDirty = false;          // a build with a reset pass has used the first map since the allocation: the
@@ -462,15 +463,16 @@ struct IdxPlugin final : d3d_plugin {
     blockMapBytes(g, cap, &recBytes, &chunkBytes);
     if (!recBytes) return false;
     const size_t stateBytes = mapStateWords(chunkBytes) * 4;
+    const size_t listBytes = subM ? 2 * sizeof(uint32_t) * static_cast<size_t>(cap > 0 ? cap : 1) : 0;
     auto have = [&]() {
-      return link->mapRecords.bytes >= 2 * recBytes && link->mapChunkBase.bytes >= chunkBytes &&
+      return link->mapList.bytes >= listBytes && link->mapRecords.bytes >= 2 * recBytes && link->mapChunkBase.bytes >= chunkBytes &&
              link->mapState.bytes >= stateBytes && link->mapStride * 16 == static_cast<int64_t>(recBytes);
     };
     if (!have() && mayAllocate) {
       ++link->changes;
       link->mapStride = 0;
       if (link->mapRecords.reallocZeroed(2 * recBytes) == D3D_OK && link->mapChunkBase.reserve(chunkBytes) == D3D_OK &&
-          link->mapState.reallocZeroed(stateBytes) == D3D_OK) {
+          link->mapState.reallocZeroed(stateBytes) == D3D_OK && link->mapList.reserve(listBytes) == D3D_OK) {
         link->mapStride = static_cast<int64_t>(recBytes / 16);
         link->mapDirty = false;
       }
@@ -594,6 +596,8 @@ struct IdxPlugin final : d3d_plugin {
         side.mapChunkBase = static_cast<uint32_t*>(link->mapChunkBase.ptr);
         side.mapState = static_cast<uint32_t*>(link->mapState.ptr);
         side.mapStride = link->mapStride;
+        side.mapList = static_cast<uint32_t*>(link->mapList.ptr);
+        side.mapListRows = static_cast<int64_t>(link->mapList.bytes / (2 * sizeof(uint32_t)));
         side.mapDirty = link->mapDirty;
       }
     }

@@ -381,6 +381,43 @@ def test_persistent_index_tensor(engine):
         plugin.close()
 
 
+@pytest.mark.parametrize("counts", [(2047, 2048, 2049, 1), (6145, 0, 4096, 4097)])
+def test_listed_map_across_passes(engine, counts):
+    """A submanifold operator that keeps its maps numbers and clears the records its marking pass listed, 2048 inputs to a
+    workgroup: counts around that, rows outside the grid among them, another cloud on every pass (what one pass leaves in
+    either map would be found by the next but one); every pass equals the oracle, the table's convolution included."""
+    import torch
+    from deploy3d_amd import spconv_mm
+    from deploy3d_amd.plugin import OPT_PERSISTENT_INDEX, Plugin, TensorDesc
+    from deploy3d_amd.spconv_index import index_blob
+    grid, cap = (12, 100, 90), 6200
+    rng = np.random.default_rng(5)
+    args = ((3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1))
+    plugin = Plugin("SPConvIdx3d", index_blob(*args, (0, 0, 0), cap, True, False))
+    plugin.set_option(OPT_PERSISTENT_INDEX, 1)
+    weight = rng.standard_normal(27 * 16 * 16).astype(np.float32) * 0.1
+    feats = torch.from_numpy(rng.standard_normal((cap, 16)).astype(np.float32)).cuda()
+    coors = torch.zeros((cap, 4), dtype=torch.int32, device="cuda")
+    num = torch.zeros(1, dtype=torch.int32, device="cuda")
+    in_descs = [TensorDesc.of_tensor(coors), TensorDesc.of_tensor(num), TensorDesc.of((1, 0) + grid, torch.int32)]
+    out_descs = plugin.output_descs(in_descs)
+    outs = [torch.empty(d.shape(), dtype=torch.int32, device="cuda") for d in out_descs]
+    ws = torch.empty(max(1, plugin.workspace_size(in_descs, out_descs)), dtype=torch.uint8, device="cuda")
+    for n in counts + counts:
+        coords = random_cloud(rng, n, grid, 1) if n else np.zeros((0, 4), np.int32)
+        coords[::97, 1] = grid[0] + 3    # outside: no pair, no record
+        coors[:n] = torch.from_numpy(coords).cuda()
+        num.fill_(n)
+        plugin.enqueue(in_descs, out_descs, [coors, num, None], outs, ws)
+        got = spconv_mm(feats, num, num, outs[0], outs[1], (3, 3, 3), 16, 16, cap, True, False, weight, rulebook=plugin)
+        want = spconv_mm(feats, num, num, outs[0], outs[1], (3, 3, 3), 16, 16, cap, True, False, weight)
+        ref = oracle.rulebook(coors.cpu().numpy(), n, (1,) + grid, *args, cap, True)
+        assert int(outs[1].item()) == ref["num_index"]
+        np.testing.assert_array_equal(outs[0].cpu().numpy(), ref["index"])
+        assert torch.equal(got[:n], want[:n])
+    plugin.close()
+
+
 def test_configured_operator_captures_without_an_eager_pass(engine):
     """An operator that keeps its occupancy map between passes (persistent index tensor) reserves its two maps at
     configure: captured in a graph without ever having been enqueued eagerly, every replay - the maps take turns
