@@ -35,6 +35,9 @@
 #include "common.h"
 
 namespace d3d {
+// `value` (wavefront-uniform) in lane `lane`, `rest` in the others; the compiler has no builtin for it
+extern "C" __device__ int writeLane(int value, int lane, int rest) __asm("llvm.amdgcn.writelane.i32");
+
 namespace {
 
 constexpr unsigned long long kEmptySlot = ~0ull;
@@ -1088,7 +1091,7 @@ __device__ __forceinline__ bool tapTargetCoord(const RbGeom& g, const int c[5], 
 // rank = occupied cells in earlier chunks of records + in earlier records of the chunk + below the bit
 __device__ __forceinline__ uint32_t bmRank(const BlockMap& m, const BmRecord& r, uint32_t bit,
                                            const uint32_t* __restrict__ chunkBase, uint32_t rec) {
-  return chunkBase[rec >> m.chunkShift] + r.prefix + static_cast<uint32_t>(__popcll(r.bits & ((1ull << bit) - 1ull)));
+  return (chunkBase ? chunkBase[rec >> m.chunkShift] : 0u) + r.prefix + static_cast<uint32_t>(__popcll(r.bits & ((1ull << bit) - 1ull)));
 }
 
 // reset for the block-map path: records = 0, index tensor = -1, counters = 0
@@ -1198,8 +1201,7 @@ bmMarkInputs(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
 // 120 000 on 1.3 million 21 -> 10).  The atomics go to one address, 18 ns each: hence few, large workgroups.
 constexpr int kListThreads = 1024, kListItems = 2, kListRun = kListThreads * kListItems;
 __global__ void __launch_bounds__(kListThreads)
-bmScanList(RecRef recRef, RecList list, const int32_t* __restrict__ numActIn, int64_t cap, uint32_t* __restrict__ chunkBase,
-           uint32_t nChunks) {
+bmScanList(RecRef recRef, RecList list, const int32_t* __restrict__ numActIn, int64_t cap) {
   __shared__ uint32_t sums[kListThreads / 64];
   __shared__ unsigned long long drawn;
   const uint32_t epoch = *recRef.epoch, cur = epoch & 1u;
@@ -1208,8 +1210,6 @@ bmScanList(RecRef recRef, RecList list, const int32_t* __restrict__ numActIn, in
   const uint32_t n = static_cast<uint32_t>(liveCount(numActIn, cap)), before = list.state[4 + (cur ^ 1u)];
   const uint32_t row0 = blockIdx.x * kListRun + threadIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // prefixes are absolute here
-  for (uint32_t q = blockIdx.x * kListThreads + threadIdx.x; q < nChunks; q += gridDim.x * kListThreads) chunkBase[q] = 0u;
   uint32_t rec[kListItems], old[kListItems], count[kListItems];
 #pragma unroll
   for (int j = 0; j < kListItems; ++j) {
@@ -1274,14 +1274,6 @@ bmMarkCandidates(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const 
     const unsigned long long mask = 1ull << bit;
     if ((__builtin_nontemporal_load(&records[rec].bits) & mask) == 0) atomicOr(&records[rec].bits, mask);
   }
-}
-
-// c ? a : b on values: the operands are made opaque first, so that a choice between two elements of a local array
-// stays a register select instead of becoming a dynamically indexed (memory-resident) array.
-__device__ __forceinline__ uint32_t pick(bool c, uint32_t a, uint32_t b) {
-  asm("" : "+v"(a));
-  asm("" : "+v"(b));
-  return c ? a : b;
 }
 
 constexpr uint32_t kScanGroup = 32;  // workgroups of the scan pass that share one first-level ticket
@@ -2065,6 +2057,10 @@ bmProbeNear(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int32
 // Bound by vector instructions where inputs lie in brick order and by the fetched lines where they do not.  So what the
 // taps of a row share (its sixteen cells, the ranks in front of it) is made once per row and a tap is one population
 // count of cells, and bricks no tap reaches are not fetched: 349 000 inputs 21.5 -> 18.5 us, 1.35 million 72 -> 60 us.
+// And a tap is nine vector instructions: its store goes into a buffer that ends with the rows to be written (no branch,
+// no 64-bit address per lane), the ballot reads the row's own compare, the count goes into its lane as a scalar, the 16
+// cells of a brick row are two byte permutes, choices are masks: 18.5 -> 13.5 and 60 -> 50 us, now 3.3 TB/s of rows
+// written.  (Eight wavefronts per SIMD instead of seven spill: 62 us.)
 // Workgroup roles by block index: first the fill workgroups (-1 over the neighbour table, bandwidth-bound work
 // beside latency-bound work), then the probing workgroups, then the pass only the compaction waits for
 // (rank -> row permutation, or the output coordinates).
@@ -2081,7 +2077,16 @@ static_assert(1 << kProbeShift == kProbeThreads, "counts per workgroup");
 // from 9 000 voxels, 20 000 to 30 000 outputs: 298 -> 305 us; 120 000 voxels: 260 000 outputs 663 -> 660, with the next
 // level's 50 000 too 665).
 constexpr int64_t kTableProbeRows = 1 << 17;
-enum ProbeMode { kProbeStrided = 0, kProbeSubM = 1, kProbeTable = 2 };
+// kProbeStrided stages a row per (tap, input), kProbePacked the pairs alone (see rbCompact), kProbeDirect writes them into
+// the neighbour table at once; kProbeSubM and kProbeTable write whole rows.
+enum ProbeMode { kProbeStrided, kProbePacked, kProbeDirect, kProbeSubM, kProbeTable };
+// A buffer over `bytes` bytes from p; accesses past its end are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rowBuffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
+}
+// a where the mask's bits are set, else b: one v_bfi, and no choice between array elements for the compiler to index
+__device__ __forceinline__ uint32_t pick(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
+constexpr int64_t kMaxFixedRows = 1 << 29;   // rows of 32-bit offsets
 template <int MODE, int K1, int K2, int K3>
 __global__ void __launch_bounds__(kProbeThreads)
 bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int32_t* __restrict__ numActIn, int64_t cap,
@@ -2093,13 +2098,13 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
              uint32_t nRecords, unsigned long long* __restrict__ maskOut, int64_t nMasks, int fixTail,
              int32_t* __restrict__ nbrDirect, int64_t nbrRows, uint32_t* fillState, int handOver,
              const int32_t* __restrict__ numActSrc, int64_t srcCap, PairOffsets offsets) {
-  constexpr bool SUBM = MODE != kProbeStrided;   // staging rows whole, in the order of the rows probed for
+  constexpr bool ROWS = MODE == kProbeSubM || MODE == kProbeTable;
   const BmRecord* __restrict__ records = recRef.get();
   // Besides the staging entries the pass writes what a linked convolution reads: maskOut (SubM, staging rows =
   // rows of the mirrored table) takes the tile masks - a wavefront's 64 inputs are one 64-row tile - and fixTail
-  // has the rows between the live count and the capacity set to -1; nbrDirect (strided, index tensor unread)
-  // takes the pairs straight into the scattered table nbrDirect[tap][output row] = input row, filled with -1 by
-  // the reset pass; staging may then be null.
+  // has the rows between the live count and the capacity set to -1; nbrDirect (kProbeDirect: strided, index tensor
+  // unread) takes the pairs straight into the scattered table nbrDirect[tap][output row] = input row, filled with -1
+  // by the scan or the reset pass.
   constexpr int KP = K2 * K3, KV = K1 * KP;
   static_assert(KV <= 64, "one lane per tap keeps the wavefront's pair counts");
   __shared__ uint32_t ldsCnt[KV];
@@ -2117,7 +2122,7 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
   const uint32_t probeBlock = blockIdx.x - fillBlocks;
   if (probeBlock >= probeBlocks) {
     const uint32_t e = probeBlock - probeBlocks;
-    if (SUBM) {
+    if (ROWS) {
       permuteRow(g, m, coors, liveCount(numActIn, cap), static_cast<int64_t>(e) * kProbeThreads + threadIdx.x, records,
                  chunkBase, perm, permShuffled);
     } else {
@@ -2145,135 +2150,149 @@ bmProbeFixed(RbGeom g, BlockMap m, const int32_t* __restrict__ coors, const int3
     return;
   }
   if (threadIdx.x < KV) ldsCnt[threadIdx.x] = 0;
-  // rows below the live count get a staging entry, in the grid or not (fixTail: every row below the capacity)
-  const bool inRange = i < n || (fixTail && i < cap);
   bool live = i < n;
   int c[5] = {0, 0, 0, 0, 0};   // (b, z, y, x) in c[0], c[2..4]; c[1] is the degenerate dim
-  if (live && !loadInput(g, coors, i, c)) {
-    live = false;
-    c[0] = c[1] = c[2] = c[3] = c[4] = 0;
+  if (live) {
+    loadCoord(coors, 3, i, c);
+    live = inputInGrid(g, c);
   }
-  live = live && c[0] >= 0 && c[0] < g.shape[0] && c[1] == 0;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) c[q] = live ? c[q] : 0;
+  live = live & (static_cast<uint32_t>(c[0]) < static_cast<uint32_t>(g.shape[0]));
   // Bricks of a 3-D map are one level of 8 x 8 cells (a byte of the occupancy bits per row).  Per dim and kernel
   // position: validity and output cell; a position whose cell is invalid may point anywhere inside the group.
-  auto along = [&](int dim, int pos, int* cell) {
+  auto along = [&](int dim, int pos, int* cell) __attribute__((always_inline)) -> bool {
     const int st = g.s[dim];
-    const int ls = st >> 1 > 1 ? 2 : st >> 1;
     if constexpr (MODE == kProbeTable) {
       *cell = c[dim + 1] * st + g.p[dim] - pos;
-      return *cell >= 0 && *cell < g.shape[dim + 1];
+      return static_cast<uint32_t>(*cell) < static_cast<uint32_t>(g.shape[dim + 1]);
     }
+    const int ls = st >> 1 > 1 ? 2 : st >> 1;
     const int num = c[dim + 1] + g.p[dim] - pos;
-    *cell = num >> ls;
-    return num >= 0 && (num & (st - 1)) == 0 && *cell < g.shape[dim + 1];
+    *cell = num >> ls;   // (negative: no cell either)
+    return (static_cast<uint32_t>(*cell) < static_cast<uint32_t>(g.shape[dim + 1])) & ((num & (st - 1)) == 0);
   };
-  bool ok1[K1], ok2[K2];
+  bool ok1[K1];
+  uint32_t ok2[K2];
   int o1[K1], o2[K2];
 #pragma unroll
-  for (int q = 0; q < K1; ++q) ok1[q] = along(1, q, &o1[q]) && live;
+  for (int q = 0; q < K1; ++q) ok1[q] = along(1, q, &o1[q]) & live;
 #pragma unroll
-  for (int q = 0; q < K2; ++q) ok2[q] = along(2, q, &o2[q]);
+  for (int q = 0; q < K2; ++q) ok2[q] = along(2, q, &o2[q]) ? ~0u : 0u;
   // lower brick of the 2x2 group per dim: that of the highest kernel position (the lowest cell), clamped to 0
   int low3;
   along(3, K3 - 1, &low3);
   const int base2 = o2[K2 - 1] > 0 ? o2[K2 - 1] >> 3 : 0, base3 = low3 > 0 ? low3 >> 3 : 0;
   // Innermost dim: a row of the group's two bricks is 16 cells; `at` the cell of a position (0 if invalid), `below` the
-  // cells before it, first3 whether it lies in the first of the two bricks.
-  uint32_t at3[K3], below3[K3];
-  bool first3[K3];
+  // cells of its brick's before it, first3 whether it lies in the first of the two bricks (the highest position always).
+  uint32_t at3[K3], below3[K3], first3[K3];
 #pragma unroll
   for (int q = 0; q < K3; ++q) {
     int cell;
     const bool ok = along(3, q, &cell);
     const uint32_t pos = static_cast<uint32_t>(cell - (base3 << 3)) & 15u;
     at3[q] = ok ? 1u << pos : 0u;
-    below3[q] = (1u << pos) - 1u;
-    first3[q] = pos < 8u;
+    first3[q] = q == K3 - 1 || pos < 8u ? ~0u : 0u;
+    below3[q] = ((1u << pos) - 1u) & (0xFF00u | first3[q]);
   }
   const uint32_t levelRecords = static_cast<uint32_t>(m.nb[2]) * static_cast<uint32_t>(m.nb[3]);
   const uint32_t inLevel = static_cast<uint32_t>(base2 * m.nb[3] + base3);
   // The records of every level first (independent loads), then the taps.  A brick of the group that no position reaches
   // (three cells in a row cross into the next brick for a quarter of the inputs) and one outside the grid are replaced by
   // the first: no line is fetched for them, and no valid tap looks at them.
-  const bool need2 = ((o2[0] >> 3) > base2) && base2 + 1 < m.nb[2];
+  const bool need2 = ((o2[0] >> 3) > base2) & (base2 + 1 < m.nb[2]);
   int high3;
   along(3, 0, &high3);
-  const bool need3 = ((high3 >> 3) > base3) && base3 + 1 < m.nb[3];
-  const uint32_t step2 = need2 ? static_cast<uint32_t>(m.nb[3]) : 0u, step3 = need3 ? 1u : 0u;
-  const bool inside = live && base2 < m.nb[2] && base3 < m.nb[3];
-  uint32_t lo[K1][4], hi[K1][4], pre[K1][4];
+  const bool need3 = ((high3 >> 3) > base3) & (base3 + 1 < m.nb[3]);
+  const bool inside = live & (base2 < m.nb[2]) & (base3 < m.nb[3]);
+  const uint32_t level0 = static_cast<uint32_t>(c[0]) * static_cast<uint32_t>(m.nb[0]) * static_cast<uint32_t>(m.nb[1]);
+  uint32_t lo[K1][4], hi[K1][4], pre[K1][4], recs[K1][4];
 #pragma unroll
   for (int q1 = 0; q1 < K1; ++q1) {
-    const uint32_t rec0 = ok1[q1] && inside ? (static_cast<uint32_t>(c[0]) * static_cast<uint32_t>(m.nb[0]) * static_cast<uint32_t>(m.nb[1]) +
-                                               static_cast<uint32_t>(o1[q1])) * levelRecords + inLevel
-                                            : 0u;
+    const bool there = ok1[q1] & inside;
+    const uint32_t rec0 = there ? (level0 + static_cast<uint32_t>(o1[q1])) * levelRecords + inLevel : 0u;
+    const uint32_t step2 = (there & need2) ? static_cast<uint32_t>(m.nb[3]) : 0u, step3 = (there & need3) ? 1u : 0u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t rec = rec0 + (ok1[q1] && inside ? ((e & 2) ? step2 : 0u) + ((e & 1) ? step3 : 0u) : 0u);
-      const uint4 r = *reinterpret_cast<const uint4*>(records + rec);
-      const uint32_t base = chunkBase[rec >> m.chunkShift];
+      const uint32_t rec = rec0 + ((e & 2) ? step2 : 0u) + ((e & 1) ? step3 : 0u);
+      // (a map is at most kMaxBlockMapBytes: 32-bit offsets)
+      const uint4 r = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(records) + rec * 16u);
+      recs[q1][e] = rec;
       lo[q1][e] = r.x;
       hi[q1][e] = r.y;
-      pre[q1][e] = r.z + base;  // in-chunk prefix -> global prefix
+      pre[q1][e] = r.z;
     }
   }
-  uint32_t mine = 0;  // lane t of a wavefront counts the wavefront's pairs of tap t
-  unsigned long long hitsOfTap = 0;  // strided: which of the wavefront's inputs have tap t (lane t)
-  unsigned long long tileBits = 0;  // wavefront-uniform: (mirrored) taps that some input of the wavefront has
+  if (chunkBase) {  // in-chunk prefix -> global prefix (a listed map's prefixes are global)
+#pragma unroll
+    for (int q1 = 0; q1 < K1; ++q1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        pre[q1][e] += *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(chunkBase) + (recs[q1][e] >> m.chunkShift) * 4u);
+  }
+  int mine = 0;             // lane t of a wavefront counts the wavefront's pairs of tap t
+  int hitsLo = 0, hitsHi = 0;  // packed: which of the wavefront's inputs have tap t (lane t)
+  // SubM: a rank past the live rows is a cell of a shared map whose row a truncated strided build dropped
   const uint32_t rankLimit = static_cast<uint32_t>(MODE == kProbeTable ? liveCount(numActSrc, srcCap)
                                                                        : MODE == kProbeSubM ? n : maxNumActOut);
+  // rows below the live count get a staging entry, in the grid or not (fixTail: every row below the capacity); the others'
+  // stores lie past the end of the row's buffer
+  const uint32_t rowBytes = static_cast<uint32_t>(MODE == kProbeDirect ? nbrRows : fixTail ? cap : MODE == kProbePacked ? i0 + kProbeThreads : n) * 4u;
+  const uint32_t ownOffset = static_cast<uint32_t>(i) * 4u, waveOffset = static_cast<uint32_t>(i - lane) * 4u;
 #pragma unroll
   for (int q2 = 0; q2 < K2; ++q2) {
-    const bool up = (o2[q2] >> 3) > base2;
-    const uint32_t rowIn = static_cast<uint32_t>(o2[q2]) & 7u;            // row of the brick
-    const bool high = rowIn >= 4u;
-    const uint32_t rowShift = (rowIn & 3u) * 8u;
-    const uint32_t rowsBefore = (1u << rowShift) - 1u;                    // earlier rows of the word that holds the row
-    const uint32_t beforeLo = high ? ~0u : rowsBefore, beforeHi = high ? rowsBefore : 0u;
+    const uint32_t up = q2 < K2 - 1 && (o2[q2] >> 3) > base2 ? ~0u : 0u;  // (the highest position is in the lower bricks)
+    const uint32_t rowIn = static_cast<uint32_t>(o2[q2]) & 7u;            // row of the brick: a byte of its cells
+    const uint32_t high = static_cast<uint32_t>(static_cast<int>(rowIn << 29) >> 31);  // in the upper word
+    const uint32_t rowsBefore = (1u << ((rowIn & 3u) * 8u)) - 1u;         // earlier rows of the word that holds the row
+    const uint32_t beforeLo = high | rowsBefore, beforeHi = high & rowsBefore;
+    const uint32_t byte0 = 0x0C0C0C00u | rowIn, byte1 = 0x0C0C000Cu | (rowIn << 8);  // that byte as byte 0 / 1, zeros around
 #pragma unroll
     for (int q1 = 0; q1 < K1; ++q1) {
       // the two records of this brick row: first and second 8 cells of the 16
       const uint32_t lo0 = pick(up, lo[q1][2], lo[q1][0]), hi0 = pick(up, hi[q1][2], hi[q1][0]), pre0 = pick(up, pre[q1][2], pre[q1][0]);
       const uint32_t lo1 = pick(up, lo[q1][3], lo[q1][1]), hi1 = pick(up, hi[q1][3], hi[q1][1]), pre1 = pick(up, pre[q1][3], pre[q1][1]);
-      const uint32_t row0 = ((high ? hi0 : lo0) >> rowShift) & 0xFFu, row1 = ((high ? hi1 : lo1) >> rowShift) & 0xFFu;
-      const uint32_t cells = row0 | (row1 << 8);
+      const uint32_t cells = __builtin_amdgcn_perm(hi0, lo0, byte0) | __builtin_amdgcn_perm(hi1, lo1, byte1);
       const uint32_t rank0 = pre0 + static_cast<uint32_t>(__popc(lo0 & beforeLo)) + static_cast<uint32_t>(__popc(hi0 & beforeHi));
-      const uint32_t rank1 = pre1 + static_cast<uint32_t>(__popc(lo1 & beforeLo)) + static_cast<uint32_t>(__popc(hi1 & beforeHi)) -
-                             static_cast<uint32_t>(__popc(row0));         // counts of `cells` below a cell include row0
-      const uint32_t taken = ok1[q1] && ok2[q2] ? cells : 0u;
+      const uint32_t rank1 = pre1 + static_cast<uint32_t>(__popc(lo1 & beforeLo)) + static_cast<uint32_t>(__popc(hi1 & beforeHi));
+      const uint32_t taken = cells & (ok1[q1] ? ok2[q2] : 0u);
 #pragma unroll
       for (int q3 = 0; q3 < K3; ++q3) {
-        const uint32_t rank = (first3[q3] ? rank0 : rank1) + static_cast<uint32_t>(__popc(cells & below3[q3]));
-        // SubM: a rank past the live rows is a cell of a shared map whose row a truncated strided build dropped
-        const uint32_t row = (taken & at3[q3]) != 0u && rank < rankLimit ? rank : kNone;
+        const uint32_t rank = pick(first3[q3], rank0, rank1) + static_cast<uint32_t>(__popc(cells & below3[q3]));
+        const bool valid = ((taken & at3[q3]) != 0u) & (rank < rankLimit);
+        uint32_t row = valid ? rank : kNone;
+        asm("" : "+v"(row));   // (one compare for the ballot below, instead of `valid` made into a number and back)
         const int tap = (q1 * K2 + q2) * K3 + q3;
-        if (nbrDirect && row != kNone && row < static_cast<uint64_t>(nbrRows))
-          nbrDirect[static_cast<int64_t>(tap) * nbrRows + row] = static_cast<int32_t>(i);
-        const unsigned long long having = __ballot(row != kNone);
-        if constexpr (SUBM) {
-          if (staging && inRange) staging[static_cast<int64_t>(tap) * pitch + i] = row;
-          const uint32_t hits = static_cast<uint32_t>(__popcll(having));
-          mine = lane == tap ? hits : mine;
-          if (hits) tileBits |= 1ull << (KV - 1 - tap);
+        const unsigned long long having = __builtin_amdgcn_ballot_w64(row != kNone);
+        if constexpr (MODE == kProbePacked) {
+          const uint32_t at = valid ? waveOffset + lanesBelow(having) * 4u : kNone;
+          __builtin_amdgcn_raw_buffer_store_b32(row, rowBuffer(staging + static_cast<int64_t>(tap) * pitch, rowBytes), at, 0, 0);
+          hitsLo = writeLane(static_cast<int>(having), tap, hitsLo);
+          hitsHi = writeLane(static_cast<int>(having >> 32), tap, hitsHi);
         } else {
-          if (hitsOut) {
-            if (row != kNone) staging[static_cast<int64_t>(tap) * pitch + (i - lane) + lanesBelow(having)] = row;
-          } else if (staging && inRange) {
-            staging[static_cast<int64_t>(tap) * pitch + i] = row;
-          }
-          hitsOfTap = lane == tap ? having : hitsOfTap;
+          if constexpr (MODE == kProbeDirect)
+            __builtin_amdgcn_raw_buffer_store_b32(static_cast<uint32_t>(i), rowBuffer(nbrDirect + static_cast<int64_t>(tap) * nbrRows, rowBytes),
+                                                  row * 4u, 0, 0);
+          else
+            __builtin_amdgcn_raw_buffer_store_b32(row, rowBuffer(staging + static_cast<int64_t>(tap) * pitch, rowBytes), ownOffset, 0, 0);
+          mine = writeLane(static_cast<int>(__popcll(having)), tap, mine);
         }
       }
     }
   }
-  if (maskOut && lane == 0 && (i >> 6) < nMasks) maskOut[i >> 6] = tileBits;
-  if constexpr (!SUBM) {
-    mine = static_cast<uint32_t>(__popcll(hitsOfTap));
-    if (hitsOut && lane < KV) hitsOut[static_cast<size_t>(lane) * hitsPitch + (i >> 6)] = hitsOfTap;
+  if constexpr (MODE == kProbePacked) {
+    mine = __popc(hitsLo) + __popc(hitsHi);
+    if (lane < KV)
+      hitsOut[static_cast<size_t>(lane) * hitsPitch + (i >> 6)] =
+          static_cast<unsigned long long>(static_cast<uint32_t>(hitsHi)) << 32 | static_cast<uint32_t>(hitsLo);
+  }
+  if constexpr (ROWS) {  // the taps of the table (mirrored) that some row of the wavefront's has
+    const unsigned long long taps = __builtin_amdgcn_ballot_w64(mine != 0);
+    if (maskOut && lane == 0 && (i >> 6) < nMasks) maskOut[i >> 6] = __brevll(taps) >> (64 - KV);
   }
   if constexpr (MODE == kProbeTable) return;  // the pairs were counted from the inputs' side
   __syncthreads();  // ldsCnt zeroed
-  if (mine) atomicAdd(&ldsCnt[lane], mine);
+  if (mine) atomicAdd(&ldsCnt[lane], static_cast<uint32_t>(mine));
   __syncthreads();
   if (threadIdx.x < KV) cnt[static_cast<size_t>(threadIdx.x) * cntPitch + probeBlock] = static_cast<RbCount>(ldsCnt[threadIdx.x]);
 }
@@ -2588,7 +2607,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     side.mapWritten = !subM && mapOutside;
     const dim3 perChunk(w.nChunks > 0 ? w.nChunks : 1);
     const bool near = nearEligible(g, m);
-    const int ksel = near ? fixedKernelShape(g) : 0;
+    const int ksel = near && cap < kMaxFixedRows && nbrRows < kMaxFixedRows ? fixedKernelShape(g) : 0;
     // Two maps in turn (no reset pass) when the caller keeps the map and its state between passes and the probe
     // is the fixed-shape one, which leaves nothing else to zero; a SubM build on a shared map follows the build
     // that wrote it.
@@ -2716,7 +2735,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
     if (sharedMap) {
     } else if (list.entries) {
       hipLaunchKernelGGL(bmScanList, dim3(static_cast<unsigned>((side.mapListRows + kListRun - 1) / kListRun)), dim3(kListThreads), 0,
-                         stream, recBefore, list, numActIn, cap, chunkBase, perChunk.x);
+                         stream, recBefore, list, numActIn, cap);
     } else if (gather == 1) {
       if (ordered) D3D_LAUNCH_SCAN(true, 1); else D3D_LAUNCH_SCAN(false, 1);
     } else if (gather == 2) {
@@ -2759,8 +2778,8 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       planeFill = (planeFill * kRbThreads + kProbeThreads - 1) / kProbeThreads;
 #define D3D_LAUNCH_PROBE_PLANE(MODE, K1, K2, K3)                                                                    \
   hipLaunchKernelGGL((bmProbeFixed<MODE, K1, K2, K3>), dim3(planeFill + fixedBlocks + fixedExtra), dim3(kProbeThreads), 0, stream, \
-                     g, m, coors, numActIn, cap, pitch, recBehind, chunkBase, perm, permShuffled, maxNumActOut,   \
-                     (directScatter && skipIndex) ? nullptr : staging, packed ? hits : nullptr, w.hitsPitch, cnt, w.cntPitch, probeFillIndex, \
+                     g, m, coors, numActIn, cap, pitch, recBehind, list.entries ? nullptr : chunkBase, perm, permShuffled, maxNumActOut, \
+                     staging, hits, w.hitsPitch, cnt, w.cntPitch, probeFillIndex, \
                      nIndex, fillB, nFillB, planeFill,                                                               \
                      fixedBlocks, outCoors, w.nRecords, probeMasks ? masks : nullptr, nMasks,                        \
                      (subM && inPlace) ? 1 : 0, directScatter ? nbrOut : nullptr, nbrRows, fillState,               \
@@ -2775,13 +2794,20 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
           default: D3D_LAUNCH_PROBE_NEAR(true, 0);
         }
       } else {
+#define D3D_LAUNCH_PROBE_STRIDED(K1, K2, K3)                                      \
+  do {                                                                            \
+    if (directScatter) D3D_LAUNCH_PROBE_PLANE(kProbeDirect, K1, K2, K3);          \
+    else if (packed) D3D_LAUNCH_PROBE_PLANE(kProbePacked, K1, K2, K3);            \
+    else D3D_LAUNCH_PROBE_PLANE(kProbeStrided, K1, K2, K3);                       \
+  } while (0)
         switch (ksel) {
-          case 1: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 3, 3); break;
-          case 2: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 1, 1); break;
-          case 3: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 3, 1, 3); break;
-          case 4: D3D_LAUNCH_PROBE_PLANE(kProbeStrided, 1, 3, 3); break;
+          case 1: D3D_LAUNCH_PROBE_STRIDED(3, 3, 3); break;
+          case 2: D3D_LAUNCH_PROBE_STRIDED(3, 1, 1); break;
+          case 3: D3D_LAUNCH_PROBE_STRIDED(3, 1, 3); break;
+          case 4: D3D_LAUNCH_PROBE_STRIDED(1, 3, 3); break;
           default: D3D_LAUNCH_PROBE_NEAR(false, 0);
         }
+#undef D3D_LAUNCH_PROBE_STRIDED
       }
 #undef D3D_LAUNCH_PROBE_PLANE
       if (tableProbe) {
