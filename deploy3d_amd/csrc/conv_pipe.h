@@ -32,22 +32,12 @@ namespace convk {
 
 typedef __attribute__((address_space(3))) void* LdsVoidPtr;
 
-// Wavefronts of the largest shape of a layer of 128 output channels.  int8 128 -> 128: the wider workgroups (two wavefronts per
-// SIMD, 256 registers each) spill - 84-97 us against 33-44 on a 47 000-row layer - so only the four-wavefront shapes count.
-template <class T, int CIN>
-constexpr int pipeWaves() { return sizeof(T) == 1 && CIN == 128 ? 4 : 8; }
-
-// Whether the 48-row shape is among those a kernel chooses from: in two-byte types it takes 278 registers, which workgroups of
-// eight wavefronts do not have (256 and a spill: 59 us where it takes 45 by itself).
-template <class T> constexpr bool kPipeTall = sizeof(T) == 1;
-
-// Shapes of those layers, rows per wavefront x wavefronts: 0: 32 x 8, 1: 32 x 6, 2: 32 x 4, 3: 48 x 4.  The one that loads the
-// busiest of `cus` CUs least with `rows` rows (rounds of tiles x rows per tile); see launchPipeShape.
-template <bool FOUR_ONLY>
+// Shapes of two-byte layers of 128 output channels whose workgroups take all of them, rows per wavefront x wavefronts:
+// 0: 32 x 8, 1: 32 x 6, 2: 32 x 4, 3: 48 x 4.  The one that loads the busiest of `cus` CUs least with `rows` rows (rounds of
+// tiles x rows per tile); see launchPipeShape.
 __host__ __device__ inline int pipeShapeOf(int64_t rows, int cus) {
   auto load = [&](int tile) { return static_cast<int>((rows + static_cast<int64_t>(tile) * cus - 1) / (static_cast<int64_t>(tile) * cus)) * tile; };
   const int l8 = load(256), l6 = load(192), l4 = load(128);
-  if (FOUR_ONLY) return l4 < l6 ? 2 : 3;
   int best = l6 < l8 ? 1 : 0;
   if (l4 < (best ? l6 : l8)) best = 2;
   return best == 1 && l6 <= 192 ? 3 : best;
@@ -55,7 +45,7 @@ __host__ __device__ inline int pipeShapeOf(int64_t rows, int cus) {
 
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
 // ceil(outRows / 64) (a workgroup reads the masks of a whole tile at once); null = every tap of every tile.
-template <class T, int CIN, int COUT, int MT, int WAVES>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
 __device__ __forceinline__ void
 pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
           const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch,
@@ -70,10 +60,11 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   constexpr int WM = 16 * MT, TM = WAVES * WM;
   constexpr int GL = WM / RPI;                                 // gather instructions per step
   constexpr int GPM = 16 / RPI;                                // gathers that cover the 16 rows of one row group
-  constexpr int NT = COUT / 16;
+  constexpr int NT = CO / 16;
+  constexpr int COLS = COUT / CO;                              // workgroups that share a tile, CO output channels each
   constexpr int KK = CS * ES / 64;                             // MFMAs along K per step: 64 bytes of a row each
   constexpr int NQ = KK * NT;                                  // MFMAs per row group and step
-  constexpr int WCH = CS * COUT * ES / 16;                     // 16-byte chunks of one step's weights
+  constexpr int WCH = CS * CO * ES / 16;                       // 16-byte chunks of one step's weights
   constexpr int WL = (WCH + THREADS - 1) / THREADS;            // weight loads per wavefront and step
   constexpr int NWB = 3;                                       // weight buffers
   constexpr int NI = 4;                                        // index ring depth (steps)
@@ -118,7 +109,8 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   // past the live rows; inside an XCD, workgroups take tiles round robin ----
   const TileOrder order(static_cast<int>((outRows + TM - 1) / TM), static_cast<int>((liveOutRows(numActOut, outRows) + TM - 1) / TM), xcdShift,
                         blockIdx.x & ((1 << xcdShift) - 1));
-  const int firstLocal = blockIdx.x >> xcdShift, strideLocal = blocks >> xcdShift;
+  const int firstLocal = (blockIdx.x >> xcdShift) / COLS, strideLocal = (blocks >> xcdShift) / COLS;
+  const int part = (blockIdx.x >> xcdShift) % COLS;      // which CO of the output channels
   const int nMine = firstLocal < order.count() ? (order.count() - 1 - firstLocal) / strideLocal + 1 : 0;
   if (nMine <= 0) return;                                // workgroup-uniform
   auto tileAt = [&](int pos) __attribute__((always_inline)) { return order.tile(firstLocal + pos * strideLocal); };
@@ -215,9 +207,11 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     __builtin_amdgcn_raw_ptr_buffer_load_lds(inBuf, (LdsVoidPtr)(stage + slot * SLOTS + j * 64), 16, off, 0, 0, 0);
   };
   auto weightLoad = [&](int q, int s, int buf) __attribute__((always_inline)) {
-    const u32x4* wk = reinterpret_cast<const u32x4*>(wf) + static_cast<size_t>(s) * WCH;
+    const u32x4* wk = reinterpret_cast<const u32x4*>(wf) + static_cast<size_t>(s) * (WCH * COLS);
     const int base = (q * THREADS + wave * 64) % WCH;  // wavefronts past the slice repeat a part of it: same bytes
-    __builtin_amdgcn_global_load_lds(wk + base + lane, wLds + buf * WCH + base, 16, 0, 0);
+    // fragments lie in the order (K, channel tile): the workgroup's NT of the COLS * NT tiles of every K
+    const int from = COLS == 1 ? base : (base / (NT * 64) * COLS + part) * (NT * 64) + base % (NT * 64);
+    __builtin_amdgcn_global_load_lds(wk + from + lane, wLds + buf * WCH + base, 16, 0, 0);
   };
   auto readRowGroup = [&](F (&dst)[KK], int m, int slot) __attribute__((always_inline)) {
     const int n = m * 16 + r16;
@@ -238,7 +232,7 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     if constexpr (ES == 4) {
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        const int col = n * 16 + kgrp * 4;
+        const int col = part * CO + n * 16 + kgrp * 4;
         const float4v b = bias ? *reinterpret_cast<const float4v*>(bias + col) : float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -256,12 +250,12 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     } else {
 #pragma unroll
     for (int n = 0; n < NT; n += 2) {
-      const int col0 = n * 16 + kgrp * 4, col1 = col0 + 16;
+      const int col0 = part * CO + n * 16 + kgrp * 4, col1 = col0 + 16;
       const float4v b0 = bias ? *reinterpret_cast<const float4v*>(bias + col0) : float4v{0.f, 0.f, 0.f, 0.f};
       const float4v b1 = bias ? *reinterpret_cast<const float4v*>(bias + col1) : float4v{0.f, 0.f, 0.f, 0.f};
       // channels this lane stores after the swaps: tile n for even 16-lane rows, tile n+1 for odd ones; the
       // first or second half of the tile's 16 channels by lane row / 2
-      const int outCol = (n + (kgrp & 1)) * 16 + (kgrp >> 1) * 8;
+      const int outCol = part * CO + (n + (kgrp & 1)) * 16 + (kgrp >> 1) * 8;
       if constexpr (ES == 1) {
         // int8: q = clamp(rint(float(acc) * m[c] + bq[c])), lower bound 0 with the fused ReLU; a lane's 4 channels
         // are one dword, and one swap hands every lane 8 consecutive channels.  One channel tile at a time, so that
@@ -436,46 +430,37 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   waitVmcnt<0>();                                   // loads issued for steps that do not exist, and the stores
 }
 
-template <class T, int CIN, int COUT, int MT, int WAVES>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
 __global__ void __launch_bounds__(64 * WAVES)
 convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
          const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
          const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
          int xcdShift, const int32_t* __restrict__ numActOut) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  pipeTiles<T, CIN, COUT, MT, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+  pipeTiles<T, CIN, COUT, MT, WAVES, CO>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
                                      relu, xcdShift, numActOut, gridDim.x);
 }
 
-// The workgroup shape chosen here, by the rows that are live, for layers whose time is that of a few rounds of tiles (see
-// launchPipeShape): the host knows the capacity only.  Wavefronts past the shape's end at once.
-template <class T, int CIN, int COUT, int MOST>
-__global__ void __launch_bounds__(64 * MOST)
+// The same with the shape (0, 1 or 2: 48-row wavefronts take 278 registers, which workgroups of eight do not have) chosen by
+// the live rows; the host knows the capacity only.  Wavefronts past the shape's end at once.
+template <class T, int CIN, int COUT>
+__global__ void __launch_bounds__(512)
 convPipeByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
                const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
                const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
                int xcdShift, const int32_t* __restrict__ numActOut, int cus) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int shape = pipeShapeOf<MOST == 4>(liveOutRows(numActOut, outRows), cus);
-#define D3D_PIPE_BODY(MT, WAVES)                                                                                        \
+  const int shape = pipeShapeOf(liveOutRows(numActOut, outRows), cus);
+#define D3D_PIPE_BODY(WAVES)                                                                                            \
   {                                                                                                                     \
     if (wave >= WAVES) return;                                                                                          \
-    pipeTiles<T, CIN, COUT, MT, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol,    \
-                                       inRows, outRows, relu, xcdShift, numActOut, WAVES == 4 && MT == 3 ? cus : gridDim.x); \
+    pipeTiles<T, CIN, COUT, 2, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol,     \
+                                      inRows, outRows, relu, xcdShift, numActOut, gridDim.x);                           \
   }
-  if constexpr (kPipeTall<T>) {
-    if (shape == 3) {
-      if (blockIdx.x >= static_cast<unsigned>(cus)) return;   // one round: a tile per CU, none beside another
-      D3D_PIPE_BODY(3, 4)
-      return;
-    }
-  }
-  if (shape == 2) D3D_PIPE_BODY(2, 4)
-  else if constexpr (MOST == 8) {
-    if (shape == 0) D3D_PIPE_BODY(2, 8)
-    else D3D_PIPE_BODY(2, 6)
-  }
+  if (shape == 2) D3D_PIPE_BODY(4)
+  else if (shape == 0) D3D_PIPE_BODY(8)
+  else D3D_PIPE_BODY(6)
 #undef D3D_PIPE_BODY
 }
 
@@ -495,33 +480,30 @@ inline bool pipeTakes(const ConvArgs& a, int64_t pitch, size_t rowBytes, int til
 
 template <class T, int CIN, int COUT>
 int32_t launchPipeByRows(const ConvArgs& a, hipStream_t stream) {
-  constexpr int WAVES = pipeWaves<T, CIN>();
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
   if (!pipeTakes(a, pitch, CIN * sizeof(T), 256)) return D3D_ERR_UNSUPPORTED;
-  constexpr size_t wide = pipeLds<T, CIN, COUT>(2, WAVES), tall = kPipeTall<T> ? pipeLds<T, CIN, COUT>(3, 4) : 0;
-  constexpr size_t lds = wide > tall ? wide : tall;
+  constexpr size_t lds = pipeLds<T, CIN, COUT>(2, 8);
   static_assert(lds <= kLdsLimit, "every shape fits a CU");
   static std::atomic<size_t> granted{64 * 1024};
-  const int32_t rc = grantLds(&convPipeByRows<T, CIN, COUT, WAVES>, lds, &granted);
+  const int32_t rc = grantLds(&convPipeByRows<T, CIN, COUT>, lds, &granted);
   if (rc != D3D_OK) return rc;
   const ChipLayout chip = chipLayout();
-  const int nXcd = 1 << chip.xcdShift, cus = chip.cus / nXcd * nXcd;
-  const int perCu = 2 * lds <= kLdsLimit ? 2 : 1;
-  hipLaunchKernelGGL((convPipeByRows<T, CIN, COUT, WAVES>), dim3(static_cast<unsigned>(cus * perCu)), dim3(64 * WAVES), lds, stream,
+  const int nXcd = 1 << chip.xcdShift, cus = chip.cus / nXcd * nXcd, perCu = kLdsLimit / lds > 1 ? 2 : 1;
+  hipLaunchKernelGGL((convPipeByRows<T, CIN, COUT>), dim3(static_cast<unsigned>(cus * perCu)), dim3(512), lds, stream,
                      static_cast<const T*>(a.in), static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias,
                      a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift,
                      a.numActOut, cus);
   return D3D_OK;
 }
 
-template <class T, int CIN, int COUT, int MT, int WAVES>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
 int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
-  constexpr int TM = 16 * MT * WAVES;
-  constexpr size_t lds = pipeLds<T, CIN, COUT>(MT, WAVES);
+  constexpr int TM = 16 * MT * WAVES, COLS = COUT / CO;
+  constexpr size_t lds = pipeLds<T, CIN, CO>(MT, WAVES);
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
   if (lds > kLdsLimit || !pipeTakes(a, pitch, CIN * sizeof(T), TM)) return D3D_ERR_UNSUPPORTED;
   static std::atomic<size_t> granted{64 * 1024};
-  const int32_t rc = grantLds(&convPipe<T, CIN, COUT, MT, WAVES>, lds, &granted);
+  const int32_t rc = grantLds(&convPipe<T, CIN, COUT, MT, WAVES, CO>, lds, &granted);
   if (rc != D3D_OK) return rc;
   const int tiles = static_cast<int>((a.outRows + TM - 1) / TM);
   // persistent workgroups: as many as the CUs can hold at this LDS footprint, never more than there are tiles
@@ -530,9 +512,10 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   if (perCu < 1) perCu = 1;
   const ChipLayout chip = chipLayout();
   const int nXcd = 1 << chip.xcdShift;
-  int blocks = (tiles + nXcd - 1) / nXcd * nXcd;
-  if (blocks > chip.cus / nXcd * nXcd * perCu) blocks = chip.cus / nXcd * nXcd * perCu;
-  hipLaunchKernelGGL((convPipe<T, CIN, COUT, MT, WAVES>), dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES),
+  int blocks = (tiles + nXcd - 1) / nXcd * nXcd * COLS;
+  const int most = chip.cus * perCu / (nXcd * COLS) * (nXcd * COLS);
+  if (blocks > most) blocks = most;
+  hipLaunchKernelGGL((convPipe<T, CIN, COUT, MT, WAVES, CO>), dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES),
                      lds, stream, static_cast<const T*>(a.in), static_cast<T*>(a.out),
                      static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks,
                      a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut);
@@ -549,11 +532,8 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
 // (a stage row holding the neighbours under two taps side by side, the step of a 64-channel layer) measured slower
 // on 32 -> 64 in every tile shape tried (45-57 us against 36): the stage doubles, one workgroup fits a CU instead of
 // two, and the layer needs the wavefronts more than the longer steps.
-// Layers with few
-// rows (the 128-channel stages: 47 000 rows are 186 tiles of 256 rows for 256 CUs) pick the workgroup shape by
-// tile count: the time of a layer that fits one round is that of ONE tile, so 248 tiles of 192 rows beat 186 of
-// 256 (48 us against 55), and there four wavefronts of 48 rows - one per SIMD, three 16-row groups each - beat
-// six of 32 rows (45 us against 48).
+// Layers of 128 output channels pick the shape by the row count: the time of a layer that fits one round is that of ONE
+// tile.
 template <class T, int CIN, int COUT>
 int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   // shapes go by the bytes of an input row (the stage) and by the output channels (the accumulators): an int8 layer
@@ -579,40 +559,41 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     }
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else if constexpr (COUT >= 128) {
-    // 8, 6 or 4 wavefronts of 32 rows: the workgroup size whose tiles load the busiest CU least (rounds of tiles
-    // over the 256 CUs x rows per tile).  A layer that fits ONE round of 192-row tiles takes them as four
-    // wavefronts of 48 rows - one per SIMD - instead of six of 32, which load two SIMDs twice as much as the
-    // others (conv4_x: 45 us against 48); over several rounds the eight-wavefront shapes hide their waits better
-    // (a 64 -> 128 layer of 10 rounds: 105 us with 8 x 32 rows, 138 us with 4 x 48).
-    // Fewer rows than one round of 64-row tiles take those, two wavefronts each (128 -> 128 with 10 200 rows: 29 us
-    // against 33 with 128-row tiles; with 23 000 rows, more than a round, 41 against 34).
-    if constexpr (sizeof(T) == 2 && CIN >= 64)
-      if (a.outRows <= 64 * static_cast<int64_t>(chipLayout().cus) && !debugEnv("D3D_CONV_PIPE_SHAPE"))
-        return launchPipeCfg<T, CIN, COUT, 2, 2>(a, stream);
-    static const int kCand[4][2] = {{32, 8}, {32, 6}, {32, 4}, {48, 4}};
-    constexpr bool FOUR_ONLY = pipeWaves<T, CIN>() == 4;
-    const char* const force = debugEnv("D3D_CONV_PIPE_SHAPE");  // "rows,wavefronts" of one candidate (tests)
-    // More than a round of the largest tiles: the shape is chosen from the live rows (convPipeByRows; fp16, us: 128 -> 128 with
-    // 190 000 rows at a capacity of 237 000 183 -> 154, at 199 500 202 -> 160, 64 -> 128 104 -> 88; what the host would choose
-    // at the live count takes the same).  Below, that kernel has nothing better to choose in two-byte types: 48-row
-    // wavefronts need a launch of their own, and 32 x 6 in it is no faster than 32 x 8 (53 us).  int8 128 -> 128 has two
-    // shapes, both in it: 47 500 rows at a capacity of 59 400 43 -> 33.
-    if (!force && a.outRows > (FOUR_ONLY ? 128 : 256) * static_cast<int64_t>(chipLayout().cus))
-      return launchPipeByRows<T, CIN, COUT>(a, stream);
-    int best = pipeShapeOf<FOUR_ONLY>(a.outRows, chipLayout().cus);
-    if (force) {
-      for (int c = FOUR_ONLY ? 2 : 0; c < 4; ++c)
-        if (std::atoi(force) == kCand[c][0] && std::strchr(force, ',') &&
-            std::atoi(std::strchr(force, ',') + 1) == kCand[c][1])
-          best = c;
-    }
-    if (best == 2) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
-    if (best == 3) return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
-    if constexpr (!FOUR_ONLY) {
+    const int64_t cus = chipLayout().cus;
+    const char* const force = debugEnv("D3D_CONV_PIPE_SHAPE");  // "rows,wavefronts" (tests)
+    const int rows = force ? std::atoi(force) : 0, waves = force && std::strchr(force, ',') ? std::atoi(std::strchr(force, ',') + 1) : 0;
+    if constexpr (sizeof(T) == 1 || CIN >= 64) {
+      // One workgroup of four wavefronts per CU that takes all 128 channels adds the time of its LDS reads (each wavefront
+      // reads a step's whole weight slice) to that of its MFMAs: without MFMAs, gathers and weight loads a 24 000-row layer
+      // still took 21 of 34 us.  So a tile's channels are shared out to workgroups of 64 (with few rows, 32): two workgroups
+      // of half the slices fit a CU and each computes while the other reads.  us of 128 -> 128 and of 64 -> 128 with all
+      // channels / shared out, fp16: 10 500 rows 30 / 23 and 21 / 16, 24 500 rows 34.5 / 29.5 and 24 / 19, 38 000 rows
+      // 44 / 41 and 30 / 26, 47 500 rows 50.5 / 45 and 32 / 29, 97 000 rows 91 / 75 and 56 / 50, 190 000 rows 134 / 137 and
+      // 89 / 90 (its three-tap column layer 33 / 27); int8: 22 / 19.5, 27 / 25, 32 / 27.5, 51 / 44, 89 / 80.  The wider tile
+      // wins where it fits as many workgroups to a CU: the lines are whole rounds of one and of two workgroups per CU.
+      if (!force && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);   // 29 -> 18 us
+      if ((!force && (a.outRows <= 64 * cus || (a.outRows > 96 * cus && a.outRows <= 128 * cus))) || (rows == 32 && waves == 4))
+        return launchPipeCfg<T, CIN, COUT, 2, 4, 64>(a, stream);
+      // Past one round of two 192-row workgroups per CU a few of them would have a second tile (55 000 rows: 70 us by the
+      // rounds, 53 with 256-row tiles): up to 288 rows per CU the two-byte layers choose by the live rows.  (Six percent of
+      // head-room above the line: a capacity is above its live rows.)
+      if (sizeof(T) == 1 || (!force && (a.outRows <= 204 * cus || a.outRows > 288 * cus)) || (rows == 48 && waves == 4))
+        return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
+      if constexpr (sizeof(T) > 1) return launchPipeByRows<T, CIN, COUT>(a, stream);
+      return D3D_ERR_UNSUPPORTED;
+    } else {
+      // 32 -> 128: 8, 6 or 4 wavefronts of 32 rows, or 4 of 48: the workgroup size whose tiles load the busiest CU least
+      // (rounds of tiles over the 256 CUs x rows per tile), by the live rows past one round of the largest
+      if (!force && a.outRows > 256 * cus) return launchPipeByRows<T, CIN, COUT>(a, stream);
+      static const int kCand[4][2] = {{32, 8}, {32, 6}, {32, 4}, {48, 4}};
+      int best = pipeShapeOf(a.outRows, static_cast<int>(cus));
+      for (int c = 0; c < 4; ++c)
+        if (rows == kCand[c][0] && waves == kCand[c][1]) best = c;
+      if (best == 0) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
       if (best == 1) return launchPipeCfg<T, CIN, COUT, 2, 6>(a, stream);
-      return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+      if (best == 2) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
+      return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
     }
-    return D3D_ERR_UNSUPPORTED;
   } else if constexpr (RB == 64 && COUT == 32) {
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else {

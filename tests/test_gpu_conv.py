@@ -397,6 +397,14 @@ def test_pipelined_tile_shapes_by_row_count(engine, cin, cout):
         run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, ("float16", "bfloat16")[k % 2], True, relu=True)
 
 
+@pytest.mark.parametrize("cin,dtype", [(64, "bfloat16"), (128, "float16")])
+def test_output_channels_shared_out_by_row_count(engine, cin, dtype):
+    """128 output channels in workgroups of 32 or 64 of them: row counts on both sides of the lines (32, 96, 204 and 288 rows
+    per CU) at which the tile or the share changes."""
+    for n in (32 * 256, 32 * 256 + 1, 96 * 256, 96 * 256 + 1, 204 * 256 + 1, 288 * 256 + 1):
+        run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, dtype, True, relu=True)
+
+
 @pytest.mark.parametrize("levels", [1, 13, 14])
 def test_map_sizes_around_the_scan_forms(engine, levels):
     """Occupancy maps of 50 x 50 bricks per level, on both sides of the 32 768 records at which their scan takes another

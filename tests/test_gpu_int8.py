@@ -101,6 +101,13 @@ def test_int8_pipelined_tile_shape_by_live_rows(engine, cin):
         run_int8(n, (16, 128, 128), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, True, True, cap_extra=76011 - n)
 
 
+@pytest.mark.parametrize("cin", [64, 128])
+def test_int8_output_channels_shared_out_by_row_count(engine, cin):
+    """128 output channels in workgroups of 32 or 64 of them: row counts on both sides of the lines of the shapes."""
+    for n in (32 * 256, 32 * 256 + 1, 64 * 256 + 1, 96 * 256 + 1, 128 * 256 + 1):
+        run_int8(n, (16, 120, 120), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, True, True)
+
+
 @pytest.mark.parametrize("cin,cout", [(64, 32), (64, 64), (128, 64), (128, 128)])
 def test_int8_pipelined_and_barrier_per_tap_kernels_agree_with_the_oracle(engine, monkeypatch, cin, cout):
     """The same layer on the pipelined kernel (the default from 64 input channels up), across several tiles per
