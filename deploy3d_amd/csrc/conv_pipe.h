@@ -506,9 +506,11 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   const int32_t rc = grantLds(&convPipe<T, CIN, COUT, MT, WAVES, CO>, lds, &granted);
   if (rc != D3D_OK) return rc;
   const int tiles = static_cast<int>((a.outRows + TM - 1) / TM);
-  // persistent workgroups: as many as the CUs can hold at this LDS footprint, never more than there are tiles
+  // persistent workgroups: as many as the CUs can hold at this LDS footprint, never more than there are tiles (three where
+  // they fit: int8 64 -> 64 127 us with two, 121 with three on 1.07 million rows, 31 and 28 on 190 000; fp16 32 -> 64 153 and
+  // 147, 28.7 and 26)
   int perCu = static_cast<int>(kLdsLimit / lds);
-  if (perCu > 2) perCu = 2;
+  if (perCu > 3) perCu = 3;
   if (perCu < 1) perCu = 1;
   const ChipLayout chip = chipLayout();
   const int nXcd = 1 << chip.xcdShift;
@@ -541,12 +543,17 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   constexpr int RB = CIN * static_cast<int>(sizeof(T));
   if constexpr (sizeof(T) == 4) {
     // fp32: a step's MFMAs take eight times the cycles of a two-byte step with the same bytes, so the matrix pipe is
-    // the bound and the tile only has to spread over the CUs: 128 rows (two workgroups per CU) up to 64 output
-    // channels, eight wavefronts at 128, where one workgroup's weights leave no room for a second.  64 -> 64 with
-    // 150 000 rows runs in 285 us = 118 TFLOP/s of issued MFMAs against the 157 of the pipe (630 us on the vector
-    // kernel); skipping a 16-row group's MFMAs when none of its rows has the tap gained 15-20 us on strided and
+    // the bound and the tile only has to spread over the CUs: 128 rows, two or three workgroups per CU (16 -> 128: eight
+    // wavefronts).  64 -> 64 with 150 000 rows runs at 130 TFLOP/s of issued MFMAs against the 157 of the pipe (630 us on
+    // the vector kernel); skipping a 16-row group's MFMAs when none of its rows has the tap gained 15-20 us on strided and
     // inverse layers and cost as much on the dense ones: the barrier waits for the fullest group either way
-    if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+    // Layers of 64 and 128 output channels share a tile's channels out to workgroups of 32: with the matrix pipe as the bound
+    // a layer's time goes by the workgroups of the fullest CU, and smaller ones spread more evenly (64 -> 64, 144 000 rows,
+    // 4.4 tiles of all channels to a CU: 264 -> 254 us, 10 000-voxel encoder-decoder 110 -> 90, 32 -> 64 there 60 -> 51, a
+    // VoxelNet's from 30 000 voxels 114 -> 119 and 214 -> 214; 128 -> 128, 47 000 rows, 70 of 100 CUs with a tile of all
+    // channels: 413 -> 289, 16 500 rows 412 -> 172)
+    if constexpr (COUT >= 64 && CIN >= 32) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);
+    else if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
     else return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
   } else if constexpr (RB == 128 && COUT == 64) {
     // 512-row tiles; few rows take the smallest of 128, 256 and 512 whose tiles still fit one round of the CUs (64 -> 64:

@@ -405,6 +405,15 @@ def test_output_channels_shared_out_by_row_count(engine, cin, dtype):
         run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, dtype, True, relu=True)
 
 
+@pytest.mark.parametrize("cin,cout", [(32, 64), (64, 64), (32, 128), (64, 128), (128, 128)])
+def test_float_output_channels_shared_out(engine, cin, cout):
+    """fp32 layers whose output channels go to workgroups of 32: less than a tile, a tile and one row more, and more tiles
+    than workgroups (64 -> 64)."""
+    for n in (100, 128, 129, 3001) + ((70000,) if cin == cout == 64 else ()):
+        run_case(n, (16, 200, 200) if n > 9000 else (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, "float32", True,
+                 relu=True, cap_extra=n % 50)
+
+
 @pytest.mark.parametrize("levels", [1, 13, 14])
 def test_map_sizes_around_the_scan_forms(engine, levels):
     """Occupancy maps of 50 x 50 bricks per level, on both sides of the 32 768 records at which their scan takes another
