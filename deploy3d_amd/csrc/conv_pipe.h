@@ -206,12 +206,17 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     const uint32_t off = (static_cast<uint32_t>(idx) << ROWSHIFT) + partOff;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(inBuf, (LdsVoidPtr)(stage + slot * SLOTS + j * 64), 16, off, 0, 0, 0);
   };
+  // Buffer loads, not global ones: the compiler takes a global load into LDS for a flat access that may be pending in either
+  // memory, and from then on waits for ALL outstanding LDS reads where it needs the oldest - the reads meant to run in the
+  // shadow of a group's MFMAs were waited for in front of them (fp16 128 -> 128, 24 500 rows 28 -> 25.5 us, 190 000 rows
+  // 135 -> 125; 64 -> 64, 262 000 rows 59.5 -> 57.5; fp32 64 -> 64, 144 000 rows 253 -> 238).
+  const __amdgpu_buffer_rsrc_t wBuf = makeRawBuffer(wf, static_cast<uint32_t>(kVol * KS) * (WCH * COLS * 16u));
   auto weightLoad = [&](int q, int s, int buf) __attribute__((always_inline)) {
-    const u32x4* wk = reinterpret_cast<const u32x4*>(wf) + static_cast<size_t>(s) * (WCH * COLS);
     const int base = (q * THREADS + wave * 64) % WCH;  // wavefronts past the slice repeat a part of it: same bytes
     // fragments lie in the order (K, channel tile): the workgroup's NT of the COLS * NT tiles of every K
     const int from = COLS == 1 ? base : (base / (NT * 64) * COLS + part) * (NT * 64) + base % (NT * 64);
-    __builtin_amdgcn_global_load_lds(wk + from + lane, wLds + buf * WCH + base, 16, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wBuf, (LdsVoidPtr)(wLds + buf * WCH + base), 16, lane * 16,
+                                             (s * (WCH * COLS) + from) * 16, 0, 0);
   };
   auto readRowGroup = [&](F (&dst)[KK], int m, int slot) __attribute__((always_inline)) {
     const int n = m * 16 + r16;
