@@ -469,6 +469,27 @@ convPipeByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restric
 #undef D3D_PIPE_BODY
 }
 
+// 64 output channels: eight wavefronts of 64 rows, or of 48 where rounds of those tiles leave the CUs clearly less to do (with
+// many rounds the wider tile is the better one whatever their number).
+__host__ __device__ inline bool pipeTakes48(int64_t rows, int cus) {
+  auto load = [&](int tile) { return (rows + static_cast<int64_t>(tile) * cus - 1) / (static_cast<int64_t>(tile) * cus) * tile; };
+  return 10 * load(384) < 9 * load(512);
+}
+template <class T, int CIN, int COUT>
+__global__ void __launch_bounds__(512)
+convPipeNarrowByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
+                     const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
+                     const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
+                     int xcdShift, const int32_t* __restrict__ numActOut, int cus) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if (pipeTakes48(liveOutRows(numActOut, outRows), cus))
+    pipeTiles<T, CIN, COUT, 3, 8>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+                                  relu, xcdShift, numActOut, gridDim.x);
+  else
+    pipeTiles<T, CIN, COUT, 4, 8>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+                                  relu, xcdShift, numActOut, gridDim.x);
+}
+
 // LDS of a shape: three weight slices, two stages and four steps of indices per wavefront.
 template <class T, int CIN, int COUT>
 constexpr size_t pipeLds(int mt, int waves) {
@@ -484,17 +505,25 @@ inline bool pipeTakes(const ConvArgs& a, int64_t pitch, size_t rowBytes, int til
 }
 
 template <class T, int CIN, int COUT>
+constexpr auto pipeByRowsKernel() {
+  if constexpr (COUT < 128) return &convPipeNarrowByRows<T, CIN, COUT>;
+  else return &convPipeByRows<T, CIN, COUT>;
+}
+
+template <class T, int CIN, int COUT>
 int32_t launchPipeByRows(const ConvArgs& a, hipStream_t stream) {
+  constexpr bool NARROW = COUT < 128;
+  constexpr auto kernel = pipeByRowsKernel<T, CIN, COUT>();
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
-  if (!pipeTakes(a, pitch, CIN * sizeof(T), 256)) return D3D_ERR_UNSUPPORTED;
-  constexpr size_t lds = pipeLds<T, CIN, COUT>(2, 8);
+  if (!pipeTakes(a, pitch, CIN * sizeof(T), 512)) return D3D_ERR_UNSUPPORTED;
+  constexpr size_t lds = pipeLds<T, CIN, COUT>(NARROW ? 4 : 2, 8);
   static_assert(lds <= kLdsLimit, "every shape fits a CU");
   static std::atomic<size_t> granted{64 * 1024};
-  const int32_t rc = grantLds(&convPipeByRows<T, CIN, COUT>, lds, &granted);
+  const int32_t rc = grantLds(kernel, lds, &granted);
   if (rc != D3D_OK) return rc;
   const ChipLayout chip = chipLayout();
   const int nXcd = 1 << chip.xcdShift, cus = chip.cus / nXcd * nXcd, perCu = kLdsLimit / lds > 1 ? 2 : 1;
-  hipLaunchKernelGGL((convPipeByRows<T, CIN, COUT>), dim3(static_cast<unsigned>(cus * perCu)), dim3(512), lds, stream,
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(cus * perCu)), dim3(512), lds, stream,
                      static_cast<const T*>(a.in), static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias,
                      a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift,
                      a.numActOut, cus);
@@ -561,13 +590,16 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     else if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
     else return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
   } else if constexpr (RB == 128 && COUT == 64) {
-    // 512-row tiles; few rows take the smallest of 128, 256 and 512 whose tiles still fit one round of the CUs (64 -> 64:
+    // 512- or 384-row tiles; few rows take the smallest of 128, 256 and 512 whose tiles still fit one round of the CUs (64 -> 64:
     // 15 600 rows 16 us against 25 with 512-row tiles, 43 000 rows 19 against 26; with 118 000 rows, more than one round
     // of 256-row tiles, those take 35 against 30)
     if constexpr (sizeof(T) == 2) {
       const int64_t cus = chipLayout().cus;
       if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
       if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+      // 384-row tiles by the live rows: 196 000 rows, one and a half rounds of 512, two of 384, 52 -> 46 us; 262 000, two
+      // rounds of 512, stay at 60 (64 with 384)
+      if constexpr (CIN * sizeof(T) == 128) return launchPipeByRows<T, CIN, COUT>(a, stream);
     }
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else if constexpr (COUT >= 128) {

@@ -414,6 +414,14 @@ def test_float_output_channels_shared_out(engine, cin, cout):
                  relu=True, cap_extra=n % 50)
 
 
+@pytest.mark.parametrize("n", [70000, 98304, 98305, 140000])
+def test_pipelined_tiles_of_64_channels_by_live_rows(engine, n):
+    """64 -> 64 beyond 256 rows per CU: 384-row tiles while they take a round less (up to 98 304 rows), else 512-row ones, by
+    the live rows of one capacity."""
+    run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), 64, 64, "bfloat16" if n % 2 else "float16", True, relu=True,
+             cap_extra=150001 - n)
+
+
 @pytest.mark.parametrize("levels", [1, 13, 14])
 def test_map_sizes_around_the_scan_forms(engine, levels):
     """Occupancy maps of 50 x 50 bricks per level, on both sides of the 32 768 records at which their scan takes another
