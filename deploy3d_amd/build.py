@@ -107,7 +107,8 @@ def build_engine(verbose=False, incremental=False, jobs=None):
 def build_peaks():
     """The measured-peaks microbenchmark (dense MFMA loop, streaming copy), a standalone program bench.py runs."""
     os.makedirs(LIBS, exist_ok=True)
-    _run([_hipcc(), "--offload-arch=gfx950", "-O3", "-std=c++17", os.path.join(CSRC, "peaks.hip"), "-o", PEAKS_BIN])
+    _run([_hipcc(), "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+          "-packed-fp32-ops", os.path.join(CSRC, "peaks.hip"), "-o", PEAKS_BIN])
     return PEAKS_BIN
 
 
