@@ -91,7 +91,7 @@ struct RbWorkspace {
                           // fixed-shape probe: the output rows alone, packed per (tap, 64 inputs), with
   size_t hits;            // u64 [kVol, hitsPitch] which of the 64 inputs they belong to (block map, strided only)
   uint32_t hitsPitch;
-  size_t offsets;
+  size_t offsets;         // u32 [kVol, offsetPitch] where the pairs of a (tap, block of 512 inputs) go (block map)
   uint32_t offsetPitch;
   size_t ownCnt;          // hash: u32 [kVol, nBlocks] owned outputs per (tap, chunk) (strided only);  block map: chunk totals
   size_t cnt;             // u16 [kVol, cntPitch] valid pairs per (tap, block of 256 or 1024 inputs)
@@ -111,14 +111,15 @@ struct RbSide {
                                         // row, -1 elsewhere; 16-byte aligned; null = not wanted
   int64_t nbrRows = 0;
   unsigned long long* masks = nullptr;  // [nMasks] bit t of masks[r / 64]: some output row of 64r..64r+63 has tap t;
-                                        // written with the table of a SubM rulebook when kVol <= 64 (entries past
-                                        // the rows read 0), see masksWritten
+                                        // written with the table of a SubM rulebook, and of a strided one looked up in
+                                        // its source's map, when kVol <= 64 (entries past the rows read 0), see
+                                        // masksWritten
   int64_t nMasks = 0;
   uint32_t* fillState = nullptr;        // 2 words: end of the used part of the index tensor after the previous
                                         // pass / after this pass
   bool incrementalFill = false;         // the index tensor still holds the previous pass that used this fillState:
                                         // only the slots that pass used and this one does not are set to -1
-  bool masksWritten = false;            // out: this build wrote `masks` (SubM rulebooks with a mirrored table)
+  bool masksWritten = false;            // out: this build wrote `masks`
   bool skipIndex = false;               // nothing reads the index tensor but convolutions that read nbr: where the
                                         // build can write nbr (and masks) without compacting, it leaves the index
                                         // tensor unwritten (numIndex is still written)
