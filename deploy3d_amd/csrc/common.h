@@ -225,7 +225,7 @@ bool convUsesMfma(int32_t dtype, int cin, int cout);
 // output channels qualify), else cin itself; and the kernel that widens rows to it with zero channels.
 int paddedMfmaChannels(int32_t dtype, int cin, int cout);
 // True when the layer's kernel reads rows of `cin` stored channels as they are although its MFMA contracts
-// paddedMfmaChannels() of them (ConvArgs::rowChannels): no widened copy of the input is needed.
+// paddedMfmaChannels() of them (ConvArgs::rowChannels): no widened copy of an input on 16 bytes is needed.
 bool convReadsNarrowRows(int32_t dtype, int kVol, int cin, int cout);
 int32_t launchPadRows(const void* in, int64_t rows, int inBytes, int outBytes, void* out, hipStream_t stream);
 

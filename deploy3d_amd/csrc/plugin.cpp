@@ -848,10 +848,10 @@ struct MMPlugin final : d3d_plugin {
       }
     }
     // Capacities are known here: reserve what enqueue would otherwise have to allocate on first use - the rows of a
-    // narrow layer widened to the MFMA channel count, and the derived table of a node that has no link (or is an
+    // narrow layer widened to the MFMA channel count (also of one whose kernel reads them as stored: an input off 16
+    // bytes is widened, and addresses are not known here), and the derived table of a node that has no link (or is an
     // inverse convolution, whose table is always derived).
-    if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && dev->cinMfma > cin &&
-        !convReadsNarrowRows(dtype, kernelVol, cin, cout)) {
+    if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && dev->cinMfma > cin) {
       if (!widened) widened = std::make_shared<DeviceBuffer>();
       const void* const before = widened->ptr;
       const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * dev->cinMfma * dtypeBytes(dtype));

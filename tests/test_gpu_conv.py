@@ -554,3 +554,52 @@ def test_an_unprepared_node_is_refused_under_capture(engine):
     graph, err = captured(fresh)
     assert err is None
     assert torch.equal(replayed(graph), eager)
+
+
+@pytest.mark.parametrize("cin,dtype", [(5, "int8"), (8, "int8"), (16, "int8"), (5, "float16"), (12, "bfloat16")])
+def test_narrow_rows_off_16_bytes_under_capture(engine, cin, dtype):
+    """Layers whose rows are read as stored widen them instead when the input is a view off 16 bytes.  A node configured from
+    its descriptors, which name no address, has reserved those rows: its first enqueue may be a captured one."""
+    from deploy3d_amd.plugin import Plugin, TensorDesc
+    from deploy3d_amd.spconv_mm import mm_blob, run_mm
+    rng = np.random.default_rng(79)
+    grid, ksize, cout = (10, 36, 30), (3, 3, 3), 16
+    coords = random_cloud(rng, 2000, grid, 1)
+    n = len(coords)
+    rb = gpu_rulebook(coords, n, grid, 1, ksize, (1, 1, 1), (1, 1, 1), (1, 1, 1), n, True)
+    w = (rng.standard_normal((27, cin, cout)) / np.sqrt(27 * cin)).astype(np.float32)
+    scales = {}
+    if dtype == "int8":
+        s_in, s_out = np.float32(0.043), np.float32(0.057)
+        scales = dict(act_scale_in=float(s_in), act_scale_out=float(s_out))
+        feats = rng.integers(-128, 128, (n, cin)).astype(np.int8)
+        w_q, s_w = oracle.quantize_weights(w)
+        ref = oracle.requantize(oracle.conv_i8(feats, w_q, rb["index"], rb["num_index"], n),
+                                *oracle.requant_params(s_in, s_w, s_out, None), False)
+        tdtype = torch.int8
+    else:
+        feats, w = round_to(rng.standard_normal((n, cin)), dtype), round_to(w, dtype)
+        ref = oracle.conv(feats, w, None, rb["index"], rb["num_index"], n, acc="f64")
+        tdtype = TORCH_DTYPE[dtype]
+    store = torch.zeros((n + 1) * cin + 16, dtype=tdtype, device="cuda")
+    at = 1 if (cin * store.element_size()) % 16 == 0 else cin
+    x = store[at:at + n * cin].view(n, cin)
+    assert x.data_ptr() % 16 != 0
+    x.copy_(torch.from_numpy(feats).to(tdtype))
+    out = torch.zeros((n, cout), dtype=tdtype, device="cuda")
+    args = (x, rb["num_act_in"], rb["num_act_in"], rb["dev"][0], rb["dev"][1])
+    plugin = Plugin("SPConvMM", mm_blob(ksize, cin, cout, n, True, False, w, None, **scales))
+    in_descs = [TensorDesc.of_tensor(t) for t in args]
+    plugin.configure(in_descs, plugin.output_descs(in_descs))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run_mm(plugin, *args, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.float().cpu().numpy()
+        if dtype == "int8":
+            np.testing.assert_array_equal(got, ref)
+        else:
+            check_close(got, ref, dtype)
