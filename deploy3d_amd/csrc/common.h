@@ -88,15 +88,16 @@ struct RbWorkspace {
   size_t table;           // hash: u64 [slots] key<<32 | value;  block map: records [nRecords]
   size_t ids;             // hash: u32 [slots] output row of an occupied slot (strided only);  block map: perm [cap] (SubM)
   size_t staging;         // u32 [kVol, pitch] per (tap, input): slot, then output row, or ~0;  strided builds of the
-                          // fixed-shape probe: the output rows alone, packed per (tap, 64 inputs), with
-  size_t hits;            // u64 [kVol, hitsPitch] which of the 64 inputs they belong to (block map, strided only)
-  uint32_t hitsPitch;
-  size_t offsets;         // u32 [kVol, offsetPitch] where the pairs of a (tap, block of 512 inputs) go (block map)
-  uint32_t offsetPitch;
+                          // fixed-shape probe, given `hits`: the output rows alone, packed per (tap, 64 inputs)
   size_t ownCnt;          // hash: u32 [kVol, nBlocks] owned outputs per (tap, chunk) (strided only);  block map: chunk totals
   size_t cnt;             // u16 [kVol, cntPitch] valid pairs per (tap, block of 256 or 1024 inputs)
   size_t totals;          // u32 [2, kVol]  valid pairs per tap; owned outputs per tap
-  size_t total;           // bytes
+  size_t total;           // bytes the build cannot do without; behind them (block map), what makes it faster:
+  size_t hits;            // u64 [kVol, hitsPitch] which of 64 inputs have the tap (strided only)
+  uint32_t hitsPitch;
+  size_t offsets;         // u32 [kVol, offsetPitch] where the pairs of a (tap, block of 512 inputs) go
+  uint32_t offsetPitch;
+  size_t totalWanted;     // bytes with these; a workspace of less than that is used without them
 };
 
 // Plan for the structure that will be used given `workspaceBytes` of workspace.

@@ -2406,21 +2406,22 @@ RbWorkspace planWith(const RbGeom& g, int64_t cap, bool subM, bool blockMap) {
   }
   w.staging = off;
   off = alignUp(off + static_cast<size_t>(g.kVol) * w.pitch * 4);
-  w.hits = off;    // strided builds of the fixed-shape probe: u64 [kVol, hitsPitch], the inputs of 64 that have the tap
-  w.hitsPitch = static_cast<uint32_t>((cap + kProbeThreads - 1) / kProbeThreads * (kProbeThreads / 64));
-  if (blockMap && !subM) off = alignUp(off + static_cast<size_t>(g.kVol) * w.hitsPitch * 8);
   // pairs per (tap, block of inputs): rows of cntPitch words, one per 256 inputs (the fixed-shape probe) or per
   // 1024 (the others, which use the head of each row)
   w.cntPitch = static_cast<uint32_t>(((cap + kRbThreads - 1) / kRbThreads + 7) / 8 * 8);
-  w.offsets = off; // u32 [kVol, offsetPitch] where the pairs of a (tap, block) go
-  w.offsetPitch = static_cast<uint32_t>((cap + 8191) / 8192 * 16);
-  if (blockMap) off = alignUp(off + static_cast<size_t>(g.kVol) * w.offsetPitch * 4);
   w.cnt = off;     // RbCount [kVol, cntPitch], followed (the counters are cleared as one range) by
   off = alignUp(off + static_cast<size_t>(g.kVol) * w.cntPitch * sizeof(RbCount), 16);
   w.totals = off;  // [kVol, kTotalSlots] valid pairs per tap in partial sums, [kVol] owned outputs per tap, "rows not
                    // in rank order" flag, scan ticket, first-level scan tickets
   off = alignUp(off + totalsWords(g.kVol, w.nChunks) * 4);
   w.total = off;
+  w.hits = off;    // strided builds of the fixed-shape probe: u64 [kVol, hitsPitch], the inputs of 64 that have the tap
+  w.hitsPitch = static_cast<uint32_t>((cap + kProbeThreads - 1) / kProbeThreads * (kProbeThreads / 64));
+  if (blockMap && !subM) off = alignUp(off + static_cast<size_t>(g.kVol) * w.hitsPitch * 8);
+  w.offsets = off; // u32 [kVol, offsetPitch] where the pairs of a (tap, block) go
+  w.offsetPitch = static_cast<uint32_t>((cap + 8191) / 8192 * 16);
+  if (blockMap) off = alignUp(off + static_cast<size_t>(g.kVol) * w.offsetPitch * 4);
+  w.totalWanted = off;
   return w;
 }
 
@@ -2471,9 +2472,9 @@ void blockMapBytes(const RbGeom& g, int64_t cap, size_t* records, size_t* chunkB
 
 size_t rulebookWorkspaceBytes(const RbGeom& g, int64_t cap, bool subM, bool gridKnown) {
   // enough for either structure, so the choice at enqueue time is free
-  size_t need = planWith(g, cap, subM, false).total;
+  size_t need = planWith(g, cap, subM, false).totalWanted;
   if (gridKnown && blockMapFits(g)) {
-    const size_t bm = planWith(g, cap, subM, true).total;
+    const size_t bm = planWith(g, cap, subM, true).totalWanted;
     if (bm > need) need = bm;
   }
   return need;
@@ -2588,6 +2589,9 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
   bool needReset = true;                      // a reset pass opens the build
   bool tableProbe = false;                    // the table is written by a probe of the source map (see below)
   bool packed = false;                        // staging holds the pairs alone, packed per 64 inputs
+  // A workspace that lacks the room for them (the fixed scratch array just below its limit) does without the packed staging
+  // and the places of the pairs, which cost 3 % and 0.2 % of it.
+  const bool withPlaces = workspaceBytes >= w.totalWanted;
   auto* const hits = reinterpret_cast<unsigned long long*>(ws + w.hits);
   const PairOffsets offsets{reinterpret_cast<uint32_t*>(ws + w.offsets), w.offsetPitch, numIndex, fillState};
   int cntShift = 8;                           // log2 of the inputs one entry of cnt covers
@@ -2661,7 +2665,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
       }
     }
     // ... and its table comes from that map too, row by row of the output (tableProbe below).
-    tableProbe = gather == 1 && !side.skipIndex && nbrOut && nbrRows == maxNumActOut && nbrRows >= kTableProbeRows;
+    tableProbe = withPlaces && gather == 1 && !side.skipIndex && nbrOut && nbrRows == maxNumActOut && nbrRows >= kTableProbeRows;
     if (tableProbe && side.masks && g.kVol <= 64) {
       masks = side.masks;
       nMasks = side.nMasks;
@@ -2767,7 +2771,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
                      nIndex, fillB, nFillB, quads, outCoors, w.nRecords)
       // (where the compaction scatters into the table packing costs more than the staging rows it saves: 34 -> 44 us for
       // 480 000 unsorted inputs)
-      packed = ksel != 0 && !subM && !skipIndex && !fillB;
+      packed = withPlaces && ksel != 0 && !subM && !skipIndex && !fillB;
       // fixed kernel shapes: K1 threads per input; fill workgroups only for what there is to fill
       const int64_t fillItems = (probeFillIndex ? nIndex : 0) + nFillB;
       uint32_t planeFill = static_cast<uint32_t>((fillItems / 4 + kRbThreads - 1) / kRbThreads);
@@ -2867,7 +2871,7 @@ int32_t launchRulebook(const RbGeom& g, bool subM, const int32_t* coors, const i
                        static_cast<int64_t>(g.kVol) * nbrRows);
   // with the index tensor unwritten only a build that may have to turn ranks into rows needs the whole grid; the
   // others launch the one workgroup that writes numIndex
-  const bool withOffsets = !skipIndex && cntShift == kProbeShift && (tableProbe || cap >= kOffsetRows);
+  const bool withOffsets = withPlaces && !skipIndex && cntShift == kProbeShift && (tableProbe || cap >= kOffsetRows);
   const int64_t compactRun = static_cast<int64_t>(compactThreads(withOffsets) / 64) << cntShift;  // a wavefront per block of counts
   const dim3 allSpans(static_cast<unsigned>((cap + compactRun - 1) / compactRun > 0 ? (cap + compactRun - 1) / compactRun : 1),
                       g.kVol);

@@ -117,6 +117,25 @@ def test_static_scratch_limits(engine):
     assert e.value.status == -1
 
 
+@pytest.mark.parametrize("subm,cap", [(True, 596992), (False, 616448)])
+def test_static_scratch_just_below_its_limit(engine, subm, cap):
+    """Capacities whose rulebook fits the array (staging, map, counts: 67.0 and 66.9 of its 67.1 MB) but not together with what
+    a build uses where there is room for it: the same tensors as with a caller's workspace."""
+    from deploy3d_amd import Plugin
+    from deploy3d_amd.spconv_index import index_blob
+    grid = (12, 96, 96) if subm else (41, 400, 400)
+    coords = random_cloud(np.random.default_rng(76), 30000, grid, 1)
+    max_out = cap if subm else 8 * len(coords)
+    blob = index_blob((3, 3, 3), (1, 1, 1) if subm else (2, 2, 2), (1, 1, 1), (1, 1, 1), (0, 0, 0), max_out, subm, False)
+    want = _index_outputs(Plugin("SPConvIdx3d", blob), coords, cap, grid, None)
+    got = _index_outputs(Plugin("SPConvIdx3d", blob), coords, cap, grid, "static")
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    if not subm:
+        n_out = int(want[3].item())
+        assert int(got[3].item()) == n_out and 0 < n_out <= max_out
+        assert torch.equal(got[2][:n_out], want[2][:n_out])
+
+
 def test_static_enqueue_allocates_nothing(engine):
     """The entry point's promise itself: free device memory is the same before and after static calls (operators made
     and tensors allocated beforehand), also for a strided operator that keeps a map for a linked submanifold
