@@ -227,7 +227,7 @@ bool convUsesMfma(int32_t dtype, int cin, int cout);
 int paddedMfmaChannels(int32_t dtype, int cin, int cout);
 // True when the layer's kernel reads rows of `cin` stored channels as they are although its MFMA contracts
 // paddedMfmaChannels() of them (ConvArgs::rowChannels): no widened copy of an input on 16 bytes is needed.
-bool convReadsNarrowRows(int32_t dtype, int kVol, int cin, int cout);
+bool convReadsNarrowRows(int32_t dtype, int kVol, int cin, int cout, int64_t inRows);
 int32_t launchPadRows(const void* in, int64_t rows, int inBytes, int outBytes, void* out, hipStream_t stream);
 
 // Elementwise steps of a schedule (elementwise.hip): out = a + b for n elements of `dtype` (float, half, bf16; the sum of the

@@ -330,7 +330,7 @@ convMfma(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
 }
 
 // Rows of 64 bytes (fp32 layers of 16 channels, two-byte ones of 32 -> 16), and what conv_taps.h leaves: kernel volumes above 32,
-// rows of 9 to 15 channels, inputs of 3 GB and more.
+// rows of 9 to 15 channels, inputs of 3 GB and more (int8 rows below 16 channels are widened there).
 // Small layers: the weights of ALL taps fit in LDS.  A workgroup loads them once and then lives on: each of
 // its wavefronts walks, on its own, over groups of 16 output rows (group index strided by the number of
 // wavefronts in the grid), with a private slice of the neighbour table, its own list of the taps that occur
@@ -1207,14 +1207,11 @@ int32_t launchInt8Cout(const ConvArgs& a, hipStream_t stream) {
       if (a.cout == 32) return launchInt8Resident<32, 32, 16>(a, stream);
       return D3D_ERR_UNSUPPORTED;
     }
-    if (a.rowChannels > 0 && a.rowChannels <= 8) {
+    if (a.rowChannels > 0) {  // at most eight: convTaps alone
       if (a.cout == 16) rc = launchTaps<int8_t, 0, 16, 16>(a, stream);
       if (a.cout == 32) rc = launchTaps<int8_t, 0, 16, 32>(a, stream);
-      if (rc != D3D_ERR_UNSUPPORTED) return rc;
-      if (a.cout == 16) return launchInt8Resident<32, 16, -1>(a, stream);
-      if (a.cout == 32) return launchInt8Resident<32, 32, -1>(a, stream);
+      return rc;
     }
-    if (a.rowChannels > 0) return D3D_ERR_UNSUPPORTED;
     if (a.staged == 0) {
       if (a.cout == 16) rc = launchTaps<int8_t, 32, 32, 16>(a, stream);
       if (a.cout == 32) rc = launchTaps<int8_t, 32, 32, 32>(a, stream);
@@ -1228,7 +1225,12 @@ int32_t launchInt8Cout(const ConvArgs& a, hipStream_t stream) {
   }
   switch (a.cout) {
     case 16: if constexpr (CIN * 16 >= 1024) return launchStaged<int8_t, CIN, 16>(a, stream); break;
-    case 32: return launchStaged<int8_t, CIN, 32>(a, stream);
+    case 32: {
+      const int32_t rc = launchStaged<int8_t, CIN, 32>(a, stream);
+      if constexpr (CIN == 32)  // rows past its 32-bit offsets, with tile masks
+        if (rc == D3D_ERR_UNSUPPORTED) return launchInt8Resident<32, 32>(a, stream);
+      return rc;
+    }
     case 64: return launchStaged<int8_t, CIN, 64>(a, stream);
     case 128: return launchStaged<int8_t, CIN, 128>(a, stream);
   }

@@ -232,13 +232,14 @@ inline size_t tapsLds(int kVol, int tapBytes, int cout) {
 
 inline bool tapsFit(int kVol, int tapBytes, int cout) { return kVol <= 32 && tapsLds(kVol, tapBytes, cout) <= kLdsLimit; }
 
+// 32-bit row offsets, with room above them for the one of an absent neighbour
+inline bool tapsReach(int64_t rows, uint64_t rowBytes) { return static_cast<uint64_t>(rows) * rowBytes < 0xBFFF0000ull; }
+
 template <class T, int RB, int CB, int COUT, int QC>
 int32_t launchTapsCfg(const ConvArgs& a, hipStream_t stream) {
   constexpr int WAVES = kTapsWaves;
   const size_t lds = tapsLds(a.kVol, CB, COUT);
-  if (!tapsFit(a.kVol, CB, COUT)) return D3D_ERR_UNSUPPORTED;
-  const uint64_t rowBytes = RB ? RB : a.rowChannels * sizeof(T);
-  if (static_cast<uint64_t>(a.inRows) * rowBytes >= 0xBFFF0000ull) return D3D_ERR_UNSUPPORTED;  // 32-bit row offsets
+  if (!tapsFit(a.kVol, CB, COUT) || !tapsReach(a.inRows, RB ? RB : a.rowChannels * sizeof(T))) return D3D_ERR_UNSUPPORTED;
   static std::atomic<size_t> granted{64 * 1024};
   const int32_t rc = grantLds(&convTaps<T, RB, CB, COUT, QC, WAVES>, lds, &granted);
   if (rc != D3D_OK) return rc;

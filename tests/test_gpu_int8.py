@@ -117,6 +117,36 @@ def test_int8_pipelined_and_barrier_per_tap_kernels_agree_with_the_oracle(engine
     run_int8(3001, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, True, False)
 
 
+@pytest.mark.parametrize("cout", [16, 32])
+def test_int8_narrow_rows_of_3_gb(engine, cout):
+    """Rows of 8 channels whose offsets no longer fit the kernel that reads them as stored are widened: three gathers, the
+    last row among them, from 402.7 million rows."""
+    from deploy3d_amd.plugin import Plugin
+    from deploy3d_amd.spconv_mm import mm_blob, run_mm
+    rows, cin, n_out = 3 << 27, 8, 20
+    rng = np.random.default_rng(8)
+    x = torch.zeros((rows, cin), dtype=torch.int8, device="cuda")
+    picks = [rows - 1, 5, (1 << 28) + 77]
+    values = rng.integers(-128, 128, (3, cin)).astype(np.int8)
+    for r, v in zip(picks, values):
+        x[r] = torch.from_numpy(v).cuda()
+    index = np.full((3, 128), -1, np.int32)
+    index[:, :3] = [picks, [0, 17, 9], [0, 0, 0]]
+    w = rng.standard_normal((1, cin, cout)).astype(np.float32)
+    s_in, s_out = np.float32(0.043), np.float32(0.057)
+    w_q, s_w = oracle.quantize_weights(w)
+    acc = np.zeros((n_out, cout), np.int32)
+    acc[[0, 17, 9]] = values.astype(np.int32) @ w_q[0].astype(np.int32)
+    want = oracle.requantize(acc, *oracle.requant_params(s_in, s_w, s_out, None), False)
+    num = torch.tensor([n_out], dtype=torch.int32, device="cuda")
+    plugin = Plugin("SPConvMM", mm_blob((1, 1, 1), cin, cout, n_out, False, False, w, None, act_scale_in=float(s_in),
+                                        act_scale_out=float(s_out)))
+    out = run_mm(plugin, x, num, num, torch.from_numpy(index).cuda(), torch.tensor([128], dtype=torch.int32, device="cuda"))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), want)
+    plugin.close()
+
+
 def test_int8_unsupported_channels_report_status(engine):
     from deploy3d_amd import EngineError
     with pytest.raises(EngineError) as e:
