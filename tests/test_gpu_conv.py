@@ -140,14 +140,20 @@ def test_fp32_layers_no_mfma_takes_are_not_widened(engine):
     16-channel copy of them (256 MB)."""
     from deploy3d_amd import Plugin, TensorDesc
     from deploy3d_amd.spconv_mm import mm_blob
-    rows = 1 << 22
-    op = Plugin("SPConvMM", mm_blob((5, 5, 5), 5, 16, 64, False, False, np.zeros(125 * 5 * 16, np.float32)))
-    ins = [TensorDesc.of((rows, 5), torch.float32), TensorDesc.of((1,), torch.int32), TensorDesc.of((1,), torch.int32),
-           TensorDesc.of((3, 125 * (rows + 128)), torch.int32), TensorDesc.of((1,), torch.int32)]
-    torch.cuda.synchronize()
+
+    def configured(rows):
+        op = Plugin("SPConvMM", mm_blob((5, 5, 5), 5, 16, 64, False, False, np.zeros(125 * 5 * 16, np.float32)))
+        ins = [TensorDesc.of((rows, 5), torch.float32), TensorDesc.of((1,), torch.int32), TensorDesc.of((1,), torch.int32),
+               TensorDesc.of((3, 125 * (rows + 128)), torch.int32), TensorDesc.of((1,), torch.int32)]
+        op.configure(ins, op.output_descs(ins))
+        torch.cuda.synchronize()
+        return op
+
+    small = configured(64)      # what the library loads and allocates once
     before = torch.cuda.mem_get_info()[0]
-    op.configure(ins, op.output_descs(ins))
+    large = configured(1 << 22)
     assert before - torch.cuda.mem_get_info()[0] < 128 << 20
+    small.close(), large.close()
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
