@@ -21,7 +21,6 @@
 // Gathers and index loads are buffer loads: an absent neighbour (-1) or a row past the input produces an
 // out-of-range offset, for which the hardware delivers zeros - no zero row, no select, one VALU per gather.
 #pragma once
-#include <cstdlib>
 #include <cstring>
 #include <type_traits>
 
@@ -32,15 +31,13 @@ namespace convk {
 
 typedef __attribute__((address_space(3))) void* LdsVoidPtr;
 
-// Shapes of two-byte layers of 128 output channels whose workgroups take all of them, rows per wavefront x wavefronts:
-// 0: 32 x 8, 1: 32 x 6, 2: 32 x 4, 3: 48 x 4.  The one that loads the busiest of `cus` CUs least with `rows` rows (rounds of
-// tiles x rows per tile); see launchPipeShape.
-__host__ __device__ inline int pipeShapeOf(int64_t rows, int cus) {
+// Workgroups that take all 128 output channels of their rows, in wavefronts of 32 rows: the tile (256, 192 or 128 rows) that
+// loads the busiest of `cus` CUs least with `rows` rows (rounds of tiles x rows per tile); see launchPipeShape.
+__device__ inline int pipeTileRows(int64_t rows, int cus) {
   auto load = [&](int tile) { return static_cast<int>((rows + static_cast<int64_t>(tile) * cus - 1) / (static_cast<int64_t>(tile) * cus)) * tile; };
   const int l8 = load(256), l6 = load(192), l4 = load(128);
-  int best = l6 < l8 ? 1 : 0;
-  if (l4 < (best ? l6 : l8)) best = 2;
-  return best == 1 && l6 <= 192 ? 3 : best;
+  const int best = l6 < l8 ? 192 : 256;
+  return l4 < (l6 < l8 ? l6 : l8) ? 128 : best;
 }
 
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
@@ -446,8 +443,8 @@ convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf
                                      relu, xcdShift, numActOut, gridDim.x);
 }
 
-// The same with the shape (0, 1 or 2: 48-row wavefronts take 278 registers, which workgroups of eight do not have) chosen by
-// the live rows; the host knows the capacity only.  Wavefronts past the shape's end at once.
+// The same with the tile chosen by the live rows (wavefronts of 32 rows: those of 48 take 278 registers, which workgroups of
+// eight do not have); the host knows the capacity only.  Wavefronts past the tile's end at once.
 template <class T, int CIN, int COUT>
 __global__ void __launch_bounds__(512)
 convPipeByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
@@ -456,15 +453,15 @@ convPipeByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restric
                int xcdShift, const int32_t* __restrict__ numActOut, int cus) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int shape = pipeShapeOf(liveOutRows(numActOut, outRows), cus);
+  const int tile = pipeTileRows(liveOutRows(numActOut, outRows), cus);
 #define D3D_PIPE_BODY(WAVES)                                                                                            \
   {                                                                                                                     \
     if (wave >= WAVES) return;                                                                                          \
     pipeTiles<T, CIN, COUT, 2, WAVES>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol,     \
                                       inRows, outRows, relu, xcdShift, numActOut, gridDim.x);                           \
   }
-  if (shape == 2) D3D_PIPE_BODY(4)
-  else if (shape == 0) D3D_PIPE_BODY(8)
+  if (tile == 128) D3D_PIPE_BODY(4)
+  else if (tile == 256) D3D_PIPE_BODY(8)
   else D3D_PIPE_BODY(6)
 #undef D3D_PIPE_BODY
 }
@@ -599,13 +596,16 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
       // 384-row tiles by the live rows: 196 000 rows, one and a half rounds of 512, two of 384, 52 -> 46 us; 262 000, two
       // rounds of 512, stay at 60 (64 with 384)
-      if constexpr (CIN * sizeof(T) == 128) return launchPipeByRows<T, CIN, COUT>(a, stream);
+      return launchPipeByRows<T, CIN, COUT>(a, stream);
+    } else {
+      return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
     }
-    return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
   } else if constexpr (COUT >= 128) {
     const int64_t cus = chipLayout().cus;
-    const char* const force = debugEnv("D3D_CONV_PIPE_SHAPE");  // "rows,wavefronts" (tests)
-    const int rows = force ? std::atoi(force) : 0, waves = force && std::strchr(force, ',') ? std::atoi(std::strchr(force, ',') + 1) : 0;
+    // D3D_CONV_PIPE_SHAPE=rows,wavefronts (tests): a shape the layer has whatever the rows (rows per wavefront); others, and
+    // what the kernels choose by the live rows, are not forced
+    const char* const env = debugEnv("D3D_CONV_PIPE_SHAPE");
+    auto forced = [&](const char* shape) { return env && std::strcmp(env, shape) == 0; };
     if constexpr (sizeof(T) == 1 || CIN >= 64) {
       // One workgroup of four wavefronts per CU that takes all 128 channels adds the time of its LDS reads (each wavefront
       // reads a step's whole weight slice) to that of its MFMAs: without MFMAs, gathers and weight loads a 24 000-row layer
@@ -615,28 +615,24 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       // 44 / 41 and 30 / 26, 47 500 rows 50.5 / 45 and 32 / 29, 97 000 rows 91 / 75 and 56 / 50, 190 000 rows 134 / 137 and
       // 89 / 90 (its three-tap column layer 33 / 27); int8: 22 / 19.5, 27 / 25, 32 / 27.5, 51 / 44, 89 / 80.  The wider tile
       // wins where it fits as many workgroups to a CU: the lines are whole rounds of one and of two workgroups per CU.
-      if (!force && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);   // 29 -> 18 us
-      if ((!force && (a.outRows <= 64 * cus || (a.outRows > 96 * cus && a.outRows <= 128 * cus))) || (rows == 32 && waves == 4))
+      const bool shared4 = forced("32,4"), shared3 = forced("48,4"), free = !shared4 && !shared3;
+      if (free && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);   // 29 -> 18 us
+      if (shared4 || (free && (a.outRows <= 64 * cus || (a.outRows > 96 * cus && a.outRows <= 128 * cus))))
         return launchPipeCfg<T, CIN, COUT, 2, 4, 64>(a, stream);
       // Past one round of two 192-row workgroups per CU a few of them would have a second tile (55 000 rows: 70 us by the
       // rounds, 53 with 256-row tiles): up to 288 rows per CU the two-byte layers choose by the live rows.  (Six percent of
       // head-room above the line: a capacity is above its live rows.)
-      if (sizeof(T) == 1 || (!force && (a.outRows <= 204 * cus || a.outRows > 288 * cus)) || (rows == 48 && waves == 4))
-        return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
-      if constexpr (sizeof(T) > 1) return launchPipeByRows<T, CIN, COUT>(a, stream);
-      return D3D_ERR_UNSUPPORTED;
+      if constexpr (sizeof(T) > 1)
+        if (free && a.outRows > 204 * cus && a.outRows <= 288 * cus) return launchPipeByRows<T, CIN, COUT>(a, stream);
+      return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
     } else {
-      // 32 -> 128: 8, 6 or 4 wavefronts of 32 rows, or 4 of 48: the workgroup size whose tiles load the busiest CU least
-      // (rounds of tiles over the 256 CUs x rows per tile), by the live rows past one round of the largest
-      if (!force && a.outRows > 256 * cus) return launchPipeByRows<T, CIN, COUT>(a, stream);
-      static const int kCand[4][2] = {{32, 8}, {32, 6}, {32, 4}, {48, 4}};
-      int best = pipeShapeOf(a.outRows, static_cast<int>(cus));
-      for (int c = 0; c < 4; ++c)
-        if (rows == kCand[c][0] && waves == kCand[c][1]) best = c;
-      if (best == 0) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
-      if (best == 1) return launchPipeCfg<T, CIN, COUT, 2, 6>(a, stream);
-      if (best == 2) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
-      return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
+      // 32 -> 128: one round of the smallest tile that has one (128 or 256 rows in wavefronts of 32, 192 in wavefronts of 48);
+      // beyond, the tile that loads the busiest CU least, by the live rows
+      const bool rows128 = forced("32,4"), rows192 = forced("48,4"), rows256 = forced("32,8"), free = !rows128 && !rows192 && !rows256;
+      if (rows128 || (free && a.outRows <= 128 * cus)) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
+      if (rows192 || (free && a.outRows <= 192 * cus)) return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
+      if (rows256 || (free && a.outRows <= 256 * cus)) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+      return launchPipeByRows<T, CIN, COUT>(a, stream);
     }
   } else if constexpr (RB == 64 && COUT == 32) {
     return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);

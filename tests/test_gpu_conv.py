@@ -33,19 +33,22 @@ def check_close(got, ref, dtype):
 
 
 def run_case(n, grid, ksize, stride, padding, cin, cout, dtype, subm, with_bias=True, relu=False, inverse=False,
-             seed=0, cap_extra=0, link=True):
+             seed=0, cap_extra=0, link=True, room=0):
     """link: the convolution is linked to the rulebook operator and reads the table that operator wrote (an inverse
-    convolution never does); otherwise it derives the table from the index tensor, as an unlinked node does."""
+    convolution never does); otherwise it derives the table from the index tensor, as an unlinked node does.
+    cap_extra: input rows past the live ones; room (SubM): input and output rows past the live ones, as in a network (the
+    table comes with tile masks then)."""
     from deploy3d_amd import spconv_mm
     rng = np.random.default_rng(seed + n + cin * 7 + cout)
     coords = random_cloud(rng, n, grid, 1)
     n = len(coords)
     kvol = int(np.prod(ksize))
     dil = (1,) * len(ksize)
-    max_out = n if subm else n * 8
-    rb = gpu_rulebook(coords, n, grid, 1, ksize, stride, padding, dil, max_out, subm, cap=n + cap_extra, link=link)
+    cap = n + cap_extra + room
+    max_out = n + room if subm else n * 8
+    rb = gpu_rulebook(coords, n, grid, 1, ksize, stride, padding, dil, max_out, subm, cap=cap, link=link)
     n_out = n if subm else rb["num_act_out"]
-    in_rows, out_rows = (n + cap_extra, max_out) if not inverse else (max_out, n + cap_extra)
+    in_rows, out_rows = (cap, max_out) if not inverse else (max_out, cap)
     feats = round_to(rng.standard_normal((in_rows, cin)), dtype)
     w = round_to(rng.standard_normal((kvol, cin, cout)) / np.sqrt(kvol * cin), dtype)
     b = round_to(rng.standard_normal(cout), dtype) if with_bias else None
@@ -372,27 +375,30 @@ def test_mfma_tile_sizes(engine, monkeypatch, tile_rows, cin, cout):
     run_case(3001, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, "float16", True, relu=True)
 
 
-@pytest.mark.parametrize("shape", ["32,8", "32,6", "32,4", "48,4"])
-@pytest.mark.parametrize("cin,cout,dtype", [(32, 128, "float16"), (64, 128, "float16"), (128, 128, "float16"),
-                                            (128, 128, "bfloat16")])
-def test_pipelined_tile_shapes_of_wide_layers(engine, monkeypatch, shape, cin, cout, dtype):
-    """The four workgroup shapes (rows per wavefront, wavefronts) the pipelined kernel chooses from for 128 output
-    channels by row count - 48-row wavefronts (three 16-row groups: the register sets alternate across steps) among
-    them - each forced on a SubM layer (tile masks) and a strided one, and once on a layer with more tiles than
-    workgroups, where the pipeline runs across tiles."""
+@pytest.mark.parametrize("cin,cout,dtype,shape",
+                         [(32, 128, "float16", "32,8")] +
+                         [(cin, 128, dtype, shape) for shape in ("32,4", "48,4")
+                          for cin, dtype in ((32, "float16"), (64, "float16"), (128, "float16"), (128, "bfloat16"))])
+def test_pipelined_tile_shapes_of_wide_layers(engine, monkeypatch, cin, cout, dtype, shape):
+    """The workgroup shapes (rows per wavefront, wavefronts) that the host chooses from for 128 output channels by row count -
+    48-row wavefronts (three 16-row groups: the register sets alternate across steps) among them - each forced on a SubM
+    layer with rows past the live ones (tile masks) and a strided one, and once on a layer with more tiles than workgroups,
+    where the pipeline runs across tiles.  Eight wavefronts of 32 rows are the host's choice for 32 -> 128 alone; from 64 input
+    channels on the live rows choose them (the next test)."""
     monkeypatch.setenv("D3D_CONV_PIPE_SHAPE", shape)
-    run_case(9001, (12, 48, 40), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=True, cap_extra=50)
-    if cin == 64:
+    run_case(9001, (12, 48, 40), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=True, room=51)
+    if cin == 64 or shape == "32,8":
         run_case(5000, (12, 48, 40), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False)
         run_case(70000, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, relu=True)
 
 
 @pytest.mark.parametrize("cin,dtype", [(32, "float16"), (64, "bfloat16"), (128, "float16")])
 def test_pipelined_tile_shape_by_live_rows(engine, cin, dtype):
-    """Capacities above 256 rows per CU: the kernel chooses its workgroup shape by the live rows - here one round of 128-row
-    tiles, one of 192, one of 256, and several - and serves the rows past them whatever it chose."""
-    for n in (30000, 45000, 60000, 75000):
-        run_case(n, (16, 128, 128), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, dtype, True, relu=True, cap_extra=76011 - n)
+    """A capacity at which the kernel chooses its tile by the live rows (above 256 rows per CU, from 64 input channels on 204
+    to 288) - here one round of 128-row tiles, one of 192, one of 256, and several - and serves the rows past them whatever it
+    chose."""
+    for n in (30000, 45000, 60000, 72000):
+        run_case(n, (16, 128, 128), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, 128, dtype, True, relu=True, room=73011 - n)
 
 
 @pytest.mark.parametrize("cin,cout", [(32, 64), (64, 64), (64, 128), (128, 128)])
@@ -422,10 +428,10 @@ def test_float_output_channels_shared_out(engine, cin, cout):
 
 @pytest.mark.parametrize("n", [70000, 98304, 98305, 140000])
 def test_pipelined_tiles_of_64_channels_by_live_rows(engine, n):
-    """64 -> 64 beyond 256 rows per CU: 384-row tiles while they take a round less (up to 98 304 rows), else 512-row ones, by
-    the live rows of one capacity."""
+    """64 -> 64 beyond 256 rows per CU, the live rows of one capacity: 384-row tiles where their rounds take clearly less (up to
+    98 304 rows and again at 140 000), else 512-row ones."""
     run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), 64, 64, "bfloat16" if n % 2 else "float16", True, relu=True,
-             cap_extra=150001 - n)
+             room=150001 - n)
 
 
 @pytest.mark.parametrize("levels", [1, 13, 14])
@@ -469,8 +475,14 @@ def test_inverse(engine, subm, dtype):
     run_case(2500, (10, 36, 30), (3, 3, 3), stride, (1, 1, 1), 32, 16, dtype, subm, inverse=True)
 
 
-def test_capacity_rows_beyond_live(engine):
-    run_case(2500, (10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1), 32, 32, "float16", True, cap_extra=777)
+@pytest.mark.parametrize("cin,cout,dtype", [(5, 16, "float16"), (16, 16, "float16"), (32, 32, "float16"), (32, 64, "bfloat16"),
+                                            (64, 64, "float16"), (128, 128, "float16"), (16, 16, "float32"), (64, 64, "float32")])
+def test_capacity_rows_beyond_live(engine, cin, cout, dtype):
+    """Input rows past the live ones, and output rows too (with tile masks), as many as a quarter of the rows and a few tiles."""
+    geometry = ((10, 36, 30), (3, 3, 3), (1, 1, 1), (1, 1, 1))
+    run_case(2500, *geometry, cin, cout, dtype, True, cap_extra=777)
+    for room in (3, 776, 2300):
+        run_case(2500, *geometry, cin, cout, dtype, True, relu=True, room=room)
 
 
 def test_bit_reproducible(engine):
