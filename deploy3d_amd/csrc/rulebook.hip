@@ -35,8 +35,14 @@
 #include "common.h"
 
 namespace d3d {
-// `value` (wavefront-uniform) in lane `lane`, `rest` in the others; the compiler has no builtin for it
+// `value` (wavefront-uniform) in lane `lane`, `rest` in the others.  A compiler without a builtin for it is handed the
+// intrinsic by its name; one that has neither fails to build (there `lane == own ? value : rest` says the same in three vector
+// instructions instead of one).
+#if __has_builtin(__builtin_amdgcn_writelane)
+__device__ __forceinline__ int writeLane(int value, int lane, int rest) { return __builtin_amdgcn_writelane(value, lane, rest); }
+#else
 extern "C" __device__ int writeLane(int value, int lane, int rest) __asm("llvm.amdgcn.writelane.i32");
+#endif
 
 namespace {
 
