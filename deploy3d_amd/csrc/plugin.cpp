@@ -71,7 +71,9 @@ struct DeviceBuffer {
     }
     D3D_HIP_CHECK(hipMalloc(&ptr, n));
     bytes = n;
+    // hipMemset returns before the null stream has done it, and the callers' streams need not wait for that one
     D3D_HIP_CHECK(hipMemset(ptr, 0, n));
+    D3D_HIP_CHECK(hipStreamSynchronize(nullptr));
     return D3D_OK;
   }
   int32_t upload(const void* src, size_t n) {
@@ -690,7 +692,7 @@ const void* zeroRow() {
   std::lock_guard<std::mutex> lock(m);
   if (!buf) {
     auto* b = new DeviceBuffer();
-    if (b->reserve(1024) != D3D_OK || hipMemset(b->ptr, 0, 1024) != hipSuccess) {
+    if (b->reallocZeroed(1024) != D3D_OK) {
       delete b;
       return nullptr;
     }

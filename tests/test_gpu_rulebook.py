@@ -418,6 +418,49 @@ def test_listed_map_across_passes(engine, counts):
     plugin.close()
 
 
+def test_first_pass_beside_work_on_the_null_stream(engine):
+    """What an operator keeps between passes is allocated and zeroed on first use.  With the null stream busy, a first pass on
+    a stream that does not wait for it finds that memory zeroed, and so do the passes behind it: a smaller cloud, whose index
+    tensor is cleared by what the pass before left in the state, and another one."""
+    import torch
+    from deploy3d_amd.plugin import OPT_PERSISTENT_INDEX, Plugin, TensorDesc
+    from deploy3d_amd.spconv_index import index_blob
+    grid, cap = (12, 100, 90), 6000
+    rng = np.random.default_rng(81)
+    args = ((3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1))
+    coords = [random_cloud(rng, n, grid, 1) for n in (6000, 300, 2500)]
+    inputs = [torch.from_numpy(c).cuda() for c in coords]
+    in_descs = [TensorDesc.of((cap, 4), torch.int32), TensorDesc.of((1,), torch.int32), TensorDesc.of((1, 0) + grid, torch.int32)]
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(5000000)       # 50 ms on the null stream
+    with torch.cuda.stream(stream):
+        plugin = Plugin("SPConvIdx3d", index_blob(*args, (0, 0, 0), 8 * cap, False, False))
+        subm = Plugin("SPConvIdx3d", index_blob(args[0], (1, 1, 1), args[2], args[3], (0, 0, 0), 8 * cap, True, False))
+        plugin.set_option(OPT_PERSISTENT_INDEX, 1)
+        subm.link_coords(plugin)
+        out_descs = plugin.output_descs(in_descs)
+        outs = [torch.empty(d.shape(), dtype=torch.int32, device="cuda") for d in out_descs[:4]] + [None]
+        ws = torch.empty(plugin.workspace_size(in_descs, out_descs), dtype=torch.uint8, device="cuda")
+        coors = torch.zeros((cap, 4), dtype=torch.int32, device="cuda")
+        num = torch.zeros(1, dtype=torch.int32, device="cuda")
+        for c, rows in zip(inputs, coords):
+            coors[:len(c)].copy_(c)
+            num.fill_(len(c))
+            plugin.enqueue(in_descs, out_descs, [coors, num, None], outs, ws)
+            stream.synchronize()
+            ref = oracle.rulebook(coors.cpu().numpy(), len(c), [1] + list(out_descs[4].shape()[2:]), *args, 8 * cap, False)
+            index, ni = outs[0].cpu().numpy(), int(outs[1].item())
+            assert ni == ref["num_index"] and (index[:, ni:] == -1).all()
+            got = oracle.canonical(index, ni, outs[2].cpu().numpy(), int(outs[3].item()))
+            want = oracle.canonical(ref["index"], ref["num_index"], ref["out_coors"], ref["num_act_out"])
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a, b)
+    torch.cuda.synchronize()
+    subm.link_coords(None)
+    plugin.close(), subm.close()
+
+
 def test_configured_operator_captures_without_an_eager_pass(engine):
     """An operator that keeps its occupancy map between passes (persistent index tensor) reserves its two maps at
     configure: captured in a graph without ever having been enqueued eagerly, every replay - the maps take turns
