@@ -728,11 +728,19 @@ int stagedOverride() {
 constexpr uint32_t kExtMagic = 0x58443344u;  // "D3DX"
 constexpr size_t kMMHeader = 19;
 
+// The weights on the device, converted for each feature type that was asked for: written once and never again, since kernels
+// in flight and captured graphs of another type go on reading theirs.
 struct MMDeviceWeights {
-  int32_t dtype = -1;
-  std::atomic<uint64_t> changes{0};  // uploads so far
-  int cinMfma = 0;  // input channels of the packed MFMA weights (cin widened with zero rows), 0 = no MFMA copy
-  DeviceBuffer f32, mfma, bias, requantM;  // int8: bias holds bias / s_out, requantM holds s_in * s_w[c] / s_out
+  struct Converted {
+    std::atomic<bool> ready{false};
+    int cinMfma = 0;  // input channels of the packed MFMA weights (cin widened with zero rows), 0 = no MFMA copy
+    DeviceBuffer f32, mfma, bias, requantM;  // int8: bias holds bias / s_out, requantM holds s_in * s_w[c] / s_out
+  };
+  std::atomic<uint64_t> changes{0};  // conversions so far
+  Converted& of(int32_t dtype) { return types[dtype == D3D_FLOAT ? 0 : dtype == D3D_HALF ? 1 : dtype == D3D_BF16 ? 2 : 3]; }
+
+ private:
+  Converted types[4];
 };
 
 struct MMPlugin final : d3d_plugin {
@@ -841,22 +849,24 @@ struct MMPlugin final : d3d_plugin {
       setError("SPConvMM: feature dtype %d not implemented", dtype);
       return D3D_ERR_UNSUPPORTED;
     }
+    MMDeviceWeights::Converted& weights = dev->of(dtype);
     {
       std::lock_guard<std::mutex> lock(*devMutex);
-      if (dev->dtype != dtype) {
+      if (!weights.ready) {
         ++dev->changes;
-        const int32_t rc = dtype == D3D_INT8 ? configureInt8() : configureFloat(dtype);
+        const int32_t rc = dtype == D3D_INT8 ? configureInt8(weights) : configureFloat(dtype, weights);
         if (rc != D3D_OK) return rc;
+        weights.ready = true;
       }
     }
     // Capacities are known here: reserve what enqueue would otherwise have to allocate on first use - the rows of a
     // narrow layer widened to the MFMA channel count (also of one whose kernel reads them as stored: an input off 16
     // bytes is widened, and addresses are not known here), and the derived table of a node that has no link (or is an
     // inverse convolution, whose table is always derived).
-    if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && dev->cinMfma > cin) {
+    if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && weights.cinMfma > cin) {
       if (!widened) widened = std::make_shared<DeviceBuffer>();
       const void* const before = widened->ptr;
-      const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * dev->cinMfma * dtypeBytes(dtype));
+      const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * weights.cinMfma * dtypeBytes(dtype));
       if (widened->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
@@ -870,7 +880,7 @@ struct MMPlugin final : d3d_plugin {
     return D3D_OK;
   }
 
-  int32_t configureFloat(int32_t dtype) {
+  int32_t configureFloat(int32_t dtype, MMDeviceWeights::Converted& to) {
     const size_t nW = static_cast<size_t>(kernelVol) * cin * cout;
     std::vector<float> w(nW), b(withBias ? cout : 0);
     std::memcpy(w.data(), blob.data() + weightOffset, nW * 4);
@@ -909,29 +919,28 @@ struct MMPlugin final : d3d_plugin {
       uint32_t bits;
       v = rnd(v, &bits);
     }
-    int32_t rc = dev->f32.upload(w.data(), nW * 4);
+    int32_t rc = to.f32.upload(w.data(), nW * 4);
     if (rc != D3D_OK) return rc;
     if (!packed.empty()) {
-      rc = dev->mfma.upload(packed.data(), packed.size());
+      rc = to.mfma.upload(packed.data(), packed.size());
       if (rc != D3D_OK) return rc;
     }
     if (withBias) {
-      rc = dev->bias.upload(b.data(), b.size() * 4);
+      rc = to.bias.upload(b.data(), b.size() * 4);
       if (rc != D3D_OK) return rc;
     }
     if (!zeroRow()) {
       setError("SPConvMM: could not allocate the zero row");
       return D3D_ERR_DEVICE;
     }
-    dev->cinMfma = mfma ? cinP : 0;
-    dev->dtype = dtype;
+    to.cinMfma = mfma ? cinP : 0;
     return D3D_OK;
   }
 
   // int8 (no counterpart in the reference): symmetric per-output-channel weights, s_w[c] = max|W[:,:,c]| / 127,
   // q = clamp(rint(w / s_w)); the epilogue computes clamp(rint(float(acc) * m[c] + bq[c])) with
   // m[c] = float(s_in * s_w[c] / s_out) and bq[c] = float(bias[c] / s_out), all three quotients in double.
-  int32_t configureInt8() {
+  int32_t configureInt8(MMDeviceWeights::Converted& to) {
     if (!(actScaleIn > 0.f) || !(actScaleOut > 0.f)) {
       setError("SPConvMM: int8 needs positive activation scales in the extension record");
       return D3D_ERR_UNSUPPORTED;
@@ -970,16 +979,15 @@ struct MMPlugin final : d3d_plugin {
           const size_t dst = (((static_cast<size_t>(k) * kkN + kk) * nt + co / 16) * 64 + lane) * kg + j;
           packed[dst] = static_cast<int8_t>(q);
         }
-    int32_t rc = dev->mfma.upload(packed.data(), packed.size());
-    if (rc == D3D_OK) rc = dev->requantM.upload(m.data(), m.size() * 4);
-    if (rc == D3D_OK) rc = dev->bias.upload(bq.data(), bq.size() * 4);
+    int32_t rc = to.mfma.upload(packed.data(), packed.size());
+    if (rc == D3D_OK) rc = to.requantM.upload(m.data(), m.size() * 4);
+    if (rc == D3D_OK) rc = to.bias.upload(bq.data(), bq.size() * 4);
     if (rc != D3D_OK) return rc;
     if (!zeroRow()) {
       setError("SPConvMM: could not allocate the zero row");
       return D3D_ERR_DEVICE;
     }
-    dev->cinMfma = cinP;
-    dev->dtype = D3D_INT8;
+    to.cinMfma = cinP;
     return D3D_OK;
   }
 
@@ -1005,7 +1013,8 @@ struct MMPlugin final : d3d_plugin {
       setError("SPConvMM: expected inFeats [*, %d], index [3, *], outFeats [*, %d]", cin, cout);
       return D3D_ERR_BAD_ARG;
     }
-    if (dev->dtype != dtype) {  // a plugin enqueued without configurePlugin, or with another dtype
+    const MMDeviceWeights::Converted& weights = dev->of(dtype);
+    if (!weights.ready) {  // a plugin enqueued without configurePlugin, or with another dtype
       if (streamIsCapturing(stream)) {  // converting and uploading the weights allocates and synchronises
         setError("SPConvMM: the node was not configured for this feature type before the capture (call "
                  "d3d_configure, or enqueue it once, first)");
@@ -1071,16 +1080,16 @@ struct MMPlugin final : d3d_plugin {
     a.inNarrow = inputs[0];
     a.cinNarrow = cin;
     a.staged = stagedOverride();
-    if (dev->cinMfma > cin && a.staged == 0 && convReadsNarrowRows(dtype, kernelVol, cin, cout, a.inRows) &&
+    if (weights.cinMfma > cin && a.staged == 0 && convReadsNarrowRows(dtype, kernelVol, cin, cout, a.inRows) &&
         ((reinterpret_cast<uintptr_t>(inputs[0]) | reinterpret_cast<uintptr_t>(outputs[0])) & 15) == 0 &&
         (dtype == D3D_INT8 || debugEnv("D3D_CONV_NO_PAD") == nullptr) && tileRowsOverride() == 0) {
-      a.cin = dev->cinMfma;       // the kernel reads the rows as they are and multiplies zeros for the rest
+      a.cin = weights.cinMfma;       // the kernel reads the rows as they are and multiplies zeros for the rest
       a.rowChannels = cin;
-    } else if (dev->cinMfma > cin && (dtype == D3D_INT8 || ((reinterpret_cast<uintptr_t>(outputs[0]) & 15) == 0 &&
+    } else if (weights.cinMfma > cin && (dtype == D3D_INT8 || ((reinterpret_cast<uintptr_t>(outputs[0]) & 15) == 0 &&
                                                      debugEnv("D3D_CONV_NO_PAD") == nullptr))) {  // narrow layer: widen the rows, then MFMA
       if (!widened) widened = std::make_shared<DeviceBuffer>();
       const int es = dtypeBytes(dtype);
-      const size_t wideBytes = static_cast<size_t>(a.inRows > 0 ? a.inRows : 1) * dev->cinMfma * es;
+      const size_t wideBytes = static_cast<size_t>(a.inRows > 0 ? a.inRows : 1) * weights.cinMfma * es;
       if (widened->bytes < wideBytes && streamIsCapturing(stream)) {
         setError("SPConvMM: %zu bytes for the widened input rows were not reserved before the capture", wideBytes);
         return D3D_ERR_UNSUPPORTED;
@@ -1088,16 +1097,16 @@ struct MMPlugin final : d3d_plugin {
       if (widened->bytes < wideBytes) ++changes;
       rc = widened->reserve(wideBytes);
       if (rc != D3D_OK) return rc;
-      rc = launchPadRows(inputs[0], a.inRows, cin * es, dev->cinMfma * es, widened->ptr, stream);
+      rc = launchPadRows(inputs[0], a.inRows, cin * es, weights.cinMfma * es, widened->ptr, stream);
       if (rc != D3D_OK) return rc;
       a.in = widened->ptr;
-      a.cin = dev->cinMfma;
+      a.cin = weights.cinMfma;
     }
     a.out = outputs[0];
-    a.weightsF32 = static_cast<const float*>(dev->f32.ptr);
-    a.weightsMfma = dev->cinMfma > 0 ? dev->mfma.ptr : nullptr;
-    a.bias = (withBias || dtype == D3D_INT8) ? static_cast<const float*>(dev->bias.ptr) : nullptr;
-    a.requantM = dtype == D3D_INT8 ? static_cast<const float*>(dev->requantM.ptr) : nullptr;
+    a.weightsF32 = static_cast<const float*>(weights.f32.ptr);
+    a.weightsMfma = weights.cinMfma > 0 ? weights.mfma.ptr : nullptr;
+    a.bias = (withBias || dtype == D3D_INT8) ? static_cast<const float*>(weights.bias.ptr) : nullptr;
+    a.requantM = dtype == D3D_INT8 ? static_cast<const float*>(weights.requantM.ptr) : nullptr;
     a.nbr = nbr;
     a.tileMasks = masks;
     a.numActOut = static_cast<const int32_t*>(inputs[2]);

@@ -110,7 +110,8 @@ int32_t d3d_supports_format(const d3d_plugin* p, int32_t pos, const d3d_tensor_d
                             int32_t nb_out);
 
 /* configurePlugin (mm_trt.cu:127-142): converts the fp32 weights of the blob to
- * the feature dtype of in[0] and uploads them (synchronous, default stream). */
+ * the feature dtype of in[0] and uploads them (synchronous, default stream), once for each dtype: launches and captured
+ * graphs of another dtype keep theirs. */
 int32_t d3d_configure(d3d_plugin* p, const d3d_tensor_desc* in, int32_t nb_in, const d3d_tensor_desc* out,
                       int32_t nb_out);
 

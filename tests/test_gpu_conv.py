@@ -621,3 +621,34 @@ def test_narrow_rows_off_16_bytes_under_capture(engine, cin, dtype):
             np.testing.assert_array_equal(got, ref)
         else:
             check_close(got, ref, dtype)
+
+
+def test_a_captured_layer_keeps_its_weights_when_another_type_is_run(engine):
+    """The weights are converted once for each feature type: a graph captured with fp16 features replays with the fp16 weights
+    after the same node has run bf16 and fp32 features, and each type gives its own result whatever ran before."""
+    from deploy3d_amd.plugin import Plugin
+    from deploy3d_amd.spconv_mm import mm_blob, run_mm
+    rng = np.random.default_rng(80)
+    grid, ksize, c = (10, 36, 30), (3, 3, 3), 64
+    coords = random_cloud(rng, 2000, grid, 1)
+    n = len(coords)
+    rb = gpu_rulebook(coords, n, grid, 1, ksize, (1, 1, 1), (1, 1, 1), (1, 1, 1), n, True)
+    w, b = rng.standard_normal((27, c, c)) / np.sqrt(27 * c), rng.standard_normal(c)
+    feats = rng.standard_normal((n, c))
+    plugin = Plugin("SPConvMM", mm_blob(ksize, c, c, n, True, False, w, b))
+    clone = plugin.clone()      # shares the weights
+    x = {t: torch.from_numpy(round_to(feats, t)).to(device="cuda", dtype=TORCH_DTYPE[t]) for t in TORCH_DTYPE}
+    ref = {t: oracle.conv(x[t].float().cpu().numpy(), round_to(w, t), round_to(b, t), rb["index"], rb["num_index"], n, acc="f64")
+           for t in TORCH_DTYPE}
+    rest = (rb["num_act_in"], rb["num_act_in"], rb["dev"][0], rb["dev"][1])
+    run_mm(plugin, x["float16"], *rest)
+    out = torch.empty((n, c), dtype=torch.float16, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run_mm(plugin, x["float16"], *rest, out=out)
+    for t in ("float16", "bfloat16", "float32", "float16"):
+        check_close(run_mm(clone if t == "bfloat16" else plugin, x[t], *rest).float().cpu().numpy(), ref[t], t)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check_close(out.float().cpu().numpy(), ref["float16"], "float16")
