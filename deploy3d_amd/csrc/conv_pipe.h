@@ -579,10 +579,10 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     // the vector kernel); skipping a 16-row group's MFMAs when none of its rows has the tap gained 15-20 us on strided and
     // inverse layers and cost as much on the dense ones: the barrier waits for the fullest group either way
     // Layers of 64 and 128 output channels share a tile's channels out to workgroups of 32: with the matrix pipe as the bound
-    // a layer's time goes by the workgroups of the fullest CU, and smaller ones spread more evenly (64 -> 64, 144 000 rows,
-    // 4.4 tiles of all channels to a CU: 264 -> 254 us, 10 000-voxel encoder-decoder 110 -> 90, 32 -> 64 there 60 -> 51, a
-    // VoxelNet's from 30 000 voxels 114 -> 119 and 214 -> 214; 128 -> 128, 47 000 rows, 70 of 100 CUs with a tile of all
-    // channels: 413 -> 289, 16 500 rows 412 -> 172)
+    // a layer's time goes by the workgroups of the fullest CU, and smaller ones spread more evenly.  us with all channels /
+    // shared out: 64 -> 64, 30 000 rows 64 / 61, 118 000 212 / 203, 144 000 (4.4 tiles of all channels to a CU) 260 / 238,
+    // 261 000 402 / 398; 32 -> 64, 262 000 rows 208 / 207; 128 -> 128, 17 000 rows 409 / 163, 40 000 (a 256-row tile of all channels on
+    // 156 of 256 CUs) 409 / 274, 47 500 410 / 324
     if constexpr (COUT >= 64 && CIN >= 32) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);
     else if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
     else return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
@@ -611,17 +611,23 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       // reads a step's whole weight slice) to that of its MFMAs: without MFMAs, gathers and weight loads a 24 000-row layer
       // still took 21 of 34 us.  So a tile's channels are shared out to workgroups of 64 (with few rows, 32): two workgroups
       // of half the slices fit a CU and each computes while the other reads.  us of 128 -> 128 and of 64 -> 128 with all
-      // channels / shared out, fp16: 10 500 rows 30 / 23 and 21 / 16, 24 500 rows 34.5 / 29.5 and 24 / 19, 38 000 rows
-      // 44 / 41 and 30 / 26, 47 500 rows 50.5 / 45 and 32 / 29, 97 000 rows 91 / 75 and 56 / 50, 190 000 rows 134 / 137 and
-      // 89 / 90 (its three-tap column layer 33 / 27); int8: 22 / 19.5, 27 / 25, 32 / 27.5, 51 / 44, 89 / 80.  The wider tile
-      // wins where it fits as many workgroups to a CU: the lines are whole rounds of one and of two workgroups per CU.
+      // channels / shared out, fp16: 11 000 rows 33 / 22 and 22 / 15, 17 500 rows 31 / 25.5 and 20 / 17, 23 500 rows 32 / 27
+      // and 23 / 18, 40 000 rows 42 / 41 and 29.5 / 26, 47 500 rows 44 / 43.5 and 29 / 28, 95 000 rows 87 / 73 and 54.5 / 48,
+      // 188 000 rows 127 / 134 and 87 / 85.5 (the three-tap column layer behind it 32 / 26); int8: 22.5 / 16 and 17 / 13.5, 21 / 17
+      // and 15 / 13.5, 21 / 18 and 18 / 14, 26 / 24.5 and 21.5 / 18.5, 27.5 / 25.5 and 20 / 20, 50 / 42 and 28.5 / 34, 87 / 79 and
+      // 51 / 57.  From 188 000 rows on 128 -> 128 gives back 5 % in two-byte types, and 64 -> 128 a tenth in int8: over the layers
+      // of a network (two of the one, one of the other and a column layer) as much is won, so no further line is drawn.
+      // The wider tile wins where it fits as many workgroups to a CU: the lines are whole rounds of one and of two per CU.
       const bool shared4 = forced("32,4"), shared3 = forced("48,4"), free = !shared4 && !shared3;
       if (free && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);   // 29 -> 18 us
       if (shared4 || (free && (a.outRows <= 64 * cus || (a.outRows > 96 * cus && a.outRows <= 128 * cus))))
         return launchPipeCfg<T, CIN, COUT, 2, 4, 64>(a, stream);
-      // Past one round of two 192-row workgroups per CU a few of them would have a second tile (55 000 rows: 70 us by the
-      // rounds, 53 with 256-row tiles): up to 288 rows per CU the two-byte layers choose by the live rows.  (Six percent of
-      // head-room above the line: a capacity is above its live rows.)
+      // Past one round of two 192-row workgroups per CU (49 152 rows) a few of them have a second tile, 50 000 live rows take
+      // 61 us, 55 000 70, where 256-row tiles of all channels take 52 and 53: up to 288 rows per CU the two-byte layers choose
+      // by the live rows.  The line is drawn at the capacity, six percent above the round, since a capacity is above its live
+      // rows, and that suits one head-room: 47 500 live rows take 44 us under the line and 51 above it (capacities of 1.25 and
+      // 1.5 times, where the shared-out tile would take 45), 50 000 live rows below the line take the 61.  The kernel that
+      // chooses on the device does not hold the shared-out shape.
       if constexpr (sizeof(T) > 1)
         if (free && a.outRows > 204 * cus && a.outRows <= 288 * cus) return launchPipeByRows<T, CIN, COUT>(a, stream);
       return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
