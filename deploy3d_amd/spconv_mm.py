@@ -86,6 +86,10 @@ def spconv_mm(in_feats, num_act_in, num_act_out, index, num_index, kernel_size, 
     ``rulebook``, the SPConvIdx operator instance that wrote ``index`` (``spconv_index.index_plugin``): the
     convolution is linked to it and reads the neighbour table that operator wrote instead of deriving one from the
     index tensor (which is what happens without it, and for any tensor that operator did not write last).
+
+    Calls with the same attributes and weights run one operator instance, which keeps that table: they are to run in order
+    (one stream, or streams that wait for each other; one thread at a time).  Passes that overlap take ``run_mm`` with clones
+    of the instance.
     """
     size = int(kernel_size) if np.isscalar(kernel_size) else tuple(kernel_size)
     plugin = _plugin_of((size, int(in_channels), int(out_channels), int(max_num_act_out), bool(subm), bool(inverse),

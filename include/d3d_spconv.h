@@ -120,7 +120,8 @@ size_t d3d_workspace_size(const d3d_plugin* p, const d3d_tensor_desc* in, int32_
                           int32_t nb_out);
 
 /* enqueue (index_trt.cu:188-248, mm_trt.cu:149-205).  `stream` is a hipStream_t.
- * Stream-ordered, no host synchronisation: live counts are read on the device.
+ * Stream-ordered, no host synchronisation: live counts are read on the device.  A handle's enqueues run in order (one
+ * stream, or streams that wait for each other): what it derives and keeps is its own.
  *
  * SPConvIdx{N}d  inputs : 0 inCoors int32 [cap, N+1] (b, spatial...), 1 numActIn int32 [1],
  *                         2 inSpatialShape (dims [B, 0, spatial...] only; pointer unused)
