@@ -685,20 +685,25 @@ struct IdxPlugin final : d3d_plugin {
   }
 };
 
-// One zero-filled device row shared by every convolution: the source of gathers for absent neighbours.
+// One zero-filled row on each device, shared by the device's convolutions: the source of gathers for absent neighbours.  (A
+// row of another device would be no memory of the kernel's own.)
 const void* zeroRow() {
+  constexpr int kMaxDevices = 64;
   static std::mutex m;
-  static DeviceBuffer* buf = nullptr;  // lives until the process ends
+  static DeviceBuffer* rows[kMaxDevices] = {};  // live until the process ends
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lock(m);
-  if (!buf) {
+  DeviceBuffer*& row = rows[device];
+  if (!row) {
     auto* b = new DeviceBuffer();
     if (b->reallocZeroed(1024) != D3D_OK) {
       delete b;
       return nullptr;
     }
-    buf = b;
+    row = b;
   }
-  return buf->ptr;
+  return row->ptr;
 }
 
 // Tuning / test hook: D3D_CONV_TILE_ROWS = rows per workgroup of the weight-streaming MFMA convolution
