@@ -40,9 +40,99 @@ __device__ inline int pipeTileRows(int64_t rows, int cus) {
   return l4 < (l6 < l8 ? l6 : l8) ? 128 : best;
 }
 
+// The tiles one of `per` workgroups of an XCD takes, in order.  A tile's time goes by the taps its rows have (27, or 18 and 9
+// in the outer levels of a scene), and a layer ends with its busiest workgroup.  Where workgroups take several tiles and masks
+// say what those hold, the tiles of an XCD are ranked by their taps, most first, and dealt back and forth: one with a heavy
+// tile gets a light one with it.  XCDs take runs of CHUNK tiles in turn instead of a contiguous eighth each, which could be
+// all heavy: levels of a scene are contiguous.  Each wavefront ranks for itself, 64 tiles to a register, and keeps its
+// workgroup's list in the lanes of one register.
+// Otherwise (no masks, at most ROUNDS tiles each or more than a list holds) XCD x takes the x-th contiguous part (TileOrder).
+// fp32 layers, bound by the matrix pipe, are dealt from the second tile on: steps of the busiest workgroup / of the average
+// one 153 / 110 contiguous and 120 / 110 dealt for 64 -> 64 with 260 000 rows, 407 -> 344 us; 118 000 rows 208 -> 174.  The
+// other types gain from the fifth tile on (64 -> 64, 1.04 million rows, 216 / 174 -> 180 / 174 steps: fp16 232 -> 217 us, int8
+// 123 -> 114) and not before: with two tiles each (260 000 rows, 54 / 44 -> 45 / 44) the part runs at a lower clock when no CU
+// is idle, the XCDs read 20 % more lines from each other's parts, and it was 58.7 against 59.2 us alone and 25 us of 630 lost
+// in a pass whose rulebooks had run on the CUs that finished early.
+constexpr int kDealRounds = 4;
+template <int PER, int CHUNK, int ROUNDS>                // ROUNDS = 0: never dealt
+struct TileDeal {
+  static constexpr int SLOTS = 4;                        // registers of tiles ranked together
+  TileOrder order;
+  int first, per, mine, list;                            // list: lane p holds the p-th of `mine` dealt tiles
+  bool dealt;
+  __device__ __forceinline__ TileDeal(int tiles, int live, int xcdShift, int xcd, int first_, int per_,
+                                      const unsigned long long* __restrict__ tileMasks, int kVol, unsigned long long allTaps, int lane)
+      : order(tiles, live, xcdShift, xcd), first(first_), per(per_), mine(0), list(0), dealt(false) {
+    if constexpr (ROUNDS > 0) deal(xcdShift, xcd, tileMasks, kVol, allTaps, lane);
+  }
+  __device__ __forceinline__ void deal(int xcdShift, int xcd, const unsigned long long* __restrict__ tileMasks, int kVol,
+                                       unsigned long long allTaps, int lane) {
+    const int live = order.liveTiles, wgs = per << xcdShift;
+    if (!tileMasks || live <= ROUNDS * wgs || live > 32 * wgs || per > 192) return;
+    dealt = true;
+    const int chunks = (live + CHUNK - 1) / CHUNK;
+    int lx = ((chunks - xcd + order.nXcd - 1) >> xcdShift) * CHUNK;   // chunks xcd, xcd + nXcd, ...; the last one may be short
+    if (((chunks - 1) & (order.nXcd - 1)) == xcd) lx -= chunks * CHUNK - live;
+    if (lx < 0) lx = 0;
+    for (int from = 0; from < lx; from += 64 * SLOTS) {
+      int taps[SLOTS], at[SLOTS], rank[SLOTS];
+#pragma unroll
+      for (int s = 0; s < SLOTS; ++s) {
+        const int local = from + s * 64 + lane;
+        at[s] = ((local / CHUNK << xcdShift) + xcd) * CHUNK + local % CHUNK;
+        taps[s] = -1;
+        rank[s] = 0;
+        if (local < lx) {
+          unsigned long long m = 0;
+#pragma unroll
+          for (int e = 0; e < PER; ++e) m |= tileMasks[static_cast<int64_t>(at[s]) * PER + e];
+          taps[s] = __builtin_popcountll(m & allTaps);
+        }
+      }
+      int base = 0;
+      for (int c = kVol; c >= 0; --c) {
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+          const unsigned long long b = __ballot(taps[s] == c);
+          if (b) {
+            const int before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(b >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(b), 0u));
+            if (taps[s] == c) rank[s] = base + before;
+            base += __builtin_popcountll(b);
+          }
+        }
+      }
+      const int had = mine;
+#pragma unroll
+      for (int s = 0; s < SLOTS; ++s) {
+        const int round = rank[s] / per, place = rank[s] - round * per;
+        unsigned long long b = __ballot(taps[s] >= 0 && place == (round & 1 ? per - 1 - first : first));
+        for (; b; b &= b - 1) {
+          const int l = __builtin_ctzll(b);
+          const int pos = had + __builtin_amdgcn_readlane(round, l), t = __builtin_amdgcn_readlane(at[s], l);
+          if (lane == pos) list = t;
+          ++mine;
+        }
+      }
+    }
+    mine = __builtin_amdgcn_readfirstlane(mine);
+  }
+  // tiles of this workgroup: the live ones, then its share of those past the live rows
+  __device__ __forceinline__ int count() const {
+    if constexpr (ROUNDS == 0) return first < order.count() ? (order.count() - 1 - first) / per + 1 : 0;
+    const int n = dealt ? order.dx : order.count();
+    return mine + (first < n ? (n - 1 - first) / per + 1 : 0);
+  }
+  __device__ __forceinline__ bool live(int pos) const { return ROUNDS > 0 && dealt ? pos < mine : order.live(first + pos * per); }
+  __device__ __forceinline__ int tile(int pos) const {
+    if (ROUNDS == 0 || !dealt) return order.tile(first + pos * per);
+    if (pos < mine) return __builtin_amdgcn_readlane(list, pos);
+    return order.liveTiles + (first + (pos - mine) * per) * order.nXcd + order.xcd;
+  }
+};
+
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
 // ceil(outRows / 64) (a workgroup reads the masks of a whole tile at once); null = every tap of every tile.
-template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false>
 __device__ __forceinline__ void
 pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
           const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch,
@@ -101,21 +191,19 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     idxRow[i] = static_cast<uint32_t>(wave * WM + (p % GL) * RPI + p / GL);
   }
 
-  // ---- this workgroup's tiles: XCD x serves the x-th contiguous part of the tiles that hold live rows
-  // (neighbouring tiles gather many of the same rows: they should meet behind one L2) and its share of the tiles
-  // past the live rows; inside an XCD, workgroups take tiles round robin ----
-  const TileOrder order(static_cast<int>((outRows + TM - 1) / TM), static_cast<int>((liveOutRows(numActOut, outRows) + TM - 1) / TM), xcdShift,
-                        blockIdx.x & ((1 << xcdShift) - 1));
-  const int firstLocal = (blockIdx.x >> xcdShift) / COLS, strideLocal = (blocks >> xcdShift) / COLS;
+  // ---- this workgroup's tiles (TileDeal) ----
   const int part = (blockIdx.x >> xcdShift) % COLS;      // which CO of the output channels
-  const int nMine = firstLocal < order.count() ? (order.count() - 1 - firstLocal) / strideLocal + 1 : 0;
-  if (nMine <= 0) return;                                // workgroup-uniform
-  auto tileAt = [&](int pos) __attribute__((always_inline)) { return order.tile(firstLocal + pos * strideLocal); };
   const unsigned long long allTaps = kVol >= 64 ? ~0ull : ((1ull << kVol) - 1ull);
+  const TileDeal<PER, (TM < 2048 ? 2048 / TM : 1), DEAL ? (ES == 4 ? 1 : kDealRounds) : 0> deal(
+      static_cast<int>((outRows + TM - 1) / TM), static_cast<int>((liveOutRows(numActOut, outRows) + TM - 1) / TM), xcdShift,
+      blockIdx.x & ((1 << xcdShift) - 1), (blockIdx.x >> xcdShift) / COLS, (blocks >> xcdShift) / COLS, tileMasks, kVol, allTaps, lane);
+  const int nMine = deal.count();
+  if (nMine <= 0) return;                                // workgroup-uniform
+  auto tileAt = [&](int pos) __attribute__((always_inline)) { return deal.tile(pos); };
   // taps of the workgroup's pos-th tile; a tile without any tap still takes one step (tap 0: all rows absent)
   auto maskAt = [&](int pos) __attribute__((always_inline)) -> unsigned long long {
     if (pos >= nMine) return 0ull;
-    if (!order.live(firstLocal + pos * strideLocal)) return 1ull;   // no live row: one step of absent neighbours
+    if (!deal.live(pos)) return 1ull;                    // no live row: one step of absent neighbours
     unsigned long long m = allTaps;
     if (tileMasks) {
       const unsigned long long* p = tileMasks + static_cast<int64_t>(tileAt(pos)) * PER;
@@ -432,14 +520,14 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   waitVmcnt<0>();                                   // loads issued for steps that do not exist, and the stores
 }
 
-template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false>
 __global__ void __launch_bounds__(64 * WAVES)
 convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
          const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
          const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
          int xcdShift, const int32_t* __restrict__ numActOut) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  pipeTiles<T, CIN, COUT, MT, WAVES, CO>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+  pipeTiles<T, CIN, COUT, MT, WAVES, CO, DEAL>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
                                      relu, xcdShift, numActOut, gridDim.x);
 }
 
@@ -533,9 +621,6 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   constexpr size_t lds = pipeLds<T, CIN, CO>(MT, WAVES);
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
   if (lds > kLdsLimit || !pipeTakes(a, pitch, CIN * sizeof(T), TM)) return D3D_ERR_UNSUPPORTED;
-  static std::atomic<size_t> granted{64 * 1024};
-  const int32_t rc = grantLds(&convPipe<T, CIN, COUT, MT, WAVES, CO>, lds, &granted);
-  if (rc != D3D_OK) return rc;
   const int tiles = static_cast<int>((a.outRows + TM - 1) / TM);
   // persistent workgroups: as many as the CUs can hold at this LDS footprint, never more than there are tiles (three where
   // they fit: int8 64 -> 64 127 us with two, 121 with three on 1.07 million rows, 31 and 28 on 190 000; fp16 32 -> 64 153 and
@@ -548,11 +633,23 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   int blocks = (tiles + nXcd - 1) / nXcd * nXcd * COLS;
   const int most = chip.cus * perCu / (nXcd * COLS) * (nXcd * COLS);
   if (blocks > most) blocks = most;
-  hipLaunchKernelGGL((convPipe<T, CIN, COUT, MT, WAVES, CO>), dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES),
-                     lds, stream, static_cast<const T*>(a.in), static_cast<T*>(a.out),
-                     static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror, a.tileMasks,
-                     a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut);
-  return D3D_OK;
+  auto launch = [&](auto kernel, std::atomic<size_t>* granted) -> int32_t {
+    const int32_t rc = grantLds(kernel, lds, granted);
+    if (rc != D3D_OK) return rc;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), lds, stream, static_cast<const T*>(a.in),
+                       static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror,
+                       a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut);
+    return D3D_OK;
+  };
+  static std::atomic<size_t> granted{64 * 1024};
+  // an instantiation of its own: the list costs the others registers they use (260 000 rows, 64 -> 64: 1 % of a pass).  The
+  // two-byte and int8 tiles of 32-row wavefronts are for few rows and never get there
+  if constexpr (sizeof(T) == 4 || MT > 2) {
+    static std::atomic<size_t> grantedDeal{64 * 1024};
+    if (a.tileMasks && tiles > (sizeof(T) == 4 ? 1 : kDealRounds) * (blocks / COLS))
+      return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, true>, &grantedDeal);
+  }
+  return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, false>, &granted);
 }
 
 // Configuration per layer shape, measured on the layers of a VoxelNet backbone (120k voxels): rows per wavefront
@@ -594,6 +691,7 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       const int64_t cus = chipLayout().cus;
       if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
       if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
+      if (a.tileMasks && a.outRows > kDealRounds * 512 * cus) return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
       // 384-row tiles by the live rows: 196 000 rows, one and a half rounds of 512, two of 384, 52 -> 46 us; 262 000, two
       // rounds of 512, stay at 60 (64 with 384)
       return launchPipeByRows<T, CIN, COUT>(a, stream);

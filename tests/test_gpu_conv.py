@@ -652,3 +652,38 @@ def test_a_captured_layer_keeps_its_weights_when_another_type_is_run(engine):
         graph.replay()
         torch.cuda.synchronize()
         check_close(out.float().cpu().numpy(), ref["float16"], "float16")
+
+
+@pytest.mark.parametrize("cin,dtype,n,room", [(64, "float32", 50000, 0), (64, "float32", 70001, 9000), (128, "float32", 30011, 300),
+                                              (64, "float16", 524999, 0), (128, "bfloat16", 197001, 4000),
+                                              (64, "int8", 790003, 10000)])
+def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
+    """Which workgroup takes a tile changes nothing: with tile masks (a linked node) tiles are dealt by their taps, without
+    (the table derived from the same index tensor) they are taken in order.  Levels hold different shares of their cells, so
+    tiles hold 9 to 27 taps.  Bit for bit, rows past the live ones included: a tap no row has adds zeros."""
+    from deploy3d_amd import layers, synth
+    from deploy3d_amd.spconv_mm import spconv_mm
+    grid = (11, 400, 400)
+    rng = np.random.default_rng(n)
+    share = np.repeat([0.02, 0.9, 0.5, 0.0, 0.05, 0.3, 0.95, 0.4, 0.01, 0.0, 0.6], grid[1] * grid[2])
+    cells = np.flatnonzero(rng.random(len(share)) < share * n / (share.sum() * 0.9))
+    cells = cells[:n]
+    coords = np.stack([np.zeros_like(cells), cells // 160000, cells // 400 % 400, cells % 400], 1).astype(np.int32)
+    n = len(coords)
+    spec = synth.layer("l", "s", True, (3, 3, 3), cin, cin, padding=(1, 1, 1))
+    torch_dtype = dict(TORCH_DTYPE, int8=torch.int8)[dtype]
+    scales = {}
+    if dtype == "int8":
+        scales = dict(act_scale_in=0.03, act_scale_out=0.05)
+        spec.update(s_in=0.03, s_out=0.05)
+    weight, bias = synth.layer_weights(3, 0, spec)
+    feats = rng.standard_normal((n, cin), dtype=np.float32)
+    if dtype == "int8":
+        feats = synth.quantize_activations(feats, 0.03)
+    net = layers.SparseBackbone([spec], [(weight, bias)], [n + room], dtype=torch_dtype)
+    x = layers.make_input(coords, feats, grid, dtype=torch_dtype, capacity=n + room)
+    got = net.forward(x).feats.clone()
+    rb = net.rulebooks["s"]
+    want = spconv_mm(x.feats, x.num_act, x.num_act, rb.index, rb.num_index, (3, 3, 3), cin, cin, n + room, True, False,
+                     weight.reshape(-1), bias, relu=spec["relu"], **scales)
+    assert torch.equal(got, want)
