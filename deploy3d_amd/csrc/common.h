@@ -196,6 +196,7 @@ struct ConvArgs {
   int64_t nbrPitch;       // row pitch of nbr in elements; 0 = outRows
   int tapMirror;          // the table is indexed by the mirrored tap (a SubM rulebook's input-major table, see rbCompact)
   const unsigned long long* tileMasks;  // optional [ceil(outRows / 64)]: bit t set iff any of rows 64i..64i+63 has tap t
+  const int32_t* rowOrder;  // optional [outRows]: the table's row r is output row rowOrder[r] (launchOrderRows; nbr, tileMasks)
   const int32_t* numActOut;  // device int32 or null: live output rows (tiles past them only take their bias; the
                           // kernels balance the live ones over the chip)
   const void* zeros;      // device, >= 512 zero bytes: the row that absent neighbours gather
@@ -206,6 +207,19 @@ struct ConvArgs {
 };
 
 int32_t launchConv(const ConvArgs& a, hipStream_t stream);
+// Does launchConv run the layer on a kernel that takes its rows in another order (rowOrder)?
+bool convTakesRowOrder(const ConvArgs& a);
+// Puts the rows of a table (pitch outRows) into an order in which rows that have the same taps are neighbours, in place:
+// inside every window of kOrderWindow rows.  `out` (orderRowsBytes) receives the output row of every table row and the tap
+// masks of the ordered 64-row tiles.  Kernel volumes up to 32.
+constexpr int kOrderWindow = 512;
+struct RowOrder {
+  int32_t* rows;               // [outRows]
+  unsigned long long* masks;   // [whole windows / 64 + 8]
+};
+size_t orderRowsBytes(int64_t outRows);
+RowOrder orderRowsAt(void* base, int64_t outRows);
+int32_t launchOrderRows(int32_t* nbr, int kVol, int64_t outRows, const int32_t* numActOut, const RowOrder& out, hipStream_t stream);
 // The MFMA kernel family, one translation unit per storage type (conv_half.hip, conv_bf16.hip, conv_int8.hip);
 // D3D_ERR_UNSUPPORTED when no instantiation fits the layer.
 int32_t launchMfmaHalf(const ConvArgs& a, hipStream_t stream);

@@ -355,8 +355,28 @@ int32_t launchBuildNeighbours(const int32_t* index, int64_t rowLen, const int32_
   return D3D_OK;
 }
 
+// The kernels that store through rowOrder are convPipe's (conv_pipe.h) and, for fp32 and two-byte 32 -> 16, convMfmaResident.
+bool convTakesRowOrder(const ConvArgs& a) {
+  const bool aligned = ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
+  // 32-bit offsets into the table
+  if (!convUsesMfma(a.dtype, a.cin, a.cout) || !aligned || !a.weightsMfma || !a.zeros || a.pipe < 0 || a.staged != 0 ||
+      a.tileRows != 0 || a.rowChannels != 0 || static_cast<uint64_t>(a.kVol) * static_cast<uint64_t>(a.outRows) * 4 >= 0x7FFF0000ull)
+    return false;
+  const int es = a.dtype == D3D_FLOAT ? 4 : (a.dtype == D3D_INT8 ? 1 : 2);
+  if (a.cout == 16 || (es == 4 && a.cin == 16 && a.cout == 32))
+    return es == 4 ? a.cin <= 32 && floatMfmaFits(a.kVol, a.cin, a.cout) : es == 2 && a.cin == 32 && a.kVol <= 32;
+  if (es == 2 && a.cin == 32 && a.cout == 32) return false;      // convSolo
+  // what the pipelined kernel's launcher asks for, with a tile of room
+  return a.cin * es >= 64 && a.kVol <= 64 && static_cast<uint64_t>(a.inRows) * (a.cin * es) < 0xFFFF0000ull &&
+         static_cast<uint64_t>(a.outRows) + 512 < 0x3FFFFFFFull;
+}
+
 int32_t launchConv(const ConvArgs& a, hipStream_t stream) {
   if (a.outRows <= 0) return D3D_OK;
+  if (a.rowOrder && !convTakesRowOrder(a)) {
+    setError("conv: rows in another order for a layer whose kernel does not take it");
+    return D3D_ERR_UNSUPPORTED;
+  }
   int32_t rc = D3D_ERR_UNSUPPORTED;
   const bool aligned = ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
   if (a.dtype == D3D_INT8) {

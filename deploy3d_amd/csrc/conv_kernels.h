@@ -345,7 +345,7 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
                  const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr,
                  int64_t nbrPitch, int tapMirror, const T* __restrict__ zeros, int kVol, int64_t inRows,
                  int64_t outRows, int relu, int groups, int xcdShift, const int32_t* __restrict__ numActOut,
-                 int rowCh) {
+                 int rowCh, const int32_t* __restrict__ rowOrder) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int MT = 1;
   constexpr int NT = COUT / 16;
@@ -495,8 +495,9 @@ convMfmaResident(const T* __restrict__ in, T* __restrict__ out, const T* __restr
       __builtin_amdgcn_sched_barrier(0);
     }
 
-    const int64_t row = row0 + r16;
+    int64_t row = row0 + r16;
     if (row < outRows) {
+      if (rowOrder) row = rowOrder[row];
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int col = n * 16 + kgrp * 4;
@@ -1023,7 +1024,7 @@ int32_t launchMfmaResident(const ConvArgs& a, hipStream_t stream) {
                      lds, stream, static_cast<const T*>(a.in), static_cast<T*>(a.out),
                      static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr,
                      a.nbrPitch > 0 ? a.nbrPitch : a.outRows, a.tapMirror, static_cast<const T*>(a.zeros), a.kVol,
-                     a.inRows, a.outRows, a.relu, groups, chip.xcdShift, a.numActOut, a.rowChannels);
+                     a.inRows, a.outRows, a.relu, groups, chip.xcdShift, a.numActOut, a.rowChannels, a.rowOrder);
   return D3D_OK;
 }
 
@@ -1107,7 +1108,7 @@ int32_t launchMfmaOne(const ConvArgs& a, hipStream_t stream) {
     return D3D_ERR_UNSUPPORTED;
   }
   if constexpr (CIN * COUT >= 512) {
-    if (a.staged >= 0) {
+    if (a.staged >= 0 && !a.rowOrder) {
       const int32_t rc = launchStaged<T, CIN, COUT>(a, stream);
       if (rc != D3D_ERR_UNSUPPORTED) return rc;
     }

@@ -137,7 +137,7 @@ __device__ __forceinline__ void
 pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
           const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch,
           int tapMirror, const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
-          int xcdShift, const int32_t* __restrict__ numActOut, int blocks) {
+          int xcdShift, const int32_t* __restrict__ numActOut, int blocks, const int32_t* __restrict__ rowOrder = nullptr) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int ES = static_cast<int>(sizeof(T));
   constexpr int CS = CIN * ES > 128 ? 128 / ES : CIN;          // input channels per step (at most 128 bytes of a row); a tap takes KS steps
@@ -317,6 +317,12 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   // 16 bytes per lane and 64 contiguous bytes per row.
   // (fp32: 4 consecutive channels are those 16 bytes already.)
   static_assert(NT % 2 == 0 || ES == 4, "channel tiles are stored in pairs");
+  // output row of the table's row (below outRows)
+  auto outRow = [&](int64_t row) __attribute__((always_inline)) -> size_t {
+    if constexpr (DEAL)
+      if (rowOrder) return static_cast<size_t>(rowOrder[row]);
+    return static_cast<size_t>(row);
+  };
   auto storeTile = [&](int pos) __attribute__((always_inline)) {
     const int64_t row0 = static_cast<int64_t>(tileAt(pos)) * TM + wave * WM;
     if constexpr (ES == 4) {
@@ -334,7 +340,7 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
           }
           acc[m][n] = Acc{0, 0, 0, 0};
           const int64_t row = row0 + m * 16 + r16;
-          if (row < outRows) *reinterpret_cast<float4v*>(out + static_cast<size_t>(row) * COUT + col) = v;
+          if (row < outRows) *reinterpret_cast<float4v*>(out + outRow(row) * COUT + col) = v;
         }
       }
     } else {
@@ -377,7 +383,7 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
           const auto sw = __builtin_amdgcn_permlane16_swap(packed[0][m], packed[1][m], false, false);
           const u32x2 line = {sw[0], sw[1]};
           const int64_t row = row0 + m * 16 + r16;
-          if (row < outRows) *reinterpret_cast<u32x2*>(out + static_cast<size_t>(row) * COUT + outCol) = line;
+          if (row < outRows) *reinterpret_cast<u32x2*>(out + outRow(row) * COUT + outCol) = line;
         }
         __builtin_amdgcn_sched_barrier(0);
       } else {
@@ -404,7 +410,7 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
         const auto s1 = __builtin_amdgcn_permlane16_swap(a[1], c[1], false, false);
         const u32x4 line = {s0[0], s1[0], s0[1], s1[1]};
         const int64_t row = row0 + m * 16 + r16;
-        if (row < outRows) *reinterpret_cast<u32x4*>(out + static_cast<size_t>(row) * COUT + outCol) = line;
+        if (row < outRows) *reinterpret_cast<u32x4*>(out + outRow(row) * COUT + outCol) = line;
       }
       }
     }
@@ -525,10 +531,10 @@ __global__ void __launch_bounds__(64 * WAVES)
 convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
          const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
          const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
-         int xcdShift, const int32_t* __restrict__ numActOut) {
+         int xcdShift, const int32_t* __restrict__ numActOut, const int32_t* __restrict__ rowOrder) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   pipeTiles<T, CIN, COUT, MT, WAVES, CO, DEAL>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
-                                     relu, xcdShift, numActOut, gridDim.x);
+                                     relu, xcdShift, numActOut, gridDim.x, rowOrder);
 }
 
 // The same with the tile chosen by the live rows (wavefronts of 32 rows: those of 48 take 278 registers, which workgroups of
@@ -638,7 +644,7 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
     if (rc != D3D_OK) return rc;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), lds, stream, static_cast<const T*>(a.in),
                        static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror,
-                       a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut);
+                       a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut, a.rowOrder);
     return D3D_OK;
   };
   static std::atomic<size_t> granted{64 * 1024};
@@ -646,8 +652,12 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   // two-byte and int8 tiles of 32-row wavefronts are for few rows and never get there
   if constexpr (sizeof(T) == 4 || MT > 2) {
     static std::atomic<size_t> grantedDeal{64 * 1024};
-    if (a.tileMasks && tiles > (sizeof(T) == 4 ? 1 : kDealRounds) * (blocks / COLS))
+    if (a.rowOrder || (a.tileMasks && tiles > (sizeof(T) == 4 ? 1 : kDealRounds) * (blocks / COLS)))
       return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, true>, &grantedDeal);
+  }
+  if (a.rowOrder) {
+    setError("conv: a tile shape that does not take rows in another order");
+    return D3D_ERR_DEVICE;
   }
   return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, false>, &granted);
 }
@@ -669,6 +679,13 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   // shapes go by the bytes of an input row (the stage) and by the output channels (the accumulators): an int8 layer
   // takes the shape of the two-byte layer with half its input channels
   constexpr int RB = CIN * static_cast<int>(sizeof(T));
+  // rows in the order of their taps: the narrower a tile, the fewer taps it has
+  if constexpr (sizeof(T) < 4)
+    if (a.rowOrder) {
+      if constexpr (COUT >= 128 && (sizeof(T) == 1 || CIN >= 64)) return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
+      else if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
+      else return launchPipeCfg<T, CIN, COUT, 4, 4>(a, stream);
+    }
   if constexpr (sizeof(T) == 4) {
     // fp32: a step's MFMAs take eight times the cycles of a two-byte step with the same bytes, so the matrix pipe is
     // the bound and the tile only has to spread over the CUs: 128 rows, two or three workgroups per CU (16 -> 128: eight

@@ -878,12 +878,21 @@ struct MMPlugin final : d3d_plugin {
     if ((!linked || inverse) && maxNumActOut > 0) {
       if (!derived) derived = std::make_shared<DeviceBuffer>();
       const void* const before = derived->ptr;
-      const int32_t rc = derived->reserve(static_cast<size_t>(kernelVol) * static_cast<size_t>(maxNumActOut) * sizeof(int32_t));
+      const int32_t rc = derived->reserve(derivedBytes(maxNumActOut));
       if (derived->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
     return D3D_OK;
   }
+
+  // Inverse convolutions of several taps put the rows of their derived table in the order of their taps, where the layer's
+  // kernel takes that (orderRows).  A launch costs what four or five steps of a tile do: kernels of fewer than eight taps
+  // (three where rows differ along one axis) have no such steps to lose.
+  bool ordersRows() const { return inverse && kernelVol >= 8 && kernelVol <= 32; }
+  size_t derivedTableBytes(int64_t outRows) const {
+    return (static_cast<size_t>(kernelVol) * static_cast<size_t>(outRows > 0 ? outRows : 1) * sizeof(int32_t) + 15) / 16 * 16;
+  }
+  size_t derivedBytes(int64_t outRows) const { return derivedTableBytes(outRows) + (ordersRows() ? orderRowsBytes(outRows) : 0); }
 
   int32_t configureFloat(int32_t dtype, MMDeviceWeights::Converted& to) {
     const size_t nW = static_cast<size_t>(kernelVol) * cin * cout;
@@ -1055,7 +1064,7 @@ struct MMPlugin final : d3d_plugin {
     }
     if (!nbr) {  // the index tensor is all there is to go by: derive the table from it
       if (!derived) derived = std::make_shared<DeviceBuffer>();
-      const size_t bytes = static_cast<size_t>(kernelVol) * static_cast<size_t>(outRows > 0 ? outRows : 1) * sizeof(int32_t);
+      const size_t bytes = derivedBytes(outRows);
       if (derived->bytes < bytes && streamIsCapturing(stream)) {
         setError("SPConvMM: the table derived from the index tensor needs %zu bytes that were not reserved before the "
                  "capture (configure the node at these shapes, or enqueue it once, first)", bytes);
@@ -1119,6 +1128,13 @@ struct MMPlugin final : d3d_plugin {
     a.zeros = zeros;
     if (const char* e = debugEnv("D3D_CONV_PIPE")) a.pipe = e[0] == '0' ? -1 : 0;
     a.tileRows = tileRowsOverride();
+    if (ordersRows() && convTakesRowOrder(a)) {
+      const RowOrder order = orderRowsAt(static_cast<char*>(derived->ptr) + derivedTableBytes(outRows), outRows);
+      rc = launchOrderRows(static_cast<int32_t*>(derived->ptr), kernelVol, outRows, a.numActOut, order, stream);
+      if (rc != D3D_OK) return rc;
+      a.rowOrder = order.rows;
+      a.tileMasks = order.masks;
+    }
     return launchConv(a, stream);
   }
 };

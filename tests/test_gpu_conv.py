@@ -687,3 +687,38 @@ def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
     want = spconv_mm(x.feats, x.num_act, x.num_act, rb.index, rb.num_index, (3, 3, 3), cin, cin, n + room, True, False,
                      weight.reshape(-1), bias, relu=spec["relu"], **scales)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,room", [(1, 0), (63, 5), (511, 1), (512, 0), (513, 511), (3100, 1500)])
+@pytest.mark.parametrize("cin,cout,dtype", [(64, 32, "float32"), (32, 16, "float32"), (16, 128, "float32"), (64, 64, "float16"),
+                                            (32, 16, "bfloat16"), (32, 128, "float16"), (128, 128, "bfloat16")])
+def test_inverse_rows_in_the_order_of_their_taps(engine, n, room, cin, cout, dtype):
+    """Inverse convolutions sort their table's rows by taps inside windows of 512: sizes around a window's ends, live rows that
+    end in, at and windows before the capacity's end."""
+    run_case(n, (14, 60, 50), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False, inverse=True, cap_extra=room, relu=True)
+
+
+@pytest.mark.parametrize("ksize,stride,padding", [((2, 2, 2), (2, 2, 2), (0, 0, 0)), ((3, 3, 3), (3, 3, 3), (0, 0, 0)), ((4, 4, 2), (2, 2, 1), (1, 1, 0)),
+                                                  ((3, 3, 3), (1, 1, 1), (1, 1, 1)), ((3, 3, 4), (2, 2, 2), (1, 1, 1))])
+def test_inverse_rows_of_other_kernels(engine, ksize, stride, padding):
+    """Kernel volumes of 8, 27, 32 (sorted; with stride 1 nearly every row has a mask of its own) and 36 (not sorted)."""
+    for cin, cout, dtype in ((64, 32, "float16"), (32, 64, "float32")):
+        run_case(3000, (14, 60, 50), ksize, stride, padding, cin, cout, dtype, False, inverse=True, cap_extra=100)
+
+
+@pytest.mark.parametrize("cin,cout", [(64, 32), (128, 64), (64, 128)])
+def test_inverse_rows_int8(engine, cin, cout):
+    """int8 against the forward convolution of the index tensor with its gather and scatter rows exchanged, bit for bit."""
+    from deploy3d_amd.spconv_mm import spconv_mm
+    rng = np.random.default_rng(cin)
+    coords = random_cloud(rng, 5000, (14, 60, 50), 1)
+    n = len(coords)
+    rb = gpu_rulebook(coords, n, (14, 60, 50), 1, (3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1), 8 * n, False, cap=n, link=False)
+    index, num_index, _, num_out, _ = rb["dev"]
+    x = torch.from_numpy(rng.integers(-128, 128, (8 * n, cin)).astype(np.int8)).cuda()
+    w, b = rng.standard_normal(27 * cin * cout).astype(np.float32) / 40, rng.standard_normal(cout).astype(np.float32)
+    args = (num_index, (3, 3, 3), cin, cout, n, False)
+    kw = dict(act_scale_in=0.03, act_scale_out=0.05)
+    got = spconv_mm(x, num_out, rb["num_act_in"], index, *args, True, w, b, **kw)
+    want = spconv_mm(x, num_out, rb["num_act_in"], index[[1, 0, 2]].contiguous(), *args, False, w, b, **kw)
+    assert torch.equal(got, want)
