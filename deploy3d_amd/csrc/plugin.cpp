@@ -878,21 +878,29 @@ struct MMPlugin final : d3d_plugin {
     if ((!linked || inverse) && maxNumActOut > 0) {
       if (!derived) derived = std::make_shared<DeviceBuffer>();
       const void* const before = derived->ptr;
-      const int32_t rc = derived->reserve(derivedBytes(maxNumActOut));
+      const int32_t rc = derived->reserve(derivedBytes(dtype, maxNumActOut));
       if (derived->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
     return D3D_OK;
   }
 
-  // Inverse convolutions of several taps put the rows of their derived table in the order of their taps, where the layer's
-  // kernel takes that (orderRows).  A launch costs what four or five steps of a tile do: kernels of fewer than eight taps
-  // (three where rows differ along one axis) have no such steps to lose.
-  bool ordersRows() const { return inverse && kernelVol >= 8 && kernelVol <= 32; }
+  // Layers that put the rows of their derived table in the order of their taps, where their kernel takes that (orderRows):
+  // inverse convolutions, and fp32 ones of 32 channels and more, which without masks multiply every tap of every tile at the
+  // matrix pipe's rate.  us of an unlinked layer with its rulebook, fp32, unsorted / sorted: 32 -> 32, 3 000 voxels 47 / 44;
+  // 64 -> 64, 8 000 scattered voxels 68 / 48, 60 000 of a scan 173 / 125; at stride 2 32 -> 64, 60 000 of a scan 207 / 173,
+  // 64 -> 128, 100 000 scattered 1115 / 515.  Two-byte layers have less to win than the launch costs: 64 -> 64, 30 000 voxels
+  // 57 / 68, at stride 2 69 / 89, 110 000 140 / 162 (64 -> 128, 110 000 scattered voxels 217 / 203, the one case the other
+  // way).  Kernels of fewer than eight taps have too few steps to lose.
+  bool ordersRows(int32_t dtype) const {
+    return kernelVol >= 8 && kernelVol <= 32 && (inverse || (dtype == D3D_FLOAT && cin >= 32 && cout >= 32));
+  }
   size_t derivedTableBytes(int64_t outRows) const {
     return (static_cast<size_t>(kernelVol) * static_cast<size_t>(outRows > 0 ? outRows : 1) * sizeof(int32_t) + 15) / 16 * 16;
   }
-  size_t derivedBytes(int64_t outRows) const { return derivedTableBytes(outRows) + (ordersRows() ? orderRowsBytes(outRows) : 0); }
+  size_t derivedBytes(int32_t dtype, int64_t outRows) const {
+    return derivedTableBytes(outRows) + (ordersRows(dtype) ? orderRowsBytes(outRows) : 0);
+  }
 
   int32_t configureFloat(int32_t dtype, MMDeviceWeights::Converted& to) {
     const size_t nW = static_cast<size_t>(kernelVol) * cin * cout;
@@ -1064,7 +1072,7 @@ struct MMPlugin final : d3d_plugin {
     }
     if (!nbr) {  // the index tensor is all there is to go by: derive the table from it
       if (!derived) derived = std::make_shared<DeviceBuffer>();
-      const size_t bytes = derivedBytes(outRows);
+      const size_t bytes = derivedBytes(dtype, outRows);
       if (derived->bytes < bytes && streamIsCapturing(stream)) {
         setError("SPConvMM: the table derived from the index tensor needs %zu bytes that were not reserved before the "
                  "capture (configure the node at these shapes, or enqueue it once, first)", bytes);
@@ -1128,7 +1136,7 @@ struct MMPlugin final : d3d_plugin {
     a.zeros = zeros;
     if (const char* e = debugEnv("D3D_CONV_PIPE")) a.pipe = e[0] == '0' ? -1 : 0;
     a.tileRows = tileRowsOverride();
-    if (ordersRows() && convTakesRowOrder(a)) {
+    if (derived && nbr == derived->ptr && ordersRows(dtype) && convTakesRowOrder(a)) {
       const RowOrder order = orderRowsAt(static_cast<char*>(derived->ptr) + derivedTableBytes(outRows), outRows);
       rc = launchOrderRows(static_cast<int32_t*>(derived->ptr), kernelVol, outRows, a.numActOut, order, stream);
       if (rc != D3D_OK) return rc;

@@ -658,9 +658,9 @@ def test_a_captured_layer_keeps_its_weights_when_another_type_is_run(engine):
                                               (64, "float16", 524999, 0), (128, "bfloat16", 197001, 4000),
                                               (64, "int8", 790003, 10000)])
 def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
-    """Which workgroup takes a tile changes nothing: with tile masks (a linked node) tiles are dealt by their taps, without
-    (the table derived from the same index tensor) they are taken in order.  Levels hold different shares of their cells, so
-    tiles hold 9 to 27 taps.  Bit for bit, rows past the live ones included: a tap no row has adds zeros."""
+    """Which workgroup takes a tile changes nothing: a layer of many tiles, dealt to workgroups by the taps they hold, against the
+    halves of its rows, of which each has too few tiles to be dealt.  Levels hold different shares of their cells, so tiles
+    hold 9 to 27 taps.  Bit for bit, rows past the live ones included: a tap no row has adds zeros."""
     from deploy3d_amd import layers, synth
     from deploy3d_amd.spconv_mm import spconv_mm
     grid = (11, 400, 400)
@@ -684,9 +684,16 @@ def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
     x = layers.make_input(coords, feats, grid, dtype=torch_dtype, capacity=n + room)
     got = net.forward(x).feats.clone()
     rb = net.rulebooks["s"]
-    want = spconv_mm(x.feats, x.num_act, x.num_act, rb.index, rb.num_index, (3, 3, 3), cin, cin, n + room, True, False,
-                     weight.reshape(-1), bias, relu=spec["relu"], **scales)
-    assert torch.equal(got, want)
+    half = (n + room + 1) // 2
+    for lo in (0, half):
+        index = rb.index.clone()
+        index[1] -= lo
+        other = (index[1] < 0) | (index[1] >= half) | (index[2] < 0)
+        index[1:, other] = -1
+        live = torch.tensor([min(max(n - lo, 0), half)], dtype=torch.int32, device="cuda")
+        want = spconv_mm(x.feats, x.num_act, live, index, rb.num_index, (3, 3, 3), cin, cin, half, True, False,
+                         weight.reshape(-1), bias, relu=spec["relu"], **scales)
+        assert torch.equal(got[lo:lo + half], want[:n + room - lo])
 
 
 @pytest.mark.parametrize("n,room", [(1, 0), (63, 5), (511, 1), (512, 0), (513, 511), (3100, 1500)])
@@ -722,3 +729,13 @@ def test_inverse_rows_int8(engine, cin, cout):
     got = spconv_mm(x, num_out, rb["num_act_in"], index, *args, True, w, b, **kw)
     want = spconv_mm(x, num_out, rb["num_act_in"], index[[1, 0, 2]].contiguous(), *args, False, w, b, **kw)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("cin,cout", [(32, 32), (64, 64), (64, 128)])
+@pytest.mark.parametrize("n,room", [(63, 1), (700, 0), (5000, 131)])
+def test_derived_fp32_rows_in_the_order_of_their_taps(engine, cin, cout, n, room):
+    """Unlinked fp32 layers sort their derived table: sparse clouds (most tiles without most taps), with rows past the live ones;
+    a kernel volume that is not sorted."""
+    for ksize, pad in (((3, 3, 3), (1, 1, 1)), ((3, 3, 5), (1, 1, 2))):
+        run_case(n, (14, 200, 150), ksize, (1, 1, 1), pad, cin, cout, "float32", True, link=False, room=room)
+        run_case(n, (14, 200, 150), ksize, (2, 2, 2), pad, cin, cout, "float32", False, link=False, relu=True)
