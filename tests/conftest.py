@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -24,3 +25,18 @@ def engine():
     deploy3d_amd.load_library()
     assert torch.cuda.is_available(), "GPU tests need a GPU"
     return deploy3d_amd
+
+
+@pytest.fixture(autouse=True)
+def no_collection_in_a_capture(request):
+    """Python's collector runs between GPU tests, never inside one: what an earlier test left in a reference cycle (an exception's
+    traceback holds its frames) may own a HIP graph, and the destructor of torch's CUDAGraph waits for the device, which is
+    refused while a stream is captured and ends the process."""
+    if request.node.get_closest_marker("gpu") is None:
+        yield
+        return
+    gc.disable()
+    yield
+    gc.enable()
+    gc.collect()
+    gc.freeze()  # what is alive after a test (modules, fixtures, caches) is not searched again
