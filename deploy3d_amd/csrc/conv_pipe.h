@@ -132,7 +132,11 @@ struct TileDeal {
 
 // tileMasks: one 64-bit tap mask per 64 output rows, padded with zero entries to a multiple of 8 entries past
 // ceil(outRows / 64) (a workgroup reads the masks of a whole tile at once); null = every tap of every tile.
-template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false>
+//
+// SPLIT = 2: a tile is the work of two groups of WAVES wavefronts, each with half of the steps and LDS of its own (channel
+// halves of every tap where a tap takes two steps, else half of the tile's taps); the second group's sums pass through its stage
+// to the first, which adds and stores them.
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false, int SPLIT = 1>
 __device__ __forceinline__ void
 pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf,
           const float* __restrict__ bias, const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch,
@@ -165,10 +169,15 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   using F = u32x4;
   using Acc = typename Mfma<T>::Acc;
 
+  constexpr int SPT = SPLIT > 1 && KS > 1 ? KS / SPLIT : KS;   // steps of a tap in one group
+  static_assert(SPLIT == 1 || (SPLIT == 2 && !DEAL && KS <= 2 && MT * NT * 1024 <= 2 * SLOTS * 16), "two groups, whose sums fit a stage");
+
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % WAVES;
+  const int group = SPLIT > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) / WAVES : 0;
   const int r16 = lane & 15, kgrp = lane >> 4;
+  if constexpr (SPLIT > 1) smem += group * (NWB * WCH * 16 + WAVES * (2 * SLOTS * 16 + NI * WM * 4));
   u32x4* wLds = reinterpret_cast<u32x4*>(smem);                                      // [NWB][WCH]
   u32x4* stage = reinterpret_cast<u32x4*>(smem + static_cast<size_t>(NWB) * WCH * 16) + wave * 2 * SLOTS;  // [2][SLOTS]
   // ring of NI steps' neighbour indices, per wavefront, stored so that the GL indices one lane needs for its
@@ -221,14 +230,29 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
   // Past the last step the walk stays on it: the loads issued for steps that do not exist repeat valid addresses and
   // nothing in the loop has to branch on "is there such a step".
   constexpr uint32_t kLastOfTile = 1u << 31;
-  int walkPos = 0;                                   // ordinal of the walk's tile among this workgroup's
-  unsigned long long walkRem = maskAt(0), walkTaps = maskAt(1);  // taps of it still to walk; taps of the next tile
+  // (two groups: tile by tile, each with a pipeline of its own)
+  for (int firstPos = 0; firstPos < (SPLIT > 1 ? nMine : 1); ++firstPos) {
+  const int endPos = SPLIT > 1 ? firstPos + 1 : nMine;
+  int walkPos = firstPos;                            // ordinal of the walk's tile among this workgroup's
+  unsigned long long walkRem = maskAt(firstPos), walkTaps = SPLIT > 1 ? 0ull : maskAt(1);  // taps of it still to walk; taps of the next tile
+  int mySteps = 0, mostSteps = 0;                    // steps of this group / of the group that has more
+  if constexpr (SPLIT > 1) {
+    const int taps = __builtin_popcountll(walkRem);
+    mySteps = mostSteps = taps * SPT;
+    if constexpr (KS == 1) {                         // the lower half of the taps, rounded up, is the first group's
+      unsigned long long upper = walkRem;
+      for (int i = 0; i < (taps + 1) / 2; ++i) upper &= upper - 1;
+      walkRem = group ? upper : walkRem ^ upper;
+      mostSteps = (taps + 1) / 2;
+      mySteps = group ? taps / 2 : mostSteps;
+    }
+  }
   int walkTap = 0, walkPart = 0;
   // moves to the next step; returns its id (tap * KS + part), flagged when it ends its tile.  *newTile = it opens one.
   auto walkNext = [&](bool* newTile) __attribute__((always_inline)) -> uint32_t {
     *newTile = false;
     if (walkPart == 0) {
-      if (walkRem == 0 && walkPos + 1 < nMine) {
+      if (walkRem == 0 && walkPos + 1 < endPos) {
         ++walkPos;
         walkRem = walkTaps;
         walkTaps = maskAt(walkPos + 1);
@@ -239,8 +263,8 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
         walkRem &= walkRem - 1;
       }
     }
-    const uint32_t s = static_cast<uint32_t>(walkTap * KS + walkPart);
-    walkPart = walkPart + 1 == KS ? 0 : walkPart + 1;
+    const uint32_t s = static_cast<uint32_t>(walkTap * KS + walkPart + (SPT < KS ? group * SPT : 0));
+    walkPart = walkPart + 1 == SPT ? 0 : walkPart + 1;
     return s | (walkRem == 0 && walkPart == 0 ? kLastOfTile : 0u);
   };
   uint32_t ids[5];                                   // steps a .. a+4
@@ -513,6 +537,34 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
     return lastOfTile;
   };
 
+  if constexpr (SPLIT > 1) {
+    // the groups keep pace: the one with fewer steps meets the other's last barrier empty-handed
+    for (int a = 0; a < mostSteps; a += 2) {
+      if (a < mySteps) step(a, std::integral_constant<int, 0>{}, wtsA, wtsB);
+      else __builtin_amdgcn_s_barrier();
+      if (a + 1 >= mostSteps) break;
+      if (a + 1 < mySteps) step(a + 1, std::integral_constant<int, 1>{}, wtsB, wtsA);
+      else __builtin_amdgcn_s_barrier();
+    }
+    waitVmcnt<0>();                                 // loads issued for steps that do not exist: the stages are free
+    if (group) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) reinterpret_cast<Acc*>(stage)[(m * NT + n) * 64 + lane] = acc[m][n];
+    }
+    __syncthreads();
+    if (!group) {
+      const Acc* const other = reinterpret_cast<const Acc*>(reinterpret_cast<const unsigned char*>(stage) +
+                                                            NWB * WCH * 16 + WAVES * (2 * SLOTS * 16 + NI * WM * 4));
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] += other[(m * NT + n) * 64 + lane];
+      storeTile(firstPos);
+    }
+    __syncthreads();                                // the sums have been read: the next tile's rows may land
+  } else {
   for (int a = 0;; a += 2) {
     if (step(a, std::integral_constant<int, 0>{}, wtsA, wtsB)) {
       storeTile(mulPos);
@@ -523,17 +575,19 @@ pipeTiles(unsigned char* smem, const T* __restrict__ in, T* __restrict__ out, co
       if (++mulPos >= nMine) break;
     }
   }
+  }
+  }
   waitVmcnt<0>();                                   // loads issued for steps that do not exist, and the stores
 }
 
-template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false>
-__global__ void __launch_bounds__(64 * WAVES)
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, bool DEAL = false, int SPLIT = 1>
+__global__ void __launch_bounds__(64 * WAVES * SPLIT)
 convPipe(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
          const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
          const unsigned long long* __restrict__ tileMasks, int kVol, int64_t inRows, int64_t outRows, int relu,
          int xcdShift, const int32_t* __restrict__ numActOut, const int32_t* __restrict__ rowOrder) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  pipeTiles<T, CIN, COUT, MT, WAVES, CO, DEAL>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+  pipeTiles<T, CIN, COUT, MT, WAVES, CO, DEAL, SPLIT>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
                                      relu, xcdShift, numActOut, gridDim.x, rowOrder);
 }
 
@@ -621,10 +675,10 @@ int32_t launchPipeByRows(const ConvArgs& a, hipStream_t stream) {
   return D3D_OK;
 }
 
-template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT>
+template <class T, int CIN, int COUT, int MT, int WAVES, int CO = COUT, int SPLIT = 1>
 int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   constexpr int TM = 16 * MT * WAVES, COLS = COUT / CO;
-  constexpr size_t lds = pipeLds<T, CIN, CO>(MT, WAVES);
+  constexpr size_t lds = SPLIT * pipeLds<T, CIN, CO>(MT, WAVES);
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
   if (lds > kLdsLimit || !pipeTakes(a, pitch, CIN * sizeof(T), TM)) return D3D_ERR_UNSUPPORTED;
   const int tiles = static_cast<int>((a.outRows + TM - 1) / TM);
@@ -642,7 +696,7 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   auto launch = [&](auto kernel, std::atomic<size_t>* granted) -> int32_t {
     const int32_t rc = grantLds(kernel, lds, granted);
     if (rc != D3D_OK) return rc;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), lds, stream, static_cast<const T*>(a.in),
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES * SPLIT), lds, stream, static_cast<const T*>(a.in),
                        static_cast<T*>(a.out), static_cast<const T*>(a.weightsMfma), a.bias, a.requantM, a.nbr, pitch, a.tapMirror,
                        a.tileMasks, a.kVol, a.inRows, a.outRows, a.relu, chip.xcdShift, a.numActOut, a.rowOrder);
     return D3D_OK;
@@ -650,7 +704,7 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
   static std::atomic<size_t> granted{64 * 1024};
   // an instantiation of its own: the list costs the others registers they use (260 000 rows, 64 -> 64: 1 % of a pass).  The
   // two-byte and int8 tiles of 32-row wavefronts are for few rows and never get there
-  if constexpr (sizeof(T) == 4 || MT > 2) {
+  if constexpr (SPLIT == 1 && (sizeof(T) == 4 || MT > 2)) {
     static std::atomic<size_t> grantedDeal{64 * 1024};
     if (a.rowOrder || (a.tileMasks && tiles > (sizeof(T) == 4 ? 1 : kDealRounds) * (blocks / COLS)))
       return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, true>, &grantedDeal);
@@ -659,7 +713,7 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
     setError("conv: a tile shape that does not take rows in another order");
     return D3D_ERR_DEVICE;
   }
-  return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, false>, &granted);
+  return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, false, SPLIT>, &granted);
 }
 
 // Configuration per layer shape, measured on the layers of a VoxelNet backbone (120k voxels): rows per wavefront
@@ -706,7 +760,10 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
     // of 256-row tiles, those take 35 against 30)
     if constexpr (sizeof(T) == 2) {
       const int64_t cus = chipLayout().cus;
-      if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4>(a, stream);
+      // up to 192 rows per CU the steps of a tile are shared by two groups of wavefronts: one group of four leaves LDS reads and
+      // MFMAs of a SIMD's only wavefront to take turns.  43 000 rows 17.3 -> 15.4 us (256-row tiles on 169 CUs before)
+      if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 64, 2>(a, stream);
+      if (a.outRows <= 192 * cus) return launchPipeCfg<T, CIN, COUT, 3, 4, 64, 2>(a, stream);
       if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
       if (a.tileMasks && a.outRows > kDealRounds * 512 * cus) return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
       // 384-row tiles by the live rows: 196 000 rows, one and a half rounds of 512, two of 384, 52 -> 46 us; 262 000, two
@@ -734,6 +791,14 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       // of a network (two of the one, one of the other and a column layer) as much is won, so no further line is drawn.
       // The wider tile wins where it fits as many workgroups to a CU: the lines are whole rounds of one and of two per CU.
       const bool shared4 = forced("32,4"), shared3 = forced("48,4"), free = !shared4 && !shared3;
+      if constexpr (RB >= 128) {
+        // one workgroup per CU: its steps are shared by two groups of wavefronts (128 -> 128, 23 000 rows: fp16 25.8 -> 23.1 us,
+        // int8 17.5 -> 15.5; a pass of 9 000 voxels in fp16 267 -> 256 with the 64 -> 64 layers).  Bound by LDS: 60 KB of fragments
+        // and rows a step, 25 000 clocks of them in all.
+        if (free && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32, 2>(a, stream);
+        if (free && a.outRows <= 64 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 64, 2>(a, stream);
+        if (free && a.outRows <= 96 * cus) return launchPipeCfg<T, CIN, COUT, 3, 4, 64, 2>(a, stream);
+      }
       if (free && a.outRows <= 32 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 32>(a, stream);   // 29 -> 18 us
       if (shared4 || (free && (a.outRows <= 64 * cus || (a.outRows > 96 * cus && a.outRows <= 128 * cus))))
         return launchPipeCfg<T, CIN, COUT, 2, 4, 64>(a, stream);

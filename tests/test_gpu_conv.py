@@ -739,3 +739,13 @@ def test_derived_fp32_rows_in_the_order_of_their_taps(engine, cin, cout, n, room
     for ksize, pad in (((3, 3, 3), (1, 1, 1)), ((3, 3, 5), (1, 1, 2))):
         run_case(n, (14, 200, 150), ksize, (1, 1, 1), pad, cin, cout, "float32", True, link=False, room=room)
         run_case(n, (14, 200, 150), ksize, (2, 2, 2), pad, cin, cout, "float32", False, link=False, relu=True)
+
+
+@pytest.mark.parametrize("cin,cout,dtype", [(64, 64, "float16"), (64, 128, "bfloat16"), (128, 128, "float16"), (128, 128, "bfloat16")])
+@pytest.mark.parametrize("ksize,padding", [((1, 1, 1), (0, 0, 0)), ((1, 1, 2), (0, 0, 0)), ((3, 1, 1), (1, 0, 0)), ((3, 3, 3), (1, 1, 1)), ((3, 3, 7), (1, 1, 3))])
+def test_steps_of_a_tile_shared_by_two_groups(engine, cin, cout, dtype, ksize, padding):
+    """Small layers: half of a tile's taps (or of their channels) to each of two groups of wavefronts, which have one step, an even
+    and an odd number of them; tiles with fewer taps than the kernel and with none, more tiles than workgroups."""
+    run_case(700, (14, 60, 50), ksize, (1, 1, 1), padding, cin, cout, dtype, True, relu=True, room=2900)
+    run_case(700, (14, 60, 50), ksize, (2, 2, 2), padding, cin, cout, dtype, False, link=False)
+    run_case(9000, (14, 100, 90), ksize, (1, 1, 1), padding, cin, cout, dtype, True, room=7000)
