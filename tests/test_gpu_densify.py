@@ -136,3 +136,25 @@ def test_wrong_out_channels_is_an_error(engine):
                     torch.zeros(1, dtype=torch.int32, device=dev),
                     torch.empty((1, 0, 2, 4, 4), dtype=torch.int32, device=dev), 16)
     assert e.value.status == -3
+
+
+@pytest.mark.parametrize("shape,channels,dtype", [
+    ((1, 1, 8, 8), 6, "float16"),       # one whole tile in 16-byte stores, rows of 12 bytes
+    ((2, 3, 5, 16), 20, "int8"),        # second tile of a plane cut at a store's end, chunk of 20 bytes
+    ((1, 2, 4, 19), 3, "float32"),      # one channel to a word
+    ((1, 1, 10, 8), 7, "int8"),         # rows off a word: not in 16-byte stores
+    ((1, 2, 33, 24), 200, "bfloat16"),  # four channel chunks, the last one short
+    ((2, 3, 31, 48), 132, "int8"),      # a last chunk of one word
+    ((1, 4, 250, 256), 66, "float16"),  # 34 MB and an odd number of workgroups: shared out XCD by XCD
+    ((2, 2, 223, 225), 45, "float32"),  # the same, planes of an odd size
+])
+def test_wide_stores_and_large_maps(engine, shape, channels, dtype):
+    rng = np.random.default_rng(23)
+    n = min(60000, int(np.prod(shape) * 0.5))
+    if dtype == "int8":
+        feats = torch.from_numpy(rng.integers(-128, 128, (n + 5, channels), dtype=np.int8))
+        _, coords = make_case(3, n, "float32", cap=n + 5, channels=1, shape=shape)
+    else:
+        feats, coords = make_case(3, n, dtype, cap=n + 5, channels=channels, shape=shape)
+    got = _run(feats, coords, n, shape)
+    assert np.array_equal(_bits(got), oracle.bev_densify(_bits(feats), coords, n, shape))
