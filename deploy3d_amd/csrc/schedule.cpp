@@ -24,51 +24,12 @@
 #include <cstring>
 #include <mutex>
 #include <utility>
-#include <vector>
 
-#include "common.h"
-#include "d3d_spconv.h"
+#include "schedule.h"
 
-struct d3d_schedule {
-  enum Kind { kOperator, kSum, kCast };
-  struct Step {
-    Kind kind = kOperator;
-    d3d_plugin* plugin = nullptr;
-    int32_t dtype = 0;          // kSum, kCast
-    int64_t count = 0;
-    std::vector<d3d_tensor_desc> in, out;
-    std::vector<const void*> inputs;
-    std::vector<void*> outputs;
-    void* workspace = nullptr;
-    size_t workspaceBytes = 0;
-    int lane = 0;
-    std::vector<int> after;     // steps of other lanes it waits for
-    int before = -1;            // the step ahead of it on its own lane
-    hipEvent_t done = nullptr;  // recorded behind the step if a step of another lane waits for it
-  };
-  std::vector<hipStream_t> lanes;  // [0] unused: lane 0 is the caller's stream
-  std::vector<hipEvent_t> joined;  // per owned lane: its tail, for the join
-  hipEvent_t fork = nullptr;
-  std::vector<Step> steps;
-  // the pass as a graph
-  hipGraphExec_t graph = nullptr;
-  bool launched = false;        // the graph has been launched, last on launchedOn
-  hipStream_t launchedOn = nullptr;
-  uint64_t graphChanges = 0;    // the operators' change count the graph was captured at
-  uint64_t lastChanges = ~0ull; // ... and at the end of the last run
-  int steady = 0;               // runs in a row that changed nothing
-  int patience = kSteadyRuns;   // ... after which a capture is tried; doubled by every refusal, as it costs a pass
-  static constexpr int kSteadyRuns = 2, kMostPatience = 4096;
-};
+namespace d3d {
 
-namespace {
-
-int32_t hipFail(hipError_t e, const char* what) {
-  d3d::setError("schedule: %s failed: %s", what, hipGetErrorString(e));
-  return D3D_ERR_DEVICE;
-}
-
-int32_t enqueueStep(const d3d_schedule::Step& st, hipStream_t q) {
+int32_t scheduleEnqueueStep(const d3d_schedule::Step& st, hipStream_t q) {
   switch (st.kind) {
     case d3d_schedule::kSum: return d3d::launchSum(st.dtype, st.inputs[0], st.inputs[1], st.outputs[0], st.count, q);
     case d3d_schedule::kCast:
@@ -77,6 +38,42 @@ int32_t enqueueStep(const d3d_schedule::Step& st, hipStream_t q) {
       return d3d_enqueue(st.plugin, st.in.data(), st.out.data(), st.inputs.data(), st.outputs.data(), st.workspace,
                          st.workspaceBytes, q);
   }
+}
+
+// A dependency that another one implies gets no edge: every edge between branches is a wait packet in front of the kernel, 6 us
+// even when the other branch is long done (a VoxelNet backbone of 9 000 voxels: 374 us with the implied edges, 324 without;
+// 120 000 voxels: 708 and 700).
+std::vector<std::vector<int>> scheduleEdges(const d3d_schedule* s) {
+  const size_t count = s->steps.size();
+  std::vector<std::vector<int>> edges(count);
+  std::vector<std::vector<bool>> behindOf(count, std::vector<bool>(count));  // what each step comes after, directly or not
+  for (size_t i = 0; i < count; ++i) {
+    const d3d_schedule::Step& st = s->steps[i];
+    std::vector<int> direct(st.after);
+    if (st.before >= 0) direct.insert(direct.begin(), st.before);
+    for (int d : direct) {
+      behindOf[i][static_cast<size_t>(d)] = true;
+      for (size_t k = 0; k < count; ++k)
+        if (behindOf[static_cast<size_t>(d)][k]) behindOf[i][k] = true;
+    }
+    auto implied = [&](int d) {
+      for (int other : direct)
+        if (behindOf[static_cast<size_t>(other)][static_cast<size_t>(d)]) return true;
+      return false;
+    };
+    for (int d : direct)
+      if (!implied(d)) edges[i].push_back(d);
+  }
+  return edges;
+}
+
+}  // namespace d3d
+
+namespace {
+
+int32_t hipFail(hipError_t e, const char* what) {
+  d3d::setError("schedule: %s failed: %s", what, hipGetErrorString(e));
+  return D3D_ERR_DEVICE;
 }
 
 uint64_t changesOf(const d3d_schedule* s) {
@@ -187,37 +184,19 @@ bool captureGraph(d3d_schedule* s) {
   }
   const size_t count = s->steps.size();
   std::vector<std::vector<hipGraphNode_t>> tail(count);
-  // What each step comes after, directly or not.  A dependency that another one implies gets no edge: every edge
-  // between branches is a wait packet in front of the kernel, 6 us even when the other branch is long done (a
-  // VoxelNet backbone of 9 000 voxels: 374 us with the implied edges, 324 without; 120 000 voxels: 708 and 700).
-  std::vector<std::vector<bool>> behindOf(count, std::vector<bool>(count));
+  const std::vector<std::vector<int>> edges = d3d::scheduleEdges(s);
   for (size_t i = 0; ok && i < count; ++i) {
     const d3d_schedule::Step& st = s->steps[i];
-    std::vector<int> direct(st.after);
-    if (st.before >= 0) direct.insert(direct.begin(), st.before);
-    for (int d : direct) {
-      behindOf[i][static_cast<size_t>(d)] = true;
-      for (size_t k = 0; k < count; ++k)
-        if (behindOf[static_cast<size_t>(d)][k]) behindOf[i][k] = true;
-    }
-    auto implied = [&](int d) {
-      for (int other : direct)
-        if (behindOf[static_cast<size_t>(other)][static_cast<size_t>(d)]) return true;
-      return false;
-    };
     std::vector<hipGraphNode_t> deps;
-    auto behind = [&](int step) {
-      for (hipGraphNode_t n : tail[static_cast<size_t>(step)])
+    for (int d : edges[i])
+      for (hipGraphNode_t n : tail[static_cast<size_t>(d)])
         if (std::find(deps.begin(), deps.end(), n) == deps.end()) deps.push_back(n);
-    };
-    for (int d : direct)
-      if (!implied(d)) behind(d);
     if (hipStreamBeginCaptureToGraph(q, graph, deps.empty() ? nullptr : deps.data(), nullptr, deps.size(),
                                      hipStreamCaptureModeThreadLocal) != hipSuccess) {
       ok = false;
       break;
     }
-    ok = enqueueStep(st, q) == D3D_OK;
+    ok = d3d::scheduleEnqueueStep(st, q) == D3D_OK;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     const hipGraphNode_t* last = nullptr;
     size_t nLast = 0;
@@ -280,12 +259,15 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
   reapGraphs(false);
   auto* s = new d3d_schedule();
   hipError_t e = hipSuccess;
-  if (n_lanes > 1) e = hipEventCreateWithFlags(&s->fork, hipEventDisableTiming);  // one lane: no HIP object at all
   s->lanes.assign(static_cast<size_t>(n_lanes), nullptr);
   s->joined.assign(static_cast<size_t>(n_lanes), nullptr);
-  for (int l = 1; l < n_lanes && e == hipSuccess; ++l) {
-    e = hipStreamCreateWithFlags(&s->lanes[l], hipStreamNonBlocking);  // default priority
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&s->joined[l], hipEventDisableTiming);
+  if (n_lanes > 1) {  // one lane: no HIP object at all
+    const RelaxedCapture relaxed;  // (a stream of the caller's may be capturing)
+    e = hipEventCreateWithFlags(&s->fork, hipEventDisableTiming);
+    for (int l = 1; l < n_lanes && e == hipSuccess; ++l) {
+      e = hipStreamCreateWithFlags(&s->lanes[l], hipStreamNonBlocking);  // default priority
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&s->joined[l], hipEventDisableTiming);
+    }
   }
   if (e != hipSuccess) {
     d3d_schedule_destroy(s);
@@ -449,7 +431,7 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
       if (e != hipSuccess && rc == D3D_OK) rc = hipFail(e, "hipStreamWaitEvent");
     }
     if (rc == D3D_OK)  // after a failure nothing more is enqueued, but the lanes still join below
-      rc = enqueueStep(st, q);
+      rc = d3d::scheduleEnqueueStep(st, q);
     if (st.done) {
       e = hipEventRecord(st.done, q);
       if (e != hipSuccess && rc == D3D_OK) rc = hipFail(e, "hipEventRecord");

@@ -204,6 +204,7 @@ class SparseBackbone:
         self._plans = {}        # buffers of the input -> the pass on them as a native schedule (False: not possible)
         self._last = None       # (buffers of the input, what was made on them) of the pass before, if ``forward`` made it
         self._repeats = 0       # passes on those buffers in a row before it
+        self._captured, self._replaced = None, []  # the schedule last captured (see _capture) and those before it
 
     def forward(self, x):
         """One pass on ``x``; returns the last layer's SparseTensor (every layer's is in ``outputs``).
@@ -213,7 +214,8 @@ class SparseBackbone:
         pass cost the host 600 us, the graph launch 170 (making the graph costs 500 once, so a pass has to repeat
         first).  Other buffers, and a stream that is being captured, take the operators one by one."""
         if torch.cuda.is_current_stream_capturing():
-            return self._forward_steps(x)
+            return self._capture(x) or self._forward_steps(x)
+        self._replaced.clear()
         key = self._buffers_of(x)
         plan = self._plans.get(key)
         if not plan or plan.expired():
@@ -236,6 +238,44 @@ class SparseBackbone:
         self._last = (key, None)
         plan.schedule.run()
         return self._hand_out(plan.made, x, SparseTensor(x.feats, x.coors, x.num_act, x.grid))
+
+    # Captured passes of up to this many input rows are captured as a schedule's steps (d3d_schedule_capture), which leaves out the
+    # dependencies that enqueueing on side streams adds.  us a pass with side streams / as steps: fp16, 7 400 rows 259 / 241,
+    # 45 000 (bf16) 440 / 407, 63 000 492 / 462, 84 000 531 / 534, 94 500 549 / 552, 126 000 619 / 635; int8, 19 000 273 / 257,
+    # 94 500 451 / 433, 150 000 531 / 521, 189 000 748 / 773.  Large passes are bound by the sum of their kernels' demands, and a
+    # rulebook that starts earlier stretches the convolutions beside it.
+    _CAPTURE_ROWS = 73728
+    _CAPTURE_ROWS_INT8 = 163840
+
+    def _capture(self, x):
+        """The pass on ``x`` into the graph that the current stream captures, as a schedule's steps; None where the last pass
+        was not made on these buffers."""
+        rows = self._CAPTURE_ROWS_INT8 if x.feats.dtype == torch.int8 else self._CAPTURE_ROWS
+        if not self.overlap or x.capacity > rows:
+            return None
+        key = self._buffers_of(x)
+        plan = self._plans.get(key)
+        sums = [s["name"] for s in self.specs if "+" in (s.get("src") or "")]
+        if self._last is not None and self._last[0] == key and self._last[1] is not None:
+            made = rulebooks, inputs, outputs = self._last[1]
+            if sums:  # into tensors of the capture's own, which live as long as the graph
+                inputs = dict(inputs)
+                for name in sums:
+                    t = inputs[name]
+                    inputs[name] = SparseTensor(torch.empty_like(t.feats), t.coors, t.num_act, t.grid, t.batch, t.producer)
+                made = rulebooks, inputs, outputs
+            sched = self._record(made)
+        elif plan and not plan.expired() and not sums:
+            sched, made = plan.schedule, plan.made
+        else:
+            return None
+        if not sched or not sched.capture(current_stream()):
+            return None
+        sched.release((x.feats, x.coors, x.num_act))
+        self._replaced.append(self._captured)  # destroyed with the next eager pass, not while the stream captures
+        self._captured = sched
+        self._last = None
+        return self._hand_out(made, x, SparseTensor(x.feats, x.coors, x.num_act, x.grid))
 
     # What a pass left behind goes to the caller as objects of that pass's own (over the same tensors): what is rebound on
     # a result is neither in what is recorded nor in the next pass's result.  Made when asked for: 30 us for a VoxelNet pass.

@@ -29,7 +29,7 @@ EXPORTS = [
     "d3d_serialize", "d3d_holds_weights", "d3d_num_outputs", "d3d_output_dims", "d3d_output_dtype", "d3d_supports_format",
     "d3d_configure", "d3d_workspace_size", "d3d_enqueue", "d3d_last_error", "d3d_num_ops", "d3d_op_name",
     "d3d_enqueue_static", "d3d_link_rulebook", "d3d_link_coords", "d3d_set_option",
-    "d3d_schedule_create", "d3d_schedule_add", "d3d_schedule_add_sum", "d3d_schedule_add_cast", "d3d_schedule_size", "d3d_schedule_run", "d3d_schedule_destroy",
+    "d3d_schedule_create", "d3d_schedule_add", "d3d_schedule_add_sum", "d3d_schedule_add_cast", "d3d_schedule_size", "d3d_schedule_run", "d3d_schedule_capture", "d3d_schedule_destroy",
 ]
 OPT_PERSISTENT_INDEX = 1
 OPT_INDEX_UNUSED = 2
@@ -133,6 +133,8 @@ def load_library(path=None):
     lib.d3d_schedule_size.argtypes = [vp]
     lib.d3d_schedule_run.restype = i32
     lib.d3d_schedule_run.argtypes = [vp, vp]
+    lib.d3d_schedule_capture.restype = i32
+    lib.d3d_schedule_capture.argtypes = [vp, vp]
     lib.d3d_schedule_destroy.restype = None
     lib.d3d_schedule_destroy.argtypes = [vp]
     _lib = lib
@@ -408,6 +410,14 @@ class Schedule:
         if stream is None:
             stream = current_stream()
         _check(self._lib.d3d_schedule_run(self._h, ctypes.c_void_p(stream)))
+
+    def capture(self, stream=None):
+        """The steps as nodes of the graph that the stream is capturing; False where it is not (nothing is enqueued then)."""
+        rc = self._lib.d3d_schedule_capture(self._h, ctypes.c_void_p(current_stream() if stream is None else stream))
+        if STATUS_NAMES.get(rc) == "UNSUPPORTED":
+            return False
+        _check(rc)
+        return True
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None

@@ -254,6 +254,10 @@ int32_t d3d_schedule_add_cast(d3d_schedule* s, int32_t dtype, const void* a, voi
                               const int32_t* after, int32_t nb_after);
 int32_t d3d_schedule_size(const d3d_schedule* s);
 int32_t d3d_schedule_run(d3d_schedule* s, void* stream);
+/* The steps as nodes of the graph that `stream` is capturing, behind what it holds at the call; what `stream` captures next
+ * comes behind all of them.  Operators have to be configured and enqueued once before (see d3d_enqueue under capture).
+ * Refused with D3D_ERR_UNSUPPORTED, before any step, while `stream` is not capturing. */
+int32_t d3d_schedule_capture(d3d_schedule* s, void* stream);
 void d3d_schedule_destroy(d3d_schedule* s);
 
 #ifdef __cplusplus

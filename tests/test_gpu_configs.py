@@ -653,3 +653,119 @@ def test_config5_full_size_first_layers_vs_oracle(engine):
         want = ref[spec["name"]]["exact"]
         rms = float(np.sqrt(np.mean(want ** 2)))
         assert float(np.abs(got - want).max()) <= 2e-2 * rms, spec["name"]
+
+
+@pytest.mark.parametrize("dtype", ["float16", "int8"])
+def test_captured_pass_as_the_steps_of_a_schedule(engine, dtype, monkeypatch):
+    """A capture on buffers that the last eager pass ran on holds a schedule's steps (no side streams): behind what the stream
+    captured before the pass, ahead of what it captures after it, bit for bit what the pass with side streams gives, on every
+    replay, with other clouds in the same buffers and eager work between.  Above the line, and on buffers of no pass before, the
+    capture is the one with side streams."""
+    from deploy3d_amd import layers, synth
+    specs, grid = synth.voxelnet_layers(), (41, 360, 360)
+    weights = [synth.layer_weights(3, i, s) for i, s in enumerate(specs)]
+    clouds = [synth.coords_lidar(synth.seed(3, 7 + k), grid, n) for k, n in enumerate((6000, 4700, 0))]
+    rng = np.random.default_rng(4)
+    feats = [rng.standard_normal((6000, specs[0]["cin"])).astype(np.float32) for _ in clouds]
+    torch_dtype = dict(chain.TORCH_DTYPE, int8=torch.int8)[dtype]
+    if dtype == "int8":
+        for s in specs:
+            s.update(s_in=0.02, s_out=0.02)
+        feats = [synth.quantize_activations(f, 0.02) for f in feats]
+    counts = layers.measure_output_counts(specs, clouds[0], grid)
+    caps = layers.plan_capacities(specs, 6000, {k: int(1.3 * v) for k, v in counts.items()})
+    staged = [(torch.from_numpy(f).to("cuda", torch_dtype), torch.zeros((6000, 4), dtype=torch.int32, device="cuda"),
+               torch.tensor([len(c)], dtype=torch.int32, device="cuda")) for c, f in zip(clouds, feats)]
+    for c, (_, coors, _) in zip(clouds, staged):
+        coors[:len(c)] = torch.from_numpy(c).cuda()
+
+    def fill(x, k):
+        for to, source in zip((x.feats, x.coors, x.num_act), staged[k]):
+            to.copy_(source)
+
+    def build():
+        net = layers.SparseBackbone(specs, weights, caps, dtype=torch_dtype)
+        return net, layers.make_input(clouds[0], feats[0], grid, dtype=torch_dtype, capacity=6000)
+
+    plain, px = build()
+    want = []
+    for k in range(len(clouds)):
+        fill(px, k)
+        y = plain._forward_steps(px)
+        n = int(y.num_act.item())
+        want.append((n, y.feats.clone(), y.coors[:n].clone()))
+    for rows, eager_first in ((1 << 20, True), (0, True), (1 << 20, False)):
+        monkeypatch.setattr(layers.SparseBackbone, "_CAPTURE_ROWS", rows)
+        monkeypatch.setattr(layers.SparseBackbone, "_CAPTURE_ROWS_INT8", rows)
+        graph = net = y = None  # a result keeps its operators: freeing one's memory is not for a capture
+        net, x = build()
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            net.forward(x)
+            if not eager_first:
+                other = layers.SparseTensor(x.feats.clone(), x.coors, x.num_act, x.grid)
+                net.forward(other)
+            fill(x, 0)
+            source = tuple(t.clone() for t in staged[0])
+            stream.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                for to, s in zip((x.feats, x.coors, x.num_act), source):
+                    to.copy_(s)
+                y = net.forward(x)
+                doubled = y.feats.float() * 2
+        torch.cuda.synchronize()
+        assert (net._captured is not None) == (rows > 0 and eager_first)
+        if net._captured is not None:
+            assert net._captured.capture() is False  # nothing is being captured now
+        for k in (0, 1, 2, 1, 0):
+            for s, new in zip(source, staged[k]):
+                s.copy_(new)
+            y.feats.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            n, want_feats, want_coors = want[k]
+            assert int(y.num_act.item()) == n
+            assert torch.equal(y.feats, want_feats) and torch.equal(y.coors[:n], want_coors)
+            assert torch.equal(doubled, want_feats.float() * 2)
+            if rows and k == 1:
+                net.forward(x)  # eager passes in between change nothing
+                torch.cuda.synchronize()
+
+
+def test_captured_sums_are_the_capture_s_own(engine):
+    """A captured pass that adds feature maps: the sums lie in memory of the graph's own, so two captures of one network and its
+    eager passes do not share them."""
+    from deploy3d_amd import layers, synth
+    p = dict(padding=(1, 1, 1))
+    specs = [synth.layer("a", "s", True, (3, 3, 3), 16, 16, **p), synth.layer("b", "s", True, (3, 3, 3), 16, 16, **p),
+             synth.layer("c", "s", True, (3, 3, 3), 16, 16, src="b+a", **p)]
+    weights = [synth.layer_weights(3, i, s) for i, s in enumerate(specs)]
+    grid = (10, 60, 60)
+    coords = synth.coords_uniform(5, grid, 3000)
+    net = layers.SparseBackbone(specs, weights, [3000] * 3)
+    inputs, graphs, want = [], [], []
+    for k in range(2):
+        x = layers.make_input(coords, np.random.default_rng(k).standard_normal((3000, 16), dtype=np.float32), grid)
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            want.append(net._forward_steps(x).feats.clone())
+            net.forward(x)
+            stream.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                y = net.forward(x)
+        assert net._captured is not None
+        summed = net.inputs["c"].feats
+        inputs.append((x, summed))
+        graphs.append(graph)
+    assert inputs[0][1].data_ptr() != inputs[1][1].data_ptr()
+    for k in (0, 1, 0, 1):
+        for _, summed in inputs:
+            summed.zero_()
+        torch.cuda.synchronize()
+        graphs[k].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.feats, want[k])
+        assert not inputs[1 - k][1].any()
