@@ -43,8 +43,9 @@ __device__ inline int pipeTileRows(int64_t rows, int cus) {
 // The tiles one of `per` workgroups of an XCD takes, in order.  A tile's time goes by the taps its rows have (27, or 18 and 9
 // in the outer levels of a scene), and a layer ends with its busiest workgroup.  Where workgroups take several tiles and masks
 // say what those hold, the tiles of an XCD are ranked by their taps, most first, and dealt back and forth: one with a heavy
-// tile gets a light one with it.  XCDs take runs of CHUNK tiles in turn instead of a contiguous eighth each, which could be
-// all heavy: levels of a scene are contiguous.  Each wavefront ranks for itself, 64 tiles to a register, and keeps its
+// tile gets a light one with it.  XCDs take runs of up to CHUNK tiles in turn instead of a contiguous eighth each, which could
+// be all heavy: levels of a scene are contiguous.  (Runs are short enough for sixteen turns: with 16-tile runs 195 tiles are 32 for
+// five XCDs and 16 for three.)  Each wavefront ranks for itself, 64 tiles to a register, and keeps its
 // workgroup's list in the lanes of one register.
 // Otherwise (no masks, at most ROUNDS tiles each or more than a list holds) XCD x takes the x-th contiguous part (TileOrder).
 // fp32 layers, bound by the matrix pipe, are dealt from the second tile on: steps of the busiest workgroup / of the average
@@ -70,16 +71,18 @@ struct TileDeal {
     const int live = order.liveTiles, wgs = per << xcdShift;
     if (!tileMasks || live <= ROUNDS * wgs || live > 32 * wgs || per > 192) return;
     dealt = true;
-    const int chunks = (live + CHUNK - 1) / CHUNK;
-    int lx = ((chunks - xcd + order.nXcd - 1) >> xcdShift) * CHUNK;   // chunks xcd, xcd + nXcd, ...; the last one may be short
-    if (((chunks - 1) & (order.nXcd - 1)) == xcd) lx -= chunks * CHUNK - live;
+    int cs = 0;                                          // log2 of a run's tiles
+    while ((2 << cs) <= CHUNK && (2 << cs) <= live >> (xcdShift + 4)) ++cs;
+    const int chunks = ((live - 1) >> cs) + 1;
+    int lx = ((chunks - xcd + order.nXcd - 1) >> xcdShift) << cs;     // chunks xcd, xcd + nXcd, ...; the last one may be short
+    if (((chunks - 1) & (order.nXcd - 1)) == xcd) lx -= (chunks << cs) - live;
     if (lx < 0) lx = 0;
     for (int from = 0; from < lx; from += 64 * SLOTS) {
       int taps[SLOTS], at[SLOTS], rank[SLOTS];
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
         const int local = from + s * 64 + lane;
-        at[s] = ((local / CHUNK << xcdShift) + xcd) * CHUNK + local % CHUNK;
+        at[s] = ((((local >> cs) << xcdShift) + xcd) << cs) + (local & ((1 << cs) - 1));
         taps[s] = -1;
         rank[s] = 0;
         if (local < lx) {
