@@ -18,7 +18,7 @@
 // can differ in the last bits from run to run; coordinates and counts cannot.
 //
 // Three forms, chosen by size (launchVoxelize): a few thousand points fit one workgroup's LDS (one launch); otherwise
-// the table's entries carry the sums (three launches: clear, insert, emit); very many points or channels keep a table
+// records of the points carry the sums (three launches: clear, insert, emit); very many points or channels keep a table
 // of bare keys and sum in the output rows (five launches).
 #include <atomic>
 
@@ -254,105 +254,133 @@ vxSmall(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, c
 }
 
 // ---------------------------------------------------------------------------
-// The usual form: a table entry holds key and lowest point, the point that claimed it, and count and feature sums of
-// the others - one cache line per voxel for everything:
-//   { u64 key << 32 | lowest point; u32 claiming point; u32 further points; float sums[C]; pad to 16 bytes }
-// The claiming point's own features are not added here (most voxels of a scan hold one or two points, so most points
-// then cost one compare-and-swap and no other atomic): the emitting pass reads them where they are.
-// 200 000 points: 42.6 us of kernels in five launches before, 34 in three (clear 8, insert 15, emit 10), bound by the
-// random compare-and-swaps; up to 50 000 points the call is bound by its three launches on the host (18 us).
+// The usual form: a table of heads, u64 key << 32 | the point that claimed the entry, and for every point a record that
+// is its voxel's if it claimed one:
+//   { u32 lowest point; float further points; float sums[C]; pad to 16 bytes }
+// The lowest point's own features are not in the sums (most voxels of a scan hold one or two points, so most points
+// then cost one compare-and-swap and no other atomic): the emitting pass reads them where they are.  A point that takes
+// a higher one's place as the lowest adds the features of the point it displaced.  Records lie in point order: the
+// emitting pass reads those of voxels with one point in one run, and heads of 8 bytes afford a table of four per point.
+// (The count is exact: the form is for fewer than 2^24 points.)
+// 200 000 points, 135 000 of them in the grid and nearly all in voxels of their own: clear 5.8, insert 11.8, emit 7.8 us, where
+// entries of 32 bytes in a table of two per point took 8, 16.6 and 10.3: bound by the chains of compare-and-swaps, whose longest
+// went from 16 to 9 with the larger table (eight heads per point: insert 10.0, but with eight points to a voxel the call is 1 us
+// slower).  In a graph of calls 36.0 -> 24.0 us, 100 000 points 27.9 -> 18.4; eight points to a voxel 62 -> 30.6, 400 000 of them
+// with six channels 136 -> 60.  Up to 50 000 points the call is bound by its three launches on the host.
 // ---------------------------------------------------------------------------
-constexpr int kVxMaxWide = 12;  // channels an entry carries
+constexpr int kVxMaxWide = 12;  // channels a record carries
 
-__host__ __device__ constexpr int vxEntryBytes(int C) { return (16 + 4 * C + 15) / 16 * 16; }
+__host__ __device__ constexpr int vxRecordBytes(int C) { return (8 + 4 * C + 15) / 16 * 16; }
 
-// Entries empty, output rows zero (simple_mean_trt.cu:139-143), chunk states zero.
+// Heads empty, every record's lowest point its own, output rows zero (simple_mean_trt.cu:139-143), chunk states zero.
 template <int PER>
 __global__ void __launch_bounds__(kVxThreads)
-vxClearWide(uint4* table, uint32_t pieces, float* outFeats, int64_t nFeats, unsigned long long* states,
-            uint32_t nStates) {
+vxClearWide(uint4* table, uint32_t headPairs, uint4* records, uint32_t pieces, float* outFeats, int64_t nFeats,
+            unsigned long long* states, uint32_t nStates) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = tid; i < headPairs; i += stride) table[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
   for (uint32_t i = static_cast<uint32_t>(tid); i < pieces; i += static_cast<uint32_t>(stride))
-    table[i] = i % PER == 0 ? make_uint4(~0u, ~0u, 0u, 0u) : make_uint4(0u, 0u, 0u, 0u);
+    records[i] = make_uint4(i % PER == 0 ? i / PER : 0u, 0u, 0u, 0u);
   for (int64_t i = tid; i < nFeats; i += stride) outFeats[i] = 0.f;
   for (int64_t i = tid; i < nStates; i += stride) states[i] = 0ull;
 }
 
-// pointSlot[i] = entry of point i when it may be its voxel's lowest point, else none.
+// points[i] = { record of point i's voxel when i may be its lowest point, else none; key }.
 template <int CT>
 __global__ void __launch_bounds__(kVxThreads)
 vxInsertWide(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, const float* __restrict__ config, int32_t n,
-             int channels, VxGeom g, unsigned char* table, uint32_t slots, uint32_t* __restrict__ pointSlot) {
+             int channels, VxGeom g, unsigned long long* table, uint32_t slots, unsigned char* records,
+             uint2* __restrict__ points) {
   const int C = CT ? CT : channels;
-  const int32_t i = blockIdx.x * kVxThreads + threadIdx.x;
-  if (i >= n) return;
-  const VxPoint<CT> f(feats + static_cast<size_t>(i) * C, C);
+  constexpr int W = CT ? 8 : 16;     // lanes that add a point: one for the count and one per channel
+  static_assert(CT + 1 <= 8 && kVxMaxWide + 1 <= 16, "a lane per word");
+  __shared__ float words[kVxThreads * W];
+  __shared__ uint32_t homes[kVxThreads];
+  const int32_t i = blockIdx.x * kVxThreads + threadIdx.x, at = min(i, n - 1);
+  const VxPoint<CT> f(feats + static_cast<size_t>(at) * C, C);
   const VxConfig cfg(config);
-  uint32_t key, slot = kVxNone;
-  if (vxCell(f, batchIdx[i], cfg, g, &key)) {
+  uint32_t key = 0, home = kVxNone, added = kVxNone;   // the voxel's record, and the point whose features go to its sums
+  bool lowest = false;
+  if (vxCell(f, i < n ? batchIdx[at] : -1, cfg, g, &key)) {
     const unsigned long long mine = (static_cast<unsigned long long>(key) << 32) | static_cast<uint32_t>(i);
     // the hash spread over the table by its high bits: any number of slots will do
     uint32_t s = static_cast<uint32_t>((static_cast<unsigned long long>(vxMix(key)) * slots) >> 32);
     for (uint32_t tries = 0; tries < slots; ++tries) {
-      unsigned char* entry = table + static_cast<size_t>(s) * vxEntryBytes(C);
-      auto* head = reinterpret_cast<unsigned long long*>(entry);
-      const unsigned long long old = atomicCAS(head, kVxEmpty, mine);
+      const unsigned long long old = atomicCAS(table + s, kVxEmpty, mine);
       if (old == kVxEmpty) {
-        reinterpret_cast<uint32_t*>(entry)[2] = static_cast<uint32_t>(i);
-        slot = s;
+        home = static_cast<uint32_t>(i);
+        lowest = true;
         break;
       }
       if (static_cast<uint32_t>(old >> 32) == key) {
-        if (old > mine) {
-          atomicMin(head, mine);
-          slot = s;
+        home = static_cast<uint32_t>(old);
+        added = static_cast<uint32_t>(i);
+        if (added < home) {
+          const uint32_t low = atomicMin(reinterpret_cast<uint32_t*>(records + static_cast<size_t>(home) * vxRecordBytes(C)), added);
+          lowest = low > added;
+          added = max(low, added);
         }
-        float* sums = reinterpret_cast<float*>(entry + 16);
-        for (int c = 0; c < C; ++c) unsafeAtomicAdd(sums + c, f[c]);
-        atomicAdd(reinterpret_cast<uint32_t*>(entry) + 3, 1u);
         break;
       }
       s = s + 1 == slots ? 0u : s + 1;
     }
   }
-  pointSlot[i] = slot;
+  if (i < n) points[i] = make_uint2(lowest ? home : kVxNone, key);
+  // The words that a point adds are one run of 4 * (C + 1) bytes: neighbouring lanes add them together, a wavefront
+  // instruction for 64 / W points, so that memory sees one access per point and not one per word.
+  const unsigned long long adds = __ballot(added != kVxNone);
+  const int lane = threadIdx.x & 63, first = threadIdx.x & ~63, count = __popcll(adds);
+  if (added != kVxNone) {
+    const int to = first + __popcll(adds & ((1ull << lane) - 1ull));
+    homes[to] = home;
+    words[to * W] = 1.f;
+    const float* from = feats + static_cast<size_t>(added) * C;
+    for (int c = 0; c < C; ++c) words[to * W + 1 + c] = from[c];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // a wavefront reads what it wrote itself
+  __builtin_amdgcn_wave_barrier();
+  const int w = lane % W;
+  for (int p = lane / W; p < count; p += 64 / W)
+    if (w <= C)
+      unsafeAtomicAdd(reinterpret_cast<float*>(records + static_cast<size_t>(homes[first + p]) * vxRecordBytes(C) + 4) + w,
+                      words[(first + p) * W + w]);
 }
 
-constexpr unsigned long long kVxAggregate = 1ull << 32, kVxPrefix = 2ull << 32;
+constexpr unsigned long long kVxPublished = 1ull << 32;
 constexpr int kVxSpins = 1 << 16;
 
 // One chunk of 1024 points per workgroup: representatives are ranked in point order, the workgroup publishes its count,
-// reads how many the chunks before it have (64 of their states at a time, waiting for those that are not there yet),
-// and writes mean and coordinate of its own voxels.  A state is one 64-bit word, flag and value together, so relaxed
-// device-scope accesses are enough.  The wait cannot deadlock - a chunk waits for lower ones only, and those were
-// dispatched before it - and it is bounded all the same: after kVxSpins looks the wavefront counts the earlier chunks'
-// representatives itself.
+// reads how many the chunks before it have (a thread per chunk, so that all states are on their way together, waiting for
+// those that are not there yet) and writes mean and coordinate of its own voxels.  A state is one 64-bit word, flag and
+// value together, so relaxed device-scope accesses are enough.  The wait cannot deadlock - a chunk waits for lower ones
+// only, and those were dispatched before it and wait for nobody before they publish - and it is bounded all the same:
+// after kVxSpins looks the thread counts that chunk's representatives itself.
 template <int CT>
 __global__ void __launch_bounds__(kVxThreads)
-vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, const unsigned char* __restrict__ table,
-           const uint32_t* __restrict__ pointSlot, unsigned long long* states, int32_t maxNumActOut, float* __restrict__ outFeats,
+vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, const unsigned char* __restrict__ records,
+           const uint2* __restrict__ points, unsigned long long* states, int32_t maxNumActOut, float* __restrict__ outFeats,
            int32_t* __restrict__ outCoors, int32_t* __restrict__ numActOut) {
   const int C = CT ? CT : channels;
-  const size_t entryBytes = vxEntryBytes(C);
-  __shared__ uint32_t waveReps[kVxItems][kVxThreads / 64];
-  __shared__ uint32_t baseShared;
+  const size_t recordBytes = vxRecordBytes(C);
+  __shared__ uint32_t waveReps[kVxItems][kVxThreads / 64], waveBase[kVxThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t chunk = blockIdx.x;
+  uint2 point[kVxItems];
   uint4 head[kVxItems];
   bool rep[kVxItems];
-  uint32_t slot[kVxItems], below[kVxItems];
+  uint32_t below[kVxItems];
 #pragma unroll
   for (int k = 0; k < kVxItems; ++k) {
     const int64_t i = static_cast<int64_t>(chunk) * kVxChunk + k * kVxThreads + tid;
-    slot[k] = i < n ? pointSlot[i] : kVxNone;
+    point[k] = i < n ? points[i] : make_uint2(kVxNone, 0u);
   }
 #pragma unroll
   for (int k = 0; k < kVxItems; ++k)
-    head[k] = slot[k] != kVxNone ? *reinterpret_cast<const uint4*>(table + slot[k] * entryBytes) : make_uint4(0, 0, 0, 0);
+    head[k] = point[k].x != kVxNone ? *reinterpret_cast<const uint4*>(records + point[k].x * recordBytes) : make_uint4(0, 0, 0, 0);
 #pragma unroll
   for (int k = 0; k < kVxItems; ++k) {
-    rep[k] = slot[k] != kVxNone && head[k].x == chunk * kVxChunk + k * kVxThreads + tid;
+    rep[k] = point[k].x != kVxNone && head[k].x == chunk * kVxChunk + k * kVxThreads + tid;
     const unsigned long long m = __ballot(rep[k]);
     below[k] = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
     if (lane == 0) waveReps[k][wave] = static_cast<uint32_t>(__popcll(m));
@@ -368,58 +396,56 @@ vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, c
       total += waveReps[k][w];
     }
   }
-  if (wave == 0) {
-    if (lane == 0)
-      __hip_atomic_store(&states[chunk], (chunk ? kVxAggregate : kVxPrefix) | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t base = 0;
-    int spins = 0;
-    for (int64_t top = static_cast<int64_t>(chunk) - 1; top >= 0;) {
-      const int64_t p = top - lane;
-      const unsigned long long st =
-          p >= 0 ? __hip_atomic_load(&states[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kVxPrefix;
-      const unsigned long long prefixes = __ballot((st >> 32) == 2u), missing = __ballot((st >> 32) == 0u);
-      const int last = prefixes ? __builtin_ctzll(prefixes) : 63;   // lanes up to here are needed
-      if (missing & (last == 63 ? ~0ull : (2ull << last) - 1ull)) {
-        if (++spins < kVxSpins) {
-          __builtin_amdgcn_s_sleep(1);
-          continue;
-        }
-        base = 0;
-        for (int64_t q = lane; q < static_cast<int64_t>(chunk) * kVxChunk; q += 64) {
-          const uint32_t qs = pointSlot[q];
-          if (qs != kVxNone && *reinterpret_cast<const uint32_t*>(table + qs * entryBytes) == static_cast<uint32_t>(q)) ++base;
-        }
+  if (tid == 0) __hip_atomic_store(&states[chunk], kVxPublished | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float mean[kVxItems][CT ? CT : 1];   // loaded ahead of the wait for the chunks before
+  if constexpr (CT != 0) {
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) base += __shfl_xor(base, off, 64);
-        break;
-      }
-      uint32_t v = lane <= last ? static_cast<uint32_t>(st) : 0u;
+    for (int k = 0; k < kVxItems; ++k) {
+      if (!rep[k]) continue;
+      const float* f = feats + static_cast<size_t>(head[k].x) * CT;
+      const float* sums = reinterpret_cast<const float*>(records + point[k].x * recordBytes + 8);
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      base += v;
-      if (prefixes) break;
-      top -= 64;
-    }
-    if (lane == 0) {
-      if (chunk)
-        __hip_atomic_store(&states[chunk], kVxPrefix | (base + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      baseShared = base;
-      if (chunk == gridDim.x - 1)
-        *numActOut = static_cast<int32_t>(base + total < static_cast<uint32_t>(maxNumActOut) ? base + total : maxNumActOut);
+      for (int c = 0; c < CT; ++c) mean[k][c] = f[c] + (c == 0 ? __uint_as_float(head[k].z) : c == 1 ? __uint_as_float(head[k].w) : sums[c]);
     }
   }
+  uint32_t base = 0;
+  for (uint32_t p = tid; p < chunk; p += kVxThreads) {
+    unsigned long long st = 0;
+    for (int spins = 0; spins < kVxSpins; ++spins) {
+      st = __hip_atomic_load(&states[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (st) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    if (!st)
+      for (int64_t q = static_cast<int64_t>(p) * kVxChunk; q < static_cast<int64_t>(p + 1) * kVxChunk; ++q) {
+        const uint32_t at = points[q].x;
+        if (at != kVxNone && *reinterpret_cast<const uint32_t*>(records + at * recordBytes) == static_cast<uint32_t>(q)) ++st;
+      }
+    base += static_cast<uint32_t>(st);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) base += __shfl_xor(base, off, 64);
+  if (lane == 0) waveBase[wave] = base;
   __syncthreads();
-  const uint32_t base = baseShared;
+  base = 0;
+#pragma unroll
+  for (int w = 0; w < kVxThreads / 64; ++w) base += waveBase[w];
+  if (tid == 0 && chunk == gridDim.x - 1) *numActOut = static_cast<int32_t>(min(base + total, static_cast<uint32_t>(maxNumActOut)));
 #pragma unroll
   for (int k = 0; k < kVxItems; ++k) {
     const uint32_t id = base + rank[k];
     if (!rep[k] || id >= static_cast<uint32_t>(maxNumActOut)) continue;
-    const float* sums = reinterpret_cast<const float*>(table + slot[k] * entryBytes + 16);
-    const float* f = feats + static_cast<size_t>(head[k].z) * C;
     float* row = outFeats + static_cast<size_t>(id) * C;
-    const float points = static_cast<float>(head[k].w + 1u);
-    for (int c = 0; c < C; ++c) row[c] = (f[c] + sums[c]) / points;
-    reinterpret_cast<int4*>(outCoors)[id] = vxCoord(head[k].y, g);
+    const float count = __uint_as_float(head[k].y) + 1.f;
+    if constexpr (CT != 0) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) row[c] = mean[k][c] / count;
+    } else {
+      const float* sums = reinterpret_cast<const float*>(records + point[k].x * recordBytes + 8);
+      const float* f = feats + static_cast<size_t>(head[k].x) * C;
+      for (int c = 0; c < C; ++c) row[c] = (f[c] + sums[c]) / count;
+    }
+    reinterpret_cast<int4*>(outCoors)[id] = vxCoord(point[k].y, g);
   }
 }
 
@@ -586,27 +612,32 @@ uint32_t pow2AtLeast(uint64_t v) {
 size_t alignUp256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 struct VxPlan {
-  bool wide;              // entries carry the sums
+  bool wide;              // records carry the sums
   uint32_t slots, nChunks;
-  size_t table, pointSlot, local, chunkBase, counts, ticket, total;
+  size_t table, records, pointSlot, local, chunkBase, counts, ticket, total;
 };
 
-// Entries with sums are cleared and read whole (2 slots per point: 64 bytes per point at 4 channels), so the form is kept
-// to what the fixed scratch array of d3d_enqueue_static holds: about a million points at 4 channels.
+// Records are cleared and heads are 8 bytes (72 bytes per point at 3 to 6 channels, 56 with two heads per point), so the form
+// is kept to what the fixed scratch array of d3d_enqueue_static holds: about 1.2 million points at 3 to 6 channels.  Four heads per
+// point: the longest chain of taken slots decides the inserting pass (see above).
 VxPlan planVoxelize(int64_t numPts, int64_t maxNumActOut, int64_t C) {
   VxPlan p{};
   const int64_t n = numPts < 1 ? 1 : numPts;
   p.nChunks = static_cast<uint32_t>((n + kVxChunk - 1) / kVxChunk);
   if (C <= kVxMaxWide && n < (1 << 30)) {
     p.wide = true;
-    p.slots = static_cast<uint32_t>(2 * n < 1024 ? 1024 : 2 * n);  // the reference's hashSpace = 2 (simple_mean_trt.cu:110)
-    size_t off = alignUp256(static_cast<size_t>(p.slots) * vxEntryBytes(static_cast<int>(C)));
-    p.pointSlot = off;
-    off = alignUp256(off + static_cast<size_t>(n) * 4);
-    p.chunkBase = off;  // chunk states, u64
-    off = alignUp256(off + static_cast<size_t>(p.nChunks) * 8);
-    p.total = off;
-    if (p.total <= kStaticScratchBytes) return p;
+    for (int64_t perPoint = 4; perPoint >= 2; perPoint /= 2) {  // the reference's hashSpace = 2 (simple_mean_trt.cu:110)
+      p.slots = static_cast<uint32_t>(perPoint * n < 1024 ? 1024 : perPoint * n);
+      size_t off = alignUp256(static_cast<size_t>(p.slots) * 8);
+      p.records = off;
+      off = alignUp256(off + static_cast<size_t>(n) * vxRecordBytes(static_cast<int>(C)));
+      p.pointSlot = off;  // record and key of every point
+      off = alignUp256(off + static_cast<size_t>(n) * 8);
+      p.chunkBase = off;  // chunk states, u64
+      off = alignUp256(off + static_cast<size_t>(p.nChunks) * 8);
+      p.total = off;
+      if (p.total <= kStaticScratchBytes) return p;
+    }
     p = VxPlan{};
     p.nChunks = static_cast<uint32_t>((n + kVxChunk - 1) / kVxChunk);
   }
@@ -656,24 +687,26 @@ int32_t launchSmall(const VoxelizeArgs& a, const VxGeom& g, uint32_t slots, size
 
 template <int CT>
 void launchWide(const VoxelizeArgs& a, const VxPlan& p, const VxGeom& g, char* ws, hipStream_t stream) {
-  auto* table = reinterpret_cast<unsigned char*>(ws);
-  auto* pointSlot = reinterpret_cast<uint32_t*>(ws + p.pointSlot);
+  auto* table = reinterpret_cast<unsigned long long*>(ws);
+  auto* records = reinterpret_cast<unsigned char*>(ws + p.records);
+  auto* points = reinterpret_cast<uint2*>(ws + p.pointSlot);
   auto* states = reinterpret_cast<unsigned long long*>(ws + p.chunkBase);
-  const int perEntry = vxEntryBytes(a.C) / 16;
-  const int64_t pieces = static_cast<int64_t>(p.slots) * perEntry, nFeats = static_cast<int64_t>(a.maxNumActOut) * a.C;
-  int64_t blocks = (pieces + kVxThreads * 4 - 1) / (kVxThreads * 4);
+  const int perRecord = vxRecordBytes(a.C) / 16;
+  const int64_t pieces = a.numPts * perRecord, nFeats = static_cast<int64_t>(a.maxNumActOut) * a.C;
+  int64_t blocks = (pieces + p.slots / 2 + kVxThreads * 4 - 1) / (kVxThreads * 4);
   if (blocks > 4096) blocks = 4096;
 #define D3D_VX_CLEAR(PER)                                                                                                       \
   hipLaunchKernelGGL(vxClearWide<PER>, dim3(static_cast<unsigned>(blocks)), dim3(kVxThreads), 0, stream,                        \
-                     reinterpret_cast<uint4*>(table), static_cast<uint32_t>(pieces), a.outFeats, nFeats, states, p.nChunks)
-  if (perEntry == 2) D3D_VX_CLEAR(2);
-  else if (perEntry == 3) D3D_VX_CLEAR(3);
+                     reinterpret_cast<uint4*>(table), p.slots / 2, reinterpret_cast<uint4*>(records),                              \
+                     static_cast<uint32_t>(pieces), a.outFeats, nFeats, states, p.nChunks)
+  if (perRecord == 2) D3D_VX_CLEAR(2);
+  else if (perRecord == 3) D3D_VX_CLEAR(3);
   else D3D_VX_CLEAR(4);
 #undef D3D_VX_CLEAR
   hipLaunchKernelGGL(vxInsertWide<CT>, dim3(static_cast<unsigned>((a.numPts + kVxThreads - 1) / kVxThreads)), dim3(kVxThreads), 0,
-                     stream, a.feats, a.batchIdx, a.config, static_cast<int32_t>(a.numPts), a.C, g, table, p.slots, pointSlot);
+                     stream, a.feats, a.batchIdx, a.config, static_cast<int32_t>(a.numPts), a.C, g, table, p.slots, records, points);
   hipLaunchKernelGGL(vxEmitWide<CT>, dim3(p.nChunks), dim3(kVxThreads), 0, stream, a.feats, static_cast<int32_t>(a.numPts), a.C, g,
-                     table, pointSlot, states, a.maxNumActOut, a.outFeats, a.outCoors, a.numActOut);
+                     records, points, states, a.maxNumActOut, a.outFeats, a.outCoors, a.numActOut);
 }
 
 }  // namespace

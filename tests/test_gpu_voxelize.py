@@ -144,6 +144,33 @@ def test_sizes_around_the_forms(engine, n, channels, max_out):
         assert not got_f[got_n:].any()
 
 
+@pytest.mark.parametrize("n,channels", [(260, 3), (50001, 12), (930000, 5), (940000, 5), (1198000, 5), (1210000, 5)])
+def test_points_that_share_voxels(engine, n, channels):
+    """Records: about eight points to a voxel, the lowest of them anywhere among the insertions, with four table heads per
+    point, two (from 932 000 points of five channels on) and, past 1.2 million points, the form of bare keys."""
+    rng = np.random.default_rng(n)
+    side = max(4, int(round((n / 8) ** (1 / 3))))
+    pts = rng.uniform(0, side, (n, channels)).astype(np.float32)
+    cfg = np.array([0, 0, 0, 1, 1, 1], np.float32)
+    batch = np.zeros(n, np.int32)
+    cells = np.minimum(pts[:, :3].astype(np.int64), side)
+    inside = (cells < side).all(axis=1)
+    key = (cells[:, 2] * side + cells[:, 1]) * side + cells[:, 0]
+    uniq, first, inv, count = np.unique(key[inside], return_index=True, return_inverse=True, return_counts=True)
+    order = np.argsort(first)
+    got_f, got_c, got_n = _run(pts, batch, cfg, (1, side, side, side), n)
+    assert got_n == len(uniq)
+    k = uniq[order]
+    want_c = np.stack([np.zeros_like(k), k // side // side, k // side % side, k % side], axis=1)
+    assert np.array_equal(got_c[:got_n], want_c)
+    # fp32 sums of up to max(count) values below max(side, 1): each addition rounds by at most half an ulp of the sum
+    bound = side * count.max() * 2.0 ** -24 * 2
+    for c in range(channels):
+        mean = np.bincount(inv, weights=pts[inside, c].astype(np.float64)) / count
+        assert np.abs(got_f[:got_n, c] - mean[order]).max() <= bound
+    assert not got_f[got_n:].any()
+
+
 def test_wrong_dtype_is_unsupported(engine):
     from deploy3d_amd import EngineError, Plugin, TensorDesc
     from deploy3d_amd.simple_mean import simple_mean_blob
