@@ -263,6 +263,36 @@ def test_strided_operator_on_a_strided_operators_map(engine, second):
         consumer.link_coords(None)
 
 
+@pytest.mark.parametrize("grid", [(13, 90, 76), (41, 200, 180), (41, 820, 800)])
+@pytest.mark.parametrize("second", [((3, 3, 3), (2, 2, 2), (1, 1, 1)), ((3, 1, 1), (2, 1, 1), (0, 0, 0))])
+def test_strided_operator_on_a_map_whose_rows_end_inside(engine, grid, second):
+    """The producer's outputs fill its capacity: they end in the first chunk of its map's records, inside a record, with the
+    last cell (nothing cut off) and at places between; maps of one to many chunks of 64 records and of 1024.  The linked
+    operator finds what the unlinked one finds on the producer's coordinates."""
+    import torch
+    from deploy3d_amd import spconv_index_nd
+    from deploy3d_amd.spconv_index import index_plugin
+    n = 6000
+    coords = torch.from_numpy(random_cloud(np.random.default_rng(7), n, grid, 1)).cuda()
+    num = torch.tensor([len(coords)], dtype=torch.int32, device="cuda")
+    shape = torch.empty((1, 0) + grid, dtype=torch.int32, device="cuda")
+    first = ((3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1), (0, 0, 0))
+    nxt = second + ((1, 1, 1), (0, 0, 0))
+    total = int(spconv_index_nd(coords, num, shape, *first, 8 * n, False, False)[3].item())
+    for max1 in (1, 65, total // 3, total - 1, total):
+        producer, consumer = index_plugin(*first, max1, False, False), index_plugin(*nxt, 8 * n, False, False)
+        got = []
+        for linked in (True, False):
+            consumer.link_coords(producer if linked else None)
+            _, _, oc, no, osh = spconv_index_nd(coords, num, shape, *first, max1, False, False)
+            index, num_index, oc2, no2, _ = spconv_index_nd(oc, no, osh, *nxt, 8 * n, False, False)
+            assert int(no.item()) == max1
+            got.append(oracle.canonical(index.cpu().numpy(), int(num_index.item()), oc2.cpu().numpy(), int(no2.item())))
+        consumer.link_coords(None)
+        np.testing.assert_array_equal(got[0][0], got[1][0])
+        np.testing.assert_array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("max1,max2", [(32000, 1 << 17), (900, 1 << 17), (1 << 19, 1 << 17), (1 << 19, 30000)])
 def test_large_strided_operator_on_a_strided_operators_map(engine, max1, max2):
     """At capacities from 131072 outputs the table of a linked 3x3x3 stride-2 operator is looked up in the producer's map
