@@ -262,13 +262,14 @@ vxSmall(const float* __restrict__ feats, const int32_t* __restrict__ batchIdx, c
 // a higher one's place as the lowest adds the features of the point it displaced.  Records lie in point order: the
 // emitting pass reads those of voxels with one point in one run, and heads of 8 bytes afford a table of four per point.
 // (The count is exact: the form is for fewer than 2^24 points.)
-// 200 000 points, 135 000 of them in the grid and nearly all in voxels of their own: clear 5.8, insert 11.8, emit 7.8 us, where
+// 200 000 points, 135 000 of them in the grid and nearly all in voxels of their own: clear 5.8, insert 11.8, emit 6.2 us, where
 // entries of 32 bytes in a table of two per point took 8, 16.6 and 10.3: bound by the chains of compare-and-swaps, whose longest
 // went from 16 to 9 with the larger table (eight heads per point: insert 10.0, but with eight points to a voxel the call is 1 us
-// slower).  In a graph of calls 36.0 -> 24.0 us, 100 000 points 27.9 -> 18.4; eight points to a voxel 62 -> 30.6, 400 000 of them
-// with six channels 136 -> 60.  Up to 50 000 points the call is bound by its three launches on the host.
+// slower).  In a graph of calls 36.0 -> 22.8 us, 100 000 points 27.9 -> 16.9; eight points to a voxel 62 -> 28.8, 400 000 of them
+// with six channels 136 -> 55.  Up to 50 000 points the call is bound by its three launches on the host.
 // ---------------------------------------------------------------------------
 constexpr int kVxMaxWide = 12;  // channels a record carries
+constexpr int64_t kVxSmallChunks = 128 * 1024;  // most points of a call in chunks of 256 (see vxEmitWide)
 
 __host__ __device__ constexpr int vxRecordBytes(int C) { return (8 + 4 * C + 15) / 16 * 16; }
 
@@ -350,45 +351,50 @@ vxInsertWide(const float* __restrict__ feats, const int32_t* __restrict__ batchI
 constexpr unsigned long long kVxPublished = 1ull << 32;
 constexpr int kVxSpins = 1 << 16;
 
-// One chunk of 1024 points per workgroup: representatives are ranked in point order, the workgroup publishes its count,
+// One chunk of points per workgroup: representatives are ranked in point order, the workgroup publishes its count,
 // reads how many the chunks before it have (a thread per chunk, so that all states are on their way together, waiting for
 // those that are not there yet) and writes mean and coordinate of its own voxels.  A state is one 64-bit word, flag and
 // value together, so relaxed device-scope accesses are enough.  The wait cannot deadlock - a chunk waits for lower ones
 // only, and those were dispatched before it and wait for nobody before they publish - and it is bounded all the same:
 // after kVxSpins looks the thread counts that chunk's representatives itself.
-template <int CT>
+// The pass is a chain of loads (points, records, features, states), so small calls take chunks of 256 points, which fill the
+// chip: in a graph of calls 10 000 points 13.8 us with chunks of 1024, 11.9 with 512, 10.9 with 256; 50 000 15.5, 13.8, 12.7;
+// 100 000 18.2, 17.0, 16.9.  Every chunk reads the states of all before it: 200 000 points 23.8, 22.7, 23.1, 930 000 63.9, 63.4, 64.3
+// (eight points to a voxel 93.8, 93.5, 96.7).  Hence 256 up to kVxSmallChunks points and 512 beyond.
+template <int CT, int ITEMS>
 __global__ void __launch_bounds__(kVxThreads)
 vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, const unsigned char* __restrict__ records,
            const uint2* __restrict__ points, unsigned long long* states, int32_t maxNumActOut, float* __restrict__ outFeats,
            int32_t* __restrict__ outCoors, int32_t* __restrict__ numActOut) {
+  constexpr int kChunk = kVxThreads * ITEMS;
   const int C = CT ? CT : channels;
   const size_t recordBytes = vxRecordBytes(C);
-  __shared__ uint32_t waveReps[kVxItems][kVxThreads / 64], waveBase[kVxThreads / 64];
+  __shared__ uint32_t waveReps[ITEMS][kVxThreads / 64], waveBase[kVxThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t chunk = blockIdx.x;
-  uint2 point[kVxItems];
-  uint4 head[kVxItems];
-  bool rep[kVxItems];
-  uint32_t below[kVxItems];
+  uint2 point[ITEMS];
+  uint4 head[ITEMS];
+  bool rep[ITEMS];
+  uint32_t below[ITEMS];
 #pragma unroll
-  for (int k = 0; k < kVxItems; ++k) {
-    const int64_t i = static_cast<int64_t>(chunk) * kVxChunk + k * kVxThreads + tid;
+  for (int k = 0; k < ITEMS; ++k) {
+    const int64_t i = static_cast<int64_t>(chunk) * kChunk + k * kVxThreads + tid;
     point[k] = i < n ? points[i] : make_uint2(kVxNone, 0u);
   }
 #pragma unroll
-  for (int k = 0; k < kVxItems; ++k)
+  for (int k = 0; k < ITEMS; ++k)
     head[k] = point[k].x != kVxNone ? *reinterpret_cast<const uint4*>(records + point[k].x * recordBytes) : make_uint4(0, 0, 0, 0);
 #pragma unroll
-  for (int k = 0; k < kVxItems; ++k) {
-    rep[k] = point[k].x != kVxNone && head[k].x == chunk * kVxChunk + k * kVxThreads + tid;
+  for (int k = 0; k < ITEMS; ++k) {
+    rep[k] = point[k].x != kVxNone && head[k].x == chunk * kChunk + k * kVxThreads + tid;
     const unsigned long long m = __ballot(rep[k]);
     below[k] = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
     if (lane == 0) waveReps[k][wave] = static_cast<uint32_t>(__popcll(m));
   }
   __syncthreads();
-  uint32_t total = 0, rank[kVxItems];
+  uint32_t total = 0, rank[ITEMS];
 #pragma unroll
-  for (int k = 0; k < kVxItems; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     rank[k] = total + below[k];
 #pragma unroll
     for (int w = 0; w < kVxThreads / 64; ++w) {
@@ -397,10 +403,10 @@ vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, c
     }
   }
   if (tid == 0) __hip_atomic_store(&states[chunk], kVxPublished | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  float mean[kVxItems][CT ? CT : 1];   // loaded ahead of the wait for the chunks before
+  float mean[ITEMS][CT ? CT : 1];   // loaded ahead of the wait for the chunks before
   if constexpr (CT != 0) {
 #pragma unroll
-    for (int k = 0; k < kVxItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
       if (!rep[k]) continue;
       const float* f = feats + static_cast<size_t>(head[k].x) * CT;
       const float* sums = reinterpret_cast<const float*>(records + point[k].x * recordBytes + 8);
@@ -417,7 +423,7 @@ vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, c
       __builtin_amdgcn_s_sleep(1);
     }
     if (!st)
-      for (int64_t q = static_cast<int64_t>(p) * kVxChunk; q < static_cast<int64_t>(p + 1) * kVxChunk; ++q) {
+      for (int64_t q = static_cast<int64_t>(p) * kChunk; q < static_cast<int64_t>(p + 1) * kChunk; ++q) {
         const uint32_t at = points[q].x;
         if (at != kVxNone && *reinterpret_cast<const uint32_t*>(records + at * recordBytes) == static_cast<uint32_t>(q)) ++st;
       }
@@ -432,7 +438,7 @@ vxEmitWide(const float* __restrict__ feats, int32_t n, int channels, VxGeom g, c
   for (int w = 0; w < kVxThreads / 64; ++w) base += waveBase[w];
   if (tid == 0 && chunk == gridDim.x - 1) *numActOut = static_cast<int32_t>(min(base + total, static_cast<uint32_t>(maxNumActOut)));
 #pragma unroll
-  for (int k = 0; k < kVxItems; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     const uint32_t id = base + rank[k];
     if (!rep[k] || id >= static_cast<uint32_t>(maxNumActOut)) continue;
     float* row = outFeats + static_cast<size_t>(id) * C;
@@ -631,6 +637,8 @@ VxPlan planVoxelize(int64_t numPts, int64_t maxNumActOut, int64_t C) {
       size_t off = alignUp256(static_cast<size_t>(p.slots) * 8);
       p.records = off;
       off = alignUp256(off + static_cast<size_t>(n) * vxRecordBytes(static_cast<int>(C)));
+      const int64_t chunk = kVxThreads * (n <= kVxSmallChunks ? 1 : 2);
+      p.nChunks = static_cast<uint32_t>((n + chunk - 1) / chunk);
       p.pointSlot = off;  // record and key of every point
       off = alignUp256(off + static_cast<size_t>(n) * 8);
       p.chunkBase = off;  // chunk states, u64
@@ -705,7 +713,7 @@ void launchWide(const VoxelizeArgs& a, const VxPlan& p, const VxGeom& g, char* w
 #undef D3D_VX_CLEAR
   hipLaunchKernelGGL(vxInsertWide<CT>, dim3(static_cast<unsigned>((a.numPts + kVxThreads - 1) / kVxThreads)), dim3(kVxThreads), 0,
                      stream, a.feats, a.batchIdx, a.config, static_cast<int32_t>(a.numPts), a.C, g, table, p.slots, records, points);
-  hipLaunchKernelGGL(vxEmitWide<CT>, dim3(p.nChunks), dim3(kVxThreads), 0, stream, a.feats, static_cast<int32_t>(a.numPts), a.C, g,
+  hipLaunchKernelGGL((a.numPts <= kVxSmallChunks ? vxEmitWide<CT, 1> : vxEmitWide<CT, 2>), dim3(p.nChunks), dim3(kVxThreads), 0, stream, a.feats, static_cast<int32_t>(a.numPts), a.C, g,
                      records, points, states, a.maxNumActOut, a.outFeats, a.outCoors, a.numActOut);
 }
 

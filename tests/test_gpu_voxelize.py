@@ -144,10 +144,11 @@ def test_sizes_around_the_forms(engine, n, channels, max_out):
         assert not got_f[got_n:].any()
 
 
-@pytest.mark.parametrize("n,channels", [(260, 3), (50001, 12), (930000, 5), (940000, 5), (1198000, 5), (1210000, 5)])
+@pytest.mark.parametrize("n,channels", [(260, 3), (50001, 12), (131072, 4), (131073, 4), (930000, 5), (940000, 5), (1198000, 5), (1210000, 5)])
 def test_points_that_share_voxels(engine, n, channels):
     """Records: about eight points to a voxel, the lowest of them anywhere among the insertions, with four table heads per
-    point, two (from 932 000 points of five channels on) and, past 1.2 million points, the form of bare keys."""
+    point, two (from 932 000 points of five channels on) and, past 1.2 million points, the form of bare keys; chunks of 256
+    points up to 131 072."""
     rng = np.random.default_rng(n)
     side = max(4, int(round((n / 8) ** (1 / 3))))
     pts = rng.uniform(0, side, (n, channels)).astype(np.float32)
