@@ -186,10 +186,12 @@ __global__ __launch_bounds__(256) void dzGather(const uint8_t* __restrict__ feat
 template <int E>
 void launchGather(const DensifyArgs& a, const int32_t* map, dim3 grid, hipStream_t stream) {
   // Large maps go out XCD by XCD (see dzGather): 60 000 rows of 256 int8 channels into 97 MB 41 -> 31 us, 80 000 of 256 fp16 into
-  // 328 MB 142 -> 130.  Small ones keep the grid as it is: the divisions cost 0.4 us, 3 % of a map of 17 MB.
+  // 328 MB 142 -> 130.  Smaller ones keep the grid as it is: the divisions cost 0.4 us, 3 % of a map of 17 MB.  us with the grid
+  // as it is / by XCD: 34 MB of fp32 (10 000 rows) 13.7 / 15.0, 35 MB of fp16 16.5 / 15.6, 41 MB 17.35 / 17.7, 49 MB of int8
+  // 17.0 / 18.3, 41 MB 15.5 / 16.4 (before the wide stores 14.0, 17.4, 18.9, 19.6, 18.1).
   const uint32_t tiles = grid.x;
   uint32_t pieces = 0;
-  if (static_cast<size_t>(grid.x) * grid.y * grid.z >= (size_t(32) << 20) / (kTile * kChunkBytes)) {
+  if (static_cast<size_t>(grid.x) * grid.y * grid.z >= (size_t(64) << 20) / (kTile * kChunkBytes)) {
     pieces = grid.x * grid.y * grid.z;
     grid = dim3((pieces + 7) / 8 * 8);
   }

@@ -145,8 +145,8 @@ def test_wrong_out_channels_is_an_error(engine):
     ((1, 1, 10, 8), 7, "int8"),         # rows off a word: not in 16-byte stores
     ((1, 2, 33, 24), 200, "bfloat16"),  # four channel chunks, the last one short
     ((2, 3, 31, 48), 132, "int8"),      # a last chunk of one word
-    ((1, 4, 250, 256), 66, "float16"),  # 34 MB and an odd number of workgroups: shared out XCD by XCD
-    ((2, 2, 223, 225), 45, "float32"),  # the same, planes of an odd size
+    ((1, 5, 250, 252), 66, "float16"),  # 9850 workgroups, no multiple of eight: shared out XCD by XCD
+    ((2, 3, 223, 227), 45, "float32"),  # the same with 9492, planes of an odd size
 ])
 def test_wide_stores_and_large_maps(engine, shape, channels, dtype):
     rng = np.random.default_rng(23)
