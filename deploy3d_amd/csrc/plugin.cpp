@@ -878,7 +878,7 @@ struct MMPlugin final : d3d_plugin {
     if ((!linked || inverse) && maxNumActOut > 0) {
       if (!derived) derived = std::make_shared<DeviceBuffer>();
       const void* const before = derived->ptr;
-      const int32_t rc = derived->reserve(derivedBytes(dtype, maxNumActOut));
+      const int32_t rc = derived->reserve(derivedBytes(maxNumActOut));
       if (derived->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
@@ -892,14 +892,17 @@ struct MMPlugin final : d3d_plugin {
   // 64 -> 128, 100 000 scattered 1115 / 515.  Two-byte layers have less to win than the launch costs: 64 -> 64, 30 000 voxels
   // 57 / 68, at stride 2 69 / 89, 110 000 140 / 162 (64 -> 128, 110 000 scattered voxels 217 / 203, the one case the other
   // way).  Kernels of fewer than eight taps have too few steps to lose.
+  bool sortableVolume() const { return kernelVol >= 8 && kernelVol <= 32; }
   bool ordersRows(int32_t dtype) const {
-    return kernelVol >= 8 && kernelVol <= 32 && (inverse || (dtype == D3D_FLOAT && cin >= 32 && cout >= 32));
+    return sortableVolume() && (inverse || (dtype == D3D_FLOAT && cin >= 32 && cout >= 32));
   }
   size_t derivedTableBytes(int64_t outRows) const {
     return (static_cast<size_t>(kernelVol) * static_cast<size_t>(outRows > 0 ? outRows : 1) * sizeof(int32_t) + 15) / 16 * 16;
   }
-  size_t derivedBytes(int32_t dtype, int64_t outRows) const {
-    return derivedTableBytes(outRows) + (ordersRows(dtype) ? orderRowsBytes(outRows) : 0);
+  // The same for every feature type, whether it sorts its rows or not: graphs captured with one type hold the table's address, and
+  // a type that asked for more would free it under them.
+  size_t derivedBytes(int64_t outRows) const {
+    return derivedTableBytes(outRows) + (sortableVolume() ? orderRowsBytes(outRows) : 0);
   }
 
   int32_t configureFloat(int32_t dtype, MMDeviceWeights::Converted& to) {
@@ -1072,7 +1075,7 @@ struct MMPlugin final : d3d_plugin {
     }
     if (!nbr) {  // the index tensor is all there is to go by: derive the table from it
       if (!derived) derived = std::make_shared<DeviceBuffer>();
-      const size_t bytes = derivedBytes(dtype, outRows);
+      const size_t bytes = derivedBytes(outRows);
       if (derived->bytes < bytes && streamIsCapturing(stream)) {
         setError("SPConvMM: the table derived from the index tensor needs %zu bytes that were not reserved before the "
                  "capture (configure the node at these shapes, or enqueue it once, first)", bytes);
