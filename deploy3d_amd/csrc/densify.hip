@@ -19,6 +19,8 @@
 // 11.3 -> 10.2 us per call in a graph of calls, for 38 000 rows of 128 fp16
 // channels into [1, 256, 180, 180]: 26.3 MB, which a large copy moves in 5.7).
 #include "common.h"
+#include "conv_kernels.h"
+#include "densify_grid.h"
 
 namespace d3d {
 namespace {
@@ -74,14 +76,14 @@ __global__ __launch_bounds__(256) void dzMapRows(const int32_t* __restrict__ coo
 template <int E, int PACK, bool VEC>
 __global__ __launch_bounds__(256) void dzGather(const uint8_t* __restrict__ feats, const int32_t* __restrict__ map,
                                                 const int32_t* __restrict__ coors, const int32_t* __restrict__ numAct,
-                                                int32_t cap, DzGrid g, uint8_t* __restrict__ out, int C, int64_t YX, uint32_t tiles, uint32_t pieces) {
+                                                int32_t cap, DzGrid g, uint8_t* __restrict__ out, int C, int64_t YX, uint32_t tiles, uint32_t pieces, int xcdShift) {
   __shared__ int32_t rows[kTile];
   __shared__ __attribute__((aligned(16))) uint8_t tile[kTile * kPitch];
 
   const int t = threadIdx.x;
   uint32_t tileAt = blockIdx.x, planeAt = blockIdx.y, chunkAt = blockIdx.z;
   if (pieces) {   // one-dimensional: XCD x takes the x-th contiguous part, so that lines two tiles share are whole in one L2
-    const uint32_t piece = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    const uint32_t piece = (blockIdx.x & ((1u << xcdShift) - 1u)) * (gridDim.x >> xcdShift) + (blockIdx.x >> xcdShift);
     if (piece >= pieces) return;
     tileAt = piece % tiles;
     planeAt = piece / tiles % (g.B * g.Z);
@@ -184,17 +186,14 @@ __global__ __launch_bounds__(256) void dzGather(const uint8_t* __restrict__ feat
 }
 
 template <int E>
-void launchGather(const DensifyArgs& a, const int32_t* map, dim3 grid, hipStream_t stream) {
+void launchGather(const DensifyArgs& a, const int32_t* map, int64_t tiles, int64_t planes, int64_t chunks, hipStream_t stream) {
   // Large maps go out XCD by XCD (see dzGather): 60 000 rows of 256 int8 channels into 97 MB 41 -> 31 us, 80 000 of 256 fp16 into
   // 328 MB 142 -> 130.  Smaller ones keep the grid as it is: the divisions cost 0.4 us, 3 % of a map of 17 MB.  us with the grid
   // as it is / by XCD: 34 MB of fp32 (10 000 rows) 13.7 / 15.0, 35 MB of fp16 16.5 / 15.6, 41 MB 17.35 / 17.7, 49 MB of int8
   // 17.0 / 18.3, 41 MB 15.5 / 16.4 (before the wide stores 14.0, 17.4, 18.9, 19.6, 18.1).
-  const uint32_t tiles = grid.x;
-  uint32_t pieces = 0;
-  if (static_cast<size_t>(grid.x) * grid.y * grid.z >= (size_t(64) << 20) / (kTile * kChunkBytes)) {
-    pieces = grid.x * grid.y * grid.z;
-    grid = dim3((pieces + 7) / 8 * 8);
-  }
+  const int xcdShift = convk::chipLayout().xcdShift;
+  const DensifyGrid dg = densifyGrid(tiles, planes, chunks, xcdShift);
+  const dim3 grid(dg.x, dg.y, dg.z);
   const int64_t yx = static_cast<int64_t>(a.Y) * a.X;
   const bool vec = (static_cast<size_t>(a.C) * E) % 16 == 0 && reinterpret_cast<uintptr_t>(a.feats) % 16 == 0;
   const bool wide = yx % (16 / E) == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && a.C * E % 4 == 0;
@@ -203,7 +202,7 @@ void launchGather(const DensifyArgs& a, const int32_t* map, dim3 grid, hipStream
   const DzGrid g{a.B, a.Z, a.Y, a.X};
   const uint8_t* f = static_cast<const uint8_t*>(a.feats);
   uint8_t* o = static_cast<uint8_t*>(a.out);
-#define D3D_DZ(P, V) hipLaunchKernelGGL((dzGather<E, P, V>), grid, dim3(256), 0, stream, f, map, a.coors, a.numAct, a.cap, g, o, a.C, yx, tiles, pieces)
+#define D3D_DZ(P, V) hipLaunchKernelGGL((dzGather<E, P, V>), grid, dim3(256), 0, stream, f, map, a.coors, a.numAct, a.cap, g, o, a.C, yx, static_cast<uint32_t>(tiles), dg.pieces, xcdShift)
   if (wide) {
     if (vec) D3D_DZ(16 / E, true); else D3D_DZ(16 / E, false);
   } else if (pack) {
@@ -232,8 +231,7 @@ int32_t launchDensify(const DensifyArgs& a, hipStream_t stream) {
     setError("BEVDensify: elements of %d bytes not implemented", E);
     return D3D_ERR_UNSUPPORTED;
   }
-  // (2^31 workgroups of 64 cells x 128 bytes would write 16 TB)
-  if (planes > 65535 || chunks > 65535 || cells >= (int64_t(1) << 31) || tiles * planes * chunks >= (int64_t(1) << 31) - 8) {
+  if (planes > 65535 || chunks > 65535 || cells >= (int64_t(1) << 31)) {
     setError("BEVDensify: grid [%d, %d, %d, %d] x %d channels exceeds the launch limits", a.B, a.Z, a.Y, a.X, a.C);
     return D3D_ERR_BAD_ARG;
   }
@@ -249,10 +247,9 @@ int32_t launchDensify(const DensifyArgs& a, hipStream_t stream) {
   if (a.cap > 0)
     hipLaunchKernelGGL(dzMapRows, dim3(static_cast<unsigned>((a.cap + 255) / 256)), dim3(256), 0, stream, a.coors,
                        a.numAct, a.cap, DzGrid{a.B, a.Z, a.Y, a.X}, map);
-  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(planes), static_cast<unsigned>(chunks));
-  if (E == 4) launchGather<4>(a, map, grid, stream);
-  else if (E == 2) launchGather<2>(a, map, grid, stream);
-  else launchGather<1>(a, map, grid, stream);
+  if (E == 4) launchGather<4>(a, map, tiles, planes, chunks, stream);
+  else if (E == 2) launchGather<2>(a, map, tiles, planes, chunks, stream);
+  else launchGather<1>(a, map, tiles, planes, chunks, stream);
   D3D_HIP_CHECK(hipGetLastError());
   return D3D_OK;
 }
