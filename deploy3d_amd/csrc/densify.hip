@@ -25,8 +25,7 @@
 namespace d3d {
 namespace {
 
-constexpr int kTile = 64;          // cells per workgroup, consecutive in y*X + x
-constexpr int kChunkBytes = 128;   // bytes of a feature row handled by one workgroup
+constexpr int kTile = kDzTile, kChunkBytes = kDzChunkBytes;
 constexpr int kPitch = kChunkBytes + 4;  // LDS bytes per cell: an odd number of dwords
 
 struct DzGrid {
@@ -186,15 +185,11 @@ __global__ __launch_bounds__(256) void dzGather(const uint8_t* __restrict__ feat
 }
 
 template <int E>
-void launchGather(const DensifyArgs& a, const int32_t* map, int64_t tiles, int64_t planes, int64_t chunks, hipStream_t stream) {
-  // Large maps go out XCD by XCD (see dzGather): 60 000 rows of 256 int8 channels into 97 MB 41 -> 31 us, 80 000 of 256 fp16 into
-  // 328 MB 142 -> 130.  Smaller ones keep the grid as it is: the divisions cost 0.4 us, 3 % of a map of 17 MB.  us with the grid
-  // as it is / by XCD: 34 MB of fp32 (10 000 rows) 13.7 / 15.0, 35 MB of fp16 16.5 / 15.6, 41 MB 17.35 / 17.7, 49 MB of int8
-  // 17.0 / 18.3, 41 MB 15.5 / 16.4 (before the wide stores 14.0, 17.4, 18.9, 19.6, 18.1).
+void launchGather(const DensifyArgs& a, const int32_t* map, hipStream_t stream) {
   const int xcdShift = convk::chipLayout().xcdShift;
-  const DensifyGrid dg = densifyGrid(tiles, planes, chunks, xcdShift);
-  const dim3 grid(dg.x, dg.y, dg.z);
   const int64_t yx = static_cast<int64_t>(a.Y) * a.X;
+  const DensifyGrid dg = densifyGrid(yx, static_cast<int64_t>(a.B) * a.Z, a.C, E, xcdShift);
+  const dim3 grid(dg.x, dg.y, dg.z);
   const bool vec = (static_cast<size_t>(a.C) * E) % 16 == 0 && reinterpret_cast<uintptr_t>(a.feats) % 16 == 0;
   const bool wide = yx % (16 / E) == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && a.C * E % 4 == 0;
   constexpr int kPack = 4 / E;
@@ -202,7 +197,7 @@ void launchGather(const DensifyArgs& a, const int32_t* map, int64_t tiles, int64
   const DzGrid g{a.B, a.Z, a.Y, a.X};
   const uint8_t* f = static_cast<const uint8_t*>(a.feats);
   uint8_t* o = static_cast<uint8_t*>(a.out);
-#define D3D_DZ(P, V) hipLaunchKernelGGL((dzGather<E, P, V>), grid, dim3(256), 0, stream, f, map, a.coors, a.numAct, a.cap, g, o, a.C, yx, static_cast<uint32_t>(tiles), dg.pieces, xcdShift)
+#define D3D_DZ(P, V) hipLaunchKernelGGL((dzGather<E, P, V>), grid, dim3(256), 0, stream, f, map, a.coors, a.numAct, a.cap, g, o, a.C, yx, static_cast<uint32_t>((yx + kTile - 1) / kTile), dg.pieces, xcdShift)
   if (wide) {
     if (vec) D3D_DZ(16 / E, true); else D3D_DZ(16 / E, false);
   } else if (pack) {
@@ -223,7 +218,6 @@ int32_t launchDensify(const DensifyArgs& a, hipStream_t stream) {
   const int64_t cells = static_cast<int64_t>(a.B) * a.Z * a.Y * a.X;
   if (cells == 0 || a.C == 0) return D3D_OK;  // nothing to write
   const int64_t yx = static_cast<int64_t>(a.Y) * a.X;
-  const int64_t tiles = (yx + kTile - 1) / kTile;
   const int64_t planes = static_cast<int64_t>(a.B) * a.Z;
   const int E = a.elemBytes;
   const int64_t chunks = (static_cast<int64_t>(a.C) * E + kChunkBytes - 1) / kChunkBytes;
@@ -247,9 +241,9 @@ int32_t launchDensify(const DensifyArgs& a, hipStream_t stream) {
   if (a.cap > 0)
     hipLaunchKernelGGL(dzMapRows, dim3(static_cast<unsigned>((a.cap + 255) / 256)), dim3(256), 0, stream, a.coors,
                        a.numAct, a.cap, DzGrid{a.B, a.Z, a.Y, a.X}, map);
-  if (E == 4) launchGather<4>(a, map, tiles, planes, chunks, stream);
-  else if (E == 2) launchGather<2>(a, map, tiles, planes, chunks, stream);
-  else launchGather<1>(a, map, tiles, planes, chunks, stream);
+  if (E == 4) launchGather<4>(a, map, stream);
+  else if (E == 2) launchGather<2>(a, map, stream);
+  else launchGather<1>(a, map, stream);
   D3D_HIP_CHECK(hipGetLastError());
   return D3D_OK;
 }

@@ -13,21 +13,42 @@
 
 namespace {
 
-// Dense maps: every piece has a workgroup, and no dimension of a launch has 2^32 threads or more.
+// Dense maps: every piece has a workgroup, no dimension of a launch has 2^32 threads or more, and what counts for the line is the
+// map itself, not the bytes that whole chunks would have.
 int denseMaps() {
+  struct Shape {
+    int64_t yx, planes, channels;
+    int elemBytes;
+    bool byXcd;
+  };
   const int64_t k24 = int64_t(1) << 24;
-  // 2^30 cells of four int8 channels in 64 planes, and sizes around 2^24 workgroups
-  const int64_t shapes[][3] = {{262144, 64, 1}, {k24 - 1, 1, 1}, {k24 / 8 - 1, 8, 1}, {k24 / 8, 8, 1}, {k24 / 16, 4, 4}, {k24 / 8 + 1, 8, 1},
-                               {8191, 1, 1}, {8192, 1, 1}, {1, 1, 1}, {507, 2, 2}, {2704, 2, 2}, {3, 65535, 65535}};
-  for (const auto& s : shapes)
+  const Shape shapes[] = {
+      {int64_t(4096) * 4096, 64, 4, 1, false},   // 2^24 workgroups, 4.3 GB
+      {int64_t(4095) * 4095, 64, 4, 1, true},    // fewer, planes off the tiles
+      {int64_t(4097) * 4095, 64, 4, 1, false},   // more
+      {k24 * 8 - 63, 8, 2, 2, false},            // 2^24 workgroups exactly, 2^24 - 8 below
+      {(k24 / 8 - 1) * 64 - 1, 8, 2, 2, true},
+      {int64_t(300) * 320, 2, 256, 2, false},    // planes of whole lines
+      {int64_t(300) * 301, 4, 128, 2, true},
+      {int64_t(200) * 200, 4, 256, 1, false},    // planes of whole int8 tiles
+      {int64_t(300) * 300, 4, 256, 4, true},     // a line off by half
+      {int64_t(300) * 301, 2, 32, 1, false},     // 5.8 MB: 16 MB in whole chunks
+      {int64_t(300) * 301, 8, 32, 1, true},
+      {int64_t(180) * 181, 2, 256, 1, false},
+      {int64_t(181) * 182, 2, 256, 1, true},
+      {1, 1, 1, 4, false},
+      {129, 65535, 1, 1, false},
+  };
+  for (const Shape& s : shapes)
     for (int xcdShift = 0; xcdShift <= 3; ++xcdShift) {
-      const d3d::DensifyGrid g = d3d::densifyGrid(s[0], s[1], s[2], xcdShift);
+      const d3d::DensifyGrid g = d3d::densifyGrid(s.yx, s.planes, s.channels, s.elemBytes, xcdShift);
       CHECK(static_cast<uint64_t>(g.x) * 256 < (uint64_t(1) << 32) && g.y <= 65535 && g.z <= 65535);
-      const int64_t pieces = s[0] * s[1] * s[2];
+      CHECK((g.pieces != 0) == s.byXcd);
+      const int64_t tiles = (s.yx + 63) / 64, chunks = (s.channels * s.elemBytes + 127) / 128, pieces = tiles * s.planes * chunks;
       if (g.pieces) {
         CHECK(g.pieces == pieces && g.y == 1 && g.z == 1 && g.x >= pieces && g.x < pieces + (1 << xcdShift) && g.x % (1 << xcdShift) == 0);
       } else {
-        CHECK(g.x == s[0] && g.y == s[1] && g.z == s[2]);
+        CHECK(g.x == tiles && g.y == s.planes && g.z == chunks);
       }
     }
   return 0;

@@ -146,7 +146,10 @@ def test_wrong_out_channels_is_an_error(engine):
     ((1, 2, 33, 24), 200, "bfloat16"),  # four channel chunks, the last one short
     ((2, 3, 31, 48), 132, "int8"),      # a last chunk of one word
     ((1, 5, 250, 252), 66, "float16"),  # 9850 workgroups, no multiple of eight: shared out XCD by XCD
-    ((2, 3, 223, 227), 45, "float32"),  # the same with 9492, planes of an odd size
+    ((2, 3, 223, 227), 45, "float32"),  # 9492 of planes of an odd size
+    ((2, 3, 251, 253), 45, "float32"),  # 11916 of them: shared out as well
+    ((1, 2, 301, 303), 97, "int8"),     # the same with rows off a word
+    ((1, 5, 256, 250), 66, "float16"),  # as large, planes of whole lines: not shared out
 ])
 def test_wide_stores_and_large_maps(engine, shape, channels, dtype):
     rng = np.random.default_rng(23)
