@@ -217,7 +217,6 @@ size_t densifyWorkspaceBytes(int64_t B, int64_t Z, int64_t Y, int64_t X) {
 int32_t launchDensify(const DensifyArgs& a, hipStream_t stream) {
   const int64_t cells = static_cast<int64_t>(a.B) * a.Z * a.Y * a.X;
   if (cells == 0 || a.C == 0) return D3D_OK;  // nothing to write
-  const int64_t yx = static_cast<int64_t>(a.Y) * a.X;
   const int64_t planes = static_cast<int64_t>(a.B) * a.Z;
   const int E = a.elemBytes;
   const int64_t chunks = (static_cast<int64_t>(a.C) * E + kChunkBytes - 1) / kChunkBytes;

@@ -871,7 +871,7 @@ struct MMPlugin final : d3d_plugin {
     if (in[0].nb_dims == 2 && in[0].dims[0] > 0 && weights.cinMfma > cin) {
       if (!widened) widened = std::make_shared<DeviceBuffer>();
       const void* const before = widened->ptr;
-      const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * weights.cinMfma * dtypeBytes(dtype));
+      const int32_t rc = widened->reserve(static_cast<size_t>(in[0].dims[0]) * widenedRowBytes());
       if (widened->ptr != before) ++changes;
       if (rc != D3D_OK) return rc;
     }
@@ -883,6 +883,17 @@ struct MMPlugin final : d3d_plugin {
       if (rc != D3D_OK) return rc;
     }
     return D3D_OK;
+  }
+
+  // Bytes of a widened row of the type that has the longest ones: graphs captured with one type hold the rows' address, and another
+  // type's would be freed under them.
+  size_t widenedRowBytes() const {
+    size_t most = 0;
+    for (const int32_t t : {D3D_FLOAT, D3D_HALF, D3D_BF16, D3D_INT8}) {
+      const int wide = paddedMfmaChannels(t, cin, cout);
+      if (wide > cin && static_cast<size_t>(wide) * dtypeBytes(t) > most) most = static_cast<size_t>(wide) * dtypeBytes(t);
+    }
+    return most;
   }
 
   // Layers that put the rows of their derived table in the order of their taps, where their kernel takes that (orderRows):
@@ -1114,7 +1125,7 @@ struct MMPlugin final : d3d_plugin {
                                                      debugEnv("D3D_CONV_NO_PAD") == nullptr))) {  // narrow layer: widen the rows, then MFMA
       if (!widened) widened = std::make_shared<DeviceBuffer>();
       const int es = dtypeBytes(dtype);
-      const size_t wideBytes = static_cast<size_t>(a.inRows > 0 ? a.inRows : 1) * weights.cinMfma * es;
+      const size_t wideBytes = static_cast<size_t>(a.inRows > 0 ? a.inRows : 1) * widenedRowBytes();
       if (widened->bytes < wideBytes && streamIsCapturing(stream)) {
         setError("SPConvMM: %zu bytes for the widened input rows were not reserved before the capture", wideBytes);
         return D3D_ERR_UNSUPPORTED;
