@@ -22,7 +22,7 @@ SYNTH_LIB = os.path.join(LIBS, "libd3d_synth.so")
 
 ENGINE_SOURCES = ["rulebook.hip", "conv.hip", "conv_half.hip", "conv_bf16.hip", "conv_int8.hip", "conv_f32.hip", "conv_pipe_half.hip",
                   "conv_pipe_bf16.hip", "conv_pipe_int8.hip", "order.hip", "densify.hip", "voxelize.hip", "elementwise.hip", "scratch.hip", "plugin.cpp", "schedule.cpp", "schedule_capture.cpp"]
-ENGINE_HEADERS = ["common.h", "conv_kernels.h", "conv_pipe.h", "conv_solo.h", "conv_taps.h", "densify_grid.h", "schedule.h", os.path.join(ROOT, "include", "d3d_spconv.h")]
+ENGINE_HEADERS = ["common.h", "conv_kernels.h", "conv_pipe.h", "conv_solo.h", "conv_taps.h", "deal.h", "densify_grid.h", "schedule.h", os.path.join(ROOT, "include", "d3d_spconv.h")]
 # per-source extra flags
 EXTRA_FLAGS = {
     # keeps the MFMA accumulators of the pipelined kernel in VGPRs (see the header of the two files)

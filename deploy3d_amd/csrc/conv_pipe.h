@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "conv_kernels.h"
+#include "deal.h"
 
 namespace d3d {
 namespace convk {
@@ -59,7 +60,7 @@ template <int PER, int CHUNK, int ROUNDS>                // ROUNDS = 0: never de
 struct TileDeal {
   static constexpr int SLOTS = 4;                        // registers of tiles ranked together
   TileOrder order;
-  int first, per, mine, list;                            // list: lane p holds the p-th of `mine` dealt tiles
+  int first, per, mine, list;                            // list: lane p holds the tile of turn p, `mine` of them
   bool dealt;
   __device__ __forceinline__ TileDeal(int tiles, int live, int xcdShift, int xcd, int first_, int per_,
                                       const unsigned long long* __restrict__ tileMasks, int kVol, unsigned long long allTaps, int lane)
@@ -104,15 +105,14 @@ struct TileDeal {
           }
         }
       }
-      const int had = mine;
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
-        const int round = rank[s] / per, place = rank[s] - round * per;
-        unsigned long long b = __ballot(taps[s] >= 0 && place == (round & 1 ? per - 1 - first : first));
+        const DealtTile to = dealTile(from, rank[s], per);
+        unsigned long long b = __ballot(taps[s] >= 0 && to.workgroup == first);
         for (; b; b &= b - 1) {
           const int l = __builtin_ctzll(b);
-          const int pos = had + __builtin_amdgcn_readlane(round, l), t = __builtin_amdgcn_readlane(at[s], l);
-          if (lane == pos) list = t;
+          const int turn = __builtin_amdgcn_readlane(to.turn, l), t = __builtin_amdgcn_readlane(at[s], l);
+          if (lane == turn) list = t;
           ++mine;
         }
       }

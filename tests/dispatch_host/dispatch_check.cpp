@@ -1,6 +1,8 @@
 // Host check of how work is cut into workgroups: arithmetic of csrc headers that needs no GPU.
 #include <cstdio>
+#include <vector>
 
+#include "deal.h"
 #include "densify_grid.h"
 
 #define CHECK(cond)                                                                 \
@@ -54,10 +56,36 @@ int denseMaps() {
   return 0;
 }
 
+// Dealt tiles: ranked in batches of 256, each goes to one workgroup; a workgroup's turns follow one another without a gap and no
+// workgroup has two tiles more than another.
+int dealtTiles() {
+  for (int per : {1, 2, 3, 31, 32, 48, 64, 95, 96, 192})
+    for (int tiles : {1, 100, 255, 256, 257, 700, 1024, 1537, 32 * per}) {
+      std::vector<int> has(static_cast<size_t>(per), 0);
+      std::vector<std::vector<bool>> turns(static_cast<size_t>(per), std::vector<bool>(static_cast<size_t>(tiles / per) + 1));
+      for (int from = 0; from < tiles; from += 256)
+        for (int rank = 0; rank < 256 && from + rank < tiles; ++rank) {
+          const d3d::DealtTile to = d3d::dealTile(from, rank, per);
+          CHECK(to.workgroup >= 0 && to.workgroup < per && to.turn >= 0 && to.turn <= tiles / per);
+          CHECK(!turns[to.workgroup][to.turn]);
+          turns[to.workgroup][to.turn] = true;
+          ++has[to.workgroup];
+        }
+      int least = tiles, most = 0;
+      for (int w = 0; w < per; ++w) {
+        for (int t = 0; t < has[w]; ++t) CHECK(turns[w][t]);
+        least = has[w] < least ? has[w] : least;
+        most = has[w] > most ? has[w] : most;
+      }
+      CHECK(most - least <= 1);
+    }
+  return 0;
+}
+
 }  // namespace
 
 int main() {
-  if (denseMaps()) return 1;
+  if (denseMaps() || dealtTiles()) return 1;
   std::puts("dispatch_check ok");
   return 0;
 }

@@ -654,12 +654,13 @@ def test_a_captured_layer_keeps_its_weights_when_another_type_is_run(engine):
         check_close(out.float().cpu().numpy(), ref["float16"], "float16")
 
 
-@pytest.mark.parametrize("cin,dtype,n,room", [(64, "float32", 50000, 0), (64, "float32", 70001, 9000), (128, "float32", 30011, 300),
-                                              (64, "float16", 524999, 0), (128, "bfloat16", 197001, 4000),
-                                              (64, "int8", 790003, 10000)])
-def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
-    """Which workgroup takes a tile changes nothing: a layer of many tiles, dealt to workgroups by the taps they hold, against the
-    halves of its rows, of which each has too few tiles to be dealt.  Levels hold different shares of their cells, so tiles
+@pytest.mark.parametrize("cin,dtype,n,room,parts", [(64, "float32", 50000, 0, 2), (64, "float32", 70001, 9000, 2),
+                                                    (128, "float32", 30011, 300, 2), (64, "float32", 300001, 700, 7),
+                                                    (64, "float16", 524999, 0, 2), (128, "bfloat16", 197001, 4000, 2),
+                                                    (64, "int8", 790003, 10000, 2)])
+def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room, parts):
+    """Which workgroup takes a tile changes nothing: a layer of many tiles, dealt to workgroups by the taps they hold (one with more
+    tiles than are ranked together), against parts of its rows, of which each has too few tiles to be dealt.  Levels hold different shares of their cells, so tiles
     hold 9 to 27 taps.  Bit for bit, rows past the live ones included: a tap no row has adds zeros."""
     from deploy3d_amd import layers, synth
     from deploy3d_amd.spconv_mm import spconv_mm
@@ -684,16 +685,16 @@ def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room):
     x = layers.make_input(coords, feats, grid, dtype=torch_dtype, capacity=n + room)
     got = net.forward(x).feats.clone()
     rb = net.rulebooks["s"]
-    half = (n + room + 1) // 2
-    for lo in (0, half):
+    part = (n + room + parts - 1) // parts
+    for lo in range(0, n + room, part):
         index = rb.index.clone()
         index[1] -= lo
-        other = (index[1] < 0) | (index[1] >= half) | (index[2] < 0)
+        other = (index[1] < 0) | (index[1] >= part) | (index[2] < 0)
         index[1:, other] = -1
-        live = torch.tensor([min(max(n - lo, 0), half)], dtype=torch.int32, device="cuda")
-        want = spconv_mm(x.feats, x.num_act, live, index, rb.num_index, (3, 3, 3), cin, cin, half, True, False,
+        live = torch.tensor([min(max(n - lo, 0), part)], dtype=torch.int32, device="cuda")
+        want = spconv_mm(x.feats, x.num_act, live, index, rb.num_index, (3, 3, 3), cin, cin, part, True, False,
                          weight.reshape(-1), bias, relu=spec["relu"], **scales)
-        assert torch.equal(got[lo:lo + half], want[:n + room - lo])
+        assert torch.equal(got[lo:lo + part], want[:n + room - lo])
 
 
 @pytest.mark.parametrize("n,room", [(1, 0), (63, 5), (511, 1), (512, 0), (513, 511), (3100, 1500)])
