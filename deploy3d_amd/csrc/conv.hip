@@ -355,7 +355,8 @@ int32_t launchBuildNeighbours(const int32_t* index, int64_t rowLen, const int32_
   return D3D_OK;
 }
 
-// The kernels that store through rowOrder are convPipe's (conv_pipe.h) and, for fp32 and two-byte 32 -> 16, convMfmaResident.
+// The kernels that store through rowOrder are convPipe's (conv_pipe.h) for fp32 and for two-byte layers of 128 output channels, and
+// convMfmaResident for fp32 and two-byte 32 -> 16.
 bool convTakesRowOrder(const ConvArgs& a) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
   // 32-bit offsets into the table
@@ -365,7 +366,8 @@ bool convTakesRowOrder(const ConvArgs& a) {
   const int es = a.dtype == D3D_FLOAT ? 4 : (a.dtype == D3D_INT8 ? 1 : 2);
   if (a.cout == 16 || (es == 4 && a.cin == 16 && a.cout == 32))
     return es == 4 ? a.cin <= 32 && floatMfmaFits(a.kVol, a.cin, a.cout) : es == 2 && a.cin == 32 && a.kVol <= 32;
-  if (es == 2 && a.cin == 32 && a.cout == 32) return false;      // convSolo
+  // (the other two-byte shapes and int8 lose more by the sort than it gives: no instantiation takes their rows)
+  if (es == 1 || (es == 2 && (a.cout != 128 || a.cin < 64))) return false;
   // what the pipelined kernel's launcher asks for, with a tile of room
   return a.cin * es >= 64 && a.kVol <= 64 && static_cast<uint64_t>(a.inRows) * (a.cin * es) < 0xFFFF0000ull &&
          static_cast<uint64_t>(a.outRows) + 512 < 0x3FFFFFFFull;

@@ -737,12 +737,8 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
   // takes the shape of the two-byte layer with half its input channels
   constexpr int RB = CIN * static_cast<int>(sizeof(T));
   // rows in the order of their taps: the narrower a tile, the fewer taps it has
-  if constexpr (sizeof(T) < 4)
-    if (a.rowOrder) {
-      if constexpr (COUT >= 128 && (sizeof(T) == 1 || CIN >= 64)) return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
-      else if constexpr (COUT >= 128) return launchPipeCfg<T, CIN, COUT, 3, 4>(a, stream);
-      else return launchPipeCfg<T, CIN, COUT, 4, 4>(a, stream);
-    }
+  if constexpr (sizeof(T) == 2 && COUT == 128 && CIN >= 64)
+    if (a.rowOrder) return launchPipeCfg<T, CIN, COUT, 3, 4, 64>(a, stream);
   if constexpr (sizeof(T) == 4) {
     // fp32: a step's MFMAs take eight times the cycles of a two-byte step with the same bytes, so the matrix pipe is
     // the bound and the tile only has to spread over the CUs: 128 rows, two or three workgroups per CU (16 -> 128: eight

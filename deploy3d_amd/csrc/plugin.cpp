@@ -896,16 +896,34 @@ struct MMPlugin final : d3d_plugin {
     return most;
   }
 
-  // Layers that put the rows of their derived table in the order of their taps, where their kernel takes that (orderRows):
-  // inverse convolutions, and fp32 ones of 32 channels and more, which without masks multiply every tap of every tile at the
-  // matrix pipe's rate.  us of an unlinked layer with its rulebook, fp32, unsorted / sorted: 32 -> 32, 3 000 voxels 47 / 44;
-  // 64 -> 64, 8 000 scattered voxels 68 / 48, 60 000 of a scan 173 / 125; at stride 2 32 -> 64, 60 000 of a scan 207 / 173,
-  // 64 -> 128, 100 000 scattered 1115 / 515.  Two-byte layers have less to win than the launch costs: 64 -> 64, 30 000 voxels
-  // 57 / 68, at stride 2 69 / 89, 110 000 140 / 162 (64 -> 128, 110 000 scattered voxels 217 / 203, the one case the other
-  // way).  Kernels of fewer than eight taps have too few steps to lose.
+  // Does the layer put the rows of its derived table in the order of their taps (orderRows, where its kernel takes that)?  The sort
+  // and the masks cost 6-10 us; what they give is the steps a tile is spared, so the lines lie where a layer's tiles have many steps
+  // at the matrix pipe's rate, or more than one round of tiles.  us of an enqueue with its table's fill and scatter, unsorted / sorted:
+  // Inverse, from stride 2 (LiDAR-like scans; uniform clouds agree).  fp32: 64 -> 32, 8 000 rows 40.7 / 37.8, 110 000 126 / 72; 128 -> 64
+  // 80.7 / 63.9 and 392 / 172; 32 -> 16, 1 000 rows 19.5 / 21.6, 2 000 28.3 / 23.4, 110 000 59.5 / 47.6; 32 -> 32, 16 000 rows 27.2 / 33.9,
+  // 40 000 42.1 / 40.4, 110 000 76.8 / 54.8; 16 -> 16, 60 000 rows 29.6 / 30.9, 110 000 41.8 / 39.0; 16 -> 128, 60 000 rows 73 / 80.9, 75 000
+  // 129 / 125; 32 -> 64, 16 000 rows 28.6 / 34.6, 30 000 43.1 / 39.1.  Two-byte types: 32 -> 16, 2 000 rows 26 / 19.2, 60 000 32.8 / 29.3, 110 000
+  // 37.8 / 37.6; 128 -> 128, 16 000 rows 29.4 / 37.8, 60 000 62 / 65, 75 000 82.7 / 70.8, 250 000 231 / 173; 64 -> 128, 110 000 rows 67 / 63, 250 000
+  // 127 / 106; the others never: 64 -> 32, 8 000 rows 17.7 / 24, 100 000 37 / 42.5, 64 -> 64, 250 000 rows 73.5 / 89, 128 -> 64 131 / 128, 32 -> 128
+  // 83 / 87.  int8 never: 64 -> 64, 30 000 rows 20.9 / 29, 128 -> 128, 110 000 rows 70.6 / 66.5.
+  // (Inverses of stride 1, whose rows have taps of their own each, lose where a scan is dense: fp32 64 -> 32, 30 000 rows 45.8 / 53.2, uniform
+  // 45.6 / 50.2, 1 000 rows 40.1 / 31.1; the two cannot be told apart before the table is there.)
+  // Forward, fp32 only (unlinked): 64 -> 64 of a scan, 1 000 rows 40.2 / 16.8, 30 000 67.4 / 62.6, 110 000 200 / 110, uniform 30 000 66.6 / 32.5
+  // (30 000 rows that fill their grid 69 / 78.6); 32 -> 64, 8 000 rows 26.4 / 25.6, 30 000 40.4 / 41.6, 60 000 71.9 / 52.7.  32 output channels have
+  // one round of tiles up to 98 304 rows: 32 -> 32 of a scan, 8 000 rows 26.1 / 25.4, 30 000 27.9 / 34, 90 000 57.4 / 63.8, 110 000 75.6 / 58.4;
+  // 64 -> 32, 16 000 rows 41.5 / 38, 30 000 42.9 / 48.8, 90 000 93.2 / 100.4, 110 000 123.6 / 79.7.  (Uniform clouds gain there too, 32 -> 32, 30 000 rows
+  // 27.6 / 22.9: scans decide.)  Two-byte forward layers: 64 -> 64 with its rulebook, 30 000 voxels 57 / 68, 110 000 140 / 162.
+  // Kernels of fewer than eight taps have too few steps to lose.  `wide`: the input channels the kernel contracts.
   bool sortableVolume() const { return kernelVol >= 8 && kernelVol <= 32; }
-  bool ordersRows(int32_t dtype) const {
-    return sortableVolume() && (inverse || (dtype == D3D_FLOAT && cin >= 32 && cout >= 32));
+  bool ordersRows(int32_t dtype, int wide, int64_t rows) const {
+    if (!sortableVolume()) return false;
+    if (const char* e = debugEnv("D3D_CONV_ORDER")) return e[0] == '1';   // tests: wherever the kernel takes it, or nowhere
+    if (dtype == D3D_INT8) return false;
+    if (dtype != D3D_FLOAT) return inverse && (cout == 16 || (cout == 128 && wide >= 64 && rows * wide >= 1 << 23));
+    if (!inverse) return cin >= 32 && cout >= 32 && (cout > 32 || wide > 64 || rows <= (wide == 32 ? 12288 : 24576) || rows > 98304);
+    if (wide >= 64) return true;
+    if (wide == 32) return rows >= (cout == 16 ? 2048 : cout == 32 ? 32768 : cout == 64 ? 24576 : 8192);
+    return rows >= (cout == 16 ? 98304 : cout == 32 ? 2048 : cout == 64 ? 32768 : 65536);
   }
   size_t derivedTableBytes(int64_t outRows) const {
     return (static_cast<size_t>(kernelVol) * static_cast<size_t>(outRows > 0 ? outRows : 1) * sizeof(int32_t) + 15) / 16 * 16;
@@ -1150,7 +1168,7 @@ struct MMPlugin final : d3d_plugin {
     a.zeros = zeros;
     if (const char* e = debugEnv("D3D_CONV_PIPE")) a.pipe = e[0] == '0' ? -1 : 0;
     a.tileRows = tileRowsOverride();
-    if (derived && nbr == derived->ptr && ordersRows(dtype) && convTakesRowOrder(a)) {
+    if (derived && nbr == derived->ptr && ordersRows(dtype, a.cin, outRows) && convTakesRowOrder(a)) {
       const RowOrder order = orderRowsAt(static_cast<char*>(derived->ptr) + derivedTableBytes(outRows), outRows);
       rc = launchOrderRows(static_cast<int32_t*>(derived->ptr), kernelVol, outRows, a.numActOut, order, stream);
       if (rc != D3D_OK) return rc;

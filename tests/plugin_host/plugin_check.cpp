@@ -17,6 +17,7 @@ std::set<void*> freed;
 const int32_t* derivedTable = nullptr;   // the table of the last launchBuildNeighbours
 d3d::ConvArgs lastConv;                  // of the last launchConv
 bool capturing = false;
+int sorts = 0;                           // launchOrderRows so far
 int padTo = 0;                           // channels that narrow layers are widened to (0: they are not)
 }  // namespace
 
@@ -59,7 +60,10 @@ int32_t launchBuildNeighbours(const int32_t*, int64_t, const int32_t*, bool, int
   derivedTable = nbr;
   return D3D_OK;
 }
-int32_t launchOrderRows(int32_t*, int, int64_t, const int32_t*, const RowOrder&, hipStream_t) { return D3D_OK; }
+int32_t launchOrderRows(int32_t*, int, int64_t, const int32_t*, const RowOrder&, hipStream_t) {
+  ++sorts;
+  return D3D_OK;
+}
 size_t orderRowsBytes(int64_t outRows) { return static_cast<size_t>(outRows) * 5 + 128; }
 RowOrder orderRowsAt(void* base, int64_t) { return {static_cast<int32_t*>(base), static_cast<unsigned long long*>(base)}; }
 bool convTakesRowOrder(const ConvArgs&) { return true; }
@@ -178,10 +182,39 @@ int widenedRowsStay() {
     }
   return 0;
 }
+
+// Which layers sort the rows of their derived table: those that were measured to gain by it, on both sides of each line.
+int sortedLayers() {
+  struct Layer {
+    int32_t dtype, kVol, cin, cout, rows;
+    bool inverse, sorted;
+  };
+  const Layer layers[] = {
+      {D3D_FLOAT, 27, 64, 32, 300, true, true},      {D3D_FLOAT, 27, 32, 16, 2000, true, false},   {D3D_FLOAT, 27, 32, 16, 2100, true, true},
+      {D3D_FLOAT, 27, 32, 32, 30000, true, false},   {D3D_FLOAT, 27, 32, 32, 40000, true, true},   {D3D_FLOAT, 27, 16, 16, 60000, true, false},
+      {D3D_FLOAT, 27, 16, 32, 4000, true, true},     {D3D_FLOAT, 27, 16, 128, 60000, true, false}, {D3D_FLOAT, 4, 64, 32, 9000, true, false},
+      {D3D_FLOAT, 36, 64, 32, 9000, true, false},    {D3D_FLOAT, 27, 32, 32, 8000, false, true},   {D3D_FLOAT, 27, 32, 32, 30000, false, false},
+      {D3D_FLOAT, 27, 32, 32, 110000, false, true},  {D3D_FLOAT, 27, 64, 32, 16000, false, true},  {D3D_FLOAT, 27, 64, 32, 60000, false, false},
+      {D3D_FLOAT, 27, 64, 64, 30000, false, true},   {D3D_FLOAT, 27, 16, 32, 4000, false, false},  {D3D_HALF, 27, 32, 16, 300, true, true},
+      {D3D_HALF, 27, 64, 32, 100000, true, false},   {D3D_BF16, 27, 64, 64, 100000, true, false},  {D3D_BF16, 27, 128, 128, 60000, true, false},
+      {D3D_BF16, 27, 128, 128, 75000, true, true},   {D3D_HALF, 27, 64, 128, 110000, true, false}, {D3D_HALF, 27, 64, 128, 140000, true, true},
+      {D3D_HALF, 27, 128, 128, 110000, false, false}, {D3D_INT8, 27, 64, 64, 30000, true, false},  {D3D_INT8, 27, 128, 128, 110000, true, false},
+  };
+  for (const Layer& l : layers) {
+    Conv c(l.kVol, l.cin, l.cout, l.rows, l.inverse);
+    CHECK(c.plugin);
+    c.type(l.dtype);
+    sorts = 0;
+    CHECK(c.enqueue() == D3D_OK);
+    if (sorts != (l.sorted ? 1 : 0)) std::fprintf(stderr, "dtype %d, %d -> %d, %d rows, inverse %d\n", l.dtype, l.cin, l.cout, l.rows, l.inverse);
+    CHECK(sorts == (l.sorted ? 1 : 0) && (lastConv.rowOrder != nullptr) == l.sorted);
+  }
+  return 0;
+}
 }  // namespace
 
 int main() {
-  if (derivedTableStays() || widenedRowsStay()) return 1;
+  if (derivedTableStays() || widenedRowsStay() || sortedLayers()) return 1;
   std::puts("plugin_check ok");
   return 0;
 }

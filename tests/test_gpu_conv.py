@@ -706,6 +706,35 @@ def test_inverse_rows_in_the_order_of_their_taps(engine, n, room, cin, cout, dty
     run_case(n, (14, 60, 50), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False, inverse=True, cap_extra=room, relu=True)
 
 
+@pytest.mark.parametrize("n,room", [(1, 0), (63, 5), (511, 1), (512, 0), (513, 511), (3100, 1500)])
+@pytest.mark.parametrize("cin,cout,dtype", [(16, 16, "float32"), (32, 16, "float32"), (32, 32, "float32"), (16, 128, "float32"),
+                                            (32, 64, "float32"), (64, 128, "float16"), (128, 128, "bfloat16")])
+def test_sorted_rows_below_the_lines(engine, monkeypatch, n, room, cin, cout, dtype):
+    """Layers that sort their rows from a number of rows on only, made to sort few (D3D_CONV_ORDER=1), and 32-channel fp32 layers in
+    both directions of the switch."""
+    monkeypatch.setenv("D3D_CONV_ORDER", "1")
+    run_case(n, (14, 60, 50), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False, inverse=True, cap_extra=room, relu=True)
+    if (cin, cout) == (32, 32):
+        run_case(n, (14, 60, 50), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, link=False, room=room)
+        monkeypatch.setenv("D3D_CONV_ORDER", "0")
+        run_case(n, (14, 60, 50), (3, 3, 3), (1, 1, 1), (1, 1, 1), cin, cout, dtype, True, link=False, room=room)
+
+
+def test_inverse_rows_of_other_kernels_sorted(engine, monkeypatch):
+    """Kernel volumes of 8, 27 and 32 on layers that would not sort so few rows."""
+    monkeypatch.setenv("D3D_CONV_ORDER", "1")
+    for ksize, stride, padding in (((2, 2, 2), (2, 2, 2), (0, 0, 0)), ((3, 3, 3), (3, 3, 3), (0, 0, 0)), ((4, 4, 2), (2, 2, 1), (1, 1, 0)),
+                                   ((3, 3, 3), (1, 1, 1), (1, 1, 1)), ((3, 3, 4), (2, 2, 2), (1, 1, 1))):
+        for cin, cout, dtype in ((128, 128, "float16"), (32, 64, "float32")):
+            run_case(3000, (14, 60, 50), ksize, stride, padding, cin, cout, dtype, False, inverse=True, cap_extra=100)
+
+
+@pytest.mark.parametrize("cin,cout,dtype,n", [(128, 128, "float16", 66000), (64, 128, "bfloat16", 132000)])
+def test_inverse_rows_sorted_from_the_line_on(engine, cin, cout, dtype, n):
+    """Two-byte layers of 128 output channels past their lines, by themselves."""
+    run_case(n, (14, 130, 120), (3, 3, 3), (2, 2, 2), (1, 1, 1), cin, cout, dtype, False, inverse=True, relu=True)
+
+
 @pytest.mark.parametrize("ksize,stride,padding", [((2, 2, 2), (2, 2, 2), (0, 0, 0)), ((3, 3, 3), (3, 3, 3), (0, 0, 0)), ((4, 4, 2), (2, 2, 1), (1, 1, 0)),
                                                   ((3, 3, 3), (1, 1, 1), (1, 1, 1)), ((3, 3, 4), (2, 2, 2), (1, 1, 1))])
 def test_inverse_rows_of_other_kernels(engine, ksize, stride, padding):
