@@ -50,11 +50,15 @@ __device__ inline int pipeTileRows(int64_t rows, int cus) {
 // workgroup's list in the lanes of one register.
 // Otherwise (no masks, at most ROUNDS tiles each or more than a list holds) XCD x takes the x-th contiguous part (TileOrder).
 // fp32 layers, bound by the matrix pipe, are dealt from the second tile on: steps of the busiest workgroup / of the average
-// one 153 / 110 contiguous and 120 / 110 dealt for 64 -> 64 with 260 000 rows, 407 -> 344 us; 118 000 rows 208 -> 174.  The
-// other types gain from the fifth tile on (64 -> 64, 1.04 million rows, 216 / 174 -> 180 / 174 steps: fp16 232 -> 217 us, int8
-// 123 -> 114) and not before: with two tiles each (260 000 rows, 54 / 44 -> 45 / 44) the part runs at a lower clock when no CU
-// is idle, the XCDs read 20 % more lines from each other's parts, and it was 58.7 against 59.2 us alone and 25 us of 630 lost
-// in a pass whose rulebooks had run on the CUs that finished early.
+// one 153 / 110 contiguous and 120 / 110 dealt for 64 -> 64 with 260 000 rows, 407 -> 344 us; 118 000 rows 208 -> 174.  Two-byte
+// layers of 64 input channels and more gain from the fifth tile on (64 -> 64, 1.04 million rows of a network's third level, 216 / 174 ->
+// 180 / 174 steps: 228 -> 210 us; 64 -> 128 451 -> 430, 128 -> 64 431 -> 395, 128 -> 32 354 -> 327) and not before: with two tiles each
+// (260 000 rows, 54 / 44 -> 45 / 44) the part runs at a lower clock when no CU is idle, the XCDs read 20 % more lines from each other's
+// parts, and it was 58.7 against 59.2 us alone and 25 us of 630 lost in a pass whose rulebooks had run on the CUs that finished early.
+// Those lines are the price everywhere: rows in a scan's own order, whose tiles all hold much the same taps, lose by it (64 -> 64, 1.08
+// million rows 227 -> 243 us), but layers of 64 channels have a level's rows.  int8 and 32 two-byte input channels, three workgroups to
+// a CU, only pay: int8 64 -> 128, 520 000 rows 122 us contiguous, 130 dealt, 1.04 million 267 and 271, 64 -> 64 840 000 rows of scans 86
+// and 96, a level's 1.04 million 115 to 118 either way; 32 -> 64 in bf16, 1.4 million rows 214 and 216, 840 000 of scans 94 and 100.
 constexpr int kDealRounds = 4;
 template <int PER, int CHUNK, int ROUNDS>                // ROUNDS = 0: never dealt
 struct TileDeal {
@@ -705,9 +709,9 @@ int32_t launchPipeCfg(const ConvArgs& a, hipStream_t stream) {
     return D3D_OK;
   };
   static std::atomic<size_t> granted{64 * 1024};
-  // an instantiation of its own: the list costs the others registers they use (260 000 rows, 64 -> 64: 1 % of a pass).  The
-  // two-byte and int8 tiles of 32-row wavefronts are for few rows and never get there
-  if constexpr (SPLIT == 1 && (sizeof(T) == 4 || MT > 2)) {
+  // an instantiation of its own: the list costs the others registers they use (260 000 rows, 64 -> 64: 1 % of a pass).  Two-byte
+  // tiles of 32-row wavefronts are for few rows and never get there; which types gain: see TileDeal
+  if constexpr (SPLIT == 1 && (sizeof(T) == 4 || (sizeof(T) == 2 && CIN >= 64 && MT > 2))) {
     static std::atomic<size_t> grantedDeal{64 * 1024};
     if (a.rowOrder || (a.tileMasks && tiles > (sizeof(T) == 4 ? 1 : kDealRounds) * (blocks / COLS)))
       return launch(&convPipe<T, CIN, COUT, MT, WAVES, CO, true>, &grantedDeal);

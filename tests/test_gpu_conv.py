@@ -660,7 +660,8 @@ def test_a_captured_layer_keeps_its_weights_when_another_type_is_run(engine):
                                                     (64, "int8", 790003, 10000, 2)])
 def test_tiles_dealt_by_the_taps_they_hold(engine, cin, dtype, n, room, parts):
     """Which workgroup takes a tile changes nothing: a layer of many tiles, dealt to workgroups by the taps they hold (one with more
-    tiles than are ranked together), against parts of its rows, of which each has too few tiles to be dealt.  Levels hold different shares of their cells, so tiles
+    tiles than are ranked together), against parts of its rows, of which each has too few tiles to be dealt (int8 is not: several
+    contiguous tiles to a workgroup).  Levels hold different shares of their cells, so tiles
     hold 9 to 27 taps.  Bit for bit, rows past the live ones included: a tap no row has adds zeros."""
     from deploy3d_amd import layers, synth
     from deploy3d_amd.spconv_mm import spconv_mm
