@@ -627,7 +627,7 @@ __host__ __device__ inline bool pipeTakes48(int64_t rows, int cus) {
   auto load = [&](int tile) { return (rows + static_cast<int64_t>(tile) * cus - 1) / (static_cast<int64_t>(tile) * cus) * tile; };
   return 10 * load(384) < 9 * load(512);
 }
-template <class T, int CIN, int COUT>
+template <class T, int CIN, int COUT, bool DEAL>
 __global__ void __launch_bounds__(512)
 convPipeNarrowByRows(const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ wf, const float* __restrict__ bias,
                      const float* __restrict__ requantM, const int32_t* __restrict__ nbr, int64_t nbrPitch, int tapMirror,
@@ -638,8 +638,8 @@ convPipeNarrowByRows(const T* __restrict__ in, T* __restrict__ out, const T* __r
     pipeTiles<T, CIN, COUT, 3, 8>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
                                   relu, xcdShift, numActOut, gridDim.x);
   else
-    pipeTiles<T, CIN, COUT, 4, 8>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
-                                  relu, xcdShift, numActOut, gridDim.x);
+    pipeTiles<T, CIN, COUT, 4, 8, COUT, DEAL>(smem, in, out, wf, bias, requantM, nbr, nbrPitch, tapMirror, tileMasks, kVol, inRows, outRows,
+                                              relu, xcdShift, numActOut, gridDim.x);
 }
 
 // LDS of a shape: three weight slices, two stages and four steps of indices per wavefront.
@@ -656,16 +656,16 @@ inline bool pipeTakes(const ConvArgs& a, int64_t pitch, size_t rowBytes, int til
          static_cast<uint64_t>(a.outRows) + tileRows < 0x3FFFFFFFull;
 }
 
-template <class T, int CIN, int COUT>
+template <class T, int CIN, int COUT, bool DEAL>
 constexpr auto pipeByRowsKernel() {
-  if constexpr (COUT < 128) return &convPipeNarrowByRows<T, CIN, COUT>;
+  if constexpr (COUT < 128) return &convPipeNarrowByRows<T, CIN, COUT, DEAL>;
   else return &convPipeByRows<T, CIN, COUT>;
 }
 
-template <class T, int CIN, int COUT>
+template <class T, int CIN, int COUT, bool DEAL = false>
 int32_t launchPipeByRows(const ConvArgs& a, hipStream_t stream) {
   constexpr bool NARROW = COUT < 128;
-  constexpr auto kernel = pipeByRowsKernel<T, CIN, COUT>();
+  constexpr auto kernel = pipeByRowsKernel<T, CIN, COUT, DEAL>();
   const int64_t pitch = a.nbrPitch > 0 ? a.nbrPitch : a.outRows;
   if (!pipeTakes(a, pitch, CIN * sizeof(T), 512)) return D3D_ERR_UNSUPPORTED;
   constexpr size_t lds = pipeLds<T, CIN, COUT>(NARROW ? 4 : 2, 8);
@@ -768,9 +768,10 @@ int32_t launchPipeShape(const ConvArgs& a, hipStream_t stream) {
       if (a.outRows <= 128 * cus) return launchPipeCfg<T, CIN, COUT, 2, 4, 64, 2>(a, stream);
       if (a.outRows <= 192 * cus) return launchPipeCfg<T, CIN, COUT, 3, 4, 64, 2>(a, stream);
       if (a.outRows <= 256 * cus) return launchPipeCfg<T, CIN, COUT, 2, 8>(a, stream);
-      if (a.tileMasks && a.outRows > kDealRounds * 512 * cus) return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);
       // 384-row tiles by the live rows: 196 000 rows, one and a half rounds of 512, two of 384, 52 -> 46 us; 262 000, two
-      // rounds of 512, stay at 60 (64 with 384)
+      // rounds of 512, stay at 60 (64 with 384).  Capacities whose 512-row tiles may be dealt choose as well: with room for 600 000
+      // rows 196 000 live ones take 58 us, 280 000 74, and 64 and 85 in 512-row tiles
+      if (a.tileMasks && a.outRows > kDealRounds * 512 * cus) return launchPipeByRows<T, CIN, COUT, true>(a, stream);
       return launchPipeByRows<T, CIN, COUT>(a, stream);
     } else {
       return launchPipeCfg<T, CIN, COUT, 4, 8>(a, stream);

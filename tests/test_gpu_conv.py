@@ -426,6 +426,14 @@ def test_float_output_channels_shared_out(engine, cin, cout):
                  relu=True, cap_extra=n % 50)
 
 
+@pytest.mark.parametrize("n", [140000, 300000, 527000])
+def test_pipelined_tiles_of_64_channels_by_live_rows_of_a_large_capacity(engine, n):
+    """64 -> 64 at a capacity from which 512-row tiles are dealt by their taps: few enough live rows for 384-row tiles, for 512-row
+    tiles in order, and for dealt ones."""
+    run_case(n, (16, 200, 200), (3, 3, 3), (1, 1, 1), (1, 1, 1), 64, 64, "bfloat16" if n % 2000 else "float16", True, relu=True,
+             room=530001 - n)
+
+
 @pytest.mark.parametrize("n", [70000, 98304, 98305, 140000])
 def test_pipelined_tiles_of_64_channels_by_live_rows(engine, n):
     """64 -> 64 beyond 256 rows per CU, the live rows of one capacity: 384-row tiles where their rounds take clearly less (up to
