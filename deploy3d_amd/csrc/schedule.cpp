@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <utility>
 
@@ -216,6 +217,23 @@ bool captureGraph(d3d_schedule* s) {
   return ok;
 }
 
+// The streams and events of a run that enqueues step by step.
+hipError_t makeLanes(d3d_schedule* s) {
+  const RelaxedCapture relaxed;  // (a stream of the caller's may be capturing)
+  hipError_t e = hipSuccess;
+  auto event = [&](hipEvent_t& ev) {
+    if (!ev && e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  };
+  if (s->lanes.size() > 1) event(s->fork);
+  for (size_t l = 1; l < s->lanes.size(); ++l) {
+    if (!s->lanes[l] && e == hipSuccess) e = hipStreamCreateWithFlags(&s->lanes[l], hipStreamNonBlocking);  // default priority
+    event(s->joined[l]);
+  }
+  for (auto& st : s->steps)
+    if (st.awaited) event(st.done);
+  return e;
+}
+
 // The checks and lane bookkeeping that every kind of step shares; returns the step's index or a status.
 int32_t appendStep(d3d_schedule* s, d3d_schedule::Step&& st, const int32_t* after, int32_t nb_after) {
   const int me = static_cast<int>(s->steps.size());
@@ -231,10 +249,7 @@ int32_t appendStep(d3d_schedule* s, d3d_schedule::Step&& st, const int32_t* afte
   for (int32_t i = 0; i < nb_after; ++i) {
     d3d_schedule::Step& dep = s->steps[static_cast<size_t>(after[i])];
     if (dep.lane == st.lane) continue;  // stream order already holds
-    if (!dep.done) {
-      const hipError_t e = hipEventCreateWithFlags(&dep.done, hipEventDisableTiming);
-      if (e != hipSuccess) return hipFail(e, "hipEventCreateWithFlags");
-    }
+    dep.awaited = true;
     st.after.push_back(after[i]);
   }
   for (int i = me - 1; i >= 0 && st.before < 0; --i)
@@ -257,23 +272,10 @@ int32_t d3d_schedule_create(int32_t n_lanes, d3d_schedule** out) {
   }
   *out = nullptr;
   reapGraphs(false);
-  auto* s = new d3d_schedule();
-  hipError_t e = hipSuccess;
+  auto s = std::make_unique<d3d_schedule>();
   s->lanes.assign(static_cast<size_t>(n_lanes), nullptr);
   s->joined.assign(static_cast<size_t>(n_lanes), nullptr);
-  if (n_lanes > 1) {  // one lane: no HIP object at all
-    const RelaxedCapture relaxed;  // (a stream of the caller's may be capturing)
-    e = hipEventCreateWithFlags(&s->fork, hipEventDisableTiming);
-    for (int l = 1; l < n_lanes && e == hipSuccess; ++l) {
-      e = hipStreamCreateWithFlags(&s->lanes[l], hipStreamNonBlocking);  // default priority
-      if (e == hipSuccess) e = hipEventCreateWithFlags(&s->joined[l], hipEventDisableTiming);
-    }
-  }
-  if (e != hipSuccess) {
-    d3d_schedule_destroy(s);
-    return hipFail(e, "creating streams and events");
-  }
-  *out = s;
+  *out = s.release();
   return D3D_OK;
   D3D_GUARD_END(D3D_ERR_BAD_ARG)
 }
@@ -386,7 +388,7 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
   if (!s) return D3D_ERR_BAD_ARG;
   hipStream_t main = static_cast<hipStream_t>(stream);
   // A run puts event edges between streams that are not the caller's; under stream capture that is a topology
-  // this runtime has crashed on at the end of the capture.  Capture the operators' own enqueues instead.
+  // this runtime has crashed on at the end of the capture.  d3d_schedule_capture captures the steps without any.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(main, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
     d3d::setError("schedule: the stream is capturing; a schedule runs eagerly");
@@ -416,7 +418,8 @@ int32_t d3d_schedule_run(d3d_schedule* s, void* stream) {
     s->launchedOn = main;  // runs use the same tensors, so the caller orders them: the last launch is the last to end
     return D3D_OK;
   }
-  hipError_t e = hipSuccess;
+  hipError_t e = makeLanes(s);
+  if (e != hipSuccess) return hipFail(e, "creating streams and events");
   auto laneStream = [&](int lane) { return lane == 0 ? main : s->lanes[static_cast<size_t>(lane)]; };
   if (s->lanes.size() > 1) {
     e = hipEventRecord(s->fork, main);

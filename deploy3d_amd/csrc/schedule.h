@@ -22,8 +22,10 @@ struct d3d_schedule {
     int lane = 0;
     std::vector<int> after;     // steps of other lanes it waits for
     int before = -1;            // the step ahead of it on its own lane
-    hipEvent_t done = nullptr;  // recorded behind the step if a step of another lane waits for it
+    bool awaited = false;       // a step of another lane waits for it ...
+    hipEvent_t done = nullptr;  // ... through this, recorded behind it
   };
+  // made by the first run that enqueues step by step: a schedule that is only captured needs no stream and no event
   std::vector<hipStream_t> lanes;  // [0] unused: lane 0 is the caller's stream
   std::vector<hipEvent_t> joined;  // per owned lane: its tail, for the join
   hipEvent_t fork = nullptr;

@@ -1,4 +1,4 @@
-// Host check of csrc/schedule.cpp against a stand-in for the HIP runtime that keeps count: work counts as pending until
+// Host check of csrc/schedule.cpp and csrc/schedule_capture.cpp against a stand-in for the HIP runtime that keeps count: work counts as pending until
 // finish() is called, and while a stream is being captured a call that asks or waits spoils the capture - from a thread that
 // is not in the relaxed mode any such call, from a relaxed one a device-wide wait and anything that asks an event last
 // recorded on that stream (as the runtime does on a gfx950 system).  Operators are stand-ins too.  No GPU.
@@ -9,6 +9,8 @@
 #include <map>
 #include <new>
 #include <set>
+#include <utility>
+#include <vector>
 
 #include "common.h"
 #include "d3d_spconv.h"
@@ -32,6 +34,10 @@ uint64_t operatorChanges = 0;
 std::map<void*, bool> eventPending;
 std::map<void*, hipStream_t> recordedOn;
 std::set<void*> running;  // graphs launched and not finished
+// the graph that the caller captures: its nodes with what each comes behind, and what the stream's next one will
+bool capturing = false;
+std::vector<std::pair<hipGraphNode_t, std::vector<hipGraphNode_t>>> nodes;
+std::vector<hipGraphNode_t> behind;
 uintptr_t nextHandle = 16;
 void* fresh() { return reinterpret_cast<void*>(nextHandle += 16); }
 hipError_t unsafe() {
@@ -127,8 +133,19 @@ hipError_t hipStreamBeginCaptureToGraph(hipStream_t, hipGraph_t, const hipGraphN
                                         hipStreamCaptureMode) {
   return hipSuccess;
 }
-hipError_t hipStreamGetCaptureInfo_v2(hipStream_t, hipStreamCaptureStatus* st, unsigned long long*, hipGraph_t*,
+hipError_t hipStreamUpdateCaptureDependencies(hipStream_t s, hipGraphNode_t* deps, size_t n, unsigned flags) {
+  if (s != kMain || !capturing || flags != hipStreamSetCaptureDependencies) return hipErrorIllegalState;
+  behind.assign(deps, deps + n);
+  return hipSuccess;
+}
+hipError_t hipStreamGetCaptureInfo_v2(hipStream_t s, hipStreamCaptureStatus* st, unsigned long long*, hipGraph_t*,
                                       const hipGraphNode_t** deps, size_t* n) {
+  if (s == kMain) {
+    *st = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    *deps = behind.data();
+    *n = behind.size();
+    return hipSuccess;
+  }
   *st = hipStreamCaptureStatusActive;
   *deps = nullptr;
   *n = 0;
@@ -156,8 +173,14 @@ hipError_t hipGraphLaunch(hipGraphExec_t g, hipStream_t) {
 const char* d3d_plugin_type(const d3d_plugin*) { return "BEVDensify"; }
 int32_t d3d_num_outputs(const d3d_plugin*) { return 1; }
 int32_t d3d_enqueue(d3d_plugin*, const d3d_tensor_desc*, const d3d_tensor_desc*, const void* const*, void* const*, void*, size_t,
-                    void*) {
+                    void* stream) {
   ++steps;
+  if (capturing && stream == kMain) {
+    const auto node = static_cast<hipGraphNode_t>(fresh());
+    nodes.emplace_back(node, behind);
+    behind = {node};
+    return D3D_OK;
+  }
   ++pendingWork;
   return D3D_OK;
 }
@@ -263,9 +286,71 @@ int outOfHostMemory() {
   d3d_schedule_destroy(s);
   return 0;
 }
+
+// A pass of five steps: two rulebooks on lanes of their own, the second behind the first, three convolutions on lane 0, each
+// behind its rulebook (the third behind the second's again).
+d3d_schedule* pass() {
+  d3d_schedule* s = nullptr;
+  if (d3d_schedule_create(3, &s) != D3D_OK) return nullptr;
+  static d3d_tensor_desc in[4], out[1];
+  const void* ins[4] = {};
+  void* outs[1] = {};
+  auto* op = reinterpret_cast<d3d_plugin*>(16);
+  auto add = [&](int32_t lane, std::initializer_list<int32_t> after) {
+    return d3d_schedule_add(s, op, in, 4, out, 1, ins, outs, nullptr, 0, lane, after.begin(), static_cast<int32_t>(after.size()));
+  };
+  const int32_t r1 = add(1, {}), c1 = add(0, {r1}), r2 = add(2, {r1}), c2 = add(0, {r2});
+  add(0, {r2, c2});
+  (void)c1;
+  return s;
+}
+
+void beginCapture(std::vector<hipGraphNode_t> base) {
+  capturing = true;
+  captured = kMain;
+  nodes.clear();
+  behind = std::move(base);
+}
+void endCapture() {
+  capturing = false;
+  captured = nullptr;
+}
+const std::vector<hipGraphNode_t>& behindNode(size_t i) { return nodes[i].second; }
+std::vector<hipGraphNode_t> named(std::initializer_list<size_t> which) {
+  std::vector<hipGraphNode_t> v;
+  for (size_t i : which) v.push_back(nodes[i].first);
+  return v;
+}
+
+// The steps as nodes of the caller's graph: behind what the stream held or behind the steps they wait for, without edges that others
+// imply, the stream going on behind all of them; no stream and no event is made, and none is touched.
+int captureOfSteps() {
+  auto* const held = static_cast<hipGraphNode_t>(fresh());
+  auto* const held2 = static_cast<hipGraphNode_t>(fresh());
+  d3d_schedule* s = pass();
+  CHECK(s && d3d_schedule_size(s) == 5 && liveStreams == 0 && liveEvents == 0);
+  CHECK(d3d_schedule_capture(s, kMain) == D3D_ERR_UNSUPPORTED && steps >= 0);  // not capturing: nothing enqueued
+  const int before = steps;
+  beginCapture({held, held2});
+  CHECK(d3d_schedule_capture(s, kMain) == D3D_OK);
+  CHECK(steps == before + 5 && nodes.size() == 5 && liveStreams == 0 && liveEvents == 0 && !spoiled);
+  CHECK((behindNode(0) == std::vector<hipGraphNode_t>{held, held2}));
+  CHECK(behindNode(1) == named({0}) && behindNode(2) == named({0}));
+  CHECK(behindNode(3) == named({1, 2}) && behindNode(4) == named({3}) && behind == named({4}));
+  CHECK(d3d_schedule_run(s, kOther) == D3D_OK);  // the same schedule eagerly, while kMain is captured
+  CHECK(liveStreams == 2 && liveEvents > 0 && !spoiled && nodes.size() == 5);
+  CHECK(d3d_schedule_capture(s, kMain) == D3D_OK && nodes.size() == 10);  // and a second time into the same graph
+  CHECK(behindNode(5) == named({4}) && behind == named({9}));
+  endCapture();
+  finish();
+  d3d_schedule_destroy(s);
+  CHECK(liveStreams == 0 && liveEvents == 0);
+  return 0;
+}
 }  // namespace
 
 int main() {
+  if (captureOfSteps()) return 1;
   if (destroyUnderCapture() || changeWithoutWaiting() || refusedForAWhile() || outOfHostMemory()) return 1;
   std::puts("schedule_check ok");
   return 0;
