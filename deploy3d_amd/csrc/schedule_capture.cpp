@@ -37,10 +37,7 @@ extern "C" int32_t d3d_schedule_capture(d3d_schedule* s, void* stream) {
   int32_t rc = D3D_OK;
   for (size_t i = 0; rc == D3D_OK && i < s->steps.size(); ++i) {
     std::vector<hipGraphNode_t> behind;
-    for (int d : edges[i]) {
-      add(&behind, tail[static_cast<size_t>(d)]);
-      followed[static_cast<size_t>(d)] = true;
-    }
+    for (int d : edges[i]) add(&behind, tail[static_cast<size_t>(d)]);
     if (edges[i].empty()) behind = base;
     if (!comeBehind(behind)) {
       d3d::setError("schedule: the capture's dependencies could not be set");
@@ -49,8 +46,13 @@ extern "C" int32_t d3d_schedule_capture(d3d_schedule* s, void* stream) {
     }
     rc = d3d::scheduleEnqueueStep(s->steps[i], q);
     if (rc == D3D_ERR_UNSUPPORTED) rc = D3D_ERR_DEVICE;  // (that status says that nothing was captured)
-    if (rc == D3D_OK && hipStreamGetCaptureInfo_v2(q, &status, nullptr, nullptr, &nodes, &count) != hipSuccess) rc = D3D_ERR_DEVICE;
-    if (rc == D3D_OK) tail[i].assign(nodes, nodes + count);
+    // (of a step that failed as well: it may have enqueued a part of what it launches)
+    if (hipStreamGetCaptureInfo_v2(q, &status, nullptr, nullptr, &nodes, &count) != hipSuccess) {
+      rc = D3D_ERR_DEVICE;
+      break;
+    }
+    tail[i].assign(nodes, nodes + count);
+    for (int d : edges[i]) followed[static_cast<size_t>(d)] = true;
   }
   std::vector<hipGraphNode_t> last;  // the stream goes on behind all of it
   for (size_t i = 0; i < s->steps.size(); ++i)

@@ -38,6 +38,7 @@ std::set<void*> running;  // graphs launched and not finished
 bool capturing = false;
 std::vector<std::pair<hipGraphNode_t, std::vector<hipGraphNode_t>>> nodes;
 std::vector<hipGraphNode_t> behind;
+int failAt = -1, emptyAt = -1;  // the step from now that fails / that enqueues nothing
 uintptr_t nextHandle = 16;
 void* fresh() { return reinterpret_cast<void*>(nextHandle += 16); }
 hipError_t unsafe() {
@@ -174,8 +175,10 @@ const char* d3d_plugin_type(const d3d_plugin*) { return "BEVDensify"; }
 int32_t d3d_num_outputs(const d3d_plugin*) { return 1; }
 int32_t d3d_enqueue(d3d_plugin*, const d3d_tensor_desc*, const d3d_tensor_desc*, const void* const*, void* const*, void*, size_t,
                     void* stream) {
+  if (failAt >= 0 && failAt-- == 0) return D3D_ERR_UNSUPPORTED;
   ++steps;
   if (capturing && stream == kMain) {
+    if (emptyAt >= 0 && emptyAt-- == 0) return D3D_OK;
     const auto node = static_cast<hipGraphNode_t>(fresh());
     nodes.emplace_back(node, behind);
     behind = {node};
@@ -314,6 +317,7 @@ void beginCapture(std::vector<hipGraphNode_t> base) {
 void endCapture() {
   capturing = false;
   captured = nullptr;
+  failAt = emptyAt = -1;
 }
 const std::vector<hipGraphNode_t>& behindNode(size_t i) { return nodes[i].second; }
 std::vector<hipGraphNode_t> named(std::initializer_list<size_t> which) {
@@ -347,10 +351,50 @@ int captureOfSteps() {
   CHECK(liveStreams == 0 && liveEvents == 0);
   return 0;
 }
+
+// A step that fails ends the capture's steps: an error, never the status that says nothing was captured, and the stream goes on
+// behind what was.  A step that enqueues nothing stands for what it came behind.
+int captureOfFailingAndEmptySteps() {
+  auto* const held = static_cast<hipGraphNode_t>(fresh());
+  for (int at = 0; at < 5; ++at) {
+    d3d_schedule* s = pass();
+    beginCapture({held});
+    failAt = at;
+    const int32_t rc = d3d_schedule_capture(s, kMain);
+    CHECK(rc < 0 && rc != D3D_ERR_UNSUPPORTED && nodes.size() == static_cast<size_t>(at));
+    if (at == 0) CHECK(behind == std::vector<hipGraphNode_t>{held});
+    if (at == 1) CHECK(behind == named({0}));
+    if (at == 2) CHECK(behind == named({1, 0}));
+    if (at == 3) CHECK(behind == named({1, 2}));
+    if (at == 4) CHECK(behind == named({3}));
+    endCapture();
+    d3d_schedule_destroy(s);
+  }
+  d3d_schedule* s = pass();
+  beginCapture({held});
+  emptyAt = 0;  // the first rulebook
+  CHECK(d3d_schedule_capture(s, kMain) == D3D_OK && nodes.size() == 4);
+  CHECK((behindNode(0) == std::vector<hipGraphNode_t>{held}) && (behindNode(1) == std::vector<hipGraphNode_t>{held}));
+  CHECK(behindNode(2) == named({0, 1}) && behind == named({3}));
+  beginCapture({});  // a stream that holds nothing yet
+  emptyAt = 2;       // the second rulebook: the convolutions behind it come behind what it did
+  CHECK(d3d_schedule_capture(s, kMain) == D3D_OK && nodes.size() == 4);
+  CHECK(behindNode(0).empty() && behindNode(2) == named({1, 0}) && behind == named({3}));
+  endCapture();
+  d3d_schedule* none = nullptr;
+  CHECK(d3d_schedule_create(1, &none) == D3D_OK);
+  beginCapture({held});
+  CHECK(d3d_schedule_capture(none, kMain) == D3D_OK && (behind == std::vector<hipGraphNode_t>{held}));  // no steps
+  endCapture();
+  d3d_schedule_destroy(none);
+  d3d_schedule_destroy(s);
+  CHECK(liveStreams == 0 && liveEvents == 0);
+  return 0;
+}
 }  // namespace
 
 int main() {
-  if (captureOfSteps()) return 1;
+  if (captureOfSteps() || captureOfFailingAndEmptySteps()) return 1;
   if (destroyUnderCapture() || changeWithoutWaiting() || refusedForAWhile() || outOfHostMemory()) return 1;
   std::puts("schedule_check ok");
   return 0;
