@@ -19,7 +19,8 @@ __host__ __device__ inline uint32_t tapClass(uint32_t mask) { return (mask * 0x2
 // Windows of 512 rows: what a workgroup reads and writes, through one CU, is the time.  128 000 rows (14 MB in, 14 MB out) and
 // 40 000 take 16 and 15 us in windows of 2048, 11 and 10 in 1024, 10 and 7.6 in 512, while 128-row tiles hold 25, 35 and 54 % of
 // the taps and 16-row groups 14, 15 and 17: fp32 64 -> 32 behind it 46, 45.5 and 50.5 us (119 unsorted), 32 -> 16 16.7, 16.2 and
-// 15.4 (27).  Encoder-decoder of 40 000 voxels in fp32 797 -> 751, 740 and 734 us; of 100 000 in fp16 522 -> 517.
+// 15.4 (27).  Encoder-decoder of 40 000 voxels in fp32 797 -> 751, 740 and 734 us.  Which
+// layers gain by it: MMPlugin::ordersRows.
 // Rows past the live ones keep to the end of the last window that has live rows; windows behind it hold no neighbours and
 // are not read.
 template <int MAXTAPS>

@@ -212,7 +212,8 @@ class SparseBackbone:
         From the third pass in a row on the same input buffers the pass is a native schedule - one HIP-graph launch from
         its third run on - instead of operator by operator from here: the 21 operator calls and 16 events of a VoxelNet
         pass cost the host 600 us, the graph launch 170 (making the graph costs 500 once, so a pass has to repeat
-        first).  Other buffers, and a stream that is being captured, take the operators one by one."""
+        first).  Other buffers take the operators one by one.  Under capture the steps of such a schedule go into the graph
+        where the pass before was made on these buffers (see _capture), else the operators' own enqueues on side streams."""
         if torch.cuda.is_current_stream_capturing():
             return self._capture(x) or self._forward_steps(x)
         self._replaced.clear()
@@ -240,10 +241,13 @@ class SparseBackbone:
         return self._hand_out(plan.made, x, SparseTensor(x.feats, x.coors, x.num_act, x.grid))
 
     # Captured passes of up to this many input rows are captured as a schedule's steps (d3d_schedule_capture), which leaves out the
-    # dependencies that enqueueing on side streams adds.  us a pass with side streams / as steps: fp16, 7 400 rows 259 / 241,
-    # 45 000 (bf16) 440 / 407, 63 000 492 / 462, 84 000 531 / 534, 94 500 549 / 552, 126 000 619 / 635; int8, 19 000 273 / 257,
-    # 94 500 451 / 433, 150 000 531 / 521, 189 000 748 / 773.  Large passes are bound by the sum of their kernels' demands, and a
-    # rulebook that starts earlier stretches the convolutions beside it.
+    # dependencies that enqueueing on side streams adds.  us a pass with side streams / as steps, by rows of capacity, two processes
+    # each with one captured pass (they differ by 0.2 to 1 %).  VoxelNet, fp16: 7 400 rows 262 / 247, 63 000 494 / 458, 84 000 530 / 529,
+    # 126 000 607 / 615; bf16: 45 000 443 / 408, 504 000 (four scans) 2124 / 2136; int8: 150 000 528 / 516, 189 000 745 / 768, 252 000 855 / 887,
+    # 504 000 1657 / 1653 (1734 / 1678 in an earlier run); fp32: 21 000 1125 / 1119, 63 000 1673 / 1692.  Encoder-decoder: fp16, 63 000 394 / 369,
+    # bf16, 115 500 540 / 531, fp32, 75 000 931 / 924.  So the steps gain up to the lines; past them VoxelNet passes of one and two scans
+    # lose 1 to 4 % by them (a strided rulebook starts beside the SubM one of the stage before and the convolutions), four int8
+    # scans and larger encoder-decoders would gain up to 3, and fp32 VoxelNet passes of 63 000 rows pay 1 % below the line.
     _CAPTURE_ROWS = 73728
     _CAPTURE_ROWS_INT8 = 163840
 

@@ -79,6 +79,8 @@ int32_t d3d_clone(const d3d_plugin* p, d3d_plugin** out);
 
 /* destroy() (index_trt.cu:82, mm_trt.cu:82). */
 void d3d_destroy(d3d_plugin* p);
+/* (It frees the handle's device memory: not while a stream is being captured, where a free spoils the capture, and not while a
+ * graph that holds its enqueues may still be replayed.) */
 
 /* getPluginType / getPluginVersion / getPluginNamespace (index_trt.cu:165-168). */
 const char* d3d_plugin_type(const d3d_plugin* p);
@@ -236,7 +238,7 @@ int32_t d3d_set_option(d3d_plugin* p, int32_t option, int64_t value);
  *   (options, links, capacities, reserved buffers), the steps are captured into one HIP graph, which the schedule keeps and
  *   later runs launch - until something changes.  A capture that is refused is tried again after twice as many runs.
  *   Returns the first failing status; steps behind a failed one are not enqueued.  Refused with D3D_ERR_UNSUPPORTED while
- *   `stream` is capturing (capture the operators' own enqueues instead).  One thread at a time per schedule; runs use the
+ *   `stream` is capturing (d3d_schedule_capture then).  One thread at a time per schedule; runs use the
  *   same tensors, so runs on different streams are the caller's to order.
  * d3d_schedule_destroy: waits for the last run, whose stream must still exist, then frees the schedule's streams and its
  *   graph; the operators stay the caller's.  Allowed while a stream is being captured: if that is the stream of the last
