@@ -460,14 +460,11 @@ class GraphExecutor:
             raise ValueError("missing graph inputs: %s" % missing)
         if self._bound is None or self._bound["signature"] != self._signature(inputs):
             self._bind(inputs)
-        elif torch.cuda.is_current_stream_capturing():
-            # the steps of a schedule, each behind the nodes its inputs come from: rulebooks beside the convolutions
-            bound = self._bound
-            if "captured" not in bound:
-                bound["captured"] = bound.get("native") or self._record()
-            if bound["captured"] is not None and bound["captured"].capture():
-                return {v.name: self._bound["values"][v.name] for v in self.model.outputs}
-        else:
+        elif not torch.cuda.is_current_stream_capturing():
+            # (Under capture the operators are enqueued one by one, on the one stream.  Captured as a schedule's steps, each
+            # behind the nodes its inputs come from, a pass of 30 000 points in bf16 takes 400 us instead of 429, but a process
+            # that prepared and replayed several such graphs - 17 000 points, bf16 - ended with a host segmentation fault whose
+            # cause is not known: off until it is.)
             # the third pass on the same buffers and later ones: a native schedule, one graph launch from its third run
             # on (recording and capturing it costs more than a pass: passes have to repeat first)
             bound = self._bound

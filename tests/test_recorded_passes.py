@@ -180,6 +180,24 @@ def test_a_view_of_other_strides_at_the_same_address_is_bound_anew(host):
         assert torch.equal(ex.run(x=x)["y"], x.half())
 
 
+def test_a_captured_run_of_an_imported_graph_is_enqueued_operator_by_operator(host, monkeypatch):
+    """Also where the run before was on the same buffers or has become a schedule: neither is captured nor run."""
+    model = onnx_graph.Model([onnx_graph.Node("Cast", ["x"], ["y"], dict(to=onnx_graph.FLOAT16))],
+                             [onnx_graph.Value("x", onnx_graph.FLOAT, [16, 16])],
+                             [onnx_graph.Value("y", onnx_graph.FLOAT16, [16, 16])])
+    ex, x = onnx_graph.GraphExecutor(model, device="cpu"), torch.rand(16, 16)
+    monkeypatch.setattr(_HostSchedule, "capture", lambda *a: pytest.fail("captured as a schedule's steps"))
+    for eager in (2, 4):
+        for _ in range(eager):
+            ex.run(x=x)
+        host.capturing = True
+        ex._bound["values"]["y"].zero_()
+        with monkeypatch.context() as m:
+            m.setattr(_HostSchedule, "run", lambda *a: pytest.fail("a schedule does not run under capture"))
+            assert torch.equal(ex.run(x=x)["y"], x.half())
+        host.capturing = False
+
+
 def test_results_are_the_callers_own_objects(host):
     """Rebinding tensors on what a pass returned, on its outputs or rulebooks, or on the input afterwards, reaches neither
     the recorded pass nor a later result - while passes run step by step, when they are recorded, and after."""
